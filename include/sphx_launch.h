@@ -111,6 +111,36 @@ SPHX_EXPORT int sphx_vjp_f32(const float* xyz, const float* sph_grad, size_t n_s
 SPHX_EXPORT int sphx_vjp_f64(const double* xyz, const double* sph_grad, size_t n_samples, int l_max,
                              int normalized, double* xyz_grad, int accumulate, void* stream);
 
+/* The second-order products of a backward pass, without ddsph (or dsph) reaching memory. No counterpart in the
+ * reference, whose torch binding writes both arrays and sums them
+ * (sphericart-torch/python/sphericart/torch/register.py:82-175).
+ *
+ * sphx_vjp_backward_*: the derivatives of sphx_vjp_* with the upstream gradient `grad` [n_samples][3],
+ *
+ *   xyz_grad[i][b]      = sum_a grad[i][a] sum_k ddsph[i][a][b][k] * sph_grad[i][k]
+ *   sph_grad_grad[i][k] = sum_a grad[i][a] dsph[i][a][k]
+ *
+ * reads xyz, sph_grad and grad, writes xyz_grad and sph_grad_grad [n_samples][n_total].
+ *
+ * sphx_gradients_backward_*: the backward pass of values and gradients,
+ *
+ *   xyz_grad[i][b] = sum_k dsph[i][b][k] * sph_grad[i][k] + sum_a sum_k ddsph[i][a][b][k] * dsph_grad[i][a][k]
+ *
+ * reads xyz, sph_grad (NULL: no such term) and dsph_grad [n_samples][3][n_total], writes xyz_grad.
+ *
+ * Enqueued on `stream`; n_samples == 0 returns SPHX_OK. Both agree with the contraction of the arrays to rounding.
+ * Where the rows of a tile of points do not fit LDS they return SPHX_ERR_UNSUPPORTED and enqueue nothing (the first
+ * takes l_max up to 28 in float32 and 24 in float64, the second 24 and 16): such callers have sphx_forward_* and
+ * sphx_backward_second_*. */
+SPHX_EXPORT int sphx_vjp_backward_f32(const float* xyz, const float* sph_grad, const float* grad, size_t n_samples,
+                                      int l_max, int normalized, float* xyz_grad, float* sph_grad_grad, void* stream);
+SPHX_EXPORT int sphx_vjp_backward_f64(const double* xyz, const double* sph_grad, const double* grad, size_t n_samples,
+                                      int l_max, int normalized, double* xyz_grad, double* sph_grad_grad, void* stream);
+SPHX_EXPORT int sphx_gradients_backward_f32(const float* xyz, const float* sph_grad, const float* dsph_grad,
+                                            size_t n_samples, int l_max, int normalized, float* xyz_grad, void* stream);
+SPHX_EXPORT int sphx_gradients_backward_f64(const double* xyz, const double* sph_grad, const double* dsph_grad,
+                                            size_t n_samples, int l_max, int normalized, double* xyz_grad, void* stream);
+
 /* float32 arrays, evaluated in float64 and rounded once: what sphx_forward_f64
  * returns for the same points, converted to float (round to nearest even).
  * For callers that need float32 storage beyond the range of float32

@@ -30,6 +30,10 @@ LAUNCH_SYMBOLS = [
     "sphx_backward_second_f64",
     "sphx_vjp_f32",
     "sphx_vjp_f64",
+    "sphx_vjp_backward_f32",
+    "sphx_vjp_backward_f64",
+    "sphx_gradients_backward_f32",
+    "sphx_gradients_backward_f64",
     "sphx_forward_f32_via_f64",
     "sphx_forward_f32_via_f64_workspace",
     "sphx_forward_f32_via_f64_static",
@@ -79,6 +83,12 @@ def _declare(lib):
         fn = getattr(lib, f"sphx_vjp_{suffix}")
         fn.restype = c_int
         fn.argtypes = [c_void_p, c_void_p, c_size_t, c_int, c_int, c_void_p, c_int, c_void_p]
+        fn = getattr(lib, f"sphx_vjp_backward_{suffix}")
+        fn.restype = c_int
+        fn.argtypes = [c_void_p, c_void_p, c_void_p, c_size_t, c_int, c_int, c_void_p, c_void_p, c_void_p]
+        fn = getattr(lib, f"sphx_gradients_backward_{suffix}")
+        fn.restype = c_int
+        fn.argtypes = [c_void_p, c_void_p, c_void_p, c_size_t, c_int, c_int, c_void_p, c_void_p]
         fn = getattr(lib, f"sphx_prefactors_{suffix}")
         fn.restype = c_int
         fn.argtypes = [c_int, c_void_p]

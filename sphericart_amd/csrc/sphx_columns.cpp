@@ -1,0 +1,118 @@
+// Host side of columns_kernel and column_rows_kernel: their constants and the geometry of a launch.
+#include "sphx_columns.hpp"
+
+#include <cstring>
+
+#include "sphx_geometry.hpp"
+#include "sphx_plan.hpp"
+
+namespace sphx {
+
+// Q_l^m = S_{l,m} q_l^m with the leading coefficient of q in z equal to one: S = (-1)^m (2l-1)!! / (l-m)!, zero for
+// m > l. In float32 the prefactors F are used as they are in the tables of the forward kernels, their underflow from
+// l = 19 on included, so that both describe the same functions.
+template <typename T> std::vector<T> column_table_of(const T* F) {
+    auto scale = [](int l, int m) -> long double {
+        if (m > l || l < 0) return 0.0L;
+        long double s = (m & 1) ? -1.0L : 1.0L;
+        for (int k = 1; k <= l; ++k) s *= 2 * k - 1;
+        for (int k = 2; k <= l - m; ++k) s /= k;
+        return s;
+    };
+    auto b = [](int l, int m) -> long double {
+        if (l < m + 2) return 0.0L;
+        return -static_cast<long double>(l + m - 1) * (l - m - 1) / (static_cast<long double>(2 * l - 1) * (2 * l - 3));
+    };
+    std::vector<T> table(static_cast<size_t>(kColumnEntries) * kColumnEntry);
+    for (int m = 0; m <= kColumnsLMax; ++m) {
+        for (int l = m; l <= kColumnsLMax; ++l) {
+            T* t = table.data() + static_cast<size_t>(column_start(m) + l - m) * kColumnEntry;
+            const long double f = F[l * (l + 1) / 2 + m], lm = l + m;
+            t[0] = static_cast<T>(b(l, m));
+            t[1] = static_cast<T>(b(l - 1, m + 1));
+            t[2] = static_cast<T>(f * scale(l, m));
+            t[3] = static_cast<T>(f * scale(l - 1, m + 1));
+            t[4] = static_cast<T>(f * lm * scale(l - 1, m));
+            t[5] = static_cast<T>(b(l - 2, m + 2));
+            t[6] = static_cast<T>(f * scale(l - 2, m + 2));
+            t[7] = static_cast<T>(f * lm * scale(l - 2, m + 1));
+            t[8] = static_cast<T>(f * lm * (lm - 1) * scale(l - 2, m));
+        }
+    }
+    return table;
+}
+template std::vector<float> column_table_of<float>(const float*);
+template std::vector<double> column_table_of<double>(const double*);
+
+bool plan_columns(ColumnsKind kind, size_t n_samples, int l_max, size_t elem, int lds_limit, int cus, ColumnsLaunch* out) {
+    if (l_max < 0 || l_max > kColumnsLMax) return false;
+    const unsigned ny = static_cast<unsigned>((l_max + 1) * (l_max + 1)), e = static_cast<unsigned>(elem);
+    // (a row of one vector stays as it is: the division by its length that places the pads has no multiplier)
+    const unsigned vec = 16u / e, pad = ny % 2 == 0 && ny > vec ? 1u : 0u;
+    const unsigned limit = static_cast<unsigned>(lds_limit);
+    auto rounded = [&](unsigned n) { return (n + vec - 1u) / vec * vec; };
+    // (a wave's sums: 3 or 6 numbers per lane, 7 per point)
+    const unsigned sums = kind == COLUMNS_ROWS ? 7u * 16u : (kind == COLUMNS_VJP ? 3u : 6u) * 64u;
+
+    int waves = 1;
+    unsigned tile = 0, rows = 0, off_rows = 0;
+    auto lay_out = [&](unsigned t, int w) {
+        tile = t;
+        waves = w;
+        off_rows = kind == COLUMNS_ROWS ? rounded(t * (3u * ny + pad)) : 0u;
+        rows = off_rows + rounded(t * (ny + pad));
+        return (rows + static_cast<unsigned>(w - 1) * sums) * e;
+    };
+    const int forced_waves = switch_or(SW_COLUMNS_WAVES, 0), forced_tile = switch_or(SW_COLUMNS_TILE, 0);
+    unsigned bytes = 0;
+    const int most = l_max + 1 < 8 ? l_max + 1 : 8;
+    // Waves per workgroup: enough workgroups fit a CU for one to compute while another one loads, and more waves than
+    // that make a tile wait for its sums. 1M points, l_max = 1, 3, 6 in float32, us with 1 / 2 / 4 / 8 waves:
+    // 13.4 15.2 - -, 29.2 28.8 35.0 -, 86.0 74.8 66.2 86.2; 400 000 at l_max = 8 71 58 50 51; float64 alike. A tile of
+    // 16 points (rows): l_max = 3, 6, 9, 12, 37 51 - -, 66 56 75 146, 98 68 59 98, 179 110 81 87. Too few tiles for the
+    // CUs: as many waves as there are columns, up to eight (1 000 points at l_max = 6: 8.1 us with one, 4.7 with eight).
+    const size_t cu = static_cast<size_t>(cus > 0 ? cus : 1);
+    if (kind == COLUMNS_ROWS) {
+        waves = l_max < 5 ? 1 : (l_max < 8 ? 2 : 4);
+        if ((n_samples + 15) / 16 <= cu) waves = most;
+        if (forced_waves > 0) waves = forced_waves < most ? forced_waves : most;
+        bytes = lay_out(16u, waves);
+    } else {
+        waves = l_max < 3 ? 1 : (l_max < 6 ? 2 : 4);
+        // 64 points while three workgroups fit a CU, else 32 on two lanes each (200 000 points at l_max = 12: 56.6
+        // against 55.0 us in float32 where 43 KB still fit three times, 128 against 111 in float64 where 86 KB do not)
+        tile = lay_out(64u, waves) <= 160u * 1024u / 3u ? 64u : 32u;
+        if ((n_samples + 63) / 64 <= cu) {
+            tile = 32u;
+            waves = most;
+        }
+        if (forced_waves > 0) waves = forced_waves < most ? forced_waves : most;
+        if (forced_tile == 32 || forced_tile == 64) tile = static_cast<unsigned>(forced_tile);
+        bytes = lay_out(tile, waves);
+        if (bytes > limit && tile == 64u) bytes = lay_out(32u, waves);
+    }
+    while (bytes > limit && waves > 1) bytes = lay_out(tile, waves / 2); // (the largest rows leave no room for many sums)
+    if (bytes > limit) return false;
+    const size_t tiles = (n_samples + tile - 1) / tile;
+    if (tiles > 0x7fffffffull) return false;
+
+    std::memset(&out->g, 0, sizeof(out->g));
+    out->g.n_samples = n_samples;
+    out->g.n_tiles = static_cast<unsigned>(tiles);
+    out->g.tiles_per_xcd = (out->g.n_tiles + 7u) / 8u;
+    out->g.l_max = l_max;
+    out->g.ny = ny;
+    out->g.pad = pad;
+    out->g.off_rows = off_rows;
+    out->g.off_sums = rows;
+    out->g.magic_ny = magic_of(ny);
+    out->g.magic_vectors = magic_of(ny / vec ? ny / vec : 1u);
+    out->g.magic_vectors3 = magic_of(3u * ny / vec ? 3u * ny / vec : 1u);
+    out->workgroups = out->g.tiles_per_xcd * 8u;
+    out->threads = 64u * static_cast<unsigned>(waves);
+    out->lds_bytes = bytes;
+    out->groups = kind == COLUMNS_ROWS ? 4 : static_cast<int>(64u / tile);
+    return true;
+}
+
+} // namespace sphx

@@ -1,0 +1,48 @@
+// The launches of columns_kernel and column_rows_kernel, as templates over the arithmetic type; sphx_columns_f32.hip
+// and sphx_columns_f64.hip instantiate them.
+#ifndef SPHX_COLUMNS_DISPATCH_HPP
+#define SPHX_COLUMNS_DISPATCH_HPP
+
+#include "sphx_columns_kernel.hpp"
+#include "sphx_runtime.hpp"
+
+namespace sphx {
+
+template <typename Kernel, typename... Args>
+static hipError_t launch_columns(Kernel kernel, const ColumnsLaunch& l, hipStream_t stream, Args... args) {
+    if (l.lds_bytes > 64u * 1024u) {
+        unsigned unused = 0;
+        const hipError_t e = kernel_facts(reinterpret_cast<const void*>(kernel), l.threads, l.lds_bytes, &unused);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL(kernel, dim3(l.workgroups), dim3(l.threads), l.lds_bytes, stream, l.g, args...);
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t dispatch_columns(ColumnsKind kind, const ColumnsLaunch& l, bool normalized, const T* xyz, const T* sph_grad,
+                            const T* upstream, T* xyz_grad, T* sph_grad_grad, hipStream_t s) {
+    if (kind == COLUMNS_ROWS) {
+        return normalized ? launch_columns(column_rows_kernel<T, true>, l, s, xyz, sph_grad, upstream, xyz_grad)
+                          : launch_columns(column_rows_kernel<T, false>, l, s, xyz, sph_grad, upstream, xyz_grad);
+    }
+    auto go = [&](auto kernel) { return launch_columns(kernel, l, s, xyz, sph_grad, upstream, xyz_grad, sph_grad_grad); };
+    if (l.groups == 2) {
+        return normalized ? go(columns_kernel<T, true, true, 2>) : go(columns_kernel<T, false, true, 2>);
+    }
+    return normalized ? go(columns_kernel<T, true, true, 1>) : go(columns_kernel<T, false, true, 1>);
+}
+
+template <typename T> hipError_t upload_column_tables(const HostTables& t) {
+    if constexpr (sizeof(T) == 4) {
+        const std::vector<float> table = column_table_of<float>(t.f32.data());
+        return hipMemcpyToSymbol(HIP_SYMBOL(kColumns32), table.data(), table.size() * sizeof(float));
+    } else {
+        const std::vector<double> table = column_table_of<double>(t.f64.data());
+        return hipMemcpyToSymbol(HIP_SYMBOL(kColumns64), table.data(), table.size() * sizeof(double));
+    }
+}
+
+} // namespace sphx
+
+#endif

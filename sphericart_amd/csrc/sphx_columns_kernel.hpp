@@ -1,0 +1,603 @@
+// Products with the derivatives of the harmonics, summed column by column: columns_kernel (the vector-Jacobian
+// product, and its own derivatives) and column_rows_kernel (the product with gradient and second-derivative arrays).
+#ifndef SPHX_COLUMNS_KERNEL_HPP
+#define SPHX_COLUMNS_KERNEL_HPP
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+#include <type_traits>
+
+#include "sphx_columns.hpp"
+#include "sphx_tiling.hpp"
+
+namespace sphx {
+
+// ---------------------------------------------------------------------------
+// The entries (l, +m) and (l, -m) of a point are Q_l^m c_m and Q_l^m s_m times a prefactor F_l^m, and every
+// derivative of Q is another Q (sphericart/include/templates_core.hpp:129-133, 219-235, 323-387):
+//
+//   d/dx Q_l^m = x Q_{l-1}^{m+1}     d/dy Q_l^m = y Q_{l-1}^{m+1}     d/dz Q_l^m = (l+m) Q_{l-1}^m
+//
+// A sum over all entries with weights w therefore splits, at fixed m, into a few sums over l that do not involve
+// x, y, c or s,
+//
+//   A = sum_l w F Q_l^m        B = sum_l w F Q_{l-1}^{m+1}        C = sum_l w F (l+m) Q_{l-1}^m          (gradients)
+//   E = sum_l w F Q_{l-2}^{m+2}  G = sum_l w F (l+m) Q_{l-2}^{m+1}  K = sum_l w F (l+m)(l+m-1) Q_{l-2}^m  (second)
+//
+// and what depends on x, y, c_m, s_m is applied once per m ("column") instead of once per entry: six (gradients) or
+// twelve (second derivatives) multiply-adds per pair of entries instead of 30 or 250 operations. The chain rule of
+// the normalised harmonics is linear too and is applied once per point. Second derivatives never exist as numbers.
+//
+// Q runs upward in l at fixed m, one three-term recursion with the leading coefficient taken out,
+//
+//   q_l = z q_{l-1} + b_{l,m} r^2 q_{l-2},   b = -(l+m-1)(l-m-1) / ((2l-1)(2l-3)),
+//
+// whose scale is folded into the prefactors on the host (sphx_columns.cpp): |q| <= 1 on the unit sphere. m is the
+// same for all lanes of a wave, so b and the prefactors come from the scalar unit. Neighbouring columns m + 1 and
+// m + 2 run along (Q_{l-1}^{m+1}, Q_{l-2}^{m+2}): three or six operations, less than what reading every weight a
+// second and third time from LDS would take.
+//
+// The products are sums in another order than the entries' own, with fused multiply-adds: they agree with the
+// contraction of the derivative arrays to rounding.
+// ---------------------------------------------------------------------------
+
+__device__ __forceinline__ float fma_of(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fma_of(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+template <typename T> __device__ __forceinline__ const T* column_table();
+static __constant__ float kColumns32[kColumnEntries * kColumnEntry];
+static __constant__ double kColumns64[kColumnEntries * kColumnEntry];
+template <> __device__ __forceinline__ const float* column_table<float>() { return kColumns32; }
+template <> __device__ __forceinline__ const double* column_table<double>() { return kColumns64; }
+
+// Walks l = m .. L of column m and hands visit(step, l, FA, FB, FC, FE, FG, FK) the products of the prefactors with
+// the six Q above. `step` is l - m as a compile-time number while that is below 5 and 5 from there on: what is zero
+// or one by construction in the first steps takes no instruction (FB is meaningful from step 2 on, FC 1, FE 4, FG 3,
+// FK 2).
+template <typename T, bool NORM, bool SECOND, typename Visit>
+__device__ __forceinline__ void walk_column(int m, int L, T z, T r2, Visit&& visit) {
+    const T* t = column_table<T>() + column_start(m) * kColumnEntry;
+    T a1 = 0, a2 = 0, b1 = 0, b2 = 0, e1 = 0, e2 = 0;
+    auto advance = [&](T factor, T v1, T v2) { // on the unit sphere r^2 = 1
+        return fma_of(NORM ? factor : factor * r2, v2, z * v1);
+    };
+    auto one = [&](auto step, int l) {
+        constexpr int S = decltype(step)::value;
+        const T* k = t;
+        t += kColumnEntry;
+        T a, b = 0, e = 0;
+        if constexpr (S == 0) a = 1;
+        else if constexpr (S == 1) a = z;
+        else a = advance(k[0], a1, a2);
+        if constexpr (S == 2) b = 1;
+        else if constexpr (S == 3) b = z;
+        else if constexpr (S >= 4) b = advance(k[1], b1, b2);
+        if constexpr (SECOND) {
+            if constexpr (S == 4) e = 1;
+            else if constexpr (S >= 5) e = advance(k[5], e1, e2);
+        }
+        T fa = k[2], fb = 0, fc = 0, fe = 0, fg = 0, fk = 0;
+        if constexpr (S >= 1) fa *= a;
+        if constexpr (S >= 1) fc = k[4];
+        if constexpr (S >= 2) fc *= a1;
+        if constexpr (S >= 2) fb = k[3];
+        if constexpr (S >= 3) fb *= b;
+        if constexpr (SECOND) {
+            if constexpr (S >= 2) fk = k[8];
+            if constexpr (S >= 3) fk *= a2;
+            if constexpr (S >= 3) fg = k[7];
+            if constexpr (S >= 4) fg *= b1;
+            if constexpr (S >= 4) fe = k[6];
+            if constexpr (S >= 5) fe *= e;
+        }
+        visit(step, l, fa, fb, fc, fe, fg, fk);
+        a2 = a1;
+        a1 = a;
+        b2 = b1;
+        b1 = b;
+        e2 = e1;
+        e1 = e;
+    };
+    using std::integral_constant;
+    one(integral_constant<int, 0>{}, m);
+    if (m + 1 > L) return;
+    one(integral_constant<int, 1>{}, m + 1);
+    if (m + 2 > L) return;
+    one(integral_constant<int, 2>{}, m + 2);
+    if (m + 3 > L) return;
+    one(integral_constant<int, 3>{}, m + 3);
+    if (m + 4 > L) return;
+    one(integral_constant<int, 4>{}, m + 4);
+#pragma unroll 2
+    for (int l = m + 5; l <= L; ++l) one(integral_constant<int, 5>{}, l);
+}
+
+// The sums of one column and one side (entries (l, +m) or (l, -m)).
+template <typename T> struct ColumnSums {
+    T A = 0, B = 0, C = 0, E = 0, G = 0, K = 0;
+
+    template <int S, bool SECOND>
+    __device__ __forceinline__ void add(T w, T fa, T fb, T fc, T fe, T fg, T fk) {
+        A = fma_of(w, fa, A);
+        if constexpr (S >= 2) B = fma_of(w, fb, B);
+        if constexpr (S >= 1) C = fma_of(w, fc, C);
+        if constexpr (SECOND) {
+            if constexpr (S >= 4) E = fma_of(w, fe, E);
+            if constexpr (S >= 3) G = fma_of(w, fg, G);
+            if constexpr (S >= 2) K = fma_of(w, fk, K);
+        }
+    }
+};
+
+// c_m, s_m of a lane's point, walked upward in m; kept with their two predecessors.
+template <typename T> struct Azimuth {
+    T c = 1, s = 0, c1 = 0, s1 = 0, c2 = 0, s2 = 0;
+    __device__ __forceinline__ void next(T x, T y) {
+        c2 = c1;
+        s2 = s1;
+        c1 = c;
+        s1 = s;
+        const T cn = fma_of(c1, x, -(s1 * y));
+        s = fma_of(c1, y, s1 * x);
+        c = cn;
+    }
+};
+
+// What the columns of a point add up to, with x and y still factored out. u stands for c_m (entries +m) or s_m (-m),
+// u1 for c_{m-1} or s_{m-1}, w1 for -s_{m-1} or c_{m-1}, and so on one order down.
+template <typename T, bool SECOND> struct PointSums {
+    T Bu = 0, Cu = 0, A1 = 0, Aw = 0;
+    T B1 = 0, Bw = 0, C1 = 0, Cw = 0, A2 = 0, Aw2 = 0, Eu = 0, Gu = 0, Ku = 0;
+
+    __device__ __forceinline__ void add(const ColumnSums<T>& k, T fm, T u, T u1, T w1, T u2, T w2) {
+        const T p1 = fm * u1, q1 = fm * w1;
+        Bu = fma_of(k.B, u, Bu);
+        Cu = fma_of(k.C, u, Cu);
+        A1 = fma_of(k.A, p1, A1);
+        Aw = fma_of(k.A, q1, Aw);
+        if constexpr (SECOND) {
+            const T fmm = fm * (fm - 1);
+            B1 = fma_of(k.B, p1, B1);
+            Bw = fma_of(k.B, q1, Bw);
+            C1 = fma_of(k.C, p1, C1);
+            Cw = fma_of(k.C, q1, Cw);
+            A2 = fma_of(k.A, fmm * u2, A2);
+            Aw2 = fma_of(k.A, fmm * w2, Aw2);
+            Eu = fma_of(k.E, u, Eu);
+            Gu = fma_of(k.G, u, Gu);
+            Ku = fma_of(k.K, u, Ku);
+        }
+    }
+    __device__ __forceinline__ void add_plus(const ColumnSums<T>& k, T fm, const Azimuth<T>& z) {
+        add(k, fm, z.c, z.c1, -z.s1, z.c2, -z.s2);
+    }
+    __device__ __forceinline__ void add_minus(const ColumnSums<T>& k, T fm, const Azimuth<T>& z) {
+        add(k, fm, z.s, z.s1, z.c1, z.s2, z.c2);
+    }
+    __device__ __forceinline__ T gx(T x) const { return fma_of(x, Bu, A1); }
+    __device__ __forceinline__ T gy(T y) const { return fma_of(y, Bu, Aw); }
+    __device__ __forceinline__ T gz() const { return Cu; }
+    __device__ __forceinline__ T xx(T x) const { return fma_of(x, fma_of(x, Eu, 2 * B1), Bu + A2); }
+    __device__ __forceinline__ T yy(T y) const { return fma_of(y, fma_of(y, Eu, 2 * Bw), Bu - A2); }
+    __device__ __forceinline__ T xy(T x, T y) const { return fma_of(y, fma_of(x, Eu, B1), fma_of(x, Bw, Aw2)); }
+    __device__ __forceinline__ T xz(T x) const { return fma_of(x, Gu, C1); }
+    __device__ __forceinline__ T yz(T y) const { return fma_of(y, Gu, Cw); }
+    __device__ __forceinline__ T zz() const { return Ku; }
+};
+
+// Column after column to wave after wave, the direction changing every time round: the longest columns come first.
+struct Deal {
+    unsigned waves, at = 0;
+    bool down = false;
+    __device__ __forceinline__ explicit Deal(unsigned n) : waves(n) {}
+    __device__ __forceinline__ bool next(unsigned wave) {
+        const unsigned owner = down ? waves - 1u - at : at;
+        if (++at == waves) {
+            at = 0;
+            down = !down;
+        }
+        return owner == wave;
+    }
+};
+
+// `len` consecutive elements of HBM, rows of `row` elements, to LDS with the rows `row + pad` apart. pad is 0 or, for
+// even rows (a multiple of 16 bytes then), 1, so that the rows of the points start on different banks. `magic` =
+// magic_of(row in 16-byte vectors). Many 16-byte loads in flight per lane: a tile is read once, and its latency is
+// most of what a workgroup would otherwise wait for.
+template <typename T>
+__device__ __forceinline__ void rows_to_lds(const T* __restrict__ run, T* staged, unsigned len, unsigned row, unsigned pad,
+                                            unsigned magic, unsigned tid, unsigned threads) {
+    using V = typename Pack<T>::type;
+    constexpr unsigned W = Pack<T>::width;
+    if ((reinterpret_cast<uintptr_t>(run) & 15u) != 0) {
+        for (unsigned e = tid; e < len; e += threads) staged[e + pad * (e / row)] = run[e];
+        return;
+    }
+    const V* in = reinterpret_cast<const V*>(run);
+    const unsigned nvec = len / W;
+    auto put = [&](unsigned at, V v) {
+        if (pad == 0) {
+            reinterpret_cast<V*>(staged)[at] = v;
+        } else {
+            T* to = staged + at * W + __umulhi(at, magic);
+#pragma unroll
+            for (unsigned e = 0; e < W; ++e) to[e] = v[e];
+        }
+    };
+    constexpr unsigned DEPTH = 8;
+    unsigned v = tid;
+    for (; v + (DEPTH - 1) * threads < nvec; v += DEPTH * threads) {
+        V hold[DEPTH];
+#pragma unroll
+        for (unsigned u = 0; u < DEPTH; ++u) hold[u] = in[v + u * threads];
+#pragma unroll
+        for (unsigned u = 0; u < DEPTH; ++u) put(v + u * threads, hold[u]);
+    }
+    {
+        // the rest, fewer than DEPTH vectors per lane: all of them in flight as well
+        V hold[DEPTH];
+#pragma unroll
+        for (unsigned u = 0; u < DEPTH; ++u) {
+            if (v + u * threads < nvec) hold[u] = in[v + u * threads];
+        }
+#pragma unroll
+        for (unsigned u = 0; u < DEPTH; ++u) {
+            if (v + u * threads < nvec) put(v + u * threads, hold[u]);
+        }
+    }
+    for (unsigned e = nvec * W + tid; e < len; e += threads) staged[e + pad * (e / row)] = run[e]; // pad == 0 here
+}
+
+// ---------------------------------------------------------------------------
+// columns_kernel: one point per lane (GROUPS == 1, 64 points per workgroup) or per pair of lanes (GROUPS == 2, 32
+// points, one lane for the entries +m and one for -m). The tile's rows of weights pass through LDS, read from HBM with
+// consecutive lanes at consecutive addresses; the columns m are dealt to the waves, longest first in both
+// directions, and every wave walks c_m, s_m along for itself.
+//
+// SECOND == false: the vector-Jacobian product  out[i][a] (+)= sum_k dsph[i][a][k] w[i][k].
+// SECOND == true: its derivatives, for a backward pass through it with the upstream gradient `grad` [n][3]:
+//   out[i][b]  = sum_a grad[i][a] sum_k w[i][k] d^2 sph[i][k] / dx_a dx_b
+//   dw[i][k]   = sum_a grad[i][a] dsph[i][a][k]
+// dw replaces w in LDS entry by entry and leaves as one contiguous run.
+//
+// With n = x/r, P = 1 - n n^T, h = sum w grad R(n) and H = sum w hess R(n) of the polynomials R the chain rule
+// (sphericart/include/templates.hpp:572-613) summed over the entries and applied to g reads
+//   out = (P (H g' - a h) - t g' - n (h . g')) / r^2,   g' = P g, a = n . g, t = n . h,
+// and dw = (g' / r) . grad R.
+// ---------------------------------------------------------------------------
+template <typename T, bool NORM, bool SECOND, int GROUPS>
+__global__ __launch_bounds__(kColumnsThreads) void columns_kernel(Columns g, const T* __restrict__ xyz, const T* __restrict__ weights,
+                                                     const T* __restrict__ grad, T* __restrict__ out,
+                                                     T* __restrict__ dw) {
+    constexpr unsigned TILE = 64 / GROUPS;
+    T* lds = reinterpret_cast<T*>(lds_raw);
+    const unsigned tid = threadIdx.x;
+    const unsigned lane = tid & 63u;
+    const unsigned wave = __builtin_amdgcn_readfirstlane(tid >> 6); // the same for all lanes: scalar
+    const unsigned threads = blockDim.x;
+    const unsigned waves = threads >> 6;
+    const int L = g.l_max;
+    const unsigned ny = g.ny, stride = ny + g.pad;
+    // consecutive workgroups go to the XCDs in turn: one contiguous stretch of tiles for each
+    const unsigned group = (blockIdx.x & 7u) * g.tiles_per_xcd + (blockIdx.x >> 3);
+    if (group >= g.n_tiles) return;
+    const unsigned long long first = static_cast<unsigned long long>(group) * TILE;
+    const unsigned long long left = g.n_samples - first;
+    const unsigned valid = left < TILE ? static_cast<unsigned>(left) : TILE;
+    const unsigned point = lane & (TILE - 1u);
+    const bool minus = GROUPS == 2 && lane >= TILE;
+
+    rows_to_lds<T>(weights + first * ny, lds, valid * ny, ny, g.pad, g.magic_vectors, tid, threads);
+    // lanes past the last point compute on the first one's coordinates and write nothing
+    const unsigned long long mine = first + (point < valid ? point : 0u);
+    const Point<T> p = load_point<T, NORM>(xyz + mine * 3);
+    T gx = 0, gy = 0, gz = 0, along = 0;
+    if constexpr (SECOND) {
+        gx = grad[mine * 3];
+        gy = grad[mine * 3 + 1];
+        gz = grad[mine * 3 + 2];
+        if constexpr (NORM) {
+            along = fma_of(gx, p.x, fma_of(gy, p.y, gz * p.z));
+            gx = fma_of(-along, p.x, gx);
+            gy = fma_of(-along, p.y, gy);
+            gz = fma_of(-along, p.z, gz);
+        }
+    }
+    const T r2 = NORM ? T(1) : p.x2 + p.y2 + p.z2;
+    // the direction of dw, the chain rule's 1/r included
+    const T scale = NORM ? p.ir : T(1);
+    const T dx = gx * scale, dy = gy * scale, dz = gz * scale;
+    const T radial = fma_of(dx, p.x, dy * p.y);
+    __syncthreads(); // weights
+
+    PointSums<T, SECOND> sums;
+    Azimuth<T> azimuth;
+    Deal deal(waves);
+    T* row = lds + point * stride;
+    for (int m = 0; m <= L; ++m) {
+        if (m > 0) azimuth.next(p.x, p.y);
+        if (!deal.next(wave)) continue;
+        const T fm = static_cast<T>(m);
+        if constexpr (GROUPS == 1) {
+            ColumnSums<T> plus, neg;
+            T along_plus = 0, along_minus = 0;
+            if constexpr (SECOND) {
+                along_plus = fm * fma_of(dx, azimuth.c1, -(dy * azimuth.s1));
+                along_minus = fm * fma_of(dx, azimuth.s1, dy * azimuth.c1);
+            }
+            walk_column<T, NORM, SECOND>(m, L, p.z, r2, [&](auto step, int l, T fa, T fb, T fc, T fe, T fg, T fk) {
+                constexpr int S = decltype(step)::value;
+                T* mid = row + l * (l + 1);
+                const T wp = mid[m], wn = mid[-m];
+                plus.template add<S, SECOND>(wp, fa, fb, fc, fe, fg, fk);
+                neg.template add<S, SECOND>(wn, fa, fb, fc, fe, fg, fk);
+                if constexpr (SECOND) {
+                    T q = 0;
+                    if constexpr (S >= 1) q = dz * fc;
+                    if constexpr (S >= 2) q = fma_of(radial, fb, q);
+                    // (m = 0: both are the same entry, the second store is the one that counts)
+                    mid[-m] = fma_of(q, azimuth.s, fa * along_minus);
+                    mid[m] = fma_of(q, azimuth.c, fa * along_plus);
+                }
+            });
+            sums.add_plus(plus, fm, azimuth);
+            sums.add_minus(neg, fm, azimuth);
+        } else {
+            const T u = minus ? azimuth.s : azimuth.c;
+            const T u1 = minus ? azimuth.s1 : azimuth.c1, w1 = minus ? azimuth.c1 : -azimuth.s1;
+            const T u2 = minus ? azimuth.s2 : azimuth.c2, w2 = minus ? azimuth.c2 : -azimuth.s2;
+            ColumnSums<T> k;
+            const T along_u = SECOND ? fm * fma_of(dx, u1, dy * w1) : T(0);
+            const bool writes = m > 0 || !minus; // (m = 0 is one entry)
+            T* at = row + (minus ? -m : m);
+            walk_column<T, NORM, SECOND>(m, L, p.z, r2, [&](auto step, int l, T fa, T fb, T fc, T fe, T fg, T fk) {
+                constexpr int S = decltype(step)::value;
+                T* here = at + l * (l + 1);
+                k.template add<S, SECOND>(*here, fa, fb, fc, fe, fg, fk);
+                if constexpr (SECOND) {
+                    T q = 0;
+                    if constexpr (S >= 1) q = dz * fc;
+                    if constexpr (S >= 2) q = fma_of(radial, fb, q);
+                    if (writes) *here = fma_of(q, u, fa * along_u);
+                }
+            });
+            sums.add(k, fm, u, u1, w1, u2, w2);
+        }
+    }
+
+    // h, and H g': the two lanes of a point, then the waves, are added up
+    constexpr unsigned NS = SECOND ? 6 : 3;
+    T total[NS];
+    total[0] = sums.gx(p.x);
+    total[1] = sums.gy(p.y);
+    total[2] = sums.gz();
+    if constexpr (SECOND) {
+        const T hxy = sums.xy(p.x, p.y), hxz = sums.xz(p.x), hyz = sums.yz(p.y);
+        total[3] = fma_of(sums.xx(p.x), gx, fma_of(hxy, gy, hxz * gz));
+        total[4] = fma_of(hxy, gx, fma_of(sums.yy(p.y), gy, hyz * gz));
+        total[5] = fma_of(hxz, gx, fma_of(hyz, gy, sums.zz() * gz));
+    }
+    if constexpr (GROUPS == 2) {
+#pragma unroll
+        for (unsigned i = 0; i < NS; ++i) total[i] += __shfl_xor(total[i], 32);
+    }
+    T* partial = lds + g.off_sums;
+    if (wave != 0) {
+#pragma unroll
+        for (unsigned i = 0; i < NS; ++i) partial[((wave - 1u) * NS + i) * 64u + lane] = total[i];
+    }
+    if (waves > 1 || SECOND) __syncthreads(); // the waves' sums, and every entry of dw
+    if (wave == 0) {
+        for (unsigned w = 0; w + 1 < waves; ++w) {
+#pragma unroll
+            for (unsigned i = 0; i < NS; ++i) total[i] += partial[(w * NS + i) * 64u + lane];
+        }
+        T ox = total[0], oy = total[1], oz = total[2];
+        if constexpr (SECOND) {
+            ox = total[3];
+            oy = total[4];
+            oz = total[5];
+        }
+        if constexpr (NORM) {
+            const T hx = total[0], hy = total[1], hz = total[2];
+            if constexpr (SECOND) {
+                ox = fma_of(-along, hx, ox);
+                oy = fma_of(-along, hy, oy);
+                oz = fma_of(-along, hz, oz);
+            }
+            const T inward = fma_of(ox, p.x, fma_of(oy, p.y, oz * p.z));
+            ox = fma_of(-inward, p.x, ox);
+            oy = fma_of(-inward, p.y, oy);
+            oz = fma_of(-inward, p.z, oz);
+            if constexpr (SECOND) {
+                const T t = fma_of(hx, p.x, fma_of(hy, p.y, hz * p.z));
+                const T hg = fma_of(hx, gx, fma_of(hy, gy, hz * gz));
+                ox = fma_of(-t, gx, fma_of(-hg, p.x, ox)) * p.ir;
+                oy = fma_of(-t, gy, fma_of(-hg, p.y, oy)) * p.ir;
+                oz = fma_of(-t, gz, fma_of(-hg, p.z, oz)) * p.ir;
+            }
+            ox *= p.ir;
+            oy *= p.ir;
+            oz *= p.ir;
+        }
+        if (point < valid && !minus) {
+            T* to = out + mine * 3;
+            if (!SECOND && g.accumulate) {
+                ox += to[0];
+                oy += to[1];
+                oz += to[2];
+            }
+            to[0] = ox;
+            to[1] = oy;
+            to[2] = oz;
+        }
+    }
+    if constexpr (SECOND) {
+        if (g.pad == 0) {
+            copy_out<T, SPHX_STREAMING_STORES, false>(lds, dw + first * ny, valid * ny, ny, 0, 0, tid, threads);
+        } else {
+            copy_out<T, SPHX_STREAMING_STORES, true>(lds, dw + first * ny, valid * ny, ny, g.pad, g.magic_ny, tid, threads);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// column_rows_kernel: the backward pass from values and gradients,
+//
+//   out[i][b] = sum_k w[i][k] dsph[i][b][k] + sum_a sum_k v[i][a][k] ddsph[i][a][b][k],
+//
+// w (may be null) the upstream gradient of the values, v [n][3][ny] that of the gradients. Four rows of weights per
+// point fill LDS four times as fast, so a point has four lanes and a tile 16 points: a lane takes one side (+m or -m)
+// and two of the four sets of weights, (x, y) or (z, values), and all lanes run the same instructions.
+//
+// Normalised: with s = n . v_k per entry, p = v_k - n s and the polynomials' d = grad R_k, H = hess R_k, the chain rule
+// summed over the entries is
+//   out = (P sum_k (H p + (w r - s) d) - sum_k (n . d) p - n sum_k d . p) / r^2,
+// and n . d = l R_k (R_k is homogeneous of degree l): the sets are p_x, p_y, p_z and w r - s, and one more sum per set,
+// of l w F Q, serves the second term.
+// ---------------------------------------------------------------------------
+template <typename T, bool NORM>
+__global__ __launch_bounds__(kColumnsThreads) void column_rows_kernel(Columns g, const T* __restrict__ xyz, const T* __restrict__ w,
+                                                         const T* __restrict__ v, T* __restrict__ out) {
+    constexpr unsigned TILE = 16;
+    T* lds = reinterpret_cast<T*>(lds_raw);
+    const unsigned tid = threadIdx.x;
+    const unsigned lane = tid & 63u;
+    const unsigned wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const unsigned threads = blockDim.x;
+    const unsigned waves = threads >> 6;
+    const int L = g.l_max;
+    const unsigned ny = g.ny, w_stride = ny + g.pad, v_stride = 3u * ny + g.pad;
+    const unsigned group = (blockIdx.x & 7u) * g.tiles_per_xcd + (blockIdx.x >> 3);
+    if (group >= g.n_tiles) return;
+    const unsigned long long first = static_cast<unsigned long long>(group) * TILE;
+    const unsigned long long left = g.n_samples - first;
+    const unsigned valid = left < TILE ? static_cast<unsigned>(left) : TILE;
+    const unsigned point = lane & (TILE - 1u);
+    const bool minus = (lane & 16u) != 0;
+    const bool second_half = lane >= 32u; // the sets z and values
+    const bool have_w = w != nullptr;
+
+    T* w_rows = lds + g.off_rows;
+    rows_to_lds<T>(v + first * 3u * ny, lds, valid * 3u * ny, 3u * ny, g.pad, g.magic_vectors3, tid, threads);
+    if (have_w) {
+        rows_to_lds<T>(w + first * ny, w_rows, valid * ny, ny, g.pad, g.magic_vectors, tid, threads);
+    } else {
+        for (unsigned e = tid; e < TILE * w_stride; e += threads) w_rows[e] = 0;
+    }
+    const unsigned long long mine = first + (point < valid ? point : 0u);
+    const Point<T> p = load_point<T, NORM>(xyz + mine * 3);
+    const T r2 = NORM ? T(1) : p.x2 + p.y2 + p.z2;
+    // set 0 = v_a - n_a s with a = x or z; set 1 = v_y - y s or w r - s
+    const T n0 = second_half ? p.z : p.x, n1 = second_half ? T(1) : p.y;
+    const T scale1 = second_half && NORM ? 1 / p.ir : T(1);
+    __syncthreads();
+
+    PointSums<T, true> sums0, sums1;
+    T euler0 = 0, euler1 = 0; // sum of l times the set's values
+    Azimuth<T> azimuth;
+    Deal deal(waves);
+    const T* v_row = lds + point * v_stride;
+    const T* w_row = w_rows + point * w_stride;
+    for (int m = 0; m <= L; ++m) {
+        if (m > 0) azimuth.next(p.x, p.y);
+        if (!deal.next(wave)) continue;
+        const T fm = static_cast<T>(m);
+        // (m = 0 is one entry: it has s_0 = 0 and m = 0 for factors on the minus side)
+        const T u = minus ? azimuth.s : azimuth.c;
+        const T u1 = minus ? azimuth.s1 : azimuth.c1, w1 = minus ? azimuth.c1 : -azimuth.s1;
+        const T u2 = minus ? azimuth.s2 : azimuth.c2, w2 = minus ? azimuth.c2 : -azimuth.s2;
+        const int side = minus ? -m : m;
+        const T* v_at = v_row + side;
+        const T* w_at = w_row + side;
+        const T* at0 = v_at + (second_half ? 2u * ny : 0u);
+        const T* at1 = second_half ? w_at : v_at + ny;
+        ColumnSums<T> k0, k1;
+        T le0 = 0, le1 = 0;
+        walk_column<T, NORM, true>(m, L, p.z, r2, [&](auto step, int l, T fa, T fb, T fc, T fe, T fg, T fk) {
+            constexpr int S = decltype(step)::value;
+            const int at = l * (l + 1);
+            T set0, set1;
+            if constexpr (NORM) {
+                const T vx = v_at[at], vy = v_at[at + ny], vz = v_at[at + 2u * ny];
+                const T s = fma_of(vx, p.x, fma_of(vy, p.y, vz * p.z));
+                const T wk = w_at[at];
+                set0 = fma_of(-n0, s, second_half ? vz : vx);
+                set1 = fma_of(-n1, s, (second_half ? wk : vy) * scale1);
+                const T lfa = fa * static_cast<T>(l);
+                le0 = fma_of(set0, lfa, le0);
+                le1 = fma_of(set1, lfa, le1);
+            } else {
+                set0 = at0[at];
+                set1 = at1[at];
+            }
+            k0.template add<S, true>(set0, fa, fb, fc, fe, fg, fk);
+            k1.template add<S, true>(set1, fa, fb, fc, fe, fg, fk);
+        });
+        sums0.add(k0, fm, u, u1, w1, u2, w2);
+        sums1.add(k1, fm, u, u1, w1, u2, w2);
+        if constexpr (NORM) {
+            euler0 = fma_of(le0, u, euler0);
+            euler1 = fma_of(le1, u, euler1);
+        }
+    }
+
+    constexpr unsigned NS = NORM ? 7 : 3;
+    T total[NS];
+    if (!second_half) {
+        const T xy0 = sums0.xy(p.x, p.y), xy1 = sums1.xy(p.x, p.y);
+        total[0] = sums0.xx(p.x) + xy1;
+        total[1] = xy0 + sums1.yy(p.y);
+        total[2] = sums0.xz(p.x) + sums1.yz(p.y);
+        if constexpr (NORM) {
+            total[3] = sums0.gx(p.x) + sums1.gy(p.y);
+            total[4] = euler0;
+            total[5] = euler1;
+            total[6] = 0;
+        }
+    } else {
+        total[0] = sums0.xz(p.x) + sums1.gx(p.x);
+        total[1] = sums0.yz(p.y) + sums1.gy(p.y);
+        total[2] = sums0.zz() + sums1.gz();
+        if constexpr (NORM) {
+            total[3] = sums0.gz();
+            total[4] = 0;
+            total[5] = 0;
+            total[6] = euler0;
+        }
+    }
+#pragma unroll
+    for (unsigned i = 0; i < NS; ++i) {
+        total[i] += __shfl_xor(total[i], 16);
+        total[i] += __shfl_xor(total[i], 32);
+    }
+    T* partial = lds + g.off_sums;
+    if (wave != 0 && lane < TILE) {
+#pragma unroll
+        for (unsigned i = 0; i < NS; ++i) partial[((wave - 1u) * NS + i) * TILE + lane] = total[i];
+    }
+    if (waves > 1) __syncthreads();
+    if (wave == 0 && lane < valid) {
+        for (unsigned q = 0; q + 1 < waves; ++q) {
+#pragma unroll
+            for (unsigned i = 0; i < NS; ++i) total[i] += partial[(q * NS + i) * TILE + lane];
+        }
+        T ox = total[0], oy = total[1], oz = total[2];
+        if constexpr (NORM) {
+            const T inward = fma_of(ox, p.x, fma_of(oy, p.y, fma_of(oz, p.z, total[3])));
+            const T irsq = p.ir * p.ir;
+            ox = (fma_of(-inward, p.x, ox) - total[4]) * irsq;
+            oy = (fma_of(-inward, p.y, oy) - total[5]) * irsq;
+            oz = (fma_of(-inward, p.z, oz) - total[6]) * irsq;
+        }
+        T* to = out + mine * 3;
+        to[0] = ox;
+        to[1] = oy;
+        to[2] = oz;
+    }
+}
+
+} // namespace sphx
+
+#endif

@@ -20,7 +20,7 @@ int fail(int code, const std::string& what) {
 }
 
 static const char* const kSwitchNames[SW_COUNT] = {
-    "SPHX_AZ_SHIFT", "SPHX_CHUNK_SHIFT", "SPHX_GRADIENT_LANES",
+    "SPHX_AZ_SHIFT", "SPHX_CHUNK_SHIFT", "SPHX_COLUMNS_TILE", "SPHX_COLUMNS_WAVES", "SPHX_GRADIENT_LANES",
     "SPHX_GRADIENT_LANES_PARTS", "SPHX_GRADIENT_LANES_TILE", "SPHX_GRADIENT_LANES_WAVES", "SPHX_GROUP_THREADS",
     "SPHX_HESSIAN_LANES",
     "SPHX_HESSIAN_LANES_PARTS", "SPHX_HESSIAN_LANES_TILE", "SPHX_JOB_LIST",

@@ -47,6 +47,8 @@ static int prepare_device(int device) {
     SPHX_HIP(upload_wide_tables<2>(t));
     SPHX_HIP(upload_vjp_tables<float>(t));
     SPHX_HIP(upload_vjp_tables<double>(t));
+    SPHX_HIP(upload_column_tables<float>(t));
+    SPHX_HIP(upload_column_tables<double>(t));
     SPHX_HIP(hipDeviceGetAttribute(&fresh.lds_limit, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
     SPHX_HIP(hipDeviceGetAttribute(&fresh.compute_units, hipDeviceAttributeMultiprocessorCount, device));
     // The kernels deal their workgroups to eight XCDs (`blockIdx.x & 7`): on a device partitioned
@@ -283,6 +285,38 @@ static int vjp(const T* xyz, const T* sph_grad, size_t n_samples, int l_max, int
     });
 }
 
+// ---- second-order products -------------------------------------------------------------------------------
+
+// The derivatives of the fused product, and the backward pass from gradient arrays: `sph_grad` may be null in the
+// latter, `sph_grad_grad` is null there.
+template <typename T>
+static int columns(ColumnsKind kind, const T* xyz, const T* sph_grad, const T* upstream, size_t n_samples, int l_max,
+                   int normalized, T* xyz_grad, T* sph_grad_grad, void* stream) {
+    t_error.clear();
+    if (l_max < 0) return fail(SPHX_ERR_ARGUMENT, "l_max must be non-negative");
+    if (n_samples == 0) return SPHX_OK;
+    const bool both = kind == COLUMNS_VJP_BACKWARD;
+    if (xyz == nullptr || upstream == nullptr || xyz_grad == nullptr || (both && (sph_grad == nullptr || sph_grad_grad == nullptr))) {
+        return fail(SPHX_ERR_ARGUMENT, "null pointer passed to a second-order product");
+    }
+    return on_device_of(xyz, [&](int device) {
+        int status = ensure_device_ready(device);
+        if (status != SPHX_OK) return status;
+        const DeviceState& dev = g_devices[device];
+        ColumnsLaunch launch;
+        (void)refresh_switches();
+        if (!plan_columns(kind, n_samples, l_max, sizeof(T), dev.lds_limit, dev.compute_units, &launch)) {
+            return fail(SPHX_ERR_UNSUPPORTED, "no kernel for this product at l_max = " + std::to_string(l_max));
+        }
+        const hipError_t e = dispatch_columns<T>(kind, launch, normalized != 0, xyz, sph_grad, upstream, xyz_grad,
+                                                 sph_grad_grad, reinterpret_cast<hipStream_t>(stream));
+        if (e != hipSuccess) {
+            return fail(SPHX_ERR_HIP, std::string("kernel launch: ") + hipGetErrorString(e));
+        }
+        return static_cast<int>(SPHX_OK);
+    });
+}
+
 // what the device is like for a plan that is only asked about; an MI355X where there is none
 static void device_for_planning(int* lds, int* cus) {
     int device = 0;
@@ -319,6 +353,30 @@ int sphx_vjp_f32(const float* xyz, const float* sph_grad, size_t n_samples, int 
 int sphx_vjp_f64(const double* xyz, const double* sph_grad, size_t n_samples, int l_max, int normalized,
                  double* xyz_grad, int accumulate, void* stream) {
     return sphx::vjp<double>(xyz, sph_grad, n_samples, l_max, normalized, xyz_grad, accumulate, stream);
+}
+
+int sphx_vjp_backward_f32(const float* xyz, const float* sph_grad, const float* grad, size_t n_samples, int l_max,
+                          int normalized, float* xyz_grad, float* sph_grad_grad, void* stream) {
+    return sphx::columns<float>(sphx::COLUMNS_VJP_BACKWARD, xyz, sph_grad, grad, n_samples, l_max, normalized, xyz_grad,
+                                sph_grad_grad, stream);
+}
+
+int sphx_vjp_backward_f64(const double* xyz, const double* sph_grad, const double* grad, size_t n_samples, int l_max,
+                          int normalized, double* xyz_grad, double* sph_grad_grad, void* stream) {
+    return sphx::columns<double>(sphx::COLUMNS_VJP_BACKWARD, xyz, sph_grad, grad, n_samples, l_max, normalized, xyz_grad,
+                                 sph_grad_grad, stream);
+}
+
+int sphx_gradients_backward_f32(const float* xyz, const float* sph_grad, const float* dsph_grad, size_t n_samples,
+                                int l_max, int normalized, float* xyz_grad, void* stream) {
+    return sphx::columns<float>(sphx::COLUMNS_ROWS, xyz, sph_grad, dsph_grad, n_samples, l_max, normalized, xyz_grad,
+                                nullptr, stream);
+}
+
+int sphx_gradients_backward_f64(const double* xyz, const double* sph_grad, const double* dsph_grad, size_t n_samples,
+                                int l_max, int normalized, double* xyz_grad, void* stream) {
+    return sphx::columns<double>(sphx::COLUMNS_ROWS, xyz, sph_grad, dsph_grad, n_samples, l_max, normalized, xyz_grad,
+                                 nullptr, stream);
 }
 
 int sphx_device_count(void) {

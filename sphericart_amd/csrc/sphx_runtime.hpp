@@ -10,6 +10,7 @@
 #include <string>
 
 #include "../../include/sphx_launch.h"
+#include "sphx_columns.hpp"
 #include "sphx_plan.hpp"
 #include "sphx_tables.hpp"
 
@@ -95,6 +96,11 @@ hipError_t dispatch_wide(const Plan& plan, bool normalized, const float* xyz, fl
 template <typename T>
 hipError_t dispatch_vjp(const VjpPlan& plan, int l_max, bool normalized, const T* xyz, const T* sph_grad,
                         T* xyz_grad, int accumulate, hipStream_t stream);
+// columns_kernel and column_rows_kernel (sphx_columns_kernel.hpp); the pointers a kind does not use are null.
+template <typename T>
+hipError_t dispatch_columns(ColumnsKind kind, const ColumnsLaunch& launch, bool normalized, const T* xyz, const T* sph_grad,
+                            const T* upstream, T* xyz_grad, T* sph_grad_grad, hipStream_t stream);
+template <typename T> hipError_t upload_column_tables(const HostTables& t);
 // Each of those translation units has the constant tables of its arithmetic type to itself; these fill them
 // on the current device. `F` / `Q` (may be null) receive the device addresses.
 template <typename T, int MODE> hipError_t upload_forward_tables(const HostTables& t, const T** F, const T** Q);

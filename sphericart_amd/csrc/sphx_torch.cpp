@@ -15,6 +15,7 @@
 #include <ATen/core/dispatch/Dispatcher.h>
 
 #include <memory>
+#include <optional>
 #include <string>
 #include <tuple>
 
@@ -132,6 +133,73 @@ template <bool SECOND> Tensor contract(const Tensor& derivatives_in, const Tenso
     return out;
 }
 
+// What the two operators below share: xyz, the row length, and weights of a given shape on the same device.
+void check_weights(const Tensor& xyz, const Tensor& weights, at::IntArrayRef shape, const char* what) {
+    TORCH_CHECK_VALUE(weights.scalar_type() == xyz.scalar_type() && weights.device() == xyz.device(), "xyz and ", what,
+                      " must share dtype and device");
+    TORCH_CHECK_VALUE(weights.sizes() == shape, what, " must have shape ", shape);
+}
+
+// The derivatives of vjp with the upstream gradient `grad` [n, 3]: with respect to xyz and to sph_grad
+// (sphx_vjp_backward_*; from the derivative arrays where that does not reach).
+template <bool NORMALIZED>
+std::tuple<Tensor, Tensor> vjp_backward(const Tensor& xyz_in, const Tensor& sph_grad_in, const Tensor& grad_in, int64_t l_max) {
+    const bool f64 = is_double(xyz_in, "spherical harmonics");
+    TORCH_CHECK_VALUE(xyz_in.dim() == 2 && xyz_in.size(1) == 3, "xyz tensor must be a 2D array with shape `n_samples x 3`");
+    TORCH_CHECK_VALUE(l_max >= 0, "l_max must be non-negative");
+    const int64_t n = xyz_in.size(0), ny = (l_max + 1) * (l_max + 1);
+    check_weights(xyz_in, sph_grad_in, {n, ny}, "sph_grad");
+    check_weights(xyz_in, grad_in, {n, 3}, "grad");
+    const Tensor xyz = xyz_in.detach().contiguous(), sph_grad = sph_grad_in.detach().contiguous(), grad = grad_in.detach().contiguous();
+    Tensor xyz_grad = at::empty_like(xyz), sph_grad_grad = at::empty_like(sph_grad);
+    const c10::DeviceGuard guard(xyz.device());
+    const size_t count = static_cast<size_t>(n);
+    const int order = static_cast<int>(l_max);
+    const int status =
+        f64 ? sphx_vjp_backward_f64(pointer<double>(xyz), pointer<double>(sph_grad), pointer<double>(grad), count, order, NORMALIZED,
+                                    pointer<double>(xyz_grad), pointer<double>(sph_grad_grad), stream_of(xyz))
+            : sphx_vjp_backward_f32(pointer<float>(xyz), pointer<float>(sph_grad), pointer<float>(grad), count, order, NORMALIZED,
+                                    pointer<float>(xyz_grad), pointer<float>(sph_grad_grad), stream_of(xyz));
+    if (status == SPHX_ERR_UNSUPPORTED) {
+        const auto all = forward(xyz, l_max, NORMALIZED, 2);
+        return {contract<true>(std::get<2>(all), grad.unsqueeze(2) * sph_grad.unsqueeze(1)),
+                (grad.unsqueeze(2) * std::get<1>(all)).sum(1)};
+    }
+    check(status);
+    return {xyz_grad, sph_grad_grad};
+}
+
+// The backward pass of values and gradients (sphx_gradients_backward_*; from the derivative arrays where that does
+// not reach). sph_grad may be missing.
+template <bool NORMALIZED>
+Tensor gradients_backward(const Tensor& xyz_in, const std::optional<Tensor>& sph_grad_in, const Tensor& dsph_grad_in, int64_t l_max) {
+    const bool f64 = is_double(xyz_in, "spherical harmonics");
+    TORCH_CHECK_VALUE(xyz_in.dim() == 2 && xyz_in.size(1) == 3, "xyz tensor must be a 2D array with shape `n_samples x 3`");
+    TORCH_CHECK_VALUE(l_max >= 0, "l_max must be non-negative");
+    const int64_t n = xyz_in.size(0), ny = (l_max + 1) * (l_max + 1);
+    check_weights(xyz_in, dsph_grad_in, {n, 3, ny}, "dsph_grad");
+    if (sph_grad_in.has_value()) check_weights(xyz_in, *sph_grad_in, {n, ny}, "sph_grad");
+    const Tensor xyz = xyz_in.detach().contiguous(), dsph_grad = dsph_grad_in.detach().contiguous();
+    Tensor sph_grad;
+    if (sph_grad_in.has_value()) sph_grad = sph_grad_in->detach().contiguous();
+    Tensor xyz_grad = at::empty_like(xyz);
+    const c10::DeviceGuard guard(xyz.device());
+    const size_t count = static_cast<size_t>(n);
+    const int order = static_cast<int>(l_max);
+    const int status =
+        f64 ? sphx_gradients_backward_f64(pointer<double>(xyz), pointer<double>(sph_grad), pointer<double>(dsph_grad), count, order,
+                                          NORMALIZED, pointer<double>(xyz_grad), stream_of(xyz))
+            : sphx_gradients_backward_f32(pointer<float>(xyz), pointer<float>(sph_grad), pointer<float>(dsph_grad), count, order,
+                                          NORMALIZED, pointer<float>(xyz_grad), stream_of(xyz));
+    if (status == SPHX_ERR_UNSUPPORTED) {
+        const auto all = forward(xyz, l_max, NORMALIZED, 2);
+        Tensor sum = contract<true>(std::get<2>(all), dsph_grad);
+        return sph_grad.defined() ? sum + contract<false>(std::get<1>(all), sph_grad) : sum;
+    }
+    check(status);
+    return xyz_grad;
+}
+
 [[noreturn]] void no_cpu() {
     TORCH_CHECK(false, "sphericart_amd evaluates on AMD GPUs only: move the tensor to the device "
                        "(there is no CPU implementation behind these operators)");
@@ -141,6 +209,8 @@ std::tuple<Tensor, Tensor> cpu_with_gradients(const Tensor&, int64_t) { no_cpu()
 std::tuple<Tensor, Tensor, Tensor> cpu_with_hessians(const Tensor&, int64_t) { no_cpu(); }
 Tensor cpu_vjp(const Tensor&, const Tensor&, int64_t) { no_cpu(); }
 Tensor cpu_contract(const Tensor&, const Tensor&) { no_cpu(); }
+std::tuple<Tensor, Tensor> cpu_vjp_backward(const Tensor&, const Tensor&, const Tensor&, int64_t) { no_cpu(); }
+Tensor cpu_gradients_backward(const Tensor&, const std::optional<Tensor>&, const Tensor&, int64_t) { no_cpu(); }
 
 } // namespace
 
@@ -152,6 +222,8 @@ TORCH_LIBRARY(sphericart_amd, m) {
         m.def((name + "_with_gradients(Tensor xyz, int l_max) -> (Tensor, Tensor)").c_str());
         m.def((name + "_with_hessians(Tensor xyz, int l_max) -> (Tensor, Tensor, Tensor)").c_str());
         m.def((name + "_vjp(Tensor xyz, Tensor sph_grad, int l_max) -> Tensor").c_str());
+        m.def((name + "_vjp_backward(Tensor xyz, Tensor sph_grad, Tensor grad, int l_max) -> (Tensor, Tensor)").c_str());
+        m.def((name + "_gradients_backward(Tensor xyz, Tensor? sph_grad, Tensor dsph_grad, int l_max) -> Tensor").c_str());
     }
     m.def("contract_gradients(Tensor dsph, Tensor sph_grad) -> Tensor");
     m.def("contract_hessians(Tensor ddsph, Tensor dsph_grad) -> Tensor");
@@ -164,10 +236,14 @@ TORCH_LIBRARY_IMPL(sphericart_amd, CUDA, m) {
     m.impl("spherical_harmonics_with_gradients", &with_gradients<true>);
     m.impl("spherical_harmonics_with_hessians", &with_hessians<true>);
     m.impl("spherical_harmonics_vjp", &vjp<true>);
+    m.impl("spherical_harmonics_vjp_backward", &vjp_backward<true>);
+    m.impl("spherical_harmonics_gradients_backward", &gradients_backward<true>);
     m.impl("solid_harmonics", &values<false>);
     m.impl("solid_harmonics_with_gradients", &with_gradients<false>);
     m.impl("solid_harmonics_with_hessians", &with_hessians<false>);
     m.impl("solid_harmonics_vjp", &vjp<false>);
+    m.impl("solid_harmonics_vjp_backward", &vjp_backward<false>);
+    m.impl("solid_harmonics_gradients_backward", &gradients_backward<false>);
     m.impl("contract_gradients", &contract<false>);
     m.impl("contract_hessians", &contract<true>);
 }
@@ -179,6 +255,8 @@ TORCH_LIBRARY_IMPL(sphericart_amd, CPU, m) {
         m.impl((name + "_with_gradients").c_str(), &cpu_with_gradients);
         m.impl((name + "_with_hessians").c_str(), &cpu_with_hessians);
         m.impl((name + "_vjp").c_str(), &cpu_vjp);
+        m.impl((name + "_vjp_backward").c_str(), &cpu_vjp_backward);
+        m.impl((name + "_gradients_backward").c_str(), &cpu_gradients_backward);
     }
     m.impl("contract_gradients", &cpu_contract);
     m.impl("contract_hessians", &cpu_contract);

@@ -21,7 +21,10 @@ same sums in one pass over ``dsph`` / ``ddsph`` (``sphx_backward_*``) without
 the product array. The backward pass of the value operators does not build
 ``dsph`` at all: ``*_vjp`` (``sphx_vjp_*``) evaluates the gradients on the chip
 and contracts them on the fly. All of these are differentiable themselves, so
-double backward works as it does in the reference.
+double backward works as it does in the reference. A backward pass that is not
+differentiated again (grad mode is off inside it) takes ``*_vjp_backward`` and
+``*_gradients_backward`` (``sphx_vjp_backward_*``, ``sphx_gradients_backward_*``),
+which write no second derivatives either.
 """
 
 import ctypes
@@ -33,6 +36,7 @@ from .._c_lib import LIBRARY_PATH, get_library
 
 NAMESPACE = "sphericart_amd"
 _MODES = {"": 0, "_with_gradients": 1, "_with_hessians": 2}
+_UNSUPPORTED = 2  # SPHX_ERR_UNSUPPORTED
 
 # The schemas and the device implementations live in C++ (csrc/sphx_torch.cpp ->
 # libsphericart_amd_torch.so, built next to the HIP library) where that library has been built: a call
@@ -60,6 +64,8 @@ if not cpp_operators:
         _lib.define(f"{_prefix}_with_gradients(Tensor xyz, int l_max) -> (Tensor, Tensor)")
         _lib.define(f"{_prefix}_with_hessians(Tensor xyz, int l_max) -> (Tensor, Tensor, Tensor)")
         _lib.define(f"{_prefix}_vjp(Tensor xyz, Tensor sph_grad, int l_max) -> Tensor")
+        _lib.define(f"{_prefix}_vjp_backward(Tensor xyz, Tensor sph_grad, Tensor grad, int l_max) -> (Tensor, Tensor)")
+        _lib.define(f"{_prefix}_gradients_backward(Tensor xyz, Tensor? sph_grad, Tensor dsph_grad, int l_max) -> Tensor")
     _lib.define("contract_gradients(Tensor dsph, Tensor sph_grad) -> Tensor")
     _lib.define("contract_hessians(Tensor ddsph, Tensor dsph_grad) -> Tensor")
 
@@ -147,6 +153,45 @@ def _vjp(xyz, sph_grad, l_max, normalized):
     return out
 
 
+def _vjp_backward(xyz, sph_grad, grad, l_max, normalized):
+    suffix = _suffix(xyz)
+    library = get_library()
+    xyz, sph_grad, grad = (t.detach().contiguous() for t in (xyz, sph_grad, grad))
+    xyz_grad, sph_grad_grad = torch.empty_like(xyz), torch.empty_like(sph_grad)
+    with torch.cuda.device(xyz.device):
+        stream = torch.cuda.current_stream(xyz.device).cuda_stream
+        status = getattr(library, f"sphx_vjp_backward_{suffix}")(
+            _pointer(xyz), _pointer(sph_grad), _pointer(grad), xyz.shape[0], l_max, int(normalized),
+            _pointer(xyz_grad), _pointer(sph_grad_grad), ctypes.c_void_p(stream),
+        )
+    if status == _UNSUPPORTED:  # beyond the l_max of those kernels: from the derivative arrays
+        _, dsph, ddsph = _forward(xyz, l_max, normalized, 2)
+        weights = grad.unsqueeze(2) * sph_grad.unsqueeze(1)
+        return _contract("sphx_backward_second", ddsph, weights), torch.sum(grad.unsqueeze(2) * dsph, dim=1)
+    _check(status, library)
+    return xyz_grad, sph_grad_grad
+
+
+def _gradients_backward(xyz, sph_grad, dsph_grad, l_max, normalized):
+    suffix = _suffix(xyz)
+    library = get_library()
+    xyz, dsph_grad = xyz.detach().contiguous(), dsph_grad.detach().contiguous()
+    sph_grad = sph_grad.detach().contiguous() if sph_grad is not None else None
+    xyz_grad = torch.empty_like(xyz)
+    with torch.cuda.device(xyz.device):
+        stream = torch.cuda.current_stream(xyz.device).cuda_stream
+        status = getattr(library, f"sphx_gradients_backward_{suffix}")(
+            _pointer(xyz), _pointer(sph_grad), _pointer(dsph_grad), xyz.shape[0], l_max, int(normalized),
+            _pointer(xyz_grad), ctypes.c_void_p(stream),
+        )
+    if status == _UNSUPPORTED:
+        _, dsph, ddsph = _forward(xyz, l_max, normalized, 2)
+        total = _contract("sphx_backward_second", ddsph, dsph_grad)
+        return total if sph_grad is None else total + _contract("sphx_backward", dsph, sph_grad)
+    _check(status, library)
+    return xyz_grad
+
+
 def _no_cpu(*args, **kwargs):
     raise RuntimeError(
         "sphericart_amd evaluates on AMD GPUs only: move the tensor to the device "
@@ -167,8 +212,15 @@ def _register_forward(prefix, normalized):
     def vjp(xyz, sph_grad, l_max):
         return _vjp(xyz, sph_grad, l_max, normalized)
 
+    def vjp_backward(xyz, sph_grad, grad, l_max):
+        return _vjp_backward(xyz, sph_grad, grad, l_max, normalized)
+
+    def gradients_backward(xyz, sph_grad, dsph_grad, l_max):
+        return _gradients_backward(xyz, sph_grad, dsph_grad, l_max, normalized)
+
     for name, fn in ((prefix, value), (f"{prefix}_with_gradients", gradients),
-                     (f"{prefix}_with_hessians", hessians), (f"{prefix}_vjp", vjp)):
+                     (f"{prefix}_with_hessians", hessians), (f"{prefix}_vjp", vjp),
+                     (f"{prefix}_vjp_backward", vjp_backward), (f"{prefix}_gradients_backward", gradients_backward)):
         _lib.impl(name, fn, "CUDA")
         _lib.impl(name, _no_cpu, "CPU")
 
@@ -253,12 +305,25 @@ def _register_vjp(prefix):
     def fake(xyz, sph_grad, l_max):
         return xyz.new_empty((xyz.shape[0], 3))
 
+    vjp_backward = getattr(_ops, f"{prefix}_vjp_backward")
+
+    @torch.library.register_fake(f"{NAMESPACE}::{prefix}_vjp_backward")
+    def fake_backward(xyz, sph_grad, grad, l_max):
+        return torch.empty_like(xyz), torch.empty_like(sph_grad)
+
+    @torch.library.register_fake(f"{NAMESPACE}::{prefix}_gradients_backward")
+    def fake_gradients_backward(xyz, sph_grad, dsph_grad, l_max):
+        return torch.empty_like(xyz)
+
     def setup_context(ctx, inputs, output):
         xyz, sph_grad, ctx.l_max = inputs
         ctx.save_for_backward(xyz, sph_grad)
 
     def backward(ctx, grad):
         xyz, sph_grad = ctx.saved_tensors
+        if not torch.is_grad_enabled():
+            return *vjp_backward(xyz, sph_grad, grad, ctx.l_max), None
+        # a backward pass that is differentiated again: from operators that can be
         _, dsph, ddsph = hessians(xyz, ctx.l_max)
         d_xyz = d_sph_grad = None
         if ctx.needs_input_grad[0]:
@@ -290,6 +355,7 @@ def _register_value_autograd(prefix):
 
 def _register_gradients_autograd(prefix):
     hessians = getattr(_ops, f"{prefix}_with_hessians")
+    gradients_backward = getattr(_ops, f"{prefix}_gradients_backward")
 
     def setup_context(ctx, inputs, output):
         xyz, ctx.l_max = inputs
@@ -300,6 +366,8 @@ def _register_gradients_autograd(prefix):
         if not ctx.needs_input_grad[0]:
             return None, None
         xyz, dsph = ctx.saved_tensors
+        if grad_dsph is not None and not torch.is_grad_enabled():
+            return gradients_backward(xyz, grad_sph, grad_dsph, ctx.l_max), None
         xyz_grad = None
         if grad_sph is not None:
             xyz_grad = _ops.contract_gradients(dsph, grad_sph)
@@ -315,9 +383,12 @@ def _register_gradients_autograd(prefix):
 
 
 def _register_hessians_autograd(prefix):
+    gradients_backward = getattr(_ops, f"{prefix}_gradients_backward")
+
     def setup_context(ctx, inputs, output):
+        xyz, ctx.l_max = inputs
         ctx.set_materialize_grads(False)
-        ctx.save_for_backward(output[1], output[2])
+        ctx.save_for_backward(xyz, output[1], output[2])
 
     def backward(ctx, grad_sph, grad_dsph, grad_ddsph):
         if grad_ddsph is not None:
@@ -325,7 +396,9 @@ def _register_hessians_autograd(prefix):
                 "Third derivatives of the spherical harmonics with respect to "
                 "the Cartesian coordinates are not supported."
             )
-        dsph, ddsph = ctx.saved_tensors
+        xyz, dsph, ddsph = ctx.saved_tensors
+        if grad_dsph is not None and not torch.is_grad_enabled():
+            return gradients_backward(xyz, grad_sph, grad_dsph, ctx.l_max), None
         xyz_grad = None
         if grad_sph is not None:
             xyz_grad = _ops.contract_gradients(dsph, grad_sph)

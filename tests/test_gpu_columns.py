@@ -1,0 +1,127 @@
+"""columns_kernel and column_rows_kernel (sphx_vjp_backward_*, sphx_gradients_backward_*): the second-order products of
+a backward pass against the oracle's derivative arrays contracted in float64, and through torch's autograd."""
+
+import numpy as np
+import pytest
+import torch
+
+import sphericart_amd.torch as sphx_torch
+from gpu_utils import announce
+
+pytestmark = pytest.mark.gpu
+
+# Against the oracle in float64 at the same points. From l = 18 on the float32 prefactors underflow (in the reference, too,
+# and the kernels use the same ones): there the float32 oracle is the other side. Errors are relative to a point's largest
+# sum of absolute terms. The bound: a term has passed through up to l_max steps of a recursion, with a rounding or two
+# each, and a tangential derivative is the difference of numbers as large as l times it, in the oracle as here. Hence
+# l_max^2 roundings, of 2^-24 or 2^-53, and a few for l_max = 0.
+def _tolerance(dtype, l_max):
+    return (l_max + 4) ** 2 * np.finfo(dtype).eps / 2
+
+
+def _cloud(n, dtype, seed):
+    rng = np.random.default_rng(seed)
+    xyz = rng.standard_normal((n, 3)) + 0.1
+    xyz[:: 50, :2] = 0.0  # on the axis
+    return xyz.astype(dtype)
+
+
+def _expected(oracle, xyz, l_max, normalized, w, g, v):
+    exact = xyz.astype(np.float64) if l_max <= 17 else xyz
+    _, dsph, ddsph = (a.astype(np.float64) for a in oracle.compute(exact, l_max, normalized, "hessians"))
+    w, g, v = (a.astype(np.float64) for a in (w, g, v))
+
+    def both(f):
+        return f(lambda a: a), f(np.abs)
+
+    hess_w = both(lambda s: np.einsum("iabk,ik,ia->ib", s(ddsph), s(w), s(g)))
+    dw = both(lambda s: np.einsum("ia,iak->ik", s(g), s(dsph)))
+    hess_v = both(lambda s: np.einsum("iabk,iak->ib", s(ddsph), s(v)))
+    grad_w = both(lambda s: np.einsum("iak,ik->ia", s(dsph), s(w)))
+    return hess_w, dw, hess_v, grad_w
+
+
+def _close(got, want, scale, tolerance, what):
+    error = np.max(np.abs(got.cpu().numpy().astype(np.float64) - want) / (scale.max(axis=1, keepdims=True) + 1))
+    assert error <= tolerance, (what, error)
+
+
+@pytest.mark.parametrize("tile", [0, 32, 64])
+@pytest.mark.parametrize("normalized", [True, False])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_second_order_products_equal_the_oracles_arrays_contracted(library, oracle, dtype, normalized, tile, switches):
+    """l_max around the steps that a column's first entries take apart (0-5), odd and even row lengths, the largest each
+    kernel holds; points around a tile's 16, 32, 64; both tiles forced where they fit; one wave and eight."""
+    suffix = "f32" if dtype == np.float32 else "f64"
+    backward, rows = getattr(library, f"sphx_vjp_backward_{suffix}"), getattr(library, f"sphx_gradients_backward_{suffix}")
+    stream = torch.cuda.current_stream().cuda_stream
+    if tile:
+        switches("SPHX_COLUMNS_TILE", tile)
+    rng = np.random.default_rng(3)
+    for l_max in (0, 1, 2, 3, 4, 5, 6, 7, 9, 12, 16, 17, 24, 25):
+        for n, waves in ((1, 0), (15, 8), (33, 1), (65, 3), (700, 0)):
+            if waves:
+                switches("SPHX_COLUMNS_WAVES", waves)
+            announce("second-order products", suffix, normalized, tile, l_max, n, waves)
+            if l_max > 12 and n > 100:
+                continue
+            ny = (l_max + 1) ** 2
+            tolerance = _tolerance(dtype, l_max)
+            xyz = _cloud(n, dtype, l_max * 100 + n)
+            w, g, v = (rng.standard_normal(shape).astype(dtype) for shape in ((n, ny), (n, 3), (n, 3, ny)))
+            hess_w, dw, hess_v, grad_w = _expected(oracle, xyz, l_max, normalized, w, g, v)
+            d_xyz, d_g, d_v = (torch.from_numpy(a).cuda() for a in (xyz, g, v))
+            # the weights once aligned, once one element into a 16-byte vector
+            holder = torch.zeros(w.size + 1, dtype=d_xyz.dtype, device="cuda")
+            for shift in (0, 1):
+                d_w = holder[shift:shift + w.size].view(w.shape)
+                d_w.copy_(torch.from_numpy(w))
+                out, out_w = torch.full_like(d_xyz, float("nan")), torch.full((n, ny), float("nan"), dtype=d_xyz.dtype, device="cuda")
+                status = backward(d_xyz.data_ptr(), d_w.data_ptr(), d_g.data_ptr(), n, l_max, int(normalized), out.data_ptr(),
+                                  out_w.data_ptr(), stream)
+                if dtype == np.float64 and l_max > 24:
+                    assert status == 2
+                    continue
+                assert status == 0, library.sphx_last_error()
+                _close(out, *hess_w, tolerance, (l_max, n, shift, "xyz_grad"))
+                _close(out_w, *dw, tolerance, (l_max, n, shift, "sph_grad_grad"))
+                for upstream, pointer in ((True, d_w.data_ptr()), (False, None)):
+                    out = torch.full_like(d_xyz, float("nan"))
+                    status = rows(d_xyz.data_ptr(), pointer, d_v.data_ptr(), n, l_max, int(normalized), out.data_ptr(), stream)
+                    if l_max > (24 if dtype == np.float32 else 16):
+                        assert status == 2
+                        continue
+                    assert status == 0, library.sphx_last_error()
+                    _close(out, hess_v[0] + upstream * grad_w[0], hess_v[1] + upstream * grad_w[1], tolerance, (l_max, n, shift, upstream))
+            if waves:
+                switches("SPHX_COLUMNS_WAVES", 0)
+    assert backward(None, None, None, 0, 3, 1, None, None, stream) == 0
+    assert rows(None, None, None, 0, 3, 1, None, stream) == 0
+    assert backward(None, None, None, 5, 3, 1, None, None, stream) == 1
+
+
+@pytest.mark.parametrize("normalized", [True, False])
+@pytest.mark.parametrize("l_max", [3, 26])
+def test_a_backward_pass_takes_them_and_stays_differentiable(normalized, l_max):
+    """Through autograd: the pass without a graph (these kernels; at l_max = 26 the derivative arrays) gives what the
+    pass with one (operators that can be differentiated again) gives."""
+    announce("second order through autograd", normalized, l_max)
+    calculator = (sphx_torch.SphericalHarmonics if normalized else sphx_torch.SolidHarmonics)(l_max)
+    torch.manual_seed(2)
+    xyz = torch.randn(90, 3, dtype=torch.float64, device="cuda", requires_grad=True)
+    w = torch.randn(90, (l_max + 1) ** 2, dtype=torch.float64, device="cuda", requires_grad=True)
+    g, v = torch.randn_like(xyz), torch.randn(90, 3, (l_max + 1) ** 2, dtype=torch.float64, device="cuda")
+    results = []
+    for create_graph in (False, True):
+        (forces,) = torch.autograd.grad(calculator(xyz), xyz, w, create_graph=True)
+        second = torch.autograd.grad(forces, (xyz, w), g, create_graph=create_graph)
+        sph, dsph = calculator.compute_with_gradients(xyz)
+        first = torch.autograd.grad((sph, dsph), xyz, (w, v), create_graph=create_graph)
+        (only,) = torch.autograd.grad(calculator.compute_with_gradients(xyz)[1], xyz, v, create_graph=create_graph)
+        _, dsph, _ = calculator.compute_with_hessians(xyz)
+        (third,) = torch.autograd.grad(dsph, xyz, v, create_graph=create_graph)
+        results.append((*second, *first, only, third))
+        assert all(t.requires_grad == create_graph for t in results[-1])
+    for a, b in zip(*results):
+        # sums of up to 3 * 729 terms in two orders: 2e-13 of the largest
+        assert (a - b).abs().max().item() <= 2e-13 * b.abs().max().item()
