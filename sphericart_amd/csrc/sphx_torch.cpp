@@ -2,16 +2,18 @@
 // torch.ops.load_library. Host code only (no kernel): it defines the schemas of the `sphericart_amd` namespace and
 // implements them for tensors on the GPU by calling the C entry points of libsphericart_amd.so on the tensor's
 // current stream, as the reference's extension does with its calculators
-// (sphericart-torch/src/torch.cpp:237-294 _compute_raw_cuda, :367-385 TORCH_LIBRARY). Autograd, fake-tensor and vmap
-// rules stay in Python (sphericart_amd/torch/ops.py), as they do in the reference
-// (sphericart-torch/python/sphericart/torch/register.py:60-185). A call through these costs the host the
-// dispatcher, the allocation of its outputs and one C call; the same operators implemented in Python over ctypes,
-// which ops.py registers when this library has not been built, cost about twice that.
+// (sphericart-torch/src/torch.cpp:237-294 _compute_raw_cuda, :367-385 TORCH_LIBRARY). Autograd of GPU tensors is here
+// too; its rules in Python (sphericart_amd/torch/ops.py, the reference's register.py:82-185) serve the operators
+// implemented in Python and tensors without a device, as do the fake-tensor and vmap rules. A call through these costs
+// the host the dispatcher, the allocation of its outputs and one C call; the same operators implemented in Python over
+// ctypes, which ops.py registers when this library has not been built, cost about twice that.
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/library.h>
 
+#include <ATen/core/LegacyTypeDispatch.h>
 #include <ATen/core/dispatch/Dispatcher.h>
 
 #include <memory>
@@ -262,6 +264,213 @@ TORCH_LIBRARY_IMPL(sphericart_amd, CPU, m) {
     m.impl("contract_hessians", &cpu_contract);
 }
 
+// ---- autograd of GPU tensors --------------------------------------------------------------------------------
+//
+// The reference's backward formulas (sphericart-torch/python/sphericart/torch/register.py:82-175), with the products in
+// place of the derivative arrays wherever the pass is not differentiated again (grad mode is off inside it then); a pass
+// that is takes operators that are differentiable themselves. Registered for the Autograd key of the GPU, in front of
+// the Python rules of the same operators: a training step on a small structure is bound by the host, and a rule in
+// Python costs it 10 to 20 us per operator and direction (1 500 points at l_max = 6, values and their product: 79 us per
+// step with the rules in Python, 46 with these, 32 for a step of torch's own sine).
+namespace {
+
+using torch::autograd::AutogradContext;
+using torch::autograd::Function;
+using torch::autograd::variable_list;
+
+template <typename Signature> c10::TypedOperatorHandle<Signature> twin(const std::string& name) {
+    return c10::Dispatcher::singleton().findSchemaOrThrow(("sphericart_amd::" + name).c_str(), "").typed<Signature>();
+}
+
+template <bool NORMALIZED> const char* prefix_of() {
+    return NORMALIZED ? "spherical_harmonics" : "solid_harmonics";
+}
+
+using ValuesSignature = Tensor(const Tensor&, int64_t);
+using GradientsSignature = std::tuple<Tensor, Tensor>(const Tensor&, int64_t);
+using HessiansSignature = std::tuple<Tensor, Tensor, Tensor>(const Tensor&, int64_t);
+using VjpSignature = Tensor(const Tensor&, const Tensor&, int64_t);
+using VjpBackwardSignature = std::tuple<Tensor, Tensor>(const Tensor&, const Tensor&, const Tensor&, int64_t);
+using GradientsBackwardSignature = Tensor(const Tensor&, const std::optional<Tensor>&, const Tensor&, int64_t);
+using ContractSignature = Tensor(const Tensor&, const Tensor&);
+
+template <bool NORMALIZED> struct Operators {
+    static std::string name(const char* suffix) { return std::string(prefix_of<NORMALIZED>()) + suffix; }
+    static const auto& values() {
+        static const auto op = twin<ValuesSignature>(name(""));
+        return op;
+    }
+    static const auto& gradients() {
+        static const auto op = twin<GradientsSignature>(name("_with_gradients"));
+        return op;
+    }
+    static const auto& hessians() {
+        static const auto op = twin<HessiansSignature>(name("_with_hessians"));
+        return op;
+    }
+    static const auto& vjp() {
+        static const auto op = twin<VjpSignature>(name("_vjp"));
+        return op;
+    }
+    static const auto& vjp_backward() {
+        static const auto op = twin<VjpBackwardSignature>(name("_vjp_backward"));
+        return op;
+    }
+    static const auto& gradients_backward() {
+        static const auto op = twin<GradientsBackwardSignature>(name("_gradients_backward"));
+        return op;
+    }
+};
+Tensor contract_gradients(const Tensor& dsph, const Tensor& sph_grad) {
+    static const auto op = twin<ContractSignature>("contract_gradients");
+    return op.call(dsph, sph_grad);
+}
+Tensor contract_hessians(const Tensor& ddsph, const Tensor& dsph_grad) {
+    static const auto op = twin<ContractSignature>("contract_hessians");
+    return op.call(ddsph, dsph_grad);
+}
+
+std::optional<Tensor> maybe(const Tensor& tensor) {
+    return tensor.defined() ? std::optional<Tensor>(tensor) : std::nullopt;
+}
+
+template <bool NORMALIZED> struct ValuesFunction : Function<ValuesFunction<NORMALIZED>> {
+    static constexpr bool is_traceable = true;
+    static Tensor forward(AutogradContext* ctx, const Tensor& xyz, int64_t l_max) {
+        ctx->set_materialize_grads(false);
+        ctx->saved_data["l_max"] = l_max;
+        ctx->save_for_backward({xyz});
+        const at::AutoDispatchBelowAutograd guard;
+        return Operators<NORMALIZED>::values().call(xyz, l_max);
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+        if (!grads[0].defined() || !ctx->needs_input_grad(0)) return {Tensor(), Tensor()};
+        const auto saved = ctx->get_saved_variables();
+        return {Operators<NORMALIZED>::vjp().call(saved[0], grads[0], ctx->saved_data["l_max"].toInt()), Tensor()};
+    }
+};
+
+// the derivatives of the fused product xyz_grad[i, a] = sum_k dsph[i, a, k] w[i, k]
+template <bool NORMALIZED> struct VjpFunction : Function<VjpFunction<NORMALIZED>> {
+    static constexpr bool is_traceable = true;
+    static Tensor forward(AutogradContext* ctx, const Tensor& xyz, const Tensor& sph_grad, int64_t l_max) {
+        ctx->saved_data["l_max"] = l_max;
+        ctx->save_for_backward({xyz, sph_grad});
+        const at::AutoDispatchBelowAutograd guard;
+        return Operators<NORMALIZED>::vjp().call(xyz, sph_grad, l_max);
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &xyz = saved[0], &sph_grad = saved[1], &grad = grads[0];
+        const int64_t l_max = ctx->saved_data["l_max"].toInt();
+        if (!at::GradMode::is_enabled()) {
+            auto both = Operators<NORMALIZED>::vjp_backward().call(xyz, sph_grad, grad, l_max);
+            return {std::get<0>(both), std::get<1>(both), Tensor()};
+        }
+        const auto all = Operators<NORMALIZED>::hessians().call(xyz, l_max);
+        Tensor d_xyz, d_sph_grad;
+        if (ctx->needs_input_grad(0)) {
+            // d/d xyz[i, b]: sum_{a, k} grad[i, a] w[i, k] ddsph[i, a, b, k]
+            d_xyz = contract_hessians(std::get<2>(all), grad.unsqueeze(2) * sph_grad.unsqueeze(1));
+        }
+        if (ctx->needs_input_grad(1)) d_sph_grad = (grad.unsqueeze(2) * std::get<1>(all)).sum(1);
+        return {d_xyz, d_sph_grad, Tensor()};
+    }
+};
+
+// Backward from the gradients of values and gradients, either of which may be missing.
+template <bool NORMALIZED, typename Dsph, typename Ddsph>
+Tensor backward_from(const Tensor& xyz, int64_t l_max, const Tensor& grad_sph, const Tensor& grad_dsph, Dsph dsph, Ddsph ddsph) {
+    if (grad_dsph.defined() && !at::GradMode::is_enabled()) {
+        return Operators<NORMALIZED>::gradients_backward().call(xyz, maybe(grad_sph), grad_dsph, l_max);
+    }
+    Tensor sum;
+    if (grad_sph.defined()) sum = contract_gradients(dsph(), grad_sph);
+    if (grad_dsph.defined()) {
+        const Tensor extra = contract_hessians(ddsph(), grad_dsph);
+        sum = sum.defined() ? sum + extra : extra;
+    }
+    return sum;
+}
+
+template <bool NORMALIZED> struct GradientsFunction : Function<GradientsFunction<NORMALIZED>> {
+    static constexpr bool is_traceable = true;
+    static variable_list forward(AutogradContext* ctx, const Tensor& xyz, int64_t l_max) {
+        const at::AutoDispatchBelowAutograd guard;
+        const auto both = Operators<NORMALIZED>::gradients().call(xyz, l_max);
+        ctx->set_materialize_grads(false); // outputs that were not used arrive undefined
+        ctx->saved_data["l_max"] = l_max;
+        ctx->save_for_backward({xyz, std::get<1>(both)});
+        return {std::get<0>(both), std::get<1>(both)};
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+        if (!ctx->needs_input_grad(0)) return {Tensor(), Tensor()};
+        const auto saved = ctx->get_saved_variables();
+        const int64_t l_max = ctx->saved_data["l_max"].toInt();
+        return {backward_from<NORMALIZED>(saved[0], l_max, grads[0], grads[1], [&] { return saved[1]; },
+                                          [&] { return std::get<2>(Operators<NORMALIZED>::hessians().call(saved[0], l_max)); }),
+                Tensor()};
+    }
+};
+
+template <bool NORMALIZED> struct HessiansFunction : Function<HessiansFunction<NORMALIZED>> {
+    static constexpr bool is_traceable = true;
+    static variable_list forward(AutogradContext* ctx, const Tensor& xyz, int64_t l_max) {
+        const at::AutoDispatchBelowAutograd guard;
+        const auto all = Operators<NORMALIZED>::hessians().call(xyz, l_max);
+        ctx->set_materialize_grads(false);
+        ctx->saved_data["l_max"] = l_max;
+        ctx->save_for_backward({xyz, std::get<1>(all), std::get<2>(all)});
+        return {std::get<0>(all), std::get<1>(all), std::get<2>(all)};
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+        TORCH_CHECK(!grads[2].defined(), "Third derivatives of the spherical harmonics with respect to the Cartesian coordinates "
+                                         "are not supported.");
+        const auto saved = ctx->get_saved_variables();
+        return {backward_from<NORMALIZED>(saved[0], ctx->saved_data["l_max"].toInt(), grads[0], grads[1], [&] { return saved[1]; },
+                                          [&] { return saved[2]; }),
+                Tensor()};
+    }
+};
+
+// The kernels of the Autograd key: straight on where nothing asks for a gradient.
+bool records(const Tensor& a) { return at::GradMode::is_enabled() && a.requires_grad(); }
+
+template <bool NORMALIZED> Tensor autograd_values(c10::DispatchKeySet keys, const Tensor& xyz, int64_t l_max) {
+    if (records(xyz)) return ValuesFunction<NORMALIZED>::apply(xyz, l_max);
+    return Operators<NORMALIZED>::values().redispatch(keys & c10::after_autograd_keyset, xyz, l_max);
+}
+template <bool NORMALIZED>
+std::tuple<Tensor, Tensor> autograd_with_gradients(c10::DispatchKeySet keys, const Tensor& xyz, int64_t l_max) {
+    if (!records(xyz)) return Operators<NORMALIZED>::gradients().redispatch(keys & c10::after_autograd_keyset, xyz, l_max);
+    const auto both = GradientsFunction<NORMALIZED>::apply(xyz, l_max);
+    return {both[0], both[1]};
+}
+template <bool NORMALIZED>
+std::tuple<Tensor, Tensor, Tensor> autograd_with_hessians(c10::DispatchKeySet keys, const Tensor& xyz, int64_t l_max) {
+    if (!records(xyz)) return Operators<NORMALIZED>::hessians().redispatch(keys & c10::after_autograd_keyset, xyz, l_max);
+    const auto all = HessiansFunction<NORMALIZED>::apply(xyz, l_max);
+    return {all[0], all[1], all[2]};
+}
+template <bool NORMALIZED>
+Tensor autograd_vjp(c10::DispatchKeySet keys, const Tensor& xyz, const Tensor& sph_grad, int64_t l_max) {
+    if (records(xyz) || records(sph_grad)) return VjpFunction<NORMALIZED>::apply(xyz, sph_grad, l_max);
+    return Operators<NORMALIZED>::vjp().redispatch(keys & c10::after_autograd_keyset, xyz, sph_grad, l_max);
+}
+
+} // namespace
+
+TORCH_LIBRARY_IMPL(sphericart_amd, AutogradCUDA, m) {
+    m.impl("spherical_harmonics", TORCH_FN(autograd_values<true>));
+    m.impl("spherical_harmonics_with_gradients", TORCH_FN(autograd_with_gradients<true>));
+    m.impl("spherical_harmonics_with_hessians", TORCH_FN(autograd_with_hessians<true>));
+    m.impl("spherical_harmonics_vjp", TORCH_FN(autograd_vjp<true>));
+    m.impl("solid_harmonics", TORCH_FN(autograd_values<false>));
+    m.impl("solid_harmonics_with_gradients", TORCH_FN(autograd_with_gradients<false>));
+    m.impl("solid_harmonics_with_hessians", TORCH_FN(autograd_with_hessians<false>));
+    m.impl("solid_harmonics_vjp", TORCH_FN(autograd_vjp<false>));
+}
+
 // ---- the reference's namespace (sphericart-torch/src/torch.cpp:367-385) -------------------------------------
 //
 // `sphericart_torch` with the reference's eight schemas, so that code written against torch.ops.sphericart_torch.*,
@@ -272,13 +481,6 @@ TORCH_LIBRARY_IMPL(sphericart_amd, CPU, m) {
 // reference's own extension is loaded): then nothing is defined and owns_reference_namespace() says so.
 namespace {
 
-template <typename Signature> c10::TypedOperatorHandle<Signature> twin(const std::string& name) {
-    return c10::Dispatcher::singleton().findSchemaOrThrow(("sphericart_amd::" + name).c_str(), "").typed<Signature>();
-}
-
-template <bool NORMALIZED> const char* prefix_of() {
-    return NORMALIZED ? "spherical_harmonics" : "solid_harmonics";
-}
 template <bool NORMALIZED> Tensor reference_values(const Tensor& xyz, int64_t l_max) {
     static const auto op = twin<Tensor(const Tensor&, int64_t)>(prefix_of<NORMALIZED>());
     return op.call(xyz, l_max);

@@ -125,3 +125,44 @@ def test_a_backward_pass_takes_them_and_stays_differentiable(normalized, l_max):
     for a, b in zip(*results):
         # sums of up to 3 * 729 terms in two orders: 2e-13 of the largest
         assert (a - b).abs().max().item() <= 2e-13 * b.abs().max().item()
+
+
+def test_autograd_with_nothing_but_the_torch_library_loaded(tmp_path):
+    """The rules for GPU tensors are in libsphericart_amd_torch.so: a process that has loaded that library alone gets the
+    gradients, and the gradients of the gradients, that the package gets."""
+    import os
+    import subprocess
+    import sys
+
+    from sphericart_amd.torch import ops
+
+    announce("autograd, library alone")
+    code = f'''
+import sys, torch
+if sys.argv[1] == "alone":
+    torch.ops.load_library({ops.TORCH_LIBRARY_PATH!r})
+    assert "sphericart_amd" not in sys.modules
+else:
+    import sphericart_amd.torch
+torch.manual_seed(1)
+xyz = torch.randn(77, 3, dtype=torch.float64).cuda().requires_grad_()
+w = torch.randn(77, 81, dtype=torch.float64).cuda().requires_grad_()
+v = torch.randn(77, 3, 81, dtype=torch.float64).cuda()
+ops = torch.ops.sphericart_amd
+(forces,) = torch.autograd.grad(ops.spherical_harmonics(xyz, 8), xyz, w, create_graph=True)
+out = [forces, *torch.autograd.grad(forces, (xyz, w), torch.ones_like(forces))]
+sph, dsph = ops.solid_harmonics_with_gradients(xyz, 8)
+out += torch.autograd.grad((sph, dsph), xyz, (w, v))
+sph, dsph, ddsph = ops.solid_harmonics_with_hessians(xyz, 8)
+out += torch.autograd.grad((sph, dsph), xyz, (w, v))
+torch.save([t.detach().cpu() for t in out], sys.argv[2])
+'''
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    results = []
+    for who in ("alone", "package"):
+        path = str(tmp_path / who)
+        done = subprocess.run([sys.executable, "-c", code, who, path], capture_output=True, text=True, cwd=root, timeout=300)
+        assert done.returncode == 0, done.stderr
+        results.append(torch.load(path, weights_only=True))
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
