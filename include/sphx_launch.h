@@ -130,7 +130,7 @@ SPHX_EXPORT int sphx_vjp_f64(const double* xyz, const double* sph_grad, size_t n
  *
  * Enqueued on `stream`; n_samples == 0 returns SPHX_OK. Both agree with the contraction of the arrays to rounding.
  * Where the rows of a tile of points do not fit LDS they return SPHX_ERR_UNSUPPORTED and enqueue nothing (the first
- * takes l_max up to 28 in float32 and 24 in float64, the second 24 and 16): such callers have sphx_forward_* and
+ * takes l_max up to 27 in float32 and 24 in float64, the second 24 and 16): such callers have sphx_forward_* and
  * sphx_backward_second_*. */
 SPHX_EXPORT int sphx_vjp_backward_f32(const float* xyz, const float* sph_grad, const float* grad, size_t n_samples,
                                       int l_max, int normalized, float* xyz_grad, float* sph_grad_grad, void* stream);

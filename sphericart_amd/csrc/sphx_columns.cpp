@@ -51,8 +51,10 @@ bool plan_columns(ColumnsKind kind, size_t n_samples, int l_max, size_t elem, in
     const unsigned vec = 16u / e, pad = ny % 2 == 0 && ny > vec ? 1u : 0u;
     const unsigned limit = static_cast<unsigned>(lds_limit);
     auto rounded = [&](unsigned n) { return (n + vec - 1u) / vec * vec; };
-    // (a wave's sums: 3 or 6 numbers per lane, 7 per point)
+    // The sums of the waves beyond the first (3 or 6 numbers per lane, 7 per point): where dw waits in the rows for its
+    // flush they have a place of their own, else that of the rows, which are no longer needed then.
     const unsigned sums = kind == COLUMNS_ROWS ? 7u * 16u : (kind == COLUMNS_VJP ? 3u : 6u) * 64u;
+    const bool apart = kind == COLUMNS_VJP_BACKWARD;
 
     int waves = 1;
     unsigned tile = 0, rows = 0, off_rows = 0;
@@ -61,16 +63,18 @@ bool plan_columns(ColumnsKind kind, size_t n_samples, int l_max, size_t elem, in
         waves = w;
         off_rows = kind == COLUMNS_ROWS ? rounded(t * (3u * ny + pad)) : 0u;
         rows = off_rows + rounded(t * (ny + pad));
-        return (rows + static_cast<unsigned>(w - 1) * sums) * e;
+        const unsigned all = static_cast<unsigned>(w - 1) * sums;
+        return (apart ? rows + all : (rows > all ? rows : all)) * e;
     };
     const int forced_waves = switch_or(SW_COLUMNS_WAVES, 0), forced_tile = switch_or(SW_COLUMNS_TILE, 0);
     unsigned bytes = 0;
     const int most = l_max + 1 < 8 ? l_max + 1 : 8;
     // Waves per workgroup: enough workgroups fit a CU for one to compute while another one loads, and more waves than
-    // that make a tile wait for its sums. 1M points, l_max = 1, 3, 6 in float32, us with 1 / 2 / 4 / 8 waves:
-    // 13.4 15.2 - -, 29.2 28.8 35.0 -, 86.0 74.8 66.2 86.2; 400 000 at l_max = 8 71 58 50 51; float64 alike. A tile of
-    // 16 points (rows): l_max = 3, 6, 9, 12, 37 51 - -, 66 56 75 146, 98 68 59 98, 179 110 81 87. Too few tiles for the
-    // CUs: as many waves as there are columns, up to eight (1 000 points at l_max = 6: 8.1 us with one, 4.7 with eight).
+    // that make a tile wait for its sums. Derivatives of the product, 1M points, l_max = 1, 3, 6 in float32, us with
+    // 1 / 2 / 4 / 8 waves: 13.4 15.2 - -, 29.2 28.8 35.0 -, 86.0 74.8 66.2 86.2; 400 000 at l_max = 8 71 58 50 51;
+    // float64 alike. A tile of 16 points (rows): l_max = 3, 6, 9, 12, 37 51 - -, 66 56 75 146, 98 68 59 98, 179 110 81
+    // 87. Too few tiles for the CUs: as many waves as there are columns, up to eight (1 000 points at l_max = 6: 8.1 us
+    // with one, 4.7 with eight).
     const size_t cu = static_cast<size_t>(cus > 0 ? cus : 1);
     if (kind == COLUMNS_ROWS) {
         waves = l_max < 5 ? 1 : (l_max < 8 ? 2 : 4);
@@ -78,10 +82,19 @@ bool plan_columns(ColumnsKind kind, size_t n_samples, int l_max, size_t elem, in
         if (forced_waves > 0) waves = forced_waves < most ? forced_waves : most;
         bytes = lay_out(16u, waves);
     } else {
-        waves = l_max < 3 ? 1 : (l_max < 6 ? 2 : 4);
-        // 64 points while three workgroups fit a CU, else 32 on two lanes each (200 000 points at l_max = 12: 56.6
-        // against 55.0 us in float32 where 43 KB still fit three times, 128 against 111 in float64 where 86 KB do not)
-        tile = lay_out(64u, waves) <= 160u * 1024u / 3u ? 64u : 32u;
+        // 64 points while three workgroups fit a CU, else 32 on two lanes each (derivatives of the product, 200 000
+        // points at l_max = 12: 56.6 against 55.0 us in float32 where 43 KB still fit three times, 128 against 111 in
+        // float64 where 86 KB do not; the product, 100 000 at l_max = 16 in float64: 73 against 63)
+        const unsigned lds = 160u * 1024u;
+        const unsigned wide = lay_out(64u, 1) <= lds / 3u ? 64u : 32u;
+        const unsigned resident = lds / lay_out(wide, 1);
+        // four waves while many workgroups share a CU, eight below (the product, us with 4 / 8: float32 l_max = 8 27.5
+        // 34.4, 10 37.1 33.1, 20 55.4 46.6; float64 l_max = 7 76 84, 8 55 48, 10 69 74, 13 93 85). The derivatives in
+        // float64 need so many registers that eight waves would fill a CU: four unless the workgroup is alone (l_max =
+        // 8: 95 143).
+        waves = resident >= (e == 4 ? 6u : 4u) || (kind == COLUMNS_VJP_BACKWARD && e == 8 && resident > 1) ? 4 : 8;
+        if (l_max < 6) waves = l_max < 3 ? 1 : 2;
+        tile = wide;
         if ((n_samples + 63) / 64 <= cu) {
             tile = 32u;
             waves = most;
@@ -104,7 +117,7 @@ bool plan_columns(ColumnsKind kind, size_t n_samples, int l_max, size_t elem, in
     out->g.ny = ny;
     out->g.pad = pad;
     out->g.off_rows = off_rows;
-    out->g.off_sums = rows;
+    out->g.off_sums = apart ? rows : 0u;
     out->g.magic_ny = magic_of(ny);
     out->g.magic_vectors = magic_of(ny / vec ? ny / vec : 1u);
     out->g.magic_vectors3 = magic_of(3u * ny / vec ? 3u * ny / vec : 1u);

@@ -7,9 +7,9 @@
 
 namespace sphx {
 
-// The columns' table holds l <= kColumnsLMax: in float32 the prefactors stop at l = 28 anyway, in float64 the rows of
-// 32 points no longer fit LDS from l_max = 25 on.
-constexpr int kColumnsLMax = 28;
+// The columns' table holds l <= kColumnsLMax: in float32 the iterates of the forward kernels' recursion start to leave
+// the range of the type at l = 28, in float64 the rows of 32 points no longer fit LDS from l_max = 25 on.
+constexpr int kColumnsLMax = 27;
 constexpr int kColumnEntries = (kColumnsLMax + 1) * (kColumnsLMax + 2) / 2;
 // numbers per entry (l, m): b_{l,m}, b_{l-1,m+1}, the factors of A, B, C, then b_{l-2,m+2} and the factors of E, G, K
 constexpr int kColumnEntry = 9;
@@ -26,7 +26,7 @@ struct Columns {
     unsigned ny;             // (l_max + 1)^2
     unsigned pad;            // elements left free after every staged row
     unsigned off_rows;       // column_rows_kernel: where the rows of the values' weights start
-    unsigned off_sums;       // the sums of the waves beyond the first
+    unsigned off_sums;       // the sums of the waves beyond the first (0: where the rows were)
     unsigned accumulate;     // add to the output instead of overwriting it
     unsigned magic_ny, magic_vectors, magic_vectors3; // magic_of(ny), (ny in 16-byte vectors), (3 ny in vectors)
 };

@@ -27,10 +27,14 @@ hipError_t dispatch_columns(ColumnsKind kind, const ColumnsLaunch& l, bool norma
                           : launch_columns(column_rows_kernel<T, false>, l, s, xyz, sph_grad, upstream, xyz_grad);
     }
     auto go = [&](auto kernel) { return launch_columns(kernel, l, s, xyz, sph_grad, upstream, xyz_grad, sph_grad_grad); };
-    if (l.groups == 2) {
-        return normalized ? go(columns_kernel<T, true, true, 2>) : go(columns_kernel<T, false, true, 2>);
-    }
-    return normalized ? go(columns_kernel<T, true, true, 1>) : go(columns_kernel<T, false, true, 1>);
+    auto by_lanes = [&](auto second) {
+        constexpr bool SECOND = decltype(second)::value;
+        if (l.groups == 2) {
+            return normalized ? go(columns_kernel<T, true, SECOND, 2>) : go(columns_kernel<T, false, SECOND, 2>);
+        }
+        return normalized ? go(columns_kernel<T, true, SECOND, 1>) : go(columns_kernel<T, false, SECOND, 1>);
+    };
+    return kind == COLUMNS_VJP ? by_lanes(std::false_type{}) : by_lanes(std::true_type{});
 }
 
 template <typename T> hipError_t upload_column_tables(const HostTables& t) {

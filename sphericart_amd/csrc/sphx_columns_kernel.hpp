@@ -383,6 +383,7 @@ __global__ __launch_bounds__(kColumnsThreads) void columns_kernel(Columns g, con
         for (unsigned i = 0; i < NS; ++i) total[i] += __shfl_xor(total[i], 32);
     }
     T* partial = lds + g.off_sums;
+    if (!SECOND && waves > 1) __syncthreads(); // the sums take the place of the weights
     if (wave != 0) {
 #pragma unroll
         for (unsigned i = 0; i < NS; ++i) partial[((wave - 1u) * NS + i) * 64u + lane] = total[i];
@@ -573,6 +574,7 @@ __global__ __launch_bounds__(kColumnsThreads) void column_rows_kernel(Columns g,
         total[i] += __shfl_xor(total[i], 32);
     }
     T* partial = lds + g.off_sums;
+    if (waves > 1) __syncthreads(); // the sums take the place of the weights
     if (wave != 0 && lane < TILE) {
 #pragma unroll
         for (unsigned i = 0; i < NS; ++i) partial[((wave - 1u) * NS + i) * TILE + lane] = total[i];

@@ -216,12 +216,8 @@ static bool plan_values(size_t n_samples, int l_max, size_t elem, int lds_limit,
                                : (bytes > half && pack != 4 ? (elem == 4 && pack == 1 ? 12 : 16) : 8);
     int waves = switch_or(SW_VALUES_WAVES, waves_by_shape != 0 && alone ? waves_by_shape : most);
     waves = waves < 1 ? 1 : (waves > most ? most : waves);
-    // (the product's closed-form slices want at least four; values: one for the tables, one for
-    // the closed forms)
+    // (values: at least two, one for the tables, one for the closed forms)
     int want = (l_max - 6 + static_cast<int>(pack) - 1) / static_cast<int>(pack);
-    // (the product: one or two channels are best with four waves, three or four channels with three, five or
-    // six with four)
-    if (with_sums) want = want <= 2 ? 4 : (want <= 4 ? 3 : (want <= 6 ? 4 : want));
     if (!with_sums && want < 2) want = switch_or(SW_VALUES_MIN_WAVES, 2);
     out->threads = 64u * static_cast<unsigned>(want < waves ? want : waves);
     out->lds_bytes = bytes;
@@ -993,6 +989,7 @@ bool make_wide_plan(size_t n_samples, int l_max, int mode, int lds_limit, int cu
 }
 
 int make_vjp_plan(size_t n_samples, int l_max, size_t elem, int lds_limit, int cus, VjpPlan* out) {
+    // (columns_kernel takes l_max = 7 to 24, in float32 to 27: sphx_runtime.cpp)
     out->use_lanes = out->lane_groups = false;
     if (l_max > 6 && switch_or(SW_VJP_LANES, 1) != 0) {
         out->use_lanes = plan_values(n_samples, l_max, elem, lds_limit, &out->lanes, true);

@@ -40,27 +40,9 @@ constexpr ShapeRow kShapeRows[] = {
     {0, 8, 15, 15, 1, true, 0, 32, "258 225 - 257 326 347"},
     // the product, float64. 200 000 points (400 000 to l_max = 16), us: tiles in half of LDS / one workgroup per
     // CU with 8 / with up to 12 waves; from l_max = 21 with tiles of 28, 24, 20 points before they halve
-    {1, 8, 14, 14, 1, true, 12, 32, "498 287 286"},
-    {1, 8, 15, 15, 1, true, 12, 32, "519 328 324"},
-    {1, 8, 16, 16, 1, true, 12, 32, "538 383 360"},
-    {1, 8, 17, 17, 1, true, 12, 32, "289 228 214"},
-    {1, 8, 18, 18, 1, true, 12, 32, "299 261 240"},
-    {1, 8, 19, 19, 1, true, 12, 32, "315 290 272"},
-    {1, 8, 20, 20, 1, true, 12, 32, "330 336 316"},
-    {1, 8, 21, 21, 1, true, 12, 16, "588 375 364"},
-    {1, 8, 22, 22, 1, true, 12, 16, "613 444 405"},
-    {1, 8, 23, 23, 1, true, 12, 16, "627 468 464"},
-    {1, 8, 24, 24, 1, true, 12, 16, "640 565 564"},
     {1, 8, 25, 25, 1, true, 8, 16, "660 598 602"},
     {1, 8, 26, 26, 1, true, 12, 16, "675 719 661"},
     // the product, float32, the same columns (l_max = 21, 31: sixteen waves 162, 423)
-    {1, 4, 19, 19, 1, true, 12, 32, "144 153 135"},
-    {1, 4, 21, 21, 1, true, 16, 32, "181 178 172"},
-    {1, 4, 22, 22, 1, true, 8, 32, "211 168 185"},
-    {1, 4, 23, 23, 1, true, 12, 32, "216 212 201"},
-    {1, 4, 25, 25, 1, true, 12, 32, "335 274 255"},
-    {1, 4, 26, 26, 1, true, 12, 32, "340 294 276"},
-    {1, 4, 27, 27, 1, true, 8, 32, "348 289 313"},
     {1, 4, 28, 28, 1, true, 8, 32, "356 318 342"},
     {1, 4, 29, 29, 1, true, 12, 32, "385 404 370"},
     {1, 4, 30, 30, 1, true, 8, 32, "397 381 422"},

@@ -272,12 +272,22 @@ static int vjp(const T* xyz, const T* sph_grad, size_t n_samples, int l_max, int
         bool fresh = false;
         PlannedCall* call = planned_call(1, n_samples, l_max, 1, sizeof(T), normalized != 0, device, &fresh);
         if (fresh) {
-            status = make_vjp_plan(n_samples, l_max, sizeof(T), dev.lds_limit, dev.compute_units, &call->vjp);
+            // Up to l_max = 6 the sum runs over the closed forms in index order (number for number what contracting the
+            // gradients gives); beyond, columns_kernel is ahead of the kernels that form every entry
+            call->by_columns = l_max > 6 && switch_or(SW_VJP_LANES, 1) != 0 &&
+                               plan_columns(COLUMNS_VJP, n_samples, l_max, sizeof(T), dev.lds_limit, dev.compute_units,
+                                            &call->columns);
+            status = call->by_columns ? static_cast<int>(SPHX_OK)
+                                      : make_vjp_plan(n_samples, l_max, sizeof(T), dev.lds_limit, dev.compute_units, &call->vjp);
             if (status != SPHX_OK) return status;
             keep(call);
         }
-        const hipError_t e = dispatch_vjp<T>(call->vjp, l_max, normalized != 0, xyz, sph_grad, xyz_grad, accumulate,
-                                             reinterpret_cast<hipStream_t>(stream));
+        hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+        if (call->by_columns) call->columns.g.accumulate = accumulate != 0;
+        const hipError_t e = call->by_columns
+                                 ? dispatch_columns<T>(COLUMNS_VJP, call->columns, normalized != 0, xyz, sph_grad, nullptr,
+                                                       xyz_grad, nullptr, s)
+                                 : dispatch_vjp<T>(call->vjp, l_max, normalized != 0, xyz, sph_grad, xyz_grad, accumulate, s);
         if (e != hipSuccess) {
             return fail(SPHX_ERR_HIP, std::string("kernel launch: ") + hipGetErrorString(e));
         }

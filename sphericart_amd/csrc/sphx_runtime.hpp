@@ -55,6 +55,8 @@ struct PlannedCall {
     // what was planned
     Plan plan;         // kinds 0 and 2
     VjpPlan vjp;       // kind 1
+    ColumnsLaunch columns;     // kind 1 beyond the closed forms, where columns_kernel takes it,
+    bool by_columns = false;   // which this says
     bool wide = false; // kind 2: the recursion kernel covers this shape
 };
 // The slot for this shape; `*fresh` says that it has yet to be planned (by the caller, who then calls keep();
