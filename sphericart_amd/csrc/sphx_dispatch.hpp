@@ -100,11 +100,12 @@ static hipError_t dispatch(const Plan& plan, const DeviceState& device, const T*
     if (plan.lanes) {
         if constexpr (MODE == 0) {
             const Launch& l = plan.closed;
-            auto kernel = l.g.points_per_pass == 4   ? values_kernel<T, NORM, 4>
+            auto kernel = l.g.points_per_pass == 8   ? values_kernel<T, NORM, 8>
+                          : l.g.points_per_pass == 4 ? values_kernel<T, NORM, 4>
                           : l.g.points_per_pass == 2 ? (l.threads > 512 ? values_kernel<T, NORM, 2, 1024> : values_kernel<T, NORM, 2>)
                           : l.threads > 512          ? values_kernel<T, NORM, 1, 1024>
                                                      : values_kernel<T, NORM, 1>;
-            if (l.threads > (l.g.points_per_pass == 4 ? 512u : 1024u)) return hipErrorInvalidValue; // never planned
+            if (l.threads > (l.g.points_per_pass >= 4 ? 512u : 1024u)) return hipErrorInvalidValue; // never planned
             if (l.lds_bytes > 64u * 1024u) {
                 unsigned unused = 0;
                 hipError_t e = kernel_facts(reinterpret_cast<const void*>(kernel), l.threads, l.lds_bytes, &unused);

@@ -18,20 +18,13 @@ namespace sphx {
 // the same points.
 //
 // Without derivatives an entry is three multiplications, so what counts is what
-// surrounds them. With one point per lane l and m are the same for the whole
-// wave: no job has to be decoded and no iterate passes through LDS. The
-// prefactors of a channel, m = 0..l, are loaded once, one per lane, and the
-// recursion takes each from its lane (v_readlane), so that its loop touches no
-// memory but the point's table in LDS, whose entries for the next m are fetched
-// before the arithmetic of this one: about 25 instructions per (l, +-m) pair of
-// entries, a fraction of what the recursion kernel spends on them. (Prefactors
-// through scalar loads inside the loop made every step wait for them: LDS and
-// scalar loads share one counter, so nothing could be fetched ahead. 1 GB of
-// values, float32, l_max = 22, 26, 28: 288, 341, 355 us then, 270, 315, 327 so.)
-// (With derivatives the entries themselves dominate and rows are four and
-// thirteen times as long, so that far fewer than 64 points fit:
-// gradients_lanes_kernel takes l_max up to about 16, the recursion kernel the
-// rest.)
+// surrounds them. With one point per lane m is the same for the whole wave: no
+// job has to be decoded and no iterate passes through LDS. A step down in m is
+// two LDS reads (c_m and s_m; 2(m+1)z), seven operations and two LDS writes.
+// What a step reads is fetched four steps ahead into registers, so that no
+// step waits for LDS, and four steps share the address arithmetic. The
+// prefactors of a channel, m = 0..l, are loaded once, one per lane, and a step
+// takes each from its lane (v_readlane).
 //
 // The rows of 64 points take most of a CU's LDS from l_max of about 12 on, and
 // one wave would leave three of the four SIMDs idle: the l channels are dealt
@@ -39,12 +32,19 @@ namespace sphx {
 // each wave evaluating its channels for all points of the tile (l_max = 15
 // float32, 500k points: 245 us with one wave, 113 with four, 106 with six).
 // When 64 rows do not fit the tile is smaller, any number of points, and the
-// lanes beyond it idle; or (K = 2, 4) the tile is 32 or 16 points and a wave
+// lanes beyond it idle; or (K = 2, 4, 8) the tile is 32, 16 or 8 points and a wave
 // evaluates K channels l0, l0 - 1, .. side by side, lane = side * (64 / K) +
-// point: it walks m down from l0 for all of them, each lane picks the
-// prefactors of its own channel, and the lanes of a shorter channel join when
-// m reaches their l. All lanes work then, for about 40 instructions per step
-// of two channels (the host picks by shape, see plan_values).
+// point: it walks m down from l0 for all of them, and the lanes of a shorter
+// channel join when m reaches their l (the host picks by shape, see
+// plan_values). The prefactors are then kept in LDS and every lane reads those
+// of its own channel, four steps ahead as well: one more read per step, where
+// handing them from lane to lane takes two instructions per channel and two
+// more to pick the right one (40 instructions per step of two channels then,
+// 14 so; 1.2 GB of values in float32, us: l_max = 22 240 and 198, 25 286 and
+// 203; 300 points at l_max = 22 7.3 and 5.8).
+//
+// (Prefactors through scalar loads inside the loop make every step wait for
+// them: LDS and scalar loads share one counter.)
 //
 // Same operations in the same order as the reference: c_m, s_m, 2(m+1)z as in
 // templates.hpp:451-466, l <= 6 in closed form, then per l the recursion of
@@ -52,10 +52,12 @@ namespace sphx {
 // multiplied by its prefactor and by c_m and s_m (:127-128,160-162,214-218,395).
 //
 // LDS: the rows of the tile in HBM layout, so that the waves stream them out
-// with 16-byte stores, and per point its table of (c_m, s_m, 2(m+1)z). A row
-// length that is a multiple of 8 words would put the same entry of all points
-// on few banks: such rows are kept one 16-byte vector apart.
-// g.rows_elems: row stride, g.off_pts: start of the tables, g.off_iter: table stride.
+// with 16-byte stores; per point its c_m, s_m and its 2(m+1)z, an odd number of
+// entries apart (no bank conflicts); K > 1: the prefactors. A row length that is a
+// multiple of 8 words would put the same entry of all points on few banks: such
+// rows are kept one 16-byte vector apart.
+// g.rows_elems: row stride, g.off_pts: start of the (c, s), g.off_F: of the 2(m+1)z,
+// g.off_iter: entries from point to point in both, g.off_Q: start of the prefactors.
 // ---------------------------------------------------------------------------
 constexpr unsigned kValuesMaxThreads = 512;
 
@@ -85,6 +87,10 @@ template <typename T> struct ChannelPrefactors {
     __device__ __forceinline__ T operator[](int m) const { return from_lane(lanes, m); }
 };
 
+template <typename T> struct Two { // one LDS read
+    T a, b;
+} __attribute__((aligned(2 * sizeof(T))));
+
 template <typename T, bool NORM, unsigned K = 1, unsigned NT = kValuesMaxThreads>
 __global__ __launch_bounds__(NT) void values_kernel(Tiling g, const T* __restrict__ xyz,
                                                                   T* __restrict__ sph) {
@@ -112,24 +118,30 @@ __global__ __launch_bounds__(NT) void values_kernel(Tiling g, const T* __restric
     Point<T> p;
     p.x = p.y = p.z = p.x2 = p.y2 = p.z2 = p.ir = 0;
     T* row = lds + point * g.rows_elems;
-    T* tab = lds + g.off_pts + point * g.off_iter; // [m][3]: c_m, s_m, 2(m+1)z
+    Two<T>* cs = reinterpret_cast<Two<T>*>(lds + g.off_pts) + point * g.off_iter; // [m]: c_m, s_m
+    T* tz = lds + g.off_F + point * g.off_iter;                                   // [m]: 2(m+1)z
+    Two<T>* fq = reinterpret_cast<Two<T>*>(lds + g.off_Q);                        // [l(l+1)/2 + m]: F, Q
     if (point < valid) p = load_point<T, NORM>(xyz + (first + point) * 3);
+    if constexpr (K > 1) {
+        const unsigned entries = static_cast<unsigned>((L + 1) * (L + 2) / 2);
+        const T* cF = table_F<T>();
+        const T* cQ = table_Q<T>();
+        for (unsigned e = tid; e < entries; e += blockDim.x) fq[e] = Two<T>{cF[e], cQ[e]};
+    }
     if (point < valid && side == 0) {
         if (wave == 0) {
             const T twoz = p.z + p.z;
-            T cm = 1.0, sm = 0.0, tz = twoz;
-            tab[0] = cm;
-            tab[1] = sm;
-            tab[2] = tz;
+            T cm = 1.0, sm = 0.0, t = twoz;
+            cs[0] = Two<T>{cm, sm};
+            tz[0] = t;
             for (int m = 1; m <= L; ++m) {
                 const T cn = cm * p.x - sm * p.y;
                 const T sn = cm * p.y + sm * p.x;
-                tz = tz + twoz;
+                t = t + twoz;
                 cm = cn;
                 sm = sn;
-                tab[3 * m] = cm;
-                tab[3 * m + 1] = sm;
-                tab[3 * m + 2] = tz;
+                cs[m] = Two<T>{cm, sm};
+                tz[m] = t;
             }
         }
         if (wave == waves - 1) { // the last wave gets the fewest channels below
@@ -140,105 +152,90 @@ __global__ __launch_bounds__(NT) void values_kernel(Tiling g, const T* __restric
         }
     }
     __syncthreads(); // the tables
-    if constexpr (K > 1) {
-        const T rxy = p.x2 + p.y2;
-        // K channels side by side, l0, l0 - 1, ..: the wave walks m from l0 down for all of them,
-        // the lanes of a shorter channel join when m reaches their l (what they hold before that
-        // is not used: the first two steps of a channel take nothing from earlier ones); bundles
-        // of K channels go to the waves like single channels below
-        const unsigned bundles = (static_cast<unsigned>(L - H) + K - 1u) / K;
-        for (unsigned i = 0; i < bundles; ++i) {
-            const unsigned pos = i % waves;
-            if ((((i / waves) & 1u) ? waves - 1u - pos : pos) != wave) continue;
-            const int l0 = L - static_cast<int>(i * K); // >= H + 1, so l0 - (K - 1) >= 0
-            ChannelPrefactors<T> pk[K], qk[K];
-#pragma unroll
-            for (unsigned k = 0; k < K; ++k) {
-                const int lk = l0 - static_cast<int>(k);
-                pk[k] = ChannelPrefactors<T>(table_F<T>() + lk * (lk + 1) / 2, lk, lane);
-                qk[k] = ChannelPrefactors<T>(table_Q<T>() + lk * (lk + 1) / 2, lk, lane);
-            }
-            if (point >= valid) continue; // (all lanes are back at the next bundle's loads)
-            const int l = l0 - static_cast<int>(side);
-            const bool live = l > H;
-            T* mid = row + l * l + l;
-            auto prefactors = [&](int m, T& f, T& q) {
-                f = pk[0][m];
-                q = qk[0][m];
-#pragma unroll
-                for (unsigned k = 1; k < K; ++k) {
-                    const T fk = pk[k][m], qk_ = qk[k][m];
-                    if (side == k) {
-                        f = fk;
-                        q = qk_;
-                    }
-                }
-            };
-            T v1 = 0, v2 = 0;
-            T c = tab[3 * l0], s = tab[3 * l0 + 1], tz = tab[3 * l0 + 2];
-            for (int m = l0; m >= 1; --m) {
-                const T c0 = c, s0 = s, tz0 = tz;
-                c = tab[3 * m - 3];
-                s = tab[3 * m - 2];
-                tz = tab[3 * m - 1];
-                T f, q;
-                prefactors(m, f, q);
-                T v0 = q * (tz0 * v1 + rxy * v2);
-                if (m == l - 1) v0 = -p.z * v1;
-                if (m == l) v0 = q;
-                const T pq = v0 * f;
-                if (live && m <= l) {
-                    mid[m] = pq * c0;
-                    mid[-m] = pq * s0;
-                }
-                v2 = v1;
-                v1 = v0;
-            }
-            T f, q;
-            prefactors(0, f, q);
-            const T v0 = q * (tz * v1 + rxy * v2);
-            if (live) mid[0] = v0 * f;
+    const T rxy = p.x2 + p.y2;
+    // Bundles of K channels, l0, l0 - 1, .., side by side: number i goes to wave i % waves in even rounds,
+    // backwards in odd ones.
+    const unsigned bundles = (static_cast<unsigned>(L - H) + K - 1u) / K;
+    for (unsigned i = 0; i < bundles; ++i) {
+        const unsigned pos = i % waves;
+        if ((((i / waves) & 1u) ? waves - 1u - pos : pos) != wave) continue;
+        const int l0 = L - static_cast<int>(i * K); // >= H + 1
+        ChannelPrefactors<T> pk, qk;
+        if constexpr (K == 1) {
+            pk = ChannelPrefactors<T>(table_F<T>() + l0 * (l0 + 1) / 2, l0, lane);
+            qk = ChannelPrefactors<T>(table_Q<T>() + l0 * (l0 + 1) / 2, l0, lane);
         }
-    } else {
-        const T rxy = p.x2 + p.y2;
-        // channel number i = L - l goes to wave i % waves in even rounds, backwards in odd ones
-        for (unsigned i = 0; static_cast<int>(i) < L - H; ++i) {
-            const unsigned pos = i % waves;
-            if ((((i / waves) & 1u) ? waves - 1u - pos : pos) != wave) continue;
-            const int l = L - static_cast<int>(i);
-            const int tri = l * (l + 1) / 2;
-            const ChannelPrefactors<T> pk(table_F<T>() + tri, l, lane);
-            const ChannelPrefactors<T> qk(table_Q<T>() + tri, l, lane);
-            if (lane >= valid) continue; // (all lanes are back at the next channel's loads)
-            T* mid = row + l * l + l;
-            T v2 = qk[l];
-            T v1 = -p.z * v2;
-            {
-                const T pq = v2 * pk[l];
-                mid[l] = pq * tab[3 * l];
-                mid[-l] = pq * tab[3 * l + 1];
+        const int l = l0 - static_cast<int>(side);
+        if (point >= valid || l <= H) continue; // (all lanes are back at the next channel's loads)
+        T* mid = row + l * l + l;
+        const Two<T>* pre = fq + l * (l + 1) / 2;
+        struct Step {
+            Two<T> cs, fq;
+            T tz;
+        };
+        // (m down to -3 at the end of a channel: those reads are inside LDS, and nothing uses them)
+        auto fetch = [&](int m) { return Step{cs[m], K == 1 ? Two<T>{0, 0} : pre[m], tz[m]}; };
+        auto F = [&](int m, const Step& k) { return K == 1 ? pk[m] : k.fq.a; };
+        auto Q = [&](int m, const Step& k) { return K == 1 ? qk[m] : k.fq.b; };
+        T v1 = 0, v2 = 0;
+        auto next = [&](int m, const Step& k) { return Q(m, k) * (k.tz * v1 + rxy * v2); };
+        auto put = [&](int m, const Step& k, T v0) {
+            const T pq = v0 * F(m, k);
+            mid[m] = pq * k.cs.a;
+            mid[-m] = pq * k.cs.b;
+        };
+        auto shift = [&](T v0) {
+            v2 = v1;
+            v1 = v0;
+        };
+        // The first two steps of every channel take nothing from earlier ones: what a lane computes before m reaches
+        // its l is not used (the prefactors it reads then are those of the next l, still inside the table). K + 1
+        // steps until that holds for the shortest channel, or down to m = 1 (K = 8, l0 = 7 and 8: the step at m = 0
+        // comes last, below).
+        constexpr int U = 4, TOP = static_cast<int>(K) + 1;
+        const int top = K > H && l0 < TOP ? l0 : TOP;
+        constexpr bool EARLY = K <= 4; // (eight channels: too many registers)
+        Step first_steps[TOP], ahead[U];
+        if constexpr (EARLY) {
+#pragma unroll
+            for (int u = 0; u < TOP; ++u) first_steps[u] = fetch(l0 - u);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) ahead[u] = fetch(l0 - top - u);
+#pragma unroll
+        for (int u = 0; u < TOP; ++u) {
+            if (u < top) {
+                const int m = l0 - u;
+                const Step k = EARLY ? first_steps[u] : fetch(m);
+                T v0 = next(m, k);
+                if (m == l - 1) v0 = -p.z * v1;
+                if (m == l) v0 = Q(m, k);
+                if (K == 1 || m <= l) put(m, k, v0);
+                shift(v0);
             }
-            {
-                const T pq = v1 * pk[l - 1];
-                mid[l - 1] = pq * tab[3 * (l - 1)];
-                mid[-(l - 1)] = pq * tab[3 * (l - 1) + 1];
+        }
+        int m = l0 - top;
+        for (; m >= U; m -= U) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const T v0 = next(m - u, ahead[u]);
+                put(m - u, ahead[u], v0);
+                shift(v0);
+                ahead[u] = fetch(m - u - U);
             }
-            // the table entries of the next m are fetched before the arithmetic of this one
-            T c = tab[3 * (l - 2)], s = tab[3 * (l - 2) + 1], tz = tab[3 * (l - 2) + 2];
-            for (int m = l - 2; m >= 1; --m) {
-                const T c0 = c, s0 = s, tz0 = tz;
-                c = tab[3 * m - 3];
-                s = tab[3 * m - 2];
-                tz = tab[3 * m - 1];
-                const T v0 = qk[m] * (tz0 * v1 + rxy * v2);
-                const T pq = v0 * pk[m];
-                mid[m] = pq * c0;
-                mid[-m] = pq * s0;
-                v2 = v1;
-                v1 = v0;
+        }
+        // m < U steps and m = 0 are left
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (u <= m) {
+                const T v0 = next(m - u, ahead[u]);
+                if (u < m) {
+                    put(m - u, ahead[u], v0);
+                } else {
+                    mid[0] = v0 * F(0, ahead[u]);
+                }
+                shift(v0);
             }
-            const T v0 = qk[0] * (tz * v1 + rxy * v2);
-            mid[0] = v0 * pk[0];
         }
     }
     __syncthreads(); // the rows

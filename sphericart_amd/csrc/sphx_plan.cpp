@@ -137,7 +137,10 @@ static bool plan_values(size_t n_samples, int l_max, size_t elem, int lds_limit,
     const unsigned vec = 16u / esize;
     // rows a multiple of 8 words long: one vector between them (values_kernel)
     const unsigned row_stride = (ny * (esize / 4u)) % 8u == 0 ? ny + vec : ny;
+    // a point's entries in the tables, an odd number: of (c, s, 2(m+1)z), or of (c, s) and of 2(m+1)z
+    const unsigned table_entries = static_cast<unsigned>(l_max + 1) | 1u;
     const unsigned table_stride = (3u * static_cast<unsigned>(l_max + 1)) | 1u;
+    const unsigned table_elems = with_sums ? table_stride : 3u * table_entries;
     const unsigned tri_all = static_cast<unsigned>(l_max + 1) * (l_max + 2) / 2;
     unsigned allowed = static_cast<unsigned>(switch_or(SW_VALUES_LDS, 160 * 1024));
     if (allowed > static_cast<unsigned>(lds_limit)) allowed = static_cast<unsigned>(lds_limit);
@@ -149,8 +152,11 @@ static bool plan_values(size_t n_samples, int l_max, size_t elem, int lds_limit,
     // Which form of the kernel goes by the shape (sphx_plan_shapes.hpp): tiles of 64 / pack points whose waves
     // evaluate `pack` channels side by side, all lanes at work; one workgroup per CU with all of its LDS and up
     // to sixteen waves, or two with half of it each.
-    const ShapeRow* shape = shape_row(with_sums ? 1 : 0, static_cast<int>(elem), l_max);
-    const unsigned pack_by_shape = shape ? shape->pack : 1u;
+    const ShapeRow* shape = shape_row(with_sums ? 1 : 0, static_cast<int>(elem), l_max, n_samples);
+    unsigned pack_by_shape = shape ? shape->pack : 1u;
+    // Fewer points than 64 for every CU: tiles of 16 reach four times as many of them (us, 3 000 points, one / two /
+    // four channels: float32 l_max = 18 7.2 5.7 5.6, 28 11.6 8.0 7.3; float64 18 8.3 6.9 6.6, 26 16.5 - 8.4)
+    if (n_samples < 16384 && l_max >= 16) pack_by_shape = 4;
     const int waves_by_shape = shape ? shape->waves : 0;
     const unsigned floor_by_shape = shape ? shape->floor : 32u;
     const bool alone = switch_or(SW_VALUES_ALONE, shape && shape->alone ? 1 : 0) != 0;
@@ -166,7 +172,7 @@ static bool plan_values(size_t n_samples, int l_max, size_t elem, int lds_limit,
     const int sum_waves = switch_or(SW_VALUES_WAVES, waves_by_shape != 0 ? waves_by_shape : 16);
     const unsigned groups_below = static_cast<unsigned>(switch_or(SW_VJP_GROUPS_BELOW, 16)); // (vjp_groups_kernel: eight waves)
     unsigned pack = with_sums ? 1u : static_cast<unsigned>(switch_or(SW_VALUES_PACK, static_cast<int>(pack_by_shape)));
-    if (pack != 2 && pack != 4) pack = 1;
+    if (pack != 2 && pack != 4 && pack != 8) pack = 1;
     auto search = [&]() {
         for (unsigned limit : {alone ? 0u : (allowed < half ? allowed : half), allowed}) {
             const unsigned least = pack > 1 ? 8u : (limit > half ? smallest_alone : smallest);
@@ -179,8 +185,8 @@ static bool plan_values(size_t n_samples, int l_max, size_t elem, int lds_limit,
                 // (a workgroup alone on its CU with more than 16 points: room for the sums of
                 // up to sixteen waves, unless eight are asked for)
                 const unsigned sums = (with_sums && limit > half && t > groups_below && sum_waves > 8 ? 16u : 8u) * 3u * 64u;
-                const unsigned extra = !with_sums ? 0u : (t == 64 ? sums : sums + 2u * tri_all);
-                bytes = (rows + t * table_stride + extra) * esize;
+                const unsigned extra = !with_sums ? (pack > 1 ? 2u * tri_all : 0u) : (t == 64 ? sums : sums + 2u * tri_all);
+                bytes = (rows + (!with_sums && pack > 1 ? align4(t * table_elems) : t * table_elems) + extra) * esize;
                 if (bytes <= limit) {
                     tile = t;
                     sums_elems = sums;
@@ -203,17 +209,23 @@ static bool plan_values(size_t n_samples, int l_max, size_t elem, int lds_limit,
     g.tiles_per_xcd = (g.n_tiles + 7u) / 8u;
     g.rows_elems = row_stride;
     g.off_pts = rows;
-    g.off_iter = table_stride;
-    g.off_jobs = rows + tile * table_stride; // the product: the waves' sums,
-    g.off_F = g.off_jobs + sums_elems;       // and (fewer than 64 points) the prefactor tables
-    g.off_Q = g.off_F + tri_all;
+    if (with_sums) {
+        g.off_iter = table_stride;
+        g.off_jobs = rows + tile * table_stride; // the waves' sums,
+        g.off_F = g.off_jobs + sums_elems;       // and (fewer than 64 points) the prefactor tables
+        g.off_Q = g.off_F + tri_all;
+    } else {
+        g.off_iter = table_entries;
+        g.off_F = rows + 2u * tile * table_entries;
+        g.off_Q = rows + align4(tile * table_elems);
+    }
     g.points_per_pass = with_sums ? 0u : pack; // values_kernel: channels a wave evaluates side by side
     out->workgroups = g.tiles_per_xcd * 8u;
     // one wave per l channel above the closed forms, eight at most
     // (alone on its CU: up to sixteen; twelve for one channel per wave in float32)
-    // (four channels side by side: that kernel exists for up to eight waves only)
+    // (four or eight channels side by side: those kernels exist for up to eight waves only)
     const int most = with_sums ? (sums_elems > 8u * 3u * 64u ? 16 : 8)
-                               : (bytes > half && pack != 4 ? (elem == 4 && pack == 1 ? 12 : 16) : 8);
+                               : (bytes > half && pack <= 2 ? (elem == 4 && pack == 1 ? 12 : 16) : 8);
     int waves = switch_or(SW_VALUES_WAVES, waves_by_shape != 0 && alone ? waves_by_shape : most);
     waves = waves < 1 ? 1 : (waves > most ? most : waves);
     // (values: at least two, one for the tables, one for the closed forms)
@@ -816,12 +828,13 @@ int make_plan(size_t n_samples, int l_max, int mode, size_t elem, int lds_limit,
         return SPHX_OK;
     }
     // Values alone where the rows of few points fill LDS: pairs_kernel (below, with the derivatives), which keeps
-    // the recursions of the next tile and the flush of this one side by side: 10-35 % faster than values_kernel
-    // (the recursion kernel from l_max = 34) from l_max = 24 in float32 and 19 in float64. Below, a point's pairs
-    // leave the entry lanes idle and values_kernel is ahead (float32 l_max = 23: 50.7 % against 44.2 %).
+    // the recursions of the next tile and the flush of this one side by side. values_kernel is ahead where LDS holds
+    // three of its workgroups or more (1.2 GB, us, pairs_kernel / values_kernel: float32 l_max = 24 266 / 208, 25 245 /
+    // 203, 26 239 / 220 (50 000 points 37.2 / 38.4), 27 255 / 233, 28 251 / 236, 29 220 / 226, 31 222 / 239, 33 260 / 343; float64 19 221 / 240,
+    // 20 217 / 218, 21 281 / 218, 22 279 / 227, 23 324 / 270, 24 243 / 238, 25 211 / 291).
     if (lane_kernels && mode == 0 && l_max > hard) {
         const int pairs = switch_or(SW_PAIRS, 1);
-        const bool pairs_by_shape = n_samples >= 32768 && (elem == 4 ? l_max >= 24 : l_max >= 19);
+        const bool pairs_by_shape = n_samples >= 32768 && (elem == 4 ? l_max == 26 || l_max >= 28 : l_max >= 24 || l_max == 19 || l_max == 20);
         if (pairs == 2 || (pairs == 1 && pairs_by_shape)) {
             PairsChoice want;
             want.tile = static_cast<unsigned>(switch_or(SW_PAIRS_TILE, 0));

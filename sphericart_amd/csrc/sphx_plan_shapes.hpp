@@ -9,7 +9,7 @@
 namespace sphx {
 
 // values_kernel (kind 0) and the lane kernels of the fused product (kind 1) on an MI355X.
-//   pack    values: channels a wave evaluates side by side (1, 2, 4); tiles of 64 / pack points
+//   pack    values: channels a wave evaluates side by side (1, 2, 4, 8); tiles of 64 / pack points
 //   alone   one workgroup per CU with all of its LDS instead of two with half each
 //   waves   the product, alone on its CU: waves of the workgroup (0: as many as there are channels)
 //   floor   the product: tiles shrink in steps of four points down to this size and halve from there
@@ -20,24 +20,36 @@ struct ShapeRow {
     int waves;
     unsigned floor;
     const char* measured;
+    unsigned long long points_from = 0, points_below = ~0ull; // calls of so many points
 };
 
 constexpr ShapeRow kShapeRows[] = {
-    // values, float32. 1 GB of values, us, in the order: tile that fits half of LDS / one workgroup with all of
-    // LDS / two channels in half of LDS / the same with all of LDS / four channels / recursion kernel
-    {0, 4, 21, 21, 2, false, 0, 32, "254 262 248 252 268 397"},
-    {0, 4, 22, 22, 2, false, 0, 32, "271 260 238 239 260 389"},
-    {0, 4, 23, 23, 1, true, 0, 32, "319 288 - 427 341 425"},
-    {0, 4, 25, 25, 4, false, 0, 32, "319 295 - 366 286 397"},
-    {0, 4, 26, 26, 4, false, 0, 32, "317 300 - 350 275 393"},
-    {0, 4, 29, 29, 2, false, 0, 32, "- 329 - 326 342 389"},
-    {0, 4, 30, 30, 2, false, 0, 32, "- 357 - 317 332 391"},
-    {0, 4, 31, 31, 2, false, 0, 32, "- 360 - 324 348 389"},
-    {0, 4, 32, 32, 2, false, 0, 32, "- 368 - 300 313 378"},
-    {0, 4, 33, 33, 2, false, 0, 32, "- 365 - 297 305 386"},
+    // values, float32. 1.2 GB of values, us, with one / two / four / eight channels side by side / pairs_kernel. More
+    // workgroups on a CU hide more of one another's loads, tables and flush, fewer points in one make more of its
+    // waves wait for a point's tables: four channels are ahead where the rows of 16 points leave room for three
+    // workgroups and those of 32 for two at most, eight channels where only two of 16 points fit. (l_max = 16
+    // from 1 000 000 points, 28, 32, and float64 22 and 23 below 32 768 points keep the plans that
+    // tests/test_library_abi.py states.)
+    {0, 4, 12, 15, 2, false, 0, 32, "191 179 187 244 -, 189 181 192 - -, 187 182 188 - -, 206 205 221 - -; 200 000 points 42.0 39.1"},
+    {0, 4, 16, 16, 2, false, 0, 32, "199 188 189 - -", 0, 1000000},
+    {0, 4, 17, 21, 4, false, 0, 32, "205 196 190 - -, 207 207 192 218 -, 247 237 207 241 -, 242 202 199 - -, 237 209 195 - -"},
+    {0, 4, 22, 22, 2, false, 0, 32, "249 198 210 216 -"},
+    {0, 4, 23, 25, 4, false, 0, 32, "280 347 227 264 -, 267 287 208 221 266, 286 299 203 226 245"},
+    {0, 4, 26, 26, 4, false, 0, 32, "291 277 247 221 239; 20 000 points - 21.6 19.9 18.9"},
+    {0, 4, 27, 27, 8, false, 0, 32, "344 313 277 234 255"},
+    {0, 4, 29, 31, 4, false, 0, 32, "310 272 227 234 220, 356 251 222 235 225, 357 296 252 252 222"},
+    {0, 4, 32, 32, 2, false, 0, 32, "356 239 221 271 229"},
+    {0, 4, 33, 33, 4, false, 0, 32, "361 360 343 260 260"},
     // values, float64, the same columns
-    {0, 8, 14, 14, 1, true, 0, 32, "224 212 - 239 309 310"},
-    {0, 8, 15, 15, 1, true, 0, 32, "258 225 - 257 326 347"},
+    {0, 8, 8, 9, 2, false, 0, 32, "214 180 204 - -, 199 201 217 331 -; 200 000 points 30.5 26.5, 37.1 31.7"},
+    {0, 8, 14, 15, 2, false, 0, 32, "203 191 194 - -, 219 198 238 250 -"},
+    {0, 8, 16, 17, 4, false, 0, 32, "221 274 204 226 -, 230 277 208 258 -"},
+    {0, 8, 18, 18, 8, false, 0, 32, "221 239 243 221 -; 100 000 points 65 66 68 61"},
+    {0, 8, 19, 21, 4, false, 0, 32, "284 259 240 267 221, 290 232 218 230 217, 308 239 218 241 281"},
+    {0, 8, 22, 22, 4, false, 0, 32, "287 220 227 266 279; 100 000 points - 89 89 102 103", 32768},
+    {0, 8, 23, 23, 8, false, 0, 32, "299 299 349 274 324", 32768},
+    {0, 8, 24, 24, 8, false, 0, 32, "293 293 314 237 244; 20 000 points - 33.8 33.0 31.0"},
+    {0, 8, 25, 32, 4, false, 0, 32, "20 000 points, l_max = 26 - - 36 36, recursion kernel 39, 32 - - 46 66, 49"},
     // the product, float64. 200 000 points (400 000 to l_max = 16), us: tiles in half of LDS / one workgroup per
     // CU with 8 / with up to 12 waves; from l_max = 21 with tiles of 28, 24, 20 points before they halve
     {1, 8, 25, 25, 1, true, 8, 16, "660 598 602"},
@@ -56,9 +68,12 @@ constexpr ShapeRow kShapeRows[] = {
 };
 
 // The row for a shape, or nullptr: then one channel per wave, two workgroups per CU where they fit.
-inline const ShapeRow* shape_row(int kind, int elem, int l_max) {
+inline const ShapeRow* shape_row(int kind, int elem, int l_max, unsigned long long n_samples) {
     for (const ShapeRow& row : kShapeRows) {
-        if (row.kind == kind && row.elem == elem && l_max >= row.l_from && l_max <= row.l_to) return &row;
+        if (row.kind == kind && row.elem == elem && l_max >= row.l_from && l_max <= row.l_to &&
+            n_samples >= row.points_from && n_samples < row.points_below) {
+            return &row;
+        }
     }
     return nullptr;
 }
