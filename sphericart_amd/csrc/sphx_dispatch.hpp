@@ -44,7 +44,7 @@ constexpr bool kLargeGroups =
     !VJP && (MODE <= 1 || (MODE == 2 && sizeof(T) == 4) || (MODE == 2 && SPLIT && (!NORM || LIST)));
 
 template <typename T, int MODE, bool NORM, bool WHOLE, bool SPLIT, bool VJP = false, bool LIST = false,
-          typename O = T, unsigned NT = kRecursionThreads, bool TOGETHER = false>
+          typename O = T, unsigned NT = kRecursionThreads, bool TOGETHER = false, int POINTS_L = 0>
 static hipError_t launch_recursion(const Launch& l, const typename AsGiven<O>::type* xyz,
                                    typename AsGiven<O>::type* sph, typename AsGiven<O>::type* dsph,
                                    typename AsGiven<O>::type* ddsph, hipStream_t stream) {
@@ -66,9 +66,27 @@ static hipError_t launch_recursion(const Launch& l, const typename AsGiven<O>::t
             return launch_recursion<T, MODE, NORM, WHOLE, SPLIT, VJP, LIST, O, NT, true>(l, xyz, sph, dsph, ddsph, stream);
         }
     }
+    if constexpr (MODE == 2 && NORM && sizeof(T) == 4 && LIST && !SPLIT && NT == 2 * kRecursionThreads && POINTS_L == 0) {
+        // the variants with one point per lane; for odd l_max, whose rows lie one element apart, only where every array starts at a multiple of 16 bytes
+        const bool aligned = ((reinterpret_cast<uintptr_t>(sph) | reinterpret_cast<uintptr_t>(dsph) |
+                               reinterpret_cast<uintptr_t>(ddsph)) & 15u) == 0;
+        if (l.g.point_lanes != 0 && (aligned || l.g.l_max % 2 == 0)) {
+            auto with = [&](auto l_max) {
+                return launch_recursion<T, MODE, NORM, WHOLE, SPLIT, VJP, LIST, O, NT, TOGETHER, decltype(l_max)::value>(
+                    l, xyz, sph, dsph, ddsph, stream);
+            };
+            switch (l.g.l_max) {
+            case 4: return with(std::integral_constant<int, 4>{});
+            case 5: return with(std::integral_constant<int, 5>{});
+            case 6: return with(std::integral_constant<int, 6>{});
+            case 7: return with(std::integral_constant<int, 7>{});
+            default: return hipErrorInvalidValue; // never planned
+            }
+        }
+    }
     if ((l.g.together != 0) != TOGETHER) return hipErrorInvalidValue; // never planned
     if (l.threads != NT) return hipErrorInvalidValue; // never planned
-    auto kernel = recursion_kernel<T, MODE, NORM, WHOLE, SPLIT, VJP, LIST, O, NT, TOGETHER>;
+    auto kernel = recursion_kernel<T, MODE, NORM, WHOLE, SPLIT, VJP, LIST, O, NT, TOGETHER, POINTS_L>;
     // The workgroups are persistent: launch exactly as many as are resident at once (registers
     // may allow fewer per CU than LDS does), or the last ones would run alone after the rest.
     unsigned workgroups = l.workgroups;

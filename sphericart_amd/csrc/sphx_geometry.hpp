@@ -30,8 +30,9 @@ struct Tiling {
     unsigned slice_waves;   // not 0: this many waves of their own (together: and wave 0) evaluate the closed
                             // forms of l <= 6 (whole rows); 0: the slices go round all waves
     unsigned together;      // recursion_kernel, float64: 1 = the recursions run next to the entries (TOGETHER)
-    unsigned row_pad;       // recursion_kernel, whole rows: elements left free after every staged row (0 or 16 bytes' worth)
+    unsigned row_pad;       // recursion_kernel, whole rows: elements left free after every staged row (0, 16 bytes' worth or, point_lanes, 0 or 1)
     unsigned magic_ny;      // ceil(2^32 / ny)
+    unsigned point_lanes;   // recursion_kernel, normalised second derivatives: one point per lane, a job for a whole wave
     unsigned priorities;    // recursion_kernel: 1 = the waves that flush run at raised priority, 2 = those that prepare the next tile
     // LDS carve-up, in elements of T: the staged rows come first, rows_elems of them, with the
     // gradient and second-derivative rows at off_dsph and off_ddsph inside a buffer; the other

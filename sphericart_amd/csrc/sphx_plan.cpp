@@ -25,7 +25,7 @@ static const char* const kSwitchNames[SW_COUNT] = {
     "SPHX_HESSIAN_LANES",
     "SPHX_HESSIAN_LANES_PARTS", "SPHX_HESSIAN_LANES_TILE", "SPHX_JOB_LIST",
     "SPHX_PAIRS", "SPHX_PAIRS_BATCH", "SPHX_PAIRS_CHUNK", "SPHX_PAIRS_PREP_WAVES", "SPHX_PAIRS_SEQUENCE_WAVES", "SPHX_PAIRS_TILE",
-    "SPHX_PREFIX_INSIDE", "SPHX_RECURSIONS_TOGETHER", "SPHX_ROW_PAD", "SPHX_SEQUENCE_WAVES", "SPHX_SLICE_WAVES", "SPHX_SPLIT_BELOW",
+    "SPHX_POINT_LANES", "SPHX_PREFIX_INSIDE", "SPHX_RECURSIONS_TOGETHER", "SPHX_ROW_PAD", "SPHX_SEQUENCE_WAVES", "SPHX_SLICE_WAVES", "SPHX_SPLIT_BELOW",
     "SPHX_SPLIT_RATIO", "SPHX_SPLIT_SIDES", "SPHX_SPREAD_KINDS", "SPHX_TILE", "SPHX_TILE_LDS_BUDGET", "SPHX_TILE_POW2",
     "SPHX_TILE_SMALL_N", "SPHX_VALUES_ALONE", "SPHX_VALUES_LDS", "SPHX_VALUES_MIN_TILE", "SPHX_VALUES_MIN_WAVES",
     "SPHX_VALUES_PACK", "SPHX_VALUES_TILE_STEP", "SPHX_VALUES_WAVES", "SPHX_VJP_GROUPS_BELOW", "SPHX_VJP_LANES", "SPHX_VJP_MIN_TILE", "SPHX_VJP_STEP_FLOOR", "SPHX_VJP_TILE_STEP", "SPHX_WAVE_PRIORITIES",
@@ -468,7 +468,18 @@ static bool plan_recursion(size_t n_samples, int l_max, int mode, bool whole, si
     // (whole rows a multiple of 64 bytes long, l_max = 3 mod 4, would all start on one LDS bank: 16 bytes are left
     // free after each, which the flush skips; recursion_kernel, row_pad. Not below l_max = 7, where a tile can be
     // shorter than the line its end is carried in.)
-    const unsigned row_pad = whole && l_max >= 7 && (ny * osize) % 64u == 0 && switch_or(SW_ROW_PAD, 1) != 0 ? 16u / osize : 0u;
+    // One point per lane and a job for a whole wave (the POINTS_L variants of recursion_kernel, their rows an odd number
+    // of elements apart): normalised second derivatives in float32 at l_max = 4-7, where the rows of 38 to 64 points fit
+    // and the vector units are what a tile waits for. us, list of jobs / this, 20 000, 100 000 and 500 000 points: l_max = 4
+    // 14.4 / 12.5, 35.0 / 31.4, 134 / 118; 5 17.7 / 15.4, 46.8 / 43.3, 187 / 169 (177 / 183 on another box); 6 20.2 / 18.3,
+    // 60.8 / 55.2, 266 / 235; 7 29.4 / 25.8, 84 / 72, 367 / 330; 8, with 35 of 64 lanes at work, 27.7 / 30.1, 87 / 97,
+    // 395 / 415. Solid harmonics, whose jobs are mostly stores, gain below 100 000 points and lose beyond (500 000,
+    // l_max = 4-7: 111 / 128, 160 / 181, 222 / 241, 283 / 313). Fewer points than 64 for every CU leave lanes idle.
+    const bool point_lanes = mode == 2 && whole && elem == 4 && osize == 4 && normalized && threads > kRecursionThreads &&
+                             l_max >= 4 && l_max <= 7 && switch_or(SW_JOB_LIST, 2) == 2 &&
+                             switch_or(SW_POINT_LANES, n_samples >= 16384 ? 1 : 0) != 0;
+    const unsigned row_pad = point_lanes ? 1u - ny % 2u
+                             : whole && l_max >= 7 && (ny * osize) % 64u == 0 && switch_or(SW_ROW_PAD, 1) != 0 ? 16u / osize : 0u;
     const unsigned row_stride = nrow + (whole ? row_pad : nyh % (16u / osize));
     g.row_pad = row_pad;
     g.magic_ny = magic_of(ny);
@@ -683,6 +694,8 @@ static bool plan_recursion(size_t n_samples, int l_max, int mode, bool whole, si
     if (must_list || want_list == 2 || (want_list == 1 && saves_a_round) || (want_list < 0 && by_shape)) {
         g.points_per_pass = 0;
     }
+    g.point_lanes = point_lanes && !*split_sides && g.points_per_pass == 0 ? 1u : 0u;
+    if (point_lanes && g.point_lanes == 0) g.row_pad = 0; // (not the list after all: its rows lie back to back)
 
     // in front of every staging region, room for the part of a 128-byte line that precedes the
     // tile's run (recursion_kernel, flush_run)
@@ -1043,6 +1056,7 @@ std::string describe(const Plan& plan, int l_max, int mode, bool is_f64, bool no
         text += "recursion_kernel<" + head + ", " + (plan.whole ? "true" : "false") + ", " +
                 (plan.split_sides ? "true" : "false") + ", false, " +
                 (plan.rec.g.points_per_pass == 0 ? "true" : "false") + ">" + geometry(plan.rec) +
+                (plan.rec.g.point_lanes != 0 ? " (one point per lane)" : "") +
                 (plan.rec.g.together != 0 ? " (recursions next to the entries)" : "") +
                 ((plan.rec.g.priorities & 1u) != 0 ? " (flush at raised priority)" : "");
     }

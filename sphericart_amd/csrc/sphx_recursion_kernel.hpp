@@ -76,13 +76,14 @@ namespace sphx {
 // rows are rows of O, so a tile holds as many points as in the float kernel's and the flush is
 // that kernel's.
 template <typename T, int MODE, bool NORM, bool WHOLE, bool SPLIT, bool VJP = false, bool LIST = false,
-          typename O = T, unsigned NT = kRecursionThreads, bool TOGETHER = false>
+          typename O = T, unsigned NT = kRecursionThreads, bool TOGETHER = false, int POINTS_L = 0>
 __global__ __launch_bounds__(NT, MODE < 2 ? 4 : 1) void recursion_kernel(Tiling g, const O* __restrict__ xyz,
                                                                      O* __restrict__ sph,
                                                                      O* __restrict__ dsph,
                                                                      O* __restrict__ ddsph) {
     static_assert(!VJP || (MODE == 1 && !SPLIT), "the fused product is built on the gradient kernel");
     static_assert(!VJP || std::is_same<T, O>::value, "the fused product stages what it computes");
+    static_assert(POINTS_L == 0 || (LIST && MODE == 2 && WHOLE && !SPLIT && sizeof(O) == 4), "one point per lane");
     static_assert(!TOGETHER || sizeof(T) == 8, "float32 has the recursions in the flush only");
     constexpr int H = MODE == 2 ? 1 : 6;
     constexpr unsigned NYH = (H + 1) * (H + 1);
@@ -93,9 +94,9 @@ __global__ __launch_bounds__(NT, MODE < 2 ? 4 : 1) void recursion_kernel(Tiling 
     const unsigned tid = threadIdx.x;
     const unsigned lane = tid & 63u;
     const unsigned wave = __builtin_amdgcn_readfirstlane(tid >> 6); // the same for all lanes: scalar
-    const int L = g.l_max;
+    const int L = POINTS_L != 0 ? POINTS_L : g.l_max;
     const unsigned S = g.tile;
-    const unsigned ny = g.ny;
+    const unsigned ny = POINTS_L != 0 ? (POINTS_L + 1) * (POINTS_L + 1) : g.ny;
     const unsigned nrow = WHOLE ? ny : ny - NYH; // staged elements per component row
     const unsigned skip = WHOLE ? 0u : NYH;      // first staged entry of a row
     // Distance between staged rows. WHOLE == false: the rows are ny apart in HBM but only nrow
@@ -109,9 +110,12 @@ __global__ __launch_bounds__(NT, MODE < 2 ? 4 : 1) void recursion_kernel(Tiling 
     // and 12). The host then asks for 16 bytes between the staged rows, g.row_pad elements; the flush skips them
     // (flush_run). They keep a row's 16-byte vectors whole only where the arrays start at multiples of 16 bytes:
     // for other pointers the rows stay back to back.
+    // POINTS_L: rows an odd number of elements apart, so that the lanes of a wave, which store the same entry of their
+    // points, spread over all banks (the arrays then start at multiples of 16 bytes).
     const unsigned row_pad =
-        WHOLE && !VJP && ((reinterpret_cast<uintptr_t>(sph) | reinterpret_cast<uintptr_t>(dsph) |
-                           reinterpret_cast<uintptr_t>(ddsph)) & 15u) == 0
+        POINTS_L != 0 ? static_cast<unsigned>(POINTS_L % 2)
+        : WHOLE && !VJP && ((reinterpret_cast<uintptr_t>(sph) | reinterpret_cast<uintptr_t>(dsph) |
+                             reinterpret_cast<uintptr_t>(ddsph)) & 15u) == 0
             ? g.row_pad
             : 0u;
     const unsigned row_stride = WHOLE ? nrow + row_pad : nrow + skip % W16;
@@ -407,6 +411,20 @@ __global__ __launch_bounds__(NT, MODE < 2 ? 4 : 1) void recursion_kernel(Tiling 
         }
     };
 
+    // one point per lane: the jobs of this wave
+    [[maybe_unused]] unsigned jobs_from = 0, jobs_to = 0;
+    if constexpr (POINTS_L != 0) {
+        const unsigned zeros = g.kind_jobs[2], others = g.jobs_per_point - zeros;
+        const unsigned all = 2u * others + zeros;
+        const unsigned share = entry_end_wave - entry_first_wave;
+        auto begins = [&](unsigned who) -> unsigned { // the first job that begins at or after who / share of the work
+            const unsigned at = (who * all + share - 1u) / share;
+            return at <= 2u * others ? (at + 1u) / 2u : others + (at - 2u * others);
+        };
+        jobs_from = __builtin_amdgcn_readfirstlane(begins(wave - entry_first_wave));
+        jobs_to = __builtin_amdgcn_readfirstlane(begins(wave - entry_first_wave + 1u));
+    }
+
     // the entries of tile n (the entry waves)
     auto entry_stage = [&](unsigned n) {
         const unsigned valid = valid_in(n);
@@ -445,8 +463,7 @@ __global__ __launch_bounds__(NT, MODE < 2 ? 4 : 1) void recursion_kernel(Tiling 
             rows.dsph = staged + g.off_dsph + phase_dsph + s * 3 * row_stride - skip;
             rows.ddsph = staged + g.off_ddsph + phase_ddsph + s * 9 * row_stride - skip;
         };
-        auto take_job = [&](unsigned e) {
-            const unsigned packed = job_table[e];
+        auto take_job = [&](unsigned packed) {
             if constexpr (!LIST && !SPLIT) {
                 if (packed == kNoJob) return;
             }
@@ -467,6 +484,17 @@ __global__ __launch_bounds__(NT, MODE < 2 ? 4 : 1) void recursion_kernel(Tiling 
             // points, |m| = l - 1, m = 0) and by point within a kind, so that the lanes of a wave
             // share a branch of entry_job except where two kinds meet: three places per tile
             // instead of three per point.
+            if constexpr (POINTS_L != 0) {
+                // One point per lane and a job for a whole wave, l_max a constant: the job, its l and m are scalar and
+                // the offsets of its 26 staged numbers from six addresses are part of the instructions, which takes
+                // most of the 100 integer instructions out of the 350 of a job. In list order each wave takes the jobs
+                // that begin in its share of the work.
+                if (lane < valid) {
+                    take_point(lane);
+                    for (unsigned e = jobs_from; e < jobs_to; ++e) take_job(__builtin_amdgcn_readfirstlane(job_table[e]));
+                }
+                return;
+            }
             const unsigned total = valid * per_point;
             if constexpr (MODE == 0) {
                 // values: an entry is three multiplications, the order by kind does not pay
@@ -478,7 +506,7 @@ __global__ __launch_bounds__(NT, MODE < 2 ? 4 : 1) void recursion_kernel(Tiling 
                         current = s;
                         take_point(s);
                     }
-                    take_job(q - s * per_point);
+                    take_job(job_table[q - s * per_point]);
                 }
                 return;
             }
@@ -510,7 +538,7 @@ __global__ __launch_bounds__(NT, MODE < 2 ? 4 : 1) void recursion_kernel(Tiling 
                     current = s;
                     take_point(s);
                 }
-                take_job(first_job + (r - s * b));
+                take_job(job_table[first_job + (r - s * b)]);
             }
         } else {
             // One pass takes the jobs of as many points as fit side by side in the wide lanes
@@ -525,7 +553,7 @@ __global__ __launch_bounds__(NT, MODE < 2 ? 4 : 1) void recursion_kernel(Tiling 
                 const unsigned s = s0 + local;
                 if (s >= valid || local >= g.points_per_pass) continue;
                 take_point(s);
-                for (unsigned e = e_first; e < per_point; e += wide_lanes) take_job(e);
+                for (unsigned e = e_first; e < per_point; e += wide_lanes) take_job(job_table[e]);
             }
         }
     };
@@ -567,8 +595,16 @@ __global__ __launch_bounds__(NT, MODE < 2 ? 4 : 1) void recursion_kernel(Tiling 
                     V* out = reinterpret_cast<V*>(line0 + full_lo);
                     // (two or four loads in flight per lane ahead of their stores: no faster on any shape)
                     for (unsigned v = ft; v < nvec; v += count) {
-                        emit<O, SPHX_STREAMING_STORES>(*reinterpret_cast<const V*>(region + staged_at(full_lo + v * W)),
-                                                       out + v);
+                        if constexpr (POINTS_L % 2 != 0) { // (a vector lies inside one row)
+                            const O* from = region + staged_at(full_lo + v * W);
+                            V hold;
+#pragma unroll
+                            for (unsigned k = 0; k < W; ++k) hold[k] = from[k];
+                            emit<O, SPHX_STREAMING_STORES>(hold, out + v);
+                        } else {
+                            emit<O, SPHX_STREAMING_STORES>(*reinterpret_cast<const V*>(region + staged_at(full_lo + v * W)),
+                                                           out + v);
+                        }
                     }
                     tail_from = full_hi;
                 } else {
