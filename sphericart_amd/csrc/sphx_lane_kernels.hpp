@@ -21,9 +21,9 @@ namespace sphx {
 // surrounds them. With one point per lane m is the same for the whole wave: no
 // job has to be decoded and no iterate passes through LDS. A step down in m is
 // two LDS reads (c_m and s_m; 2(m+1)z), seven operations and two LDS writes.
-// What a step reads is fetched four steps ahead into registers, so that no
-// step waits for LDS, and four steps share the address arithmetic. The
-// prefactors of a channel, m = 0..l, are loaded once, one per lane, and a step
+// What a step reads is fetched ahead into registers, one step or (K > 1, below)
+// four that also share the address arithmetic, so that no step waits for LDS.
+// The prefactors of a channel, m = 0..l, are loaded once, one per lane, and a step
 // takes each from its lane (v_readlane).
 //
 // The rows of 64 points take most of a CU's LDS from l_max of about 12 on, and
@@ -192,7 +192,9 @@ __global__ __launch_bounds__(NT) void values_kernel(Tiling g, const T* __restric
         // its l is not used (the prefactors it reads then are those of the next l, still inside the table). K + 1
         // steps until that holds for the shortest channel, or down to m = 1 (K = 8, l0 = 7 and 8: the step at m = 0
         // comes last, below).
-        constexpr int U = 4, TOP = static_cast<int>(K) + 1;
+        // (K = 1: one step ahead. Larger tiles, whose workgroups leave less LDS for others to run in, were level or slower
+        // with four: 1 027 397 points at l_max = 16, solid, in float32 213 us with four, 200 with one)
+        constexpr int U = K == 1 ? 1 : 4, TOP = static_cast<int>(K) + 1;
         const int top = K > H && l0 < TOP ? l0 : TOP;
         constexpr bool EARLY = K <= 4; // (eight channels: too many registers)
         Step first_steps[TOP], ahead[U];
