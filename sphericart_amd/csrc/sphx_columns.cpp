@@ -8,35 +8,31 @@
 
 namespace sphx {
 
-// Q_l^m = S_{l,m} q_l^m with the leading coefficient of q in z equal to one: S = (-1)^m (2l-1)!! / (l-m)!, zero for
-// m > l. In float32 the prefactors F are used as they are in the tables of the forward kernels, their underflow from
-// l = 19 on included, so that both describe the same functions.
+// Q_l^m at the pole is (-1)^m (l+m)! / (2^m m! (l-m)!), zero for m > l; e_n and g_n (sphx_columns_kernel.hpp) are
+// there -(n-1)/(2m+2) and (n-2)(n-3)/((2m+2)(2m+4)), n = l - m. In float32 the prefactors F are used as they are in the
+// tables of the forward kernels, their underflow from l = 19 on included, so that both describe the same functions.
 template <typename T> std::vector<T> column_table_of(const T* F) {
-    auto scale = [](int l, int m) -> long double {
+    auto pole = [](int l, int m) -> long double {
         if (m > l || l < 0) return 0.0L;
-        long double s = (m & 1) ? -1.0L : 1.0L;
-        for (int k = 1; k <= l; ++k) s *= 2 * k - 1;
-        for (int k = 2; k <= l - m; ++k) s /= k;
-        return s;
-    };
-    auto b = [](int l, int m) -> long double {
-        if (l < m + 2) return 0.0L;
-        return -static_cast<long double>(l + m - 1) * (l - m - 1) / (static_cast<long double>(2 * l - 1) * (2 * l - 3));
+        long double q = (m & 1) ? -1.0L : 1.0L;
+        for (int k = l - m + 1; k <= l + m; ++k) q *= k;
+        for (int k = 1; k <= m; ++k) q /= 2 * k;
+        return q;
     };
     std::vector<T> table(static_cast<size_t>(kColumnEntries) * kColumnEntry);
     for (int m = 0; m <= kColumnsLMax; ++m) {
         for (int l = m; l <= kColumnsLMax; ++l) {
             T* t = table.data() + static_cast<size_t>(column_start(m) + l - m) * kColumnEntry;
-            const long double f = F[l * (l + 1) / 2 + m], lm = l + m;
-            t[0] = static_cast<T>(b(l, m));
-            t[1] = static_cast<T>(b(l - 1, m + 1));
-            t[2] = static_cast<T>(f * scale(l, m));
-            t[3] = static_cast<T>(f * scale(l - 1, m + 1));
-            t[4] = static_cast<T>(f * lm * scale(l - 1, m));
-            t[5] = static_cast<T>(b(l - 2, m + 2));
-            t[6] = static_cast<T>(f * scale(l - 2, m + 2));
-            t[7] = static_cast<T>(f * lm * scale(l - 2, m + 1));
-            t[8] = static_cast<T>(f * lm * (lm - 1) * scale(l - 2, m));
+            const int n = l - m;
+            const long double f = F[l * (l + 1) / 2 + m], lm = l + m, w = 2 * m + 2;
+            t[0] = n < 2 ? T(0) : static_cast<T>((n - 1) / lm);
+            t[1] = n < 3 ? T(0) : static_cast<T>((n - 2) / lm);
+            t[2] = static_cast<T>(f * pole(l, m));
+            t[3] = n < 2 ? T(0) : static_cast<T>(-f * pole(l - 1, m + 1) * w / (n - 1));
+            t[4] = static_cast<T>(f * lm * pole(l - 1, m));
+            t[5] = n < 4 ? T(0) : static_cast<T>(f * pole(l - 2, m + 2) * w * (w + 2) / ((n - 2) * (n - 3)));
+            t[6] = n < 3 ? T(0) : static_cast<T>(-f * lm * pole(l - 2, m + 1) * w / (n - 2));
+            t[7] = static_cast<T>(f * lm * (lm - 1) * pole(l - 2, m));
         }
     }
     return table;

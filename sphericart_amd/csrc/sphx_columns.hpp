@@ -11,8 +11,8 @@ namespace sphx {
 // the range of the type at l = 28, in float64 the rows of 32 points no longer fit LDS from l_max = 25 on.
 constexpr int kColumnsLMax = 27;
 constexpr int kColumnEntries = (kColumnsLMax + 1) * (kColumnsLMax + 2) / 2;
-// numbers per entry (l, m): b_{l,m}, b_{l-1,m+1}, the factors of A, B, C, then b_{l-2,m+2} and the factors of E, G, K
-constexpr int kColumnEntry = 9;
+// numbers per entry (l, m): the factors of e_n and g_n, those of the sums A, B, C, then E, G, K
+constexpr int kColumnEntry = 8;
 // column m lists l = m .. kColumnsLMax one after the other
 constexpr int column_start(int m) { return m * (kColumnsLMax + 1) - m * (m - 1) / 2; }
 

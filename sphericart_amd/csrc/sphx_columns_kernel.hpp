@@ -29,14 +29,20 @@ namespace sphx {
 // twelve (second derivatives) multiply-adds per pair of entries instead of 30 or 250 operations. The chain rule of
 // the normalised harmonics is linear too and is applied once per point. Second derivatives never exist as numbers.
 //
-// Q runs upward in l at fixed m, one three-term recursion with the leading coefficient taken out,
+// Q runs upward in l at fixed m. With q_n the iterate at l = m + n over its value at the pole (x = y = 0, z = 1) and
+// rho^2 = x^2 + y^2, the recursion of the Gegenbauer polynomials reads
 //
-//   q_l = z q_{l-1} + b_{l,m} r^2 q_{l-2},   b = -(l+m-1)(l-m-1) / ((2l-1)(2l-3)),
+//   e_n = (n-1)/(n+2m) (z e_{n-1} - q_{n-2})     q_n = z q_{n-1} + rho^2 e_n     g_n = (n-2)/(n+2m) (z g_{n-1} - e_{n-2})
 //
-// whose scale is folded into the prefactors on the host (sphx_columns.cpp): |q| <= 1 on the unit sphere. m is the
-// same for all lanes of a wave, so b and the prefactors come from the scalar unit. Neighbouring columns m + 1 and
-// m + 2 run along (Q_{l-1}^{m+1}, Q_{l-2}^{m+2}): three or six operations, less than what reading every weight a
-// second and third time from LDS would take.
+// and e_n, g_n are, but for factors, the neighbouring columns Q_{l-1}^{m+1} and Q_{l-2}^{m+2} that the sums ask for
+// anyway: four or six operations per step for all of them, and no weight is read a second time from LDS. Near the axis
+// a recursion in z alone has a double root and collects its roundings l^2 times over; rho^2 is a factor of its own
+// here, as in the recursion in m of the forward kernels. Error against float64 over that of the float32 arrays
+// contracted in float32, root mean square over 1 500 points, normalised, l_max = 8-17: the vector-Jacobian product
+// 0.69-0.83 within a tenth of a radian of the axis and 0.79-0.93 anywhere, the second-order products 0.71-0.92 and
+// 0.80-0.96 (q_l = z q_{l-1} + b r^2 q_{l-2} with r^2 = 1: 1.4-2.8 and 0.96-1.23). The values at the pole are folded
+// into the prefactors on the host (sphx_columns.cpp): |q| <= 1 on the unit sphere. m is the same for all lanes of a
+// wave, so the table comes from the scalar unit.
 //
 // The products are sums in another order than the entries' own, with fused multiply-adds: they agree with the
 // contraction of the derivative arrays to rounding.
@@ -54,50 +60,41 @@ template <> __device__ __forceinline__ const double* column_table<double>() { re
 // Walks l = m .. L of column m and hands visit(step, l, FA, FB, FC, FE, FG, FK) the products of the prefactors with
 // the six Q above. `step` is l - m as a compile-time number while that is below 5 and 5 from there on: what is zero
 // or one by construction in the first steps takes no instruction (FB is meaningful from step 2 on, FC 1, FE 4, FG 3,
-// FK 2).
-template <typename T, bool NORM, bool SECOND, typename Visit>
-__device__ __forceinline__ void walk_column(int m, int L, T z, T r2, Visit&& visit) {
+// FK 2). rho2 = x^2 + y^2.
+template <typename T, bool SECOND, typename Visit>
+__device__ __forceinline__ void walk_column(int m, int L, T z, T rho2, Visit&& visit) {
     const T* t = column_table<T>() + column_start(m) * kColumnEntry;
-    T a1 = 0, a2 = 0, b1 = 0, b2 = 0, e1 = 0, e2 = 0;
-    auto advance = [&](T factor, T v1, T v2) { // on the unit sphere r^2 = 1
-        return fma_of(NORM ? factor : factor * r2, v2, z * v1);
-    };
+    T q1 = 0, q2 = 0, e1 = 0, e2 = 0, g1 = 0;
     auto one = [&](auto step, int l) {
         constexpr int S = decltype(step)::value;
         const T* k = t;
         t += kColumnEntry;
-        T a, b = 0, e = 0;
-        if constexpr (S == 0) a = 1;
-        else if constexpr (S == 1) a = z;
-        else a = advance(k[0], a1, a2);
-        if constexpr (S == 2) b = 1;
-        else if constexpr (S == 3) b = z;
-        else if constexpr (S >= 4) b = advance(k[1], b1, b2);
+        T q = 1, e = 0, g = 0;
+        if constexpr (S == 2) e = -k[0];
+        else if constexpr (S >= 3) e = k[0] * fma_of(z, e1, -q2);
         if constexpr (SECOND) {
-            if constexpr (S == 4) e = 1;
-            else if constexpr (S >= 5) e = advance(k[5], e1, e2);
+            if constexpr (S == 4) g = -k[1] * e2;
+            else if constexpr (S >= 5) g = k[1] * fma_of(z, g1, -e2);
         }
+        if constexpr (S == 1) q = z;
+        else if constexpr (S >= 2) q = fma_of(rho2, e, z * q1);
         T fa = k[2], fb = 0, fc = 0, fe = 0, fg = 0, fk = 0;
-        if constexpr (S >= 1) fa *= a;
+        if constexpr (S >= 1) fa *= q;
         if constexpr (S >= 1) fc = k[4];
-        if constexpr (S >= 2) fc *= a1;
-        if constexpr (S >= 2) fb = k[3];
-        if constexpr (S >= 3) fb *= b;
+        if constexpr (S >= 2) fc *= q1;
+        if constexpr (S >= 2) fb = k[3] * e;
         if constexpr (SECOND) {
-            if constexpr (S >= 2) fk = k[8];
-            if constexpr (S >= 3) fk *= a2;
-            if constexpr (S >= 3) fg = k[7];
-            if constexpr (S >= 4) fg *= b1;
-            if constexpr (S >= 4) fe = k[6];
-            if constexpr (S >= 5) fe *= e;
+            if constexpr (S >= 2) fk = k[7];
+            if constexpr (S >= 3) fk *= q2;
+            if constexpr (S >= 3) fg = k[6] * e1;
+            if constexpr (S >= 4) fe = k[5] * g;
         }
         visit(step, l, fa, fb, fc, fe, fg, fk);
-        a2 = a1;
-        a1 = a;
-        b2 = b1;
-        b1 = b;
+        q2 = q1;
+        q1 = q;
         e2 = e1;
         e1 = e;
+        g1 = g;
     };
     using std::integral_constant;
     one(integral_constant<int, 0>{}, m);
@@ -304,7 +301,7 @@ __global__ __launch_bounds__(kColumnsThreads) void columns_kernel(Columns g, con
             gz = fma_of(-along, p.z, gz);
         }
     }
-    const T r2 = NORM ? T(1) : p.x2 + p.y2 + p.z2;
+    const T rho2 = p.x2 + p.y2;
     // the direction of dw, the chain rule's 1/r included
     const T scale = NORM ? p.ir : T(1);
     const T dx = gx * scale, dy = gy * scale, dz = gz * scale;
@@ -326,7 +323,7 @@ __global__ __launch_bounds__(kColumnsThreads) void columns_kernel(Columns g, con
                 along_plus = fm * fma_of(dx, azimuth.c1, -(dy * azimuth.s1));
                 along_minus = fm * fma_of(dx, azimuth.s1, dy * azimuth.c1);
             }
-            walk_column<T, NORM, SECOND>(m, L, p.z, r2, [&](auto step, int l, T fa, T fb, T fc, T fe, T fg, T fk) {
+            walk_column<T, SECOND>(m, L, p.z, rho2, [&](auto step, int l, T fa, T fb, T fc, T fe, T fg, T fk) {
                 constexpr int S = decltype(step)::value;
                 T* mid = row + l * (l + 1);
                 const T wp = mid[m], wn = mid[-m];
@@ -351,7 +348,7 @@ __global__ __launch_bounds__(kColumnsThreads) void columns_kernel(Columns g, con
             const T along_u = SECOND ? fm * fma_of(dx, u1, dy * w1) : T(0);
             const bool writes = m > 0 || !minus; // (m = 0 is one entry)
             T* at = row + (minus ? -m : m);
-            walk_column<T, NORM, SECOND>(m, L, p.z, r2, [&](auto step, int l, T fa, T fb, T fc, T fe, T fg, T fk) {
+            walk_column<T, SECOND>(m, L, p.z, rho2, [&](auto step, int l, T fa, T fb, T fc, T fe, T fg, T fk) {
                 constexpr int S = decltype(step)::value;
                 T* here = at + l * (l + 1);
                 k.template add<S, SECOND>(*here, fa, fb, fc, fe, fg, fk);
@@ -489,7 +486,7 @@ __global__ __launch_bounds__(kColumnsThreads) void column_rows_kernel(Columns g,
     }
     const unsigned long long mine = first + (point < valid ? point : 0u);
     const Point<T> p = load_point<T, NORM>(xyz + mine * 3);
-    const T r2 = NORM ? T(1) : p.x2 + p.y2 + p.z2;
+    const T rho2 = p.x2 + p.y2;
     // set 0 = v_a - n_a s with a = x or z; set 1 = v_y - y s or w r - s
     const T n0 = second_half ? p.z : p.x, n1 = second_half ? T(1) : p.y;
     const T scale1 = second_half && NORM ? 1 / p.ir : T(1);
@@ -516,7 +513,7 @@ __global__ __launch_bounds__(kColumnsThreads) void column_rows_kernel(Columns g,
         const T* at1 = second_half ? w_at : v_at + ny;
         ColumnSums<T> k0, k1;
         T le0 = 0, le1 = 0;
-        walk_column<T, NORM, true>(m, L, p.z, r2, [&](auto step, int l, T fa, T fb, T fc, T fe, T fg, T fk) {
+        walk_column<T, true>(m, L, p.z, rho2, [&](auto step, int l, T fa, T fb, T fc, T fe, T fg, T fk) {
             constexpr int S = decltype(step)::value;
             const int at = l * (l + 1);
             T set0, set1;
