@@ -101,8 +101,10 @@ SPHX_EXPORT int sphx_backward_second_f64(const double* ddsph, const double* dsph
  * without dsph ever reaching memory: reads xyz and sph_grad, writes xyz_grad.
  * For l_max <= 6 the sum runs over k in index order, one rounding per
  * operation: the numbers are those of sphx_forward_* followed by a sequential
- * contraction. Beyond that the terms are added in another order (lanes, then a
- * butterfly), so the result agrees with that combination to rounding only.
+ * contraction. Beyond that the terms are added in another order (columns of one
+ * m, or lanes and a butterfly), so the result agrees with that combination to
+ * rounding only; where a weight is infinite or NaN, or a sum overflows on the
+ * way, a component is what the entries' own terms add up to.
  * No counterpart in the reference, whose torch binding recomputes dsph in
  * memory for its backward pass
  * (sphericart-torch/python/sphericart/torch/register.py:96-103). */
@@ -128,7 +130,8 @@ SPHX_EXPORT int sphx_vjp_f64(const double* xyz, const double* sph_grad, size_t n
  *
  * reads xyz, sph_grad (NULL: no such term) and dsph_grad [n_samples][3][n_total], writes xyz_grad.
  *
- * Enqueued on `stream`; n_samples == 0 returns SPHX_OK. Both agree with the contraction of the arrays to rounding.
+ * Enqueued on `stream`; n_samples == 0 returns SPHX_OK. Both agree with the contraction of the arrays to rounding, and
+ * term by term where a weight is not finite. The outputs may not overlap the inputs.
  * Where the rows of a tile of points do not fit LDS they return SPHX_ERR_UNSUPPORTED and enqueue nothing (the first
  * takes l_max up to 27 in float32 and 24 in float64, the second 24 and 16): such callers have sphx_forward_* and
  * sphx_backward_second_*. */

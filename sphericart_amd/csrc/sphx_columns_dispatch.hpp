@@ -27,14 +27,15 @@ hipError_t dispatch_columns(ColumnsKind kind, const ColumnsLaunch& l, bool norma
                           : launch_columns(column_rows_kernel<T, false>, l, s, xyz, sph_grad, upstream, xyz_grad);
     }
     auto go = [&](auto kernel) { return launch_columns(kernel, l, s, xyz, sph_grad, upstream, xyz_grad, sph_grad_grad); };
-    auto by_lanes = [&](auto second) {
-        constexpr bool SECOND = decltype(second)::value;
+    auto by_lanes = [&](auto second, auto add) {
+        constexpr bool SECOND = decltype(second)::value, ADD = decltype(add)::value;
         if (l.groups == 2) {
-            return normalized ? go(columns_kernel<T, true, SECOND, 2>) : go(columns_kernel<T, false, SECOND, 2>);
+            return normalized ? go(columns_kernel<T, true, SECOND, 2, ADD>) : go(columns_kernel<T, false, SECOND, 2, ADD>);
         }
-        return normalized ? go(columns_kernel<T, true, SECOND, 1>) : go(columns_kernel<T, false, SECOND, 1>);
+        return normalized ? go(columns_kernel<T, true, SECOND, 1, ADD>) : go(columns_kernel<T, false, SECOND, 1, ADD>);
     };
-    return kind == COLUMNS_VJP ? by_lanes(std::false_type{}) : by_lanes(std::true_type{});
+    if (kind == COLUMNS_VJP_BACKWARD) return by_lanes(std::true_type{}, std::false_type{});
+    return l.g.accumulate != 0 ? by_lanes(std::false_type{}, std::true_type{}) : by_lanes(std::false_type{}, std::false_type{});
 }
 
 template <typename T> hipError_t upload_column_tables(const HostTables& t) {

@@ -183,6 +183,109 @@ template <typename T, bool SECOND> struct PointSums {
     __device__ __forceinline__ T zz() const { return Ku; }
 };
 
+// ---------------------------------------------------------------------------
+// One entry at a time, for points whose sums are not finite: an infinite weight (or one so large that a sum over a
+// column overflows) makes the sums of its column infinite, and what is then multiplied by s_0 = 0 or projected on the
+// tangent plane a NaN in all components. Entry by entry such a point gets what contracting the arrays gives: an infinite
+// number where the entry's derivative is not zero, and a NaN where it is. The test costs a call 0.05 to 0.1 us (the product
+// in small calls 1-2 %; with the entries' part in front of the stores, or with the registers it would like, 3-4 %).
+// ---------------------------------------------------------------------------
+template <typename T, bool NORM, bool SECOND> struct EntryDerivatives {
+    T d[3];    // gradient
+    T h[3][3]; // second derivatives
+
+    // (the chain rule of the normalised harmonics, templates.hpp:572-613, product by product as the arrays have it)
+    __device__ __forceinline__ EntryDerivatives(const PointSums<T, SECOND>& one, const Point<T>& p) {
+        d[0] = one.gx(p.x);
+        d[1] = one.gy(p.y);
+        d[2] = one.gz();
+        if constexpr (SECOND) {
+            h[0][0] = one.xx(p.x);
+            h[1][1] = one.yy(p.y);
+            h[2][2] = one.zz();
+            h[0][1] = h[1][0] = one.xy(p.x, p.y);
+            h[0][2] = h[2][0] = one.xz(p.x);
+            h[1][2] = h[2][1] = one.yz(p.y);
+        }
+        if constexpr (NORM) {
+            const T n[3] = {p.x, p.y, p.z};
+            const T along = d[0] * n[0] + d[1] * n[1] + d[2] * n[2];
+            if constexpr (SECOND) {
+                T hn[3];
+#pragma unroll
+                for (int a = 0; a < 3; ++a) hn[a] = n[0] * h[a][0] + n[1] * h[a][1] + n[2] * h[a][2];
+                const T nhn = n[0] * hn[0] + n[1] * hn[1] + n[2] * hn[2];
+                const T irsq = p.ir * p.ir;
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+#pragma unroll
+                    for (int b = a; b < 3; ++b) {
+                        const T both = n[a] * n[b];
+                        T of = h[a][b] - n[a] * (hn[b] + d[b]) - n[b] * (hn[a] + d[a]) + both * (3 * along + nhn);
+                        if (a == b) of -= along;
+                        h[a][b] = h[b][a] = of * irsq;
+                    }
+                }
+            }
+#pragma unroll
+            for (int a = 0; a < 3; ++a) d[a] = (d[a] - n[a] * along) * p.ir;
+        }
+    }
+};
+
+// visit(k, derivatives) for all entries k = l (l + 1) +- m.
+template <typename T, bool NORM, bool SECOND, typename Visit>
+__device__ __forceinline__ void each_entry(int L, Point<T> p, Visit&& visit) {
+    const T rho2 = p.x2 + p.y2;
+    Azimuth<T> azimuth;
+#pragma unroll 1
+    for (int m = 0; m <= L; ++m) {
+        if (m > 0) azimuth.next(p.x, p.y);
+        const T* k = column_table<T>() + column_start(m) * kColumnEntry;
+        T q1 = 0, q2 = 0, e1 = 0, e2 = 0, g1 = 0;
+#pragma unroll 1
+        for (int l = m; l <= L; ++l, k += kColumnEntry) { // (the table has zeros where walk_column takes steps apart)
+            const T e = k[0] * fma_of(p.z, e1, -q2);
+            const T g = k[1] * fma_of(p.z, g1, -e2);
+            const T q = l == m ? T(1) : fma_of(rho2, e, p.z * q1);
+            ColumnSums<T> sums;
+            sums.A = k[2] * q;
+            sums.B = k[3] * e;
+            sums.C = k[4] * q1;
+            if constexpr (SECOND) {
+                sums.E = k[5] * g;
+                sums.G = k[6] * e1;
+                sums.K = k[7] * q2;
+            }
+#pragma unroll 1
+            for (int side = 0; side < (m > 0 ? 2 : 1); ++side) {
+                // (keeps the products of the coordinates from being formed ahead of the loops: 28 registers in float64)
+                asm volatile("" : "+v"(p.x), "+v"(p.y), "+v"(p.z), "+v"(p.ir));
+                PointSums<T, SECOND> one;
+                if (side == 0) one.add_plus(sums, static_cast<T>(m), azimuth);
+                else one.add_minus(sums, static_cast<T>(m), azimuth);
+                visit(l * (l + 1) + (side == 0 ? m : -m), EntryDerivatives<T, NORM, SECOND>(one, p));
+            }
+            q2 = q1;
+            q1 = q;
+            e2 = e1;
+            e1 = e;
+            g1 = g;
+        }
+    }
+}
+
+// an infinity or a NaN among three numbers: three comparisons
+__device__ __forceinline__ bool lost_one(float a, float b, float c) {
+    return __builtin_amdgcn_classf(a, 0x207) | __builtin_amdgcn_classf(b, 0x207) | __builtin_amdgcn_classf(c, 0x207);
+}
+__device__ __forceinline__ bool lost_one(double a, double b, double c) {
+    return __builtin_amdgcn_class(a, 0x207) | __builtin_amdgcn_class(b, 0x207) | __builtin_amdgcn_class(c, 0x207);
+}
+template <typename T> __device__ __forceinline__ bool is_number(const Point<T>& p) { // (at the origin every entry is a NaN)
+    return p.x == p.x && p.y == p.y && p.z == p.z;
+}
+
 // Column after column to wave after wave, the direction changing every time round: the longest columns come first.
 struct Deal {
     unsigned waves, at = 0;
@@ -246,6 +349,13 @@ __device__ __forceinline__ void rows_to_lds(const T* __restrict__ run, T* staged
     for (unsigned e = nvec * W + tid; e < len; e += threads) staged[e + pad * (e / row)] = run[e]; // pad == 0 here
 }
 
+// Waves per SIMD that the registers are to allow: what the sums need by themselves. (The compiler allots registers for
+// the whole kernel, and the entry by entry part, which hardly ever runs, would take a wave from each.)
+template <typename T, bool NORM, bool SECOND, int GROUPS> constexpr int columns_residence() {
+    if (sizeof(T) == 8 && SECOND) return NORM ? 3 : 4;
+    return SECOND && NORM && GROUPS == 2 ? 6 : 7;
+}
+
 // ---------------------------------------------------------------------------
 // columns_kernel: one point per lane (GROUPS == 1, 64 points per workgroup) or per pair of lanes (GROUPS == 2, 32
 // points, one lane for the entries +m and one for -m). The tile's rows of weights pass through LDS, read from HBM with
@@ -263,8 +373,8 @@ __device__ __forceinline__ void rows_to_lds(const T* __restrict__ run, T* staged
 //   out = (P (H g' - a h) - t g' - n (h . g')) / r^2,   g' = P g, a = n . g, t = n . h,
 // and dw = (g' / r) . grad R.
 // ---------------------------------------------------------------------------
-template <typename T, bool NORM, bool SECOND, int GROUPS>
-__global__ __launch_bounds__(kColumnsThreads) void columns_kernel(Columns g, const T* __restrict__ xyz, const T* __restrict__ weights,
+template <typename T, bool NORM, bool SECOND, int GROUPS, bool ADD>
+__global__ __launch_bounds__(kColumnsThreads, (columns_residence<T, NORM, SECOND, GROUPS>())) void columns_kernel(Columns g, const T* __restrict__ xyz, const T* __restrict__ weights,
                                                      const T* __restrict__ grad, T* __restrict__ out,
                                                      T* __restrict__ dw) {
     constexpr unsigned TILE = 64 / GROUPS;
@@ -287,13 +397,18 @@ __global__ __launch_bounds__(kColumnsThreads) void columns_kernel(Columns g, con
 
     rows_to_lds<T>(weights + first * ny, lds, valid * ny, ny, g.pad, g.magic_vectors, tid, threads);
     // lanes past the last point compute on the first one's coordinates and write nothing
-    const unsigned long long mine = first + (point < valid ? point : 0u);
-    const Point<T> p = load_point<T, NORM>(xyz + mine * 3);
+    const unsigned mine = point < valid ? point : 0u;
+    xyz += first * 3;
+    out += first * 3;
+    if constexpr (SECOND) grad += first * 3;
+    const Point<T> p = load_point<T, NORM>(xyz + mine * 3u);
     T gx = 0, gy = 0, gz = 0, along = 0;
+    bool lost_grad = false; // any of the tile's
     if constexpr (SECOND) {
-        gx = grad[mine * 3];
-        gy = grad[mine * 3 + 1];
-        gz = grad[mine * 3 + 2];
+        gx = grad[mine * 3u];
+        gy = grad[mine * 3u + 1u];
+        gz = grad[mine * 3u + 2u];
+        lost_grad = __any(lost_one(gx, gy, gz));
         if constexpr (NORM) {
             along = fma_of(gx, p.x, fma_of(gy, p.y, gz * p.z));
             gx = fma_of(-along, p.x, gx);
@@ -380,6 +495,7 @@ __global__ __launch_bounds__(kColumnsThreads) void columns_kernel(Columns g, con
         for (unsigned i = 0; i < NS; ++i) total[i] += __shfl_xor(total[i], 32);
     }
     T* partial = lds + g.off_sums;
+    bool lost = false;
     if (!SECOND && waves > 1) __syncthreads(); // the sums take the place of the weights
     if (wave != 0) {
 #pragma unroll
@@ -420,15 +536,19 @@ __global__ __launch_bounds__(kColumnsThreads) void columns_kernel(Columns g, con
             oz *= p.ir;
         }
         if (point < valid && !minus) {
-            T* to = out + mine * 3;
-            if (!SECOND && g.accumulate) {
-                ox += to[0];
-                oy += to[1];
-                oz += to[2];
+            T* to = out + mine * 3u;
+            lost = lost_one(ox, oy, oz);
+            if constexpr (ADD) {
+                if (!lost) { // (lost: added below, to what is there)
+                    to[0] += ox;
+                    to[1] += oy;
+                    to[2] += oz;
+                }
+            } else {
+                to[0] = ox;
+                to[1] = oy;
+                to[2] = oz;
             }
-            to[0] = ox;
-            to[1] = oy;
-            to[2] = oz;
         }
     }
     if constexpr (SECOND) {
@@ -436,6 +556,39 @@ __global__ __launch_bounds__(kColumnsThreads) void columns_kernel(Columns g, con
             copy_out<T, SPHX_STREAMING_STORES, false>(lds, dw + first * ny, valid * ny, ny, 0, 0, tid, threads);
         } else {
             copy_out<T, SPHX_STREAMING_STORES, true>(lds, dw + first * ny, valid * ny, ny, g.pad, g.magic_ny, tid, threads);
+        }
+    }
+    if constexpr (SECOND) {
+        // (the same in all waves, each of which has all points of the tile: dw is written once more, after the flush)
+        if (__builtin_expect(lost_grad, 0)) {
+            __threadfence();
+            __syncthreads();
+        }
+    }
+    if (__builtin_expect(lost, 0)) {
+        const Point<T> q = load_point<T, NORM>(xyz + mine * 3u);
+        const T* w = weights + (first + mine) * ny;
+        const T* u = SECOND ? grad + mine * 3u : nullptr;
+        volatile T* to = out + mine * 3u; // (summed in memory: registers here would be paid for by every call)
+        if (!ADD || !is_number(q)) {     // (at the origin every entry is a NaN)
+            to[0] = is_number(q) ? T(0) : q.x;
+            to[1] = is_number(q) ? T(0) : q.y;
+            to[2] = is_number(q) ? T(0) : q.z;
+        }
+        if (is_number(q)) {
+            each_entry<T, NORM, SECOND>(L, q, [&](int k, const EntryDerivatives<T, NORM, SECOND>& of) {
+#pragma unroll
+                for (int b = 0; b < 3; ++b) {
+                    if constexpr (SECOND) {
+                        to[b] = to[b] + (of.h[0][b] * (u[0] * w[k]) + of.h[1][b] * (u[1] * w[k]) + of.h[2][b] * (u[2] * w[k]));
+                    } else {
+                        to[b] = to[b] + of.d[b] * w[k];
+                    }
+                }
+                if constexpr (SECOND) {
+                    if (lost_one(u[0], u[1], u[2])) dw[(first + mine) * ny + k] = u[0] * of.d[0] + u[1] * of.d[1] + u[2] * of.d[2];
+                }
+            });
         }
     }
 }
@@ -484,8 +637,10 @@ __global__ __launch_bounds__(kColumnsThreads) void column_rows_kernel(Columns g,
     } else {
         for (unsigned e = tid; e < TILE * w_stride; e += threads) w_rows[e] = 0;
     }
-    const unsigned long long mine = first + (point < valid ? point : 0u);
-    const Point<T> p = load_point<T, NORM>(xyz + mine * 3);
+    const unsigned mine = point < valid ? point : 0u;
+    xyz += first * 3;
+    out += first * 3;
+    const Point<T> p = load_point<T, NORM>(xyz + mine * 3u);
     const T rho2 = p.x2 + p.y2;
     // set 0 = v_a - n_a s with a = x or z; set 1 = v_y - y s or w r - s
     const T n0 = second_half ? p.z : p.x, n1 = second_half ? T(1) : p.y;
@@ -590,10 +745,29 @@ __global__ __launch_bounds__(kColumnsThreads) void column_rows_kernel(Columns g,
             oy = (fma_of(-inward, p.y, oy) - total[5]) * irsq;
             oz = (fma_of(-inward, p.z, oz) - total[6]) * irsq;
         }
-        T* to = out + mine * 3;
+        T* to = out + mine * 3u;
         to[0] = ox;
         to[1] = oy;
         to[2] = oz;
+        if (__builtin_expect(lost_one(ox, oy, oz), 0)) {
+            const Point<T> q = load_point<T, NORM>(xyz + mine * 3u);
+            if (!is_number(q)) return; // (at the origin every entry is a NaN)
+            const T* v_of = v + (first + mine) * 3u * ny;
+            const T* w_of = w + (first + mine) * ny;
+            volatile T* sum = to; // (as above)
+            sum[0] = 0;
+            sum[1] = 0;
+            sum[2] = 0;
+            each_entry<T, NORM, true>(L, q, [&](int k, const EntryDerivatives<T, NORM, true>& of) {
+                const T vx = v_of[k], vy = v_of[k + ny], vz = v_of[k + 2u * ny];
+#pragma unroll
+                for (int b = 0; b < 3; ++b) {
+                    T add = of.h[0][b] * vx + of.h[1][b] * vy + of.h[2][b] * vz;
+                    if (have_w) add += of.d[b] * w_of[k];
+                    sum[b] = sum[b] + add;
+                }
+            });
+        }
     }
 }
 

@@ -153,6 +153,81 @@ def test_no_further_from_64_bits_than_the_arrays_contracted(library, oracle, nor
             assert here <= there, (name, l_max, here, there)
 
 
+@pytest.mark.parametrize("tile", [32, 64])
+@pytest.mark.parametrize("normalized", [True, False])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_weights_that_are_not_finite_give_what_the_contraction_gives(library, oracle, dtype, normalized, tile, switches):
+    """Infinite and NaN weights, upstream gradients and both: every component is the infinity, the NaN or the number that
+    adding up the entries' own terms gives; a weight so large that a sum over a column overflows, where no term does,
+    gives the finite number; other points of the tile keep theirs bit for bit."""
+    suffix = "f32" if dtype == np.float32 else "f64"
+    vjp, backward, rows = (getattr(library, f"sphx_{name}_{suffix}") for name in ("vjp", "vjp_backward", "gradients_backward"))
+    switches("SPHX_COLUMNS_TILE", tile)
+    stream = torch.cuda.current_stream().cuda_stream
+    n, l_max = 150, 8
+    ny, rng = (l_max + 1) ** 2, np.random.default_rng(5)
+    xyz = rng.standard_normal((n, 3))
+    xyz = (xyz / np.linalg.norm(xyz, axis=1, keepdims=True) * (1.0 + rng.random((n, 1)))).astype(dtype)
+    xyz[100:] *= 20 if normalized else 0.25
+    w, g, v = (rng.standard_normal(shape).astype(dtype) for shape in ((n, ny), (n, 3), (n, 3, ny)))
+
+    def run():
+        d_xyz, d_w, d_g, d_v = (torch.from_numpy(a).cuda() for a in (xyz, w, g, v))
+        first, second, third = (torch.full_like(d_xyz, 7) for _ in range(3))
+        dw, shape = torch.full_like(d_w, 7), (n, l_max, int(normalized))
+        assert vjp(d_xyz.data_ptr(), d_w.data_ptr(), *shape, first.data_ptr(), 0, stream) == 0
+        added = torch.full_like(d_xyz, 7)
+        assert vjp(d_xyz.data_ptr(), d_w.data_ptr(), *shape, added.data_ptr(), 1, stream) == 0
+        for kind in (torch.isnan, torch.isposinf, torch.isneginf):
+            assert torch.equal(kind(added), kind(first))
+        assert backward(d_xyz.data_ptr(), d_w.data_ptr(), d_g.data_ptr(), *shape, second.data_ptr(), dw.data_ptr(), stream) == 0
+        assert rows(d_xyz.data_ptr(), d_w.data_ptr(), d_v.data_ptr(), *shape, third.data_ptr(), stream) == 0
+        return [t.cpu().numpy() for t in (first, second, dw, third)]
+
+    announce("weights that are not finite", suffix, normalized, tile)
+    before = run()
+    inf = np.inf
+    for i in range(0, 90, 3):  # every third point, an entry of any l and m
+        kind, k, a = i // 3 % 6, int(rng.integers(ny)), int(rng.integers(3))
+        if kind in (0, 1, 5):
+            w[i, k] = inf if kind == 0 else -inf
+        if kind in (1, 2):
+            v[i, a, k] = -inf
+        if kind in (3, 5):
+            g[i, a] = inf
+        if kind == 4:
+            w[i, k] = v[i, a, k] = g[i, a] = np.nan
+    with np.errstate(invalid="ignore"):
+        _, dsph, ddsph = oracle.compute(xyz, l_max, normalized, "hessians")
+        want = [
+            (dsph * w[:, None, :]).sum(axis=2),
+            (ddsph * (g[:, :, None] * w[:, None, :])[:, :, None, :]).sum(axis=(1, 3)),
+            (g[:, :, None] * dsph).sum(axis=1),
+            (ddsph * v[:, :, None, :]).sum(axis=(1, 3)) + (dsph * w[:, None, :]).sum(axis=2),
+        ]
+    after = run()
+    for name, got, expected, untouched in zip(("product", "its xyz_grad", "its sph_grad_grad", "rows"), after, want, before):
+        for kind in (np.isnan, np.isposinf, np.isneginf):
+            np.testing.assert_array_equal(kind(got), kind(expected), err_msg=f"{name} {kind.__name__}")
+        rest = np.ones(n, dtype=bool)
+        rest[0:90:3] = False
+        np.testing.assert_array_equal(got[rest], untouched[rest], err_msg=name)
+
+    # the largest weights there are, at entries whose derivatives are below one: points 100 to 149, far out or close in
+    w[:90] = 0
+    g[:90] = v[:90] = 1
+    most = np.finfo(dtype).max
+    for i in range(100, n):
+        w[i] = 0
+        w[i, int(rng.integers(49, ny))] = most * dtype(0.9)
+    first = run()[0]
+    exact = (dsph.astype(np.longdouble) * w.astype(np.longdouble)[:, None, :]).sum(axis=2)
+    assert (np.abs(exact[100:]) < most).all()
+    # one term each: the derivative's own error on either side, _tolerance of the point's largest
+    error = np.abs(first[100:] / most - exact[100:] / most).max(axis=1)
+    assert (error <= 2 * _tolerance(dtype, l_max) * np.abs(dsph[100:]).max(axis=(1, 2))).all()
+
+
 @pytest.mark.parametrize("normalized", [True, False])
 @pytest.mark.parametrize("l_max", [3, 26])
 def test_a_backward_pass_takes_them_and_stays_differentiable(normalized, l_max):
