@@ -134,7 +134,8 @@ SPHX_EXPORT int sphx_vjp_f64(const double* xyz, const double* sph_grad, size_t n
  * term by term where a weight is not finite. The outputs may not overlap the inputs.
  * Where the rows of a tile of points do not fit LDS they return SPHX_ERR_UNSUPPORTED and enqueue nothing (the first
  * takes l_max up to 27 in float32 and 24 in float64, the second 24 and 16): such callers have sphx_forward_* and
- * sphx_backward_second_*. */
+ * sphx_backward_second_*. sphx_second_order_supported is 1 for an l_max that the first (rows == 0) or the second takes
+ * on the current device, 0 for others. */
 SPHX_EXPORT int sphx_vjp_backward_f32(const float* xyz, const float* sph_grad, const float* grad, size_t n_samples,
                                       int l_max, int normalized, float* xyz_grad, float* sph_grad_grad, void* stream);
 SPHX_EXPORT int sphx_vjp_backward_f64(const double* xyz, const double* sph_grad, const double* grad, size_t n_samples,
@@ -143,6 +144,7 @@ SPHX_EXPORT int sphx_gradients_backward_f32(const float* xyz, const float* sph_g
                                             size_t n_samples, int l_max, int normalized, float* xyz_grad, void* stream);
 SPHX_EXPORT int sphx_gradients_backward_f64(const double* xyz, const double* sph_grad, const double* dsph_grad,
                                             size_t n_samples, int l_max, int normalized, double* xyz_grad, void* stream);
+SPHX_EXPORT int sphx_second_order_supported(int rows, int l_max, int is_f64);
 
 /* float32 arrays, evaluated in float64 and rounded once: what sphx_forward_f64
  * returns for the same points, converted to float (round to nearest even).

@@ -34,6 +34,7 @@ LAUNCH_SYMBOLS = [
     "sphx_vjp_backward_f64",
     "sphx_gradients_backward_f32",
     "sphx_gradients_backward_f64",
+    "sphx_second_order_supported",
     "sphx_forward_f32_via_f64",
     "sphx_forward_f32_via_f64_workspace",
     "sphx_forward_f32_via_f64_static",
@@ -92,6 +93,8 @@ def _declare(lib):
         fn = getattr(lib, f"sphx_prefactors_{suffix}")
         fn.restype = c_int
         fn.argtypes = [c_int, c_void_p]
+    lib.sphx_second_order_supported.restype = c_int
+    lib.sphx_second_order_supported.argtypes = [c_int, c_int, c_int]
     lib.sphx_forward_f32_via_f64.restype = c_int
     lib.sphx_forward_f32_via_f64.argtypes = [
         c_void_p, c_size_t, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]

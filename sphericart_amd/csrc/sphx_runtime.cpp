@@ -389,6 +389,15 @@ int sphx_gradients_backward_f64(const double* xyz, const double* sph_grad, const
                                  nullptr, stream);
 }
 
+int sphx_second_order_supported(int rows, int l_max, int is_f64) {
+    int lds = 0, cus = 0;
+    sphx::device_for_planning(&lds, &cus);
+    (void)sphx::refresh_switches();
+    sphx::ColumnsLaunch launch;
+    return sphx::plan_columns(rows != 0 ? sphx::COLUMNS_ROWS : sphx::COLUMNS_VJP_BACKWARD, 1, l_max,
+                              is_f64 ? sizeof(double) : sizeof(float), lds, cus, &launch);
+}
+
 int sphx_device_count(void) {
     sphx::t_error.clear();
     int n = 0;

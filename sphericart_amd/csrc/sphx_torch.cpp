@@ -330,6 +330,13 @@ Tensor contract_hessians(const Tensor& ddsph, const Tensor& dsph_grad) {
     return op.call(ddsph, dsph_grad);
 }
 
+// Whether a backward pass that is not differentiated again takes the product without the arrays; beyond its l_max the pass
+// contracts what it has saved, and forms no more than is asked for. (No size is looked at: they may be symbolic here.)
+bool without_arrays(const Tensor& xyz, int64_t l_max, bool rows) {
+    return !at::GradMode::is_enabled() &&
+           sphx_second_order_supported(rows, static_cast<int>(l_max), xyz.scalar_type() == at::kDouble) != 0;
+}
+
 std::optional<Tensor> maybe(const Tensor& tensor) {
     return tensor.defined() ? std::optional<Tensor>(tensor) : std::nullopt;
 }
@@ -363,7 +370,7 @@ template <bool NORMALIZED> struct VjpFunction : Function<VjpFunction<NORMALIZED>
         const auto saved = ctx->get_saved_variables();
         const Tensor &xyz = saved[0], &sph_grad = saved[1], &grad = grads[0];
         const int64_t l_max = ctx->saved_data["l_max"].toInt();
-        if (!at::GradMode::is_enabled()) {
+        if (without_arrays(xyz, l_max, false)) {
             auto both = Operators<NORMALIZED>::vjp_backward().call(xyz, sph_grad, grad, l_max);
             return {std::get<0>(both), std::get<1>(both), Tensor()};
         }
@@ -378,12 +385,9 @@ template <bool NORMALIZED> struct VjpFunction : Function<VjpFunction<NORMALIZED>
     }
 };
 
-// Backward from the gradients of values and gradients, either of which may be missing.
-template <bool NORMALIZED, typename Dsph, typename Ddsph>
-Tensor backward_from(const Tensor& xyz, int64_t l_max, const Tensor& grad_sph, const Tensor& grad_dsph, Dsph dsph, Ddsph ddsph) {
-    if (grad_dsph.defined() && !at::GradMode::is_enabled()) {
-        return Operators<NORMALIZED>::gradients_backward().call(xyz, maybe(grad_sph), grad_dsph, l_max);
-    }
+// Backward from the gradients of values and gradients, either of which may be missing, by the arrays.
+template <typename Dsph, typename Ddsph>
+Tensor backward_from(const Tensor& grad_sph, const Tensor& grad_dsph, Dsph dsph, Ddsph ddsph) {
     Tensor sum;
     if (grad_sph.defined()) sum = contract_gradients(dsph(), grad_sph);
     if (grad_dsph.defined()) {
@@ -406,30 +410,32 @@ template <bool NORMALIZED> struct GradientsFunction : Function<GradientsFunction
     static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
         if (!ctx->needs_input_grad(0)) return {Tensor(), Tensor()};
         const auto saved = ctx->get_saved_variables();
+        const Tensor &xyz = saved[0], &dsph = saved[1];
         const int64_t l_max = ctx->saved_data["l_max"].toInt();
-        return {backward_from<NORMALIZED>(saved[0], l_max, grads[0], grads[1], [&] { return saved[1]; },
-                                          [&] { return std::get<2>(Operators<NORMALIZED>::hessians().call(saved[0], l_max)); }),
+        if (grads[1].defined() && without_arrays(xyz, l_max, true)) {
+            return {Operators<NORMALIZED>::gradients_backward().call(xyz, maybe(grads[0]), grads[1], l_max), Tensor()};
+        }
+        return {backward_from(grads[0], grads[1], [&] { return dsph; },
+                              [&] { return std::get<2>(Operators<NORMALIZED>::hessians().call(xyz, l_max)); }),
                 Tensor()};
     }
 };
 
+// (xyz is not saved: both arrays are there, and a program may have moved its points meanwhile)
 template <bool NORMALIZED> struct HessiansFunction : Function<HessiansFunction<NORMALIZED>> {
     static constexpr bool is_traceable = true;
     static variable_list forward(AutogradContext* ctx, const Tensor& xyz, int64_t l_max) {
         const at::AutoDispatchBelowAutograd guard;
         const auto all = Operators<NORMALIZED>::hessians().call(xyz, l_max);
         ctx->set_materialize_grads(false);
-        ctx->saved_data["l_max"] = l_max;
-        ctx->save_for_backward({xyz, std::get<1>(all), std::get<2>(all)});
+        ctx->save_for_backward({std::get<1>(all), std::get<2>(all)});
         return {std::get<0>(all), std::get<1>(all), std::get<2>(all)};
     }
     static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
         TORCH_CHECK(!grads[2].defined(), "Third derivatives of the spherical harmonics with respect to the Cartesian coordinates "
                                          "are not supported.");
         const auto saved = ctx->get_saved_variables();
-        return {backward_from<NORMALIZED>(saved[0], ctx->saved_data["l_max"].toInt(), grads[0], grads[1], [&] { return saved[1]; },
-                                          [&] { return saved[2]; }),
-                Tensor()};
+        return {backward_from(grads[0], grads[1], [&] { return saved[0]; }, [&] { return saved[1]; }), Tensor()};
     }
 };
 

@@ -297,6 +297,13 @@ torch.library.register_autograd(
 
 # ---- autograd of the six operators (register.py:82-175) ----------------------
 
+def _without_arrays(xyz, l_max, rows):
+    """Whether a backward pass that is not differentiated again takes the product without the derivative arrays; beyond
+    its l_max the pass contracts what it has saved, and forms no more than is asked for."""
+    return not torch.is_grad_enabled() and bool(
+        get_library().sphx_second_order_supported(int(rows), l_max, int(xyz.dtype == torch.float64)))
+
+
 def _register_vjp(prefix):
     """Shapes and derivatives of the fused product xyz_grad[i, a] = sum_k dsph[i, a, k] w[i, k]."""
     hessians = getattr(_ops, f"{prefix}_with_hessians")
@@ -321,9 +328,9 @@ def _register_vjp(prefix):
 
     def backward(ctx, grad):
         xyz, sph_grad = ctx.saved_tensors
-        if not torch.is_grad_enabled():
+        if _without_arrays(xyz, ctx.l_max, False):
             return *vjp_backward(xyz, sph_grad, grad, ctx.l_max), None
-        # a backward pass that is differentiated again: from operators that can be
+        # a backward pass that is differentiated again (from operators that can be), or beyond the l_max of the product
         _, dsph, ddsph = hessians(xyz, ctx.l_max)
         d_xyz = d_sph_grad = None
         if ctx.needs_input_grad[0]:
@@ -366,7 +373,7 @@ def _register_gradients_autograd(prefix):
         if not ctx.needs_input_grad[0]:
             return None, None
         xyz, dsph = ctx.saved_tensors
-        if grad_dsph is not None and not torch.is_grad_enabled():
+        if grad_dsph is not None and _without_arrays(xyz, ctx.l_max, True):
             return gradients_backward(xyz, grad_sph, grad_dsph, ctx.l_max), None
         xyz_grad = None
         if grad_sph is not None:
@@ -383,12 +390,9 @@ def _register_gradients_autograd(prefix):
 
 
 def _register_hessians_autograd(prefix):
-    gradients_backward = getattr(_ops, f"{prefix}_gradients_backward")
-
     def setup_context(ctx, inputs, output):
-        xyz, ctx.l_max = inputs
         ctx.set_materialize_grads(False)
-        ctx.save_for_backward(xyz, output[1], output[2])
+        ctx.save_for_backward(output[1], output[2])  # (not xyz: a program may move its points meanwhile)
 
     def backward(ctx, grad_sph, grad_dsph, grad_ddsph):
         if grad_ddsph is not None:
@@ -396,9 +400,7 @@ def _register_hessians_autograd(prefix):
                 "Third derivatives of the spherical harmonics with respect to "
                 "the Cartesian coordinates are not supported."
             )
-        xyz, dsph, ddsph = ctx.saved_tensors
-        if grad_dsph is not None and not torch.is_grad_enabled():
-            return gradients_backward(xyz, grad_sph, grad_dsph, ctx.l_max), None
+        dsph, ddsph = ctx.saved_tensors
         xyz_grad = None
         if grad_sph is not None:
             xyz_grad = _ops.contract_gradients(dsph, grad_sph)

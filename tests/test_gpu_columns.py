@@ -255,6 +255,62 @@ def test_a_backward_pass_takes_them_and_stays_differentiable(normalized, l_max):
         assert (a - b).abs().max().item() <= 2e-13 * b.abs().max().item()
 
 
+@pytest.mark.parametrize("python_operators", ["0", "1"])
+def test_a_backward_pass_from_second_derivatives_uses_the_arrays_it_has(python_operators):
+    """The pass backward from values, gradients and second derivatives contracts the saved arrays, at an l_max of the
+    column kernels and beyond it: number for number, with the points moved in the meantime, and without another array of
+    second derivatives."""
+    import os
+    import subprocess
+    import sys
+
+    announce("backward from second derivatives", python_operators)
+    code = """
+import torch, sphericart_amd.torch
+from sphericart_amd.torch import ops as rules
+assert rules.cpp_operators == (%r == "0")
+ops = torch.ops.sphericart_amd
+for l_max in (3, 18):
+    for operator in (ops.spherical_harmonics_with_hessians, ops.solid_harmonics_with_hessians):
+        torch.manual_seed(l_max)
+        xyz = torch.randn(2000, 3, dtype=torch.float64).cuda().requires_grad_()
+        sph, dsph, ddsph = operator(xyz, l_max)
+        w, v = torch.randn_like(sph), torch.randn_like(dsph)
+        with torch.no_grad():
+            xyz += 1.0
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        (grad,) = torch.autograd.grad((sph, dsph), xyz, (w, v))
+        torch.cuda.synchronize()
+        assert torch.cuda.max_memory_allocated() - before < 0.5 * ddsph.numel() * ddsph.element_size(), l_max
+        assert torch.equal(grad, ops.contract_gradients(dsph.detach(), w) + ops.contract_hessians(ddsph.detach(), v))
+print("done")
+""" % python_operators
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    done = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, cwd=root, timeout=300,
+                          env=dict(os.environ, SPHERICART_AMD_PYTHON_OPERATORS=python_operators))
+    assert done.returncode == 0 and "done" in done.stdout, done.stderr
+
+
+def test_which_products_there_are(library):
+    """sphx_second_order_supported says what the entries then do."""
+    announce("which products")
+    for suffix, dtype in (("f32", torch.float32), ("f64", torch.float64)):
+        for l_max in (0, 16, 17, 24, 25, 27, 28):
+            ny = (l_max + 1) ** 2
+            xyz, w, v = (torch.ones(shape, dtype=dtype, device="cuda") for shape in ((5, 3), (5, ny), (5, 3, ny)))
+            out, dw = torch.empty_like(xyz), torch.empty_like(w)
+            stream, shape = torch.cuda.current_stream().cuda_stream, (5, l_max, 1)
+            first = getattr(library, f"sphx_vjp_backward_{suffix}")(
+                xyz.data_ptr(), w.data_ptr(), xyz.data_ptr(), *shape, out.data_ptr(), dw.data_ptr(), stream)
+            second = getattr(library, f"sphx_gradients_backward_{suffix}")(
+                xyz.data_ptr(), w.data_ptr(), v.data_ptr(), *shape, out.data_ptr(), stream)
+            for rows, status in ((0, first), (1, second)):
+                assert status == (0 if library.sphx_second_order_supported(rows, l_max, int(suffix == "f64")) else 2)
+    assert library.sphx_second_order_supported(0, -1, 0) == 0
+
+
 def test_autograd_with_nothing_but_the_torch_library_loaded(tmp_path):
     """The rules for GPU tensors are in libsphericart_amd_torch.so: a process that has loaded that library alone gets the
     gradients, and the gradients of the gradients, that the package gets."""
