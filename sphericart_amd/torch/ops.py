@@ -153,8 +153,22 @@ def _vjp(xyz, sph_grad, l_max, normalized):
     return out
 
 
+def _check_weights(xyz, l_max, *weights):
+    """xyz [n, 3] and (name, tensor, shape after n) of one dtype on one device: the kernels take their addresses."""
+    if xyz.dim() != 2 or xyz.shape[1] != 3:
+        raise ValueError("xyz tensor must be a 2D array with shape `n_samples x 3`")
+    if l_max < 0:
+        raise ValueError("l_max must be non-negative")
+    for name, tensor, shape in weights:
+        if tensor.dtype != xyz.dtype or tensor.device != xyz.device:
+            raise ValueError(f"xyz and {name} must share dtype and device")
+        if tuple(tensor.shape) != (xyz.shape[0], *shape):
+            raise ValueError(f"{name} must have shape {(xyz.shape[0], *shape)}")
+
+
 def _vjp_backward(xyz, sph_grad, grad, l_max, normalized):
     suffix = _suffix(xyz)
+    _check_weights(xyz, l_max, ("sph_grad", sph_grad, ((l_max + 1) ** 2,)), ("grad", grad, (3,)))
     library = get_library()
     xyz, sph_grad, grad = (t.detach().contiguous() for t in (xyz, sph_grad, grad))
     xyz_grad, sph_grad_grad = torch.empty_like(xyz), torch.empty_like(sph_grad)
@@ -174,6 +188,9 @@ def _vjp_backward(xyz, sph_grad, grad, l_max, normalized):
 
 def _gradients_backward(xyz, sph_grad, dsph_grad, l_max, normalized):
     suffix = _suffix(xyz)
+    _check_weights(xyz, l_max, ("dsph_grad", dsph_grad, (3, (l_max + 1) ** 2)))
+    if sph_grad is not None:
+        _check_weights(xyz, l_max, ("sph_grad", sph_grad, ((l_max + 1) ** 2,)))
     library = get_library()
     xyz, dsph_grad = xyz.detach().contiguous(), dsph_grad.detach().contiguous()
     sph_grad = sph_grad.detach().contiguous() if sph_grad is not None else None

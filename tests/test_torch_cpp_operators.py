@@ -42,6 +42,43 @@ def test_the_python_operators_remain_behind_a_switch():
     assert done.stdout.split()[:2] == ["False", "True"] and "[4, 3, 9]" in done.stdout
 
 
+@pytest.mark.parametrize("l_max", [0, 3])
+def test_the_python_second_order_products_refuse_what_does_not_fit(l_max):
+    """Shapes, dtypes and devices that do not belong together raise before an address is handed on, as they do in C++."""
+    from sphericart_amd.torch import ops
+
+    n, ny = 5, (l_max + 1) ** 2
+    xyz, w, g, v = (torch.zeros(shape) for shape in ((n, 3), (n, ny), (n, 3), (n, 3, ny)))
+    for kind, error, message in (
+        (lambda t: t[:-1], ValueError, "shape"),
+        (lambda t: t[..., :-1], ValueError, "shape"),
+        (lambda t: torch.cat([t, t], dim=-1), ValueError, "shape"),
+        (lambda t: t.flatten(), ValueError, "shape"),
+        (lambda t: t.double(), ValueError, "share dtype and device"),
+        (lambda t: t.to("meta"), ValueError, "share dtype and device"),
+    ):
+        with pytest.raises(error, match=message):
+            ops._vjp_backward(xyz, kind(w), g, l_max, True)
+        with pytest.raises(error, match=message):
+            ops._vjp_backward(xyz, w, kind(g), l_max, True)
+        with pytest.raises(error, match=message):
+            ops._gradients_backward(xyz, kind(w), v, l_max, True)
+        for sph_grad in (w, None):
+            with pytest.raises(error, match=message):
+                ops._gradients_backward(xyz, sph_grad, kind(v), l_max, True)
+    for bad in (xyz[:, :2], torch.zeros(n, 4), xyz.flatten(), xyz[:-1]):
+        with pytest.raises(ValueError, match="shape"):
+            ops._vjp_backward(bad, w, g, l_max, True)
+        with pytest.raises(ValueError, match="shape"):
+            ops._gradients_backward(bad, w, v, l_max, True)
+    with pytest.raises(ValueError, match="non-negative"):
+        ops._vjp_backward(xyz, torch.zeros(n, 1), g, -2, True)
+    with pytest.raises(ValueError, match="non-negative"):
+        ops._gradients_backward(xyz, None, torch.zeros(n, 3, 1), -2, True)
+    with pytest.raises(TypeError):
+        ops._vjp_backward(xyz.half(), w.half(), g.half(), l_max, True)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 def test_same_numbers_as_the_python_operators_and_the_same_errors(dtype):
