@@ -80,15 +80,22 @@ template <bool NORMALIZED> std::tuple<Tensor, Tensor, Tensor> with_hessians(cons
     return forward(xyz, l_max, NORMALIZED, 2);
 }
 
+// What the operators below share: points [n, 3], and weights of a given shape and the points' dtype on their device.
+void check_points(const Tensor& xyz, int64_t l_max) {
+    TORCH_CHECK_VALUE(xyz.dim() == 2 && xyz.size(1) == 3, "xyz tensor must be a 2D array with shape `n_samples x 3`");
+    TORCH_CHECK_VALUE(l_max >= 0, "l_max must be non-negative");
+}
+void check_weights(const Tensor& xyz, const Tensor& weights, at::IntArrayRef shape, const char* what) {
+    TORCH_CHECK_VALUE(weights.scalar_type() == xyz.scalar_type() && weights.device() == xyz.device(), "xyz and ", what,
+                      " must share dtype and device");
+    TORCH_CHECK_VALUE(weights.sizes() == shape, what, " must have shape ", shape);
+}
+
 // the product of the gradients with sph_grad without the gradient array (sphx_vjp_*)
 template <bool NORMALIZED> Tensor vjp(const Tensor& xyz_in, const Tensor& sph_grad_in, int64_t l_max) {
     const bool f64 = is_double(xyz_in, "spherical harmonics");
-    TORCH_CHECK_VALUE(sph_grad_in.scalar_type() == xyz_in.scalar_type() && sph_grad_in.device() == xyz_in.device(),
-                      "xyz and sph_grad must share dtype and device");
-    const int64_t ny = (l_max + 1) * (l_max + 1);
-    TORCH_CHECK_VALUE(xyz_in.dim() == 2 && sph_grad_in.dim() == 2 && sph_grad_in.size(0) == xyz_in.size(0) &&
-                          sph_grad_in.size(1) == ny,
-                      "sph_grad must have shape (", xyz_in.dim() == 2 ? xyz_in.size(0) : 0, ", ", ny, ")");
+    check_points(xyz_in, l_max);
+    check_weights(xyz_in, sph_grad_in, {xyz_in.size(0), (l_max + 1) * (l_max + 1)}, "sph_grad");
     const Tensor xyz = xyz_in.detach().contiguous(), sph_grad = sph_grad_in.detach().contiguous();
     Tensor out = at::empty_like(xyz);
     const c10::DeviceGuard guard(xyz.device());
@@ -135,20 +142,12 @@ template <bool SECOND> Tensor contract(const Tensor& derivatives_in, const Tenso
     return out;
 }
 
-// What the two operators below share: xyz, the row length, and weights of a given shape on the same device.
-void check_weights(const Tensor& xyz, const Tensor& weights, at::IntArrayRef shape, const char* what) {
-    TORCH_CHECK_VALUE(weights.scalar_type() == xyz.scalar_type() && weights.device() == xyz.device(), "xyz and ", what,
-                      " must share dtype and device");
-    TORCH_CHECK_VALUE(weights.sizes() == shape, what, " must have shape ", shape);
-}
-
 // The derivatives of vjp with the upstream gradient `grad` [n, 3]: with respect to xyz and to sph_grad
 // (sphx_vjp_backward_*; from the derivative arrays where that does not reach).
 template <bool NORMALIZED>
 std::tuple<Tensor, Tensor> vjp_backward(const Tensor& xyz_in, const Tensor& sph_grad_in, const Tensor& grad_in, int64_t l_max) {
     const bool f64 = is_double(xyz_in, "spherical harmonics");
-    TORCH_CHECK_VALUE(xyz_in.dim() == 2 && xyz_in.size(1) == 3, "xyz tensor must be a 2D array with shape `n_samples x 3`");
-    TORCH_CHECK_VALUE(l_max >= 0, "l_max must be non-negative");
+    check_points(xyz_in, l_max);
     const int64_t n = xyz_in.size(0), ny = (l_max + 1) * (l_max + 1);
     check_weights(xyz_in, sph_grad_in, {n, ny}, "sph_grad");
     check_weights(xyz_in, grad_in, {n, 3}, "grad");
@@ -176,8 +175,7 @@ std::tuple<Tensor, Tensor> vjp_backward(const Tensor& xyz_in, const Tensor& sph_
 template <bool NORMALIZED>
 Tensor gradients_backward(const Tensor& xyz_in, const std::optional<Tensor>& sph_grad_in, const Tensor& dsph_grad_in, int64_t l_max) {
     const bool f64 = is_double(xyz_in, "spherical harmonics");
-    TORCH_CHECK_VALUE(xyz_in.dim() == 2 && xyz_in.size(1) == 3, "xyz tensor must be a 2D array with shape `n_samples x 3`");
-    TORCH_CHECK_VALUE(l_max >= 0, "l_max must be non-negative");
+    check_points(xyz_in, l_max);
     const int64_t n = xyz_in.size(0), ny = (l_max + 1) * (l_max + 1);
     check_weights(xyz_in, dsph_grad_in, {n, 3, ny}, "dsph_grad");
     if (sph_grad_in.has_value()) check_weights(xyz_in, *sph_grad_in, {n, ny}, "sph_grad");

@@ -133,12 +133,22 @@ def _contract(name, derivatives, upstream):
     return out
 
 
+def _check_weights(xyz, l_max, *weights):
+    """xyz [n, 3] and (name, tensor, shape after n) of one dtype on one device: the kernels take their addresses."""
+    if xyz.dim() != 2 or xyz.shape[1] != 3:
+        raise ValueError("xyz tensor must be a 2D array with shape `n_samples x 3`")
+    if l_max < 0:
+        raise ValueError("l_max must be non-negative")
+    for name, tensor, shape in weights:
+        if tensor.dtype != xyz.dtype or tensor.device != xyz.device:
+            raise ValueError(f"xyz and {name} must share dtype and device")
+        if tuple(tensor.shape) != (xyz.shape[0], *shape):
+            raise ValueError(f"{name} must have shape {(xyz.shape[0], *shape)}")
+
+
 def _vjp(xyz, sph_grad, l_max, normalized):
     suffix = _suffix(xyz)
-    if sph_grad.dtype != xyz.dtype or sph_grad.device != xyz.device:
-        raise ValueError("xyz and sph_grad must share dtype and device")
-    if sph_grad.shape != (xyz.shape[0], (l_max + 1) ** 2):
-        raise ValueError(f"sph_grad must have shape {(xyz.shape[0], (l_max + 1) ** 2)}")
+    _check_weights(xyz, l_max, ("sph_grad", sph_grad, ((l_max + 1) ** 2,)))
     xyz = xyz.detach().contiguous()
     sph_grad = sph_grad.detach().contiguous()
     out = torch.empty_like(xyz)
@@ -151,19 +161,6 @@ def _vjp(xyz, sph_grad, l_max, normalized):
         )
     _check(status, library)
     return out
-
-
-def _check_weights(xyz, l_max, *weights):
-    """xyz [n, 3] and (name, tensor, shape after n) of one dtype on one device: the kernels take their addresses."""
-    if xyz.dim() != 2 or xyz.shape[1] != 3:
-        raise ValueError("xyz tensor must be a 2D array with shape `n_samples x 3`")
-    if l_max < 0:
-        raise ValueError("l_max must be non-negative")
-    for name, tensor, shape in weights:
-        if tensor.dtype != xyz.dtype or tensor.device != xyz.device:
-            raise ValueError(f"xyz and {name} must share dtype and device")
-        if tuple(tensor.shape) != (xyz.shape[0], *shape):
-            raise ValueError(f"{name} must have shape {(xyz.shape[0], *shape)}")
 
 
 def _vjp_backward(xyz, sph_grad, grad, l_max, normalized):

@@ -71,6 +71,8 @@ def test_the_python_second_order_products_refuse_what_does_not_fit(l_max):
             ops._vjp_backward(bad, w, g, l_max, True)
         with pytest.raises(ValueError, match="shape"):
             ops._gradients_backward(bad, w, v, l_max, True)
+        with pytest.raises(ValueError, match="shape"):
+            ops._vjp(bad, w, l_max, True)
     with pytest.raises(ValueError, match="non-negative"):
         ops._vjp_backward(xyz, torch.zeros(n, 1), g, -2, True)
     with pytest.raises(ValueError, match="non-negative"):
@@ -113,6 +115,9 @@ def test_same_numbers_as_the_python_operators_and_the_same_errors(dtype):
         torch.ops.sphericart_amd.spherical_harmonics(xyz, -1)
     with pytest.raises(TypeError, match="float32 and float64"):
         torch.ops.sphericart_amd.spherical_harmonics(xyz.to(torch.float16), 3)
+    for bad in (xyz[:, :2], torch.zeros(5, 4, dtype=dtype, device="cuda")):
+        with pytest.raises(ValueError, match="n_samples x 3"):
+            torch.ops.sphericart_amd.solid_harmonics_vjp(bad, torch.zeros(5, 16, dtype=dtype, device="cuda"), 3)
     with pytest.raises(ValueError, match="sph_grad must have shape"):
         torch.ops.sphericart_amd.spherical_harmonics_vjp(xyz, torch.zeros(5, 15, dtype=dtype, device="cuda"), 3)
     with pytest.raises(ValueError, match="do not contract"):
