@@ -32,7 +32,6 @@ struct Tiling {
     unsigned together;      // recursion_kernel, float64: 1 = the recursions run next to the entries (TOGETHER)
     unsigned row_pad;       // recursion_kernel, whole rows: elements left free after every staged row (0, 16 bytes' worth or, point_lanes, 0 or 1)
     unsigned magic_ny;      // ceil(2^32 / ny)
-    unsigned point_lanes;   // recursion_kernel, normalised second derivatives: one point per lane, a job for a whole wave
     unsigned priorities;    // recursion_kernel: 1 = the waves that flush run at raised priority, 2 = those that prepare the next tile
     // LDS carve-up, in elements of T: the staged rows come first, rows_elems of them, with the
     // gradient and second-derivative rows at off_dsph and off_ddsph inside a buffer; the other
@@ -48,6 +47,7 @@ struct Tiling {
     // in the job table when they are moved to wave boundaries of the entry lanes (0: they follow
     // the bulk without gaps); jobs_per_point then counts the gaps too
     unsigned kind_at[3];
+    unsigned point_lanes; // recursion_kernel, normalised second derivatives: one point per lane, a job for a whole wave
 };
 
 // a place in the job table of recursion_kernel that holds no job

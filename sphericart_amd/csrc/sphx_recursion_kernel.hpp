@@ -463,7 +463,9 @@ __global__ __launch_bounds__(NT, MODE < 2 ? 4 : 1) void recursion_kernel(Tiling 
             rows.dsph = staged + g.off_dsph + phase_dsph + s * 3 * row_stride - skip;
             rows.ddsph = staged + g.off_ddsph + phase_ddsph + s * 9 * row_stride - skip;
         };
-        auto take_job = [&](unsigned packed) {
+        auto take_job = [&](unsigned e) {
+            unsigned packed = job_table[e];
+            if constexpr (POINTS_L != 0) packed = __builtin_amdgcn_readfirstlane(packed);
             if constexpr (!LIST && !SPLIT) {
                 if (packed == kNoJob) return;
             }
@@ -491,7 +493,7 @@ __global__ __launch_bounds__(NT, MODE < 2 ? 4 : 1) void recursion_kernel(Tiling 
                 // that begin in its share of the work.
                 if (lane < valid) {
                     take_point(lane);
-                    for (unsigned e = jobs_from; e < jobs_to; ++e) take_job(__builtin_amdgcn_readfirstlane(job_table[e]));
+                    for (unsigned e = jobs_from; e < jobs_to; ++e) take_job(e);
                 }
                 return;
             }
@@ -506,7 +508,7 @@ __global__ __launch_bounds__(NT, MODE < 2 ? 4 : 1) void recursion_kernel(Tiling 
                         current = s;
                         take_point(s);
                     }
-                    take_job(job_table[q - s * per_point]);
+                    take_job(q - s * per_point);
                 }
                 return;
             }
@@ -538,7 +540,7 @@ __global__ __launch_bounds__(NT, MODE < 2 ? 4 : 1) void recursion_kernel(Tiling 
                     current = s;
                     take_point(s);
                 }
-                take_job(job_table[first_job + (r - s * b)]);
+                take_job(first_job + (r - s * b));
             }
         } else {
             // One pass takes the jobs of as many points as fit side by side in the wide lanes
@@ -553,7 +555,7 @@ __global__ __launch_bounds__(NT, MODE < 2 ? 4 : 1) void recursion_kernel(Tiling 
                 const unsigned s = s0 + local;
                 if (s >= valid || local >= g.points_per_pass) continue;
                 take_point(s);
-                for (unsigned e = e_first; e < per_point; e += wide_lanes) take_job(job_table[e]);
+                for (unsigned e = e_first; e < per_point; e += wide_lanes) take_job(e);
             }
         }
     };
