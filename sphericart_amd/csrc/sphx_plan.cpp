@@ -127,7 +127,7 @@ static void plan_closed(size_t n_samples, int l_max, int hard, int mode, size_t 
 // values_kernel: up to 64 points per workgroup, their rows and tables in LDS. Returns false when that does not
 // fit, and the recursion kernel takes over. `with_sums`: the same layout for the lane kernels of the fused
 // product, which keep no rows for HBM but the sums of their waves.
-static bool plan_values(size_t n_samples, int l_max, size_t elem, int lds_limit, Launch* out,
+static bool plan_values(size_t n_samples, int l_max, size_t elem, int lds_limit, int cus, Launch* out,
                         bool with_sums = false) {
     Tiling& g = out->g;
     std::memset(&g, 0, sizeof(g));
@@ -154,9 +154,33 @@ static bool plan_values(size_t n_samples, int l_max, size_t elem, int lds_limit,
     // to sixteen waves, or two with half of it each.
     const ShapeRow* shape = shape_row(with_sums ? 1 : 0, static_cast<int>(elem), l_max, n_samples);
     unsigned pack_by_shape = shape ? shape->pack : 1u;
-    // Fewer points than 64 for every CU: tiles of 16 reach four times as many of them (us, 3 000 points, one / two /
-    // four channels: float32 l_max = 18 7.2 5.7 5.6, 28 11.6 8.0 7.3; float64 18 8.3 6.9 6.6, 26 16.5 - 8.4)
-    if (n_samples < 16384 && l_max >= 16) pack_by_shape = 4;
+    // How often the CUs are filled with tiles of so many points and channels side by side, one after the other (LDS is
+    // handed out in pieces of 1 280 bytes).
+    auto rounds = [&](unsigned points, unsigned channels) {
+        const unsigned elems = align4(points * row_stride) + align4(points * table_elems) + (channels > 1 ? 2u * tri_all : 0u);
+        const size_t at_once = static_cast<size_t>(cus) * (allowed / ((elems * esize + 1279u) / 1280u * 1280u)) * points;
+        return at_once != 0 ? (n_samples + at_once - 1) / at_once : ~static_cast<size_t>(0); // (they do not fit)
+    };
+    const bool four_fit = rounds(16u, 4u) != ~static_cast<size_t>(0);
+    if (!with_sums && n_samples < 16384 && l_max >= 16) {
+        // Fewer points than 64 for every CU: tiles of 16 reach four times as many of them (us, 3 000 points, one / two /
+        // four channels: float32 l_max = 18 7.2 5.7 5.6, 28 11.6 8.0 7.3; float64 18 8.3 6.9 6.6, 26 16.5 - 8.4), unless
+        // that takes a round more than tiles of 8 (four / eight channels: float32 26, 9 000 points 12.4 10.4; 33, 5 000
+        // 13.7 9.8; float64 23, 4 551 and 14 000 points 13.3 10.1, 25.8 23.5; as many rounds, 23, 8 000 15.1 16.0, 25, 6 000
+        // 14.4 15.4) or, in float64, more than the one in which the largest tiles take all points with one channel per
+        // wave (four / one: 16, 14 000 points 12.4 11.7; 18, 12 000 12.4 11.8; 20, 10 000 13.1 12.6; 21, 9 000 14.3
+        // 12.9; float32 28, 10 000 14.2 15.3).
+        const unsigned largest = allowed / ((row_stride + table_elems) * esize) / 4u * 4u;
+        pack_by_shape = four_fit && rounds(8u, 8u) < rounds(16u, 4u) ? 8u : 4u;
+        if (pack_by_shape == 4 && elem == 8 && rounds(16u, 4u) > 1 && largest >= 32 && rounds(largest < 64 ? largest : 64u, 1u) == 1) {
+            pack_by_shape = 1;
+        }
+    } else if (!with_sums && pack_by_shape == 2 && rounds(64u, 1u) <= 3 && rounds(32u, 2u) > rounds(64u, 1u)) {
+        // Two channels where their tiles fill the CUs once more than whole waves of points do, and not often: one (float32,
+        // l_max = 12, us, two / one: 45 000 points 10.1 8.7, 90 000 15.6 15.0, 130 000 19.5 18.7; as many rounds, 60 000
+        // points 11.0 11.7, four and five, 200 000, 26.9 26.8).
+        pack_by_shape = 1;
+    }
     const int waves_by_shape = shape ? shape->waves : 0;
     const unsigned floor_by_shape = shape ? shape->floor : 32u;
     const bool alone = switch_or(SW_VALUES_ALONE, shape && shape->alone ? 1 : 0) != 0;
@@ -867,7 +891,7 @@ int make_plan(size_t n_samples, int l_max, int mode, size_t elem, int lds_limit,
             }
         }
     }
-    if (lane_kernels && mode == 0 && plan_values(n_samples, l_max, elem, lds_limit, &plan->closed)) {
+    if (lane_kernels && mode == 0 && plan_values(n_samples, l_max, elem, lds_limit, cus, &plan->closed)) {
         plan->lanes = true;
         return SPHX_OK;
     }
@@ -1018,7 +1042,7 @@ int make_vjp_plan(size_t n_samples, int l_max, size_t elem, int lds_limit, int c
     // (columns_kernel takes l_max = 7 to 24, in float32 to 27: sphx_runtime.cpp)
     out->use_lanes = out->lane_groups = false;
     if (l_max > 6 && switch_or(SW_VJP_LANES, 1) != 0) {
-        out->use_lanes = plan_values(n_samples, l_max, elem, lds_limit, &out->lanes, true);
+        out->use_lanes = plan_values(n_samples, l_max, elem, lds_limit, cus, &out->lanes, true);
         // groups of lanes with channels of their own pay off from tiles of 16 points down (20-25 % at l_max = 24);
         // with tiles of 32 the kernel that takes its prefactors from the scalar unit is ahead
         out->lane_groups = out->use_lanes && out->lanes.g.tile <= switch_or(SW_VJP_GROUPS_BELOW, 16);

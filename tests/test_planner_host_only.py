@@ -30,6 +30,16 @@ SHAPES = [
     (2_000, 40, 1, 1, 1, "recursion_kernel<double, 1, true, false, false, false, false>"),
     (5, 24, 2, 1, 1, "recursion_kernel<double, 2, true, true, false, false, false>"),
     (1, 0, 0, 0, 1, "closed_form_kernel<float, 0, true, 0, false>"),
+    # values: channels side by side by the rounds that the tiles take on the CUs
+    (45_000, 12, 0, 0, 1, "values_kernel<float, true, 1>"),
+    (60_000, 12, 0, 0, 1, "values_kernel<float, true, 2>"),
+    (200_000, 12, 0, 0, 1, "values_kernel<float, true, 2>"),
+    (8_000, 18, 0, 1, 1, "values_kernel<double, true, 4>"),
+    (10_000, 18, 0, 1, 1, "values_kernel<double, true, 8>"),
+    (12_000, 18, 0, 1, 1, "values_kernel<double, true, 1>"),
+    (9_000, 21, 0, 1, 1, "values_kernel<double, true, 1>"),
+    (9_000, 26, 0, 0, 1, "values_kernel<float, true, 8>"),
+    (12_000, 26, 0, 0, 1, "values_kernel<float, true, 4>"),
     # the flush at raised priority: by the table of shapes, and only with many tiles per workgroup
     (200_000, 33, 1, 0, 0, "pairs_kernel<float, 1, false>"),
     (40_000, 33, 1, 0, 0, "pairs_kernel<float, 1, false>"),
