@@ -124,4 +124,27 @@ bool plan_columns(ColumnsKind kind, size_t n_samples, int l_max, size_t elem, in
     return true;
 }
 
+// Up to l_max = 6 the sum runs over the closed forms in index order (number for number what contracting the gradients
+// gives). Beyond, columns_kernel is ahead of the kernels that form every entry, but where the lane kernel's tiles are
+// larger and so many points take it fewer rounds on the CUs: one instead of two, or, where a tile of columns_kernel leaves
+// room for nothing else on a CU (float64 from l_max = 17, float32 from 25) and a few rounds follow one another, up to
+// three for four. us, columns / lanes, rounds: float64 l_max = 17, 9 000 points 14.8 10.1 (2, 1), 17 000 27.1 23.0 (3, 2),
+// 25 900 35.3 33.7 (4, 3), 41 100 50.3 45.7 (6, 4), as against 15 000 20.4 22.4 (2, 2), 38 000 42.6 45.1 (5, 4), 200 000 205 215; float32 20,
+// 17 600 16.4 14.2 (2, 1), 19 000 18.0 20.9 (2, 2); 26, 9 000 18.5 13.6 (2, 1), 41 100 64 60 (6, 4).
+bool vjp_by_columns(size_t n_samples, int l_max, size_t elem, int lds_limit, int cus, const VjpPlan& other, ColumnsLaunch* out) {
+    if (l_max <= 6 || switch_or(SW_VJP_LANES, 1) == 0) return false;
+    if (!plan_columns(COLUMNS_VJP, n_samples, l_max, elem, lds_limit, cus, out)) return false;
+    if (!other.use_lanes) return true;
+    auto resident = [&](unsigned bytes, unsigned threads) { // workgroups on a CU (LDS is handed out in pieces of 1 280 bytes)
+        const unsigned by_lds = static_cast<unsigned>(lds_limit) / ((bytes + 1279u) / 1280u * 1280u), by_waves = 2048u / threads;
+        return by_lds < by_waves ? (by_lds > 0 ? by_lds : 1u) : by_waves;
+    };
+    auto rounds = [&](unsigned tiles, unsigned at_once) { return (tiles + at_once - 1u) / at_once; };
+    const unsigned units = static_cast<unsigned>(cus > 0 ? cus : 1);
+    const unsigned beside = resident(out->lds_bytes, out->threads);
+    const unsigned columns = rounds(out->g.n_tiles, units * beside);
+    const unsigned lanes = rounds(other.lanes.g.n_tiles, units * resident(other.lanes.lds_bytes, other.lanes.threads));
+    return !(beside == 1 ? lanes <= 4 && 10u * columns > 13u * lanes : columns == 2 && lanes == 1);
+}
+
 } // namespace sphx

@@ -46,6 +46,11 @@ enum ColumnsKind {
 // Whether the kernels take this shape, and how. Plain host arithmetic, a few dozen instructions.
 bool plan_columns(ColumnsKind kind, size_t n_samples, int l_max, size_t elem, int lds_limit, int cus, ColumnsLaunch* out);
 
+// Whether columns_kernel takes the vector-Jacobian product of this shape, for which the older kernels have `other`; then
+// `out` is its plan.
+struct VjpPlan;
+bool vjp_by_columns(size_t n_samples, int l_max, size_t elem, int lds_limit, int cus, const VjpPlan& other, ColumnsLaunch* out);
+
 // The table described above, in the arithmetic of T, made from the prefactors F of sphx_tables.hpp.
 template <typename T> std::vector<T> column_table_of(const T* F);
 

@@ -1039,7 +1039,7 @@ bool make_wide_plan(size_t n_samples, int l_max, int mode, int lds_limit, int cu
 }
 
 int make_vjp_plan(size_t n_samples, int l_max, size_t elem, int lds_limit, int cus, VjpPlan* out) {
-    // (columns_kernel takes l_max = 7 to 24, in float32 to 27: sphx_runtime.cpp)
+    // (columns_kernel takes most of l_max = 7 to 24, in float32 to 27: vjp_by_columns)
     out->use_lanes = out->lane_groups = false;
     if (l_max > 6 && switch_or(SW_VJP_LANES, 1) != 0) {
         out->use_lanes = plan_values(n_samples, l_max, elem, lds_limit, cus, &out->lanes, true);

@@ -52,9 +52,15 @@ constexpr ShapeRow kShapeRows[] = {
     {0, 8, 25, 32, 4, false, 0, 32, "20 000 points, l_max = 26 - - 36 36, recursion kernel 39, 32 - - 46 66, 49"},
     // the product, float64. 200 000 points (400 000 to l_max = 16), us: tiles in half of LDS / one workgroup per
     // CU with 8 / with up to 12 waves; from l_max = 21 with tiles of 28, 24, 20 points before they halve
+    {1, 8, 17, 17, 1, true, 12, 32, "289 228 214"},
+    {1, 8, 18, 18, 1, true, 12, 32, "299 261 240"},
+    {1, 8, 19, 19, 1, true, 12, 32, "315 290 272"},
     {1, 8, 25, 25, 1, true, 8, 16, "660 598 602"},
     {1, 8, 26, 26, 1, true, 12, 16, "675 719 661"},
     // the product, float32, the same columns (l_max = 21, 31: sixteen waves 162, 423)
+    {1, 4, 25, 25, 1, true, 12, 32, "335 274 255"},
+    {1, 4, 26, 26, 1, true, 12, 32, "340 294 276"},
+    {1, 4, 27, 27, 1, true, 8, 32, "348 289 313"},
     {1, 4, 28, 28, 1, true, 8, 32, "356 318 342"},
     {1, 4, 29, 29, 1, true, 12, 32, "385 404 370"},
     {1, 4, 30, 30, 1, true, 8, 32, "397 381 422"},

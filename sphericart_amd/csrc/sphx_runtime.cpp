@@ -272,13 +272,13 @@ static int vjp(const T* xyz, const T* sph_grad, size_t n_samples, int l_max, int
         bool fresh = false;
         PlannedCall* call = planned_call(1, n_samples, l_max, 1, sizeof(T), normalized != 0, device, &fresh);
         if (fresh) {
-            // Up to l_max = 6 the sum runs over the closed forms in index order (number for number what contracting the
-            // gradients gives); beyond, columns_kernel is ahead of the kernels that form every entry
-            call->by_columns = l_max > 6 && switch_or(SW_VJP_LANES, 1) != 0 &&
-                               plan_columns(COLUMNS_VJP, n_samples, l_max, sizeof(T), dev.lds_limit, dev.compute_units,
-                                            &call->columns);
-            status = call->by_columns ? static_cast<int>(SPHX_OK)
-                                      : make_vjp_plan(n_samples, l_max, sizeof(T), dev.lds_limit, dev.compute_units, &call->vjp);
+            status = make_vjp_plan(n_samples, l_max, sizeof(T), dev.lds_limit, dev.compute_units, &call->vjp);
+            call->by_columns = vjp_by_columns(n_samples, l_max, sizeof(T), dev.lds_limit, dev.compute_units, call->vjp,
+                                              &call->columns);
+            if (call->by_columns) {
+                status = SPHX_OK;
+                t_error.clear();
+            }
             if (status != SPHX_OK) return status;
             keep(call);
         }

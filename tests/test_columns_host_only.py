@@ -1,0 +1,42 @@
+"""The planner of the column kernels is plain host C++ (sphx_columns.cpp with sphx_plan.cpp, compiled with g++ alone): which
+kernel a vector-Jacobian product gets, and that what is planned fits."""
+
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "sphericart_amd", "csrc")
+VJP, VJP_BACKWARD, ROWS = 0, 1, 2
+
+
+@pytest.fixture(scope="module")
+def plans(tmp_path_factory):
+    binary = tmp_path_factory.mktemp("columns") / "columns_probe"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", os.path.join(ROOT, "tests", "columns_probe.cpp"),
+                    *(os.path.join(CSRC, name) for name in ("sphx_columns.cpp", "sphx_plan.cpp")), "-o", str(binary)], check=True)
+
+    def run(shapes):
+        names = "there groups workgroups threads lds tiles pad off_rows off_sums by_columns".split()
+        out = subprocess.run([str(binary)] + [str(v) for shape in shapes for v in shape], capture_output=True, text=True,
+                             check=True).stdout.splitlines()
+        assert len(out) == len(shapes)
+        return [dict(zip(names, map(int, line.split()))) for line in out]
+
+    return run
+
+
+def test_which_kernel_a_product_gets(plans):
+    """The columns beyond the closed forms, but where the lane kernel takes a round less (float64 from l_max = 17, float32
+    at 20 and from 25), up to four rounds."""
+    wanted = {
+        (1_000, 6, 4): False, (1_000, 7, 4): True, (400_003, 8, 4): True, (1_500, 24, 8): True, (1_500, 25, 8): False,
+        (1_500, 27, 4): True, (1_500, 28, 4): False,
+        (8_000, 17, 8): True, (9_000, 17, 8): False, (15_000, 17, 8): True, (17_000, 17, 8): False, (41_100, 17, 8): False,
+        (200_000, 17, 8): True, (9_000, 18, 8): False, (9_000, 19, 8): False, (9_000, 20, 8): True, (9_000, 16, 8): True,
+        (17_600, 20, 4): False, (19_000, 20, 4): True, (17_600, 19, 4): True, (9_000, 24, 4): True, (9_000, 25, 4): False,
+        (15_000, 26, 4): True, (41_100, 26, 4): False, (200_000, 26, 4): True,
+    }
+    for shape, plan in zip(wanted, plans([(VJP, *shape) for shape in wanted])):
+        assert bool(plan["by_columns"]) == wanted[shape], shape

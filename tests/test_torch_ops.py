@@ -169,6 +169,37 @@ def test_fused_vjp_beyond_the_closed_forms(library, oracle, normalized, dtype, t
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype,tol", [(np.float32, 1e-5), (np.float64, 1e-12)])
+def test_fused_vjp_of_large_calls(library, oracle, dtype, tol):
+    """Beyond 64 points for every CU the product takes tiles of 64 points and few waves, or (float64 l_max = 17, float32
+    26 here) the lane kernel where that takes a round less: the same sums, on every part of the grid."""
+    rng = np.random.default_rng(7)
+    fn = library.sphx_vjp_f32 if dtype == np.float32 else library.sphx_vjp_f64
+    stream = torch.cuda.current_stream().cuda_stream
+    for l_max, n, normalized in ((7, 17_001, True), (8, 40_003, True), (8, 33_000, False), (10, 16_500, True), (13, 16_385, False),
+                                 (17, 9_000, True), (17, 16_999, False), (17, 24_001, True), (26, 9_001, True)):
+        if l_max == 26 and dtype == np.float64:
+            continue
+        announce("fused vjp, large calls", np.dtype(dtype).name, l_max, n, normalized)
+        xyz = _points(n, dtype, seed=l_max + n)
+        weights = rng.standard_normal((n, (l_max + 1) ** 2)).astype(dtype)
+        _, dsph, _ = oracle.compute(xyz, l_max, normalized, "gradients")
+        want = oracle.backward(dsph, weights)
+        scale = np.einsum("iak,ik->ia", np.abs(dsph), np.abs(weights)) + 1
+        holder = torch.zeros(weights.size + 1, dtype=torch.from_numpy(weights).dtype, device="cuda")
+        d_xyz = torch.from_numpy(xyz).cuda()
+        for shift, accumulate in ((0, 0), (1, 1)):
+            d_w = holder[shift:shift + weights.size].view(weights.shape)
+            d_w.copy_(torch.from_numpy(weights))
+            start = rng.standard_normal((n, 3)).astype(dtype)
+            out = torch.from_numpy(start).cuda()
+            status = fn(d_xyz.data_ptr(), d_w.data_ptr(), n, l_max, int(normalized), out.data_ptr(), accumulate, stream)
+            assert status == 0, library.sphx_last_error()
+            expect = want + start if accumulate else want
+            assert np.max(np.abs(out.cpu().numpy() - expect) / scale) <= tol, (l_max, n, accumulate, shift)
+
+
+@pytest.mark.gpu
 def test_contraction_accumulates_on_request(library, oracle):
     announce("contraction accumulate flag")
     rng = np.random.default_rng(5)
