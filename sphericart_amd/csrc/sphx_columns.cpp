@@ -102,8 +102,12 @@ bool plan_columns(ColumnsKind kind, size_t n_samples, int l_max, size_t elem, in
     }
     while (bytes > limit && waves > 1) bytes = lay_out(tile, waves / 2); // (the largest rows leave no room for many sums)
     if (bytes > limit) return false;
+    // A launch holds fewer than 2^32 threads: fewer waves, where those of one wave are too many as well another path
+    // (5.4e8 points at l_max = 10 in float32, 1.07e9 with arrays: 270 and 43 GB of them)
     const size_t tiles = (n_samples + tile - 1) / tile;
-    if (tiles > 0x7fffffffull) return false;
+    auto too_many = [&]() { return (tiles + 7) / 8 * 8 > 0xffffffffull / (64u * static_cast<unsigned>(waves)); };
+    while (too_many() && waves > 1) bytes = lay_out(tile, waves / 2);
+    if (too_many()) return false;
 
     std::memset(&out->g, 0, sizeof(out->g));
     out->g.n_samples = n_samples;

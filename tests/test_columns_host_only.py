@@ -40,3 +40,31 @@ def test_which_kernel_a_product_gets(plans):
     }
     for shape, plan in zip(wanted, plans([(VJP, *shape) for shape in wanted])):
         assert bool(plan["by_columns"]) == wanted[shape], shape
+
+
+@pytest.mark.parametrize("elem", [4, 8])
+def test_what_is_planned_fits(plans, elem):
+    """Rows, pads and the sums of the waves inside LDS, tiles for all points, at most 512 threads and fewer than 2^32 in a
+    launch; and where the tables or LDS end there is no plan."""
+    reach = {VJP: 27 if elem == 4 else 24, VJP_BACKWARD: 27 if elem == 4 else 24, ROWS: 24 if elem == 4 else 16}
+    shapes = [(kind, n, l_max, elem) for kind in reach for l_max in range(31)
+              for n in (1, 15, 1_000, 16_384, 16_385, 400_003, 30_000_000, 600_000_000, 1_200_000_000, 5_000_000_000)]
+    for (kind, n, l_max, _), plan in zip(shapes, plans(shapes)):
+        if l_max > reach[kind]:
+            assert not plan["there"], (kind, n, l_max)
+            continue
+        if not plan["there"]:  # one wave per tile is too many already
+            assert n > 2**32 // (64 // (16 if kind == ROWS else 32)) - 1_000, (kind, n, l_max)
+            continue
+        assert plan["threads"] % 64 == 0 and 64 <= plan["threads"] <= 512
+        assert plan["workgroups"] % 8 == 0 and plan["workgroups"] * plan["threads"] < 2**32, (kind, n, l_max)
+        tile = 64 // plan["groups"]
+        assert plan["groups"] in ((4,) if kind == ROWS else (1, 2))
+        assert (plan["tiles"] - 1) * tile < n <= plan["tiles"] * tile and plan["workgroups"] >= plan["tiles"]
+        ny, waves = (l_max + 1) ** 2, plan["threads"] // 64
+        assert plan["pad"] in (0, 1) and (plan["pad"] == 0 or ny % (16 // elem) == 0)
+        rows = plan["off_rows"] + tile * (ny + plan["pad"])
+        assert kind != ROWS or plan["off_rows"] >= tile * (3 * ny + plan["pad"])
+        sums = (waves - 1) * (7 * 16 if kind == ROWS else (3 if kind == VJP else 6) * 64)
+        assert kind != VJP_BACKWARD or plan["off_sums"] >= rows
+        assert max(rows, plan["off_sums"] + sums) * elem <= plan["lds"] <= 160 * 1024
