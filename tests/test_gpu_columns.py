@@ -58,7 +58,7 @@ def test_second_order_products_equal_the_oracles_arrays_contracted(library, orac
     if tile:
         switches("SPHX_COLUMNS_TILE", tile)
     rng = np.random.default_rng(3)
-    for l_max in (0, 1, 2, 3, 4, 5, 6, 7, 9, 12, 16, 17, 24, 25):
+    for l_max in (0, 1, 2, 3, 4, 5, 6, 7, 9, 12, 16, 17, 24, 25, 26, 27):
         for n, waves in ((1, 0), (15, 8), (33, 1), (65, 3), (700, 0)):
             if waves:
                 switches("SPHX_COLUMNS_WAVES", waves)
@@ -98,6 +98,29 @@ def test_second_order_products_equal_the_oracles_arrays_contracted(library, orac
     assert backward(None, None, None, 0, 3, 1, None, None, stream) == 0
     assert rows(None, None, None, 0, 3, 1, None, stream) == 0
     assert backward(None, None, None, 5, 3, 1, None, None, stream) == 1
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_second_order_products_of_large_calls(library, oracle, dtype):
+    """The plans of calls with more than 64 points for every CU, as they are made: 64-point tiles and few waves for the
+    product's derivatives, the rows' waves by l_max."""
+    suffix = "f32" if dtype == np.float32 else "f64"
+    backward, rows = getattr(library, f"sphx_vjp_backward_{suffix}"), getattr(library, f"sphx_gradients_backward_{suffix}")
+    stream = torch.cuda.current_stream().cuda_stream
+    rng = np.random.default_rng(11)
+    for l_max, n, normalized in ((1, 40_001, True), (3, 16_390, False), (5, 17_003, True), (6, 33_333, True), (8, 16_401, False), (10, 16_450, True)):
+        announce("second-order products, large calls", suffix, l_max, n, normalized)
+        ny, tolerance, xyz = (l_max + 1) ** 2, _tolerance(dtype, l_max), _cloud(n, dtype, l_max)
+        w, g, v = (rng.standard_normal(shape).astype(dtype) for shape in ((n, ny), (n, 3), (n, 3, ny)))
+        hess_w, dw, hess_v, grad_w = _expected(oracle, xyz, l_max, normalized, w, g, v)
+        d_xyz, d_w, d_g, d_v = (torch.from_numpy(a).cuda() for a in (xyz, w, g, v))
+        out, out_w, out_rows = torch.full_like(d_xyz, float("nan")), torch.full_like(d_w, float("nan")), torch.full_like(d_xyz, float("nan"))
+        shape = (n, l_max, int(normalized))
+        assert backward(d_xyz.data_ptr(), d_w.data_ptr(), d_g.data_ptr(), *shape, out.data_ptr(), out_w.data_ptr(), stream) == 0
+        assert rows(d_xyz.data_ptr(), d_w.data_ptr(), d_v.data_ptr(), *shape, out_rows.data_ptr(), stream) == 0
+        _close(out, *hess_w, tolerance, (l_max, n, "xyz_grad"))
+        _close(out_w, *dw, tolerance, (l_max, n, "sph_grad_grad"))
+        _close(out_rows, hess_v[0] + grad_w[0], hess_v[1] + grad_w[1], tolerance, (l_max, n, "rows"))
 
 
 def _directions(where, n, seed):
