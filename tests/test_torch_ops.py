@@ -122,7 +122,7 @@ def test_fused_vjp_beyond_the_closed_forms(library, oracle, normalized, dtype, t
     """l_max > 6, two routes: the default ("lanes": columns_kernel, to l_max = 24 in float64 and 27 in
     float32; beyond, one point per lane with the entries kept in registers, wherever a tile of 8 points
     or more fits in LDS), or the recursion kernel contracting its staged rows ("rows"). Either adds the
-    terms in another order than the checker's loop, so the comparison is relative to the sum of absolute
+    terms in another order than the oracle's loop, so the comparison is relative to the sum of absolute
     terms."""
     if route == "rows":
         switches("SPHX_VJP_LANES", "0")
