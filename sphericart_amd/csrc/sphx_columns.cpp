@@ -26,10 +26,10 @@ template <typename T> std::vector<T> column_table_of(const T* F) {
             const int n = l - m;
             const long double f = F[l * (l + 1) / 2 + m], lm = l + m, w = 2 * m + 2;
             t[0] = n < 2 ? T(0) : static_cast<T>((n - 1) / lm);
-            t[1] = n < 3 ? T(0) : static_cast<T>((n - 2) / lm);
-            t[2] = static_cast<T>(f * pole(l, m));
-            t[3] = n < 2 ? T(0) : static_cast<T>(-f * pole(l - 1, m + 1) * w / (n - 1));
-            t[4] = static_cast<T>(f * lm * pole(l - 1, m));
+            t[4] = n < 3 ? T(0) : static_cast<T>((n - 2) / lm);
+            t[1] = static_cast<T>(f * pole(l, m));
+            t[2] = n < 2 ? T(0) : static_cast<T>(-f * pole(l - 1, m + 1) * w / (n - 1));
+            t[3] = static_cast<T>(f * lm * pole(l - 1, m));
             t[5] = n < 4 ? T(0) : static_cast<T>(f * pole(l - 2, m + 2) * w * (w + 2) / ((n - 2) * (n - 3)));
             t[6] = n < 3 ? T(0) : static_cast<T>(-f * lm * pole(l - 2, m + 1) * w / (n - 2));
             t[7] = static_cast<T>(f * lm * (lm - 1) * pole(l - 2, m));
@@ -43,8 +43,7 @@ template std::vector<double> column_table_of<double>(const double*);
 bool plan_columns(ColumnsKind kind, size_t n_samples, int l_max, size_t elem, int lds_limit, int cus, ColumnsLaunch* out) {
     if (l_max < 0 || l_max > kColumnsLMax) return false;
     const unsigned ny = static_cast<unsigned>((l_max + 1) * (l_max + 1)), e = static_cast<unsigned>(elem);
-    // (a row of one vector stays as it is: the division by its length that places the pads has no multiplier)
-    const unsigned vec = 16u / e, pad = ny % 2 == 0 && ny > vec ? 1u : 0u;
+    const unsigned vec = 16u / e, pad = columns_pad(elem, ny);
     const unsigned limit = static_cast<unsigned>(lds_limit);
     auto rounded = [&](unsigned n) { return (n + vec - 1u) / vec * vec; };
     // The sums of the waves beyond the first (3 or 6 numbers per lane, 7 per point): where dw waits in the rows for its
@@ -73,24 +72,20 @@ bool plan_columns(ColumnsKind kind, size_t n_samples, int l_max, size_t elem, in
     // with one, 4.7 with eight).
     const size_t cu = static_cast<size_t>(cus > 0 ? cus : 1);
     if (kind == COLUMNS_ROWS) {
-        waves = l_max < 5 ? 1 : (l_max < 8 ? 2 : 4);
+        waves = fixed_column_waves(kind, elem, l_max);
         if ((n_samples + 15) / 16 <= cu) waves = most;
         if (forced_waves > 0) waves = forced_waves < most ? forced_waves : most;
         bytes = lay_out(16u, waves);
     } else {
-        // 64 points while three workgroups fit a CU, else 32 on two lanes each (derivatives of the product, 200 000
-        // points at l_max = 12: 56.6 against 55.0 us in float32 where 43 KB still fit three times, 128 against 111 in
-        // float64 where 86 KB do not; the product, 100 000 at l_max = 16 in float64: 73 against 63)
-        const unsigned lds = 160u * 1024u;
-        const unsigned wide = lay_out(64u, 1) <= lds / 3u ? 64u : 32u;
-        const unsigned resident = lds / lay_out(wide, 1);
+        tile = columns_tile(elem, l_max);
+        const unsigned resident = columns_resident(elem, l_max);
         // four waves while many workgroups share a CU, eight below (the product, us with 4 / 8: float32 l_max = 8 27.5
         // 34.4, 10 37.1 33.1, 20 55.4 46.6; float64 l_max = 7 76 84, 8 55 48, 10 69 74, 13 93 85). The derivatives in
         // float64 need so many registers that eight waves would fill a CU: four unless the workgroup is alone (l_max =
         // 8: 95 143).
         waves = resident >= (e == 4 ? 6u : 4u) || (kind == COLUMNS_VJP_BACKWARD && e == 8 && resident > 1) ? 4 : 8;
         if (l_max < 6) waves = l_max < 3 ? 1 : 2;
-        tile = wide;
+        if (fixed_columns(kind, l_max)) waves = fixed_column_waves(kind, elem, l_max);
         if ((n_samples + 63) / 64 <= cu) {
             tile = 32u;
             waves = most;

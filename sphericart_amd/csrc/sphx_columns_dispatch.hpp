@@ -22,6 +22,12 @@ static hipError_t launch_columns(Kernel kernel, const ColumnsLaunch& l, hipStrea
 template <typename T>
 hipError_t dispatch_columns(ColumnsKind kind, const ColumnsLaunch& l, bool normalized, const T* xyz, const T* sph_grad,
                             const T* upstream, T* xyz_grad, T* sph_grad_grad, hipStream_t s) {
+    if (fixed_columns(kind, l.g.l_max) && fixed_columns_on(kind, sizeof(T), l.g.l_max, l.groups) && l.g.accumulate == 0) {
+        auto go = [&](auto dispatch) { return dispatch(l, normalized, xyz, sph_grad, upstream, xyz_grad, sph_grad_grad, s); };
+        if (kind == COLUMNS_VJP) return go(dispatch_columns_fixed<T, COLUMNS_VJP>);
+        if (kind == COLUMNS_VJP_BACKWARD) return go(dispatch_columns_fixed<T, COLUMNS_VJP_BACKWARD>);
+        return go(dispatch_columns_fixed<T, COLUMNS_ROWS>);
+    }
     if (kind == COLUMNS_ROWS) {
         return normalized ? launch_columns(column_rows_kernel<T, true>, l, s, xyz, sph_grad, upstream, xyz_grad)
                           : launch_columns(column_rows_kernel<T, false>, l, s, xyz, sph_grad, upstream, xyz_grad);
@@ -38,7 +44,8 @@ hipError_t dispatch_columns(ColumnsKind kind, const ColumnsLaunch& l, bool norma
     return l.g.accumulate != 0 ? by_lanes(std::false_type{}, std::true_type{}) : by_lanes(std::false_type{}, std::false_type{});
 }
 
-template <typename T> hipError_t upload_column_tables(const HostTables& t) {
+// (every translation unit has its own copy of the table: internal linkage here as well)
+template <typename T> static hipError_t fill_column_table(const HostTables& t) {
     if constexpr (sizeof(T) == 4) {
         const std::vector<float> table = column_table_of<float>(t.f32.data());
         return hipMemcpyToSymbol(HIP_SYMBOL(kColumns32), table.data(), table.size() * sizeof(float));
@@ -47,6 +54,8 @@ template <typename T> hipError_t upload_column_tables(const HostTables& t) {
         return hipMemcpyToSymbol(HIP_SYMBOL(kColumns64), table.data(), table.size() * sizeof(double));
     }
 }
+
+template <typename T> hipError_t upload_column_tables(const HostTables& t) { return fill_column_table<T>(t); }
 
 } // namespace sphx
 

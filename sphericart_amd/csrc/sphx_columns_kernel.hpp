@@ -46,6 +46,16 @@ namespace sphx {
 //
 // The products are sums in another order than the entries' own, with fused multiply-adds: they agree with the
 // contraction of the derivative arrays to rounding.
+//
+// LMAX > 0: kernels for one l_max each (fixed_columns(), sphx_columns.hpp), the same operations in the same order. What the
+// general kernel is bound by is the issue of instructions and, in small calls, the wait at every step: per step it loads the
+// entry's factors through the scalar unit and the weights from LDS, which share a counter, and waits for both (l_max = 8 in
+// float32: as many scalar as vector instructions, 31 + 30 per pair of entries). With l_max a constant a column is one run
+// of 16 instructions per pair, the loads of several steps ahead, the offsets of the weights part of the instructions, and
+// the rows come into LDS without a branch between the loads. us, general and fixed: the product, 400 000 points, float32
+// l_max = 8 27.3 22.5 (floor 20.2), 12 56 43 (41), 17 134 101 (77), float64 8 50 42 (40), 12 130 106 (81), 20 000 points
+// at 14 in float32 8.8 5.1; its derivatives, float32 8 51.6 43.9 (39.7), float64 10 169 147 (116); the rows, float32 8 144
+// 108 (77), float64 9 295 236 (177), 20 000 points 22.9 18.2.
 // ---------------------------------------------------------------------------
 
 __device__ __forceinline__ float fma_of(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
@@ -61,11 +71,17 @@ template <> __device__ __forceinline__ const double* column_table<double>() { re
 // the six Q above. `step` is l - m as a compile-time number while that is below 5 and 5 from there on: what is zero
 // or one by construction in the first steps takes no instruction (FB is meaningful from step 2 on, FC 1, FE 4, FG 3,
 // FK 2). rho2 = x^2 + y^2.
-template <typename T, bool SECOND, typename Visit>
-__device__ __forceinline__ void walk_column(int m, int L, T z, T rho2, Visit&& visit) {
+template <int... I, typename F> __host__ __device__ __forceinline__ void each_of(std::integer_sequence<int, I...>, F&& f) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+
+// LMAX > 0: m and L = LMAX are compile-time numbers (m an integral_constant), and the column is one run of
+// instructions without a branch.
+template <typename T, bool SECOND, int LMAX, typename M, typename Visit>
+__device__ __forceinline__ void walk_column(M m, int L, T z, T rho2, Visit&& visit) {
     const T* t = column_table<T>() + column_start(m) * kColumnEntry;
     T q1 = 0, q2 = 0, e1 = 0, e2 = 0, g1 = 0;
-    auto one = [&](auto step, int l) {
+    auto one = [&](auto step, auto l) {
         constexpr int S = decltype(step)::value;
         const T* k = t;
         t += kColumnEntry;
@@ -73,16 +89,16 @@ __device__ __forceinline__ void walk_column(int m, int L, T z, T rho2, Visit&& v
         if constexpr (S == 2) e = -k[0];
         else if constexpr (S >= 3) e = k[0] * fma_of(z, e1, -q2);
         if constexpr (SECOND) {
-            if constexpr (S == 4) g = -k[1] * e2;
-            else if constexpr (S >= 5) g = k[1] * fma_of(z, g1, -e2);
+            if constexpr (S == 4) g = -k[4] * e2;
+            else if constexpr (S >= 5) g = k[4] * fma_of(z, g1, -e2);
         }
         if constexpr (S == 1) q = z;
         else if constexpr (S >= 2) q = fma_of(rho2, e, z * q1);
-        T fa = k[2], fb = 0, fc = 0, fe = 0, fg = 0, fk = 0;
+        T fa = k[1], fb = 0, fc = 0, fe = 0, fg = 0, fk = 0;
         if constexpr (S >= 1) fa *= q;
-        if constexpr (S >= 1) fc = k[4];
+        if constexpr (S >= 1) fc = k[3];
         if constexpr (S >= 2) fc *= q1;
-        if constexpr (S >= 2) fb = k[3] * e;
+        if constexpr (S >= 2) fb = k[2] * e;
         if constexpr (SECOND) {
             if constexpr (S >= 2) fk = k[7];
             if constexpr (S >= 3) fk *= q2;
@@ -97,7 +113,14 @@ __device__ __forceinline__ void walk_column(int m, int L, T z, T rho2, Visit&& v
         g1 = g;
     };
     using std::integral_constant;
-    one(integral_constant<int, 0>{}, m);
+    if constexpr (LMAX > 0) {
+        each_of(std::make_integer_sequence<int, LMAX - M::value + 1>{}, [&](auto n) {
+            constexpr int N = decltype(n)::value;
+            one(integral_constant<int, (N < 5 ? N : 5)>{}, integral_constant<int, M::value + N>{});
+        });
+        return;
+    }
+    one(integral_constant<int, 0>{}, static_cast<int>(m));
     if (m + 1 > L) return;
     one(integral_constant<int, 1>{}, m + 1);
     if (m + 2 > L) return;
@@ -246,12 +269,12 @@ __device__ __forceinline__ void each_entry(int L, Point<T> p, Visit&& visit) {
 #pragma unroll 1
         for (int l = m; l <= L; ++l, k += kColumnEntry) { // (the table has zeros where walk_column takes steps apart)
             const T e = k[0] * fma_of(p.z, e1, -q2);
-            const T g = k[1] * fma_of(p.z, g1, -e2);
+            const T g = k[4] * fma_of(p.z, g1, -e2);
             const T q = l == m ? T(1) : fma_of(rho2, e, p.z * q1);
             ColumnSums<T> sums;
-            sums.A = k[2] * q;
-            sums.B = k[3] * e;
-            sums.C = k[4] * q1;
+            sums.A = k[1] * q;
+            sums.B = k[2] * e;
+            sums.C = k[3] * q1;
             if constexpr (SECOND) {
                 sums.E = k[5] * g;
                 sums.G = k[6] * e1;
@@ -301,6 +324,14 @@ struct Deal {
     }
 };
 
+// The same deal as a bit per column.
+__device__ __forceinline__ unsigned columns_of(unsigned wave, unsigned waves, int l_max) {
+    const unsigned period = 2u * waves, both = (1u << wave) | (1u << (period - 1u - wave));
+    unsigned mine = 0;
+    for (unsigned at = 0; at <= static_cast<unsigned>(l_max); at += period) mine |= both << at;
+    return mine;
+}
+
 // `len` consecutive elements of HBM, rows of `row` elements, to LDS with the rows `row + pad` apart. pad is 0 or, for
 // even rows (a multiple of 16 bytes then), 1, so that the rows of the points start on different banks. `magic` =
 // magic_of(row in 16-byte vectors). Many 16-byte loads in flight per lane: a tile is read once, and its latency is
@@ -349,9 +380,63 @@ __device__ __forceinline__ void rows_to_lds(const T* __restrict__ run, T* staged
     for (unsigned e = nvec * W + tid; e < len; e += threads) staged[e + pad * (e / row)] = run[e]; // pad == 0 here
 }
 
+// The same with the rows' length and pad compile-time numbers and without a branch between the loads: issue() sends the
+// loads of ROUNDS vectors per lane, put() stores them, then the next ROUNDS. A lane that has run out of vectors loads and
+// stores the last one once more.
+template <typename T, unsigned ROW, unsigned PAD, unsigned ROUNDS> struct FixedRows {
+    using V = typename Pack<T>::type;
+    static constexpr unsigned W = Pack<T>::width;
+    static_assert(ROW >= W && (PAD == 0 || ROW % W == 0), "padded rows are whole vectors");
+    const T* __restrict__ run;
+    T* staged;
+    unsigned len, threads, last, at;
+    bool vectors;
+    V hold[ROUNDS];
+    __device__ __forceinline__ FixedRows(const T* run_, T* staged_, unsigned points, unsigned tid, unsigned threads_)
+        : run(run_), staged(staged_), len(points * ROW), threads(threads_), last(points * ROW / W - 1u), at(tid),
+          vectors((reinterpret_cast<uintptr_t>(run_) & 15u) == 0) {}
+    __device__ __forceinline__ unsigned clamped(unsigned u) const {
+        const unsigned v = at + u * threads;
+        return v < last ? v : last;
+    }
+    __device__ __forceinline__ void issue() {
+        if (!vectors) return;
+#pragma unroll
+        for (unsigned u = 0; u < ROUNDS; ++u) hold[u] = reinterpret_cast<const V*>(run)[clamped(u)];
+    }
+    __device__ __forceinline__ void put() {
+        if (!vectors) return;
+#pragma unroll
+        for (unsigned u = 0; u < ROUNDS; ++u) {
+            const unsigned v = clamped(u);
+            if constexpr (PAD == 0) {
+                reinterpret_cast<V*>(staged)[v] = hold[u];
+            } else {
+                T* to = staged + v * W + PAD * (v / (ROW / W));
+#pragma unroll
+                for (unsigned e = 0; e < W; ++e) to[e] = hold[u][e];
+            }
+        }
+        at += ROUNDS * threads;
+    }
+    // what the first issue() and put() have left
+    __device__ __forceinline__ void rest(unsigned tid) {
+        if (!vectors) {
+            for (unsigned e = tid; e < len; e += threads) staged[e + PAD * (e / ROW)] = run[e];
+            return;
+        }
+        while (at - tid <= last) { // (the same for all lanes)
+            issue();
+            put();
+        }
+        for (unsigned e = (last + 1u) * W + tid; e < len; e += threads) staged[e] = run[e]; // PAD == 0 here
+    }
+};
+
 // Waves per SIMD that the registers are to allow: what the sums need by themselves. (The compiler allots registers for
 // the whole kernel, and the entry by entry part, which hardly ever runs, would take a wave from each.)
-template <typename T, bool NORM, bool SECOND, int GROUPS> constexpr int columns_residence() {
+template <typename T, bool NORM, bool SECOND, int GROUPS, int LMAX> constexpr int columns_residence() {
+    if (LMAX > 0) return sizeof(T) == 4 ? (SECOND ? 5 : 6) : (SECOND ? 3 : 4); // (a column's loads are under way together)
     if (sizeof(T) == 8 && SECOND) return NORM ? 3 : 4;
     return SECOND && NORM && GROUPS == 2 ? 6 : 7;
 }
@@ -373,8 +458,8 @@ template <typename T, bool NORM, bool SECOND, int GROUPS> constexpr int columns_
 //   out = (P (H g' - a h) - t g' - n (h . g')) / r^2,   g' = P g, a = n . g, t = n . h,
 // and dw = (g' / r) . grad R.
 // ---------------------------------------------------------------------------
-template <typename T, bool NORM, bool SECOND, int GROUPS, bool ADD>
-__global__ __launch_bounds__(kColumnsThreads, (columns_residence<T, NORM, SECOND, GROUPS>())) void columns_kernel(Columns g, const T* __restrict__ xyz, const T* __restrict__ weights,
+template <typename T, bool NORM, bool SECOND, int GROUPS, bool ADD, int LMAX = 0>
+__global__ __launch_bounds__(kColumnsThreads, (columns_residence<T, NORM, SECOND, GROUPS, LMAX>())) void columns_kernel(Columns g, const T* __restrict__ xyz, const T* __restrict__ weights,
                                                      const T* __restrict__ grad, T* __restrict__ out,
                                                      T* __restrict__ dw) {
     constexpr unsigned TILE = 64 / GROUPS;
@@ -384,8 +469,9 @@ __global__ __launch_bounds__(kColumnsThreads, (columns_residence<T, NORM, SECOND
     const unsigned wave = __builtin_amdgcn_readfirstlane(tid >> 6); // the same for all lanes: scalar
     const unsigned threads = blockDim.x;
     const unsigned waves = threads >> 6;
-    const int L = g.l_max;
-    const unsigned ny = g.ny, stride = ny + g.pad;
+    const int L = LMAX > 0 ? LMAX : g.l_max;
+    const unsigned ny = LMAX > 0 ? (LMAX + 1) * (LMAX + 1) : g.ny;
+    const unsigned pad = LMAX > 0 ? columns_pad(sizeof(T), ny) : g.pad, stride = ny + pad;
     // consecutive workgroups go to the XCDs in turn: one contiguous stretch of tiles for each
     const unsigned group = (blockIdx.x & 7u) * g.tiles_per_xcd + (blockIdx.x >> 3);
     if (group >= g.n_tiles) return;
@@ -395,13 +481,27 @@ __global__ __launch_bounds__(kColumnsThreads, (columns_residence<T, NORM, SECOND
     const unsigned point = lane & (TILE - 1u);
     const bool minus = GROUPS == 2 && lane >= TILE;
 
-    rows_to_lds<T>(weights + first * ny, lds, valid * ny, ny, g.pad, g.magic_vectors, tid, threads);
     // lanes past the last point compute on the first one's coordinates and write nothing
     const unsigned mine = point < valid ? point : 0u;
     xyz += first * 3;
     out += first * 3;
     if constexpr (SECOND) grad += first * 3;
-    const Point<T> p = load_point<T, NORM>(xyz + mine * 3u);
+    Point<T> p;
+    if constexpr (LMAX > 0) {
+        constexpr unsigned ROW = (LMAX + 1) * (LMAX + 1);
+        constexpr int KIND = SECOND ? COLUMNS_VJP_BACKWARD : COLUMNS_VJP;
+        // (all loads of the tile under way before the first is waited for)
+        const T raw[3] = {xyz[mine * 3u], xyz[mine * 3u + 1u], xyz[mine * 3u + 2u]};
+        FixedRows<T, ROW, columns_pad(sizeof(T), ROW), column_rounds(KIND, sizeof(T), LMAX, TILE * ROW)> rows(
+            weights + first * ny, lds, valid, tid, threads);
+        rows.issue();
+        p = load_point<T, NORM>(raw);
+        rows.put();
+        rows.rest(tid);
+    } else {
+        rows_to_lds<T>(weights + first * ny, lds, valid * ny, ny, g.pad, g.magic_vectors, tid, threads);
+        p = load_point<T, NORM>(xyz + mine * 3u);
+    }
     T gx = 0, gy = 0, gz = 0, along = 0;
     bool lost_grad = false; // any of the tile's
     if constexpr (SECOND) {
@@ -425,12 +525,9 @@ __global__ __launch_bounds__(kColumnsThreads, (columns_residence<T, NORM, SECOND
 
     PointSums<T, SECOND> sums;
     Azimuth<T> azimuth;
-    Deal deal(waves);
     T* row = lds + point * stride;
-    for (int m = 0; m <= L; ++m) {
-        if (m > 0) azimuth.next(p.x, p.y);
-        if (!deal.next(wave)) continue;
-        const T fm = static_cast<T>(m);
+    auto column = [&](auto m) {
+        const T fm = static_cast<T>(static_cast<int>(m));
         if constexpr (GROUPS == 1) {
             ColumnSums<T> plus, neg;
             T along_plus = 0, along_minus = 0;
@@ -438,7 +535,7 @@ __global__ __launch_bounds__(kColumnsThreads, (columns_residence<T, NORM, SECOND
                 along_plus = fm * fma_of(dx, azimuth.c1, -(dy * azimuth.s1));
                 along_minus = fm * fma_of(dx, azimuth.s1, dy * azimuth.c1);
             }
-            walk_column<T, SECOND>(m, L, p.z, rho2, [&](auto step, int l, T fa, T fb, T fc, T fe, T fg, T fk) {
+            walk_column<T, SECOND, LMAX>(m, L, p.z, rho2, [&](auto step, auto l, T fa, T fb, T fc, T fe, T fg, T fk) {
                 constexpr int S = decltype(step)::value;
                 T* mid = row + l * (l + 1);
                 const T wp = mid[m], wn = mid[-m];
@@ -463,7 +560,7 @@ __global__ __launch_bounds__(kColumnsThreads, (columns_residence<T, NORM, SECOND
             const T along_u = SECOND ? fm * fma_of(dx, u1, dy * w1) : T(0);
             const bool writes = m > 0 || !minus; // (m = 0 is one entry)
             T* at = row + (minus ? -m : m);
-            walk_column<T, SECOND>(m, L, p.z, rho2, [&](auto step, int l, T fa, T fb, T fc, T fe, T fg, T fk) {
+            walk_column<T, SECOND, LMAX>(m, L, p.z, rho2, [&](auto step, auto l, T fa, T fb, T fc, T fe, T fg, T fk) {
                 constexpr int S = decltype(step)::value;
                 T* here = at + l * (l + 1);
                 k.template add<S, SECOND>(*here, fa, fb, fc, fe, fg, fk);
@@ -475,6 +572,19 @@ __global__ __launch_bounds__(kColumnsThreads, (columns_residence<T, NORM, SECOND
                 }
             });
             sums.add(k, fm, u, u1, w1, u2, w2);
+        }
+    };
+    if constexpr (LMAX > 0) {
+        const unsigned mine = columns_of(wave, waves, LMAX);
+        each_of(std::make_integer_sequence<int, LMAX + 1>{}, [&](auto m) {
+            if constexpr (m.value > 0) azimuth.next(p.x, p.y);
+            if ((mine >> m.value) & 1u) column(m);
+        });
+    } else {
+        Deal deal(waves);
+        for (int m = 0; m <= L; ++m) {
+            if (m > 0) azimuth.next(p.x, p.y);
+            if (deal.next(wave)) column(m);
         }
     }
 
@@ -552,10 +662,10 @@ __global__ __launch_bounds__(kColumnsThreads, (columns_residence<T, NORM, SECOND
         }
     }
     if constexpr (SECOND) {
-        if (g.pad == 0) {
+        if (pad == 0) {
             copy_out<T, SPHX_STREAMING_STORES, false>(lds, dw + first * ny, valid * ny, ny, 0, 0, tid, threads);
         } else {
-            copy_out<T, SPHX_STREAMING_STORES, true>(lds, dw + first * ny, valid * ny, ny, g.pad, g.magic_ny, tid, threads);
+            copy_out<T, SPHX_STREAMING_STORES, true>(lds, dw + first * ny, valid * ny, ny, pad, g.magic_ny, tid, threads);
         }
     }
     if constexpr (SECOND) {
@@ -608,7 +718,7 @@ __global__ __launch_bounds__(kColumnsThreads, (columns_residence<T, NORM, SECOND
 // and n . d = l R_k (R_k is homogeneous of degree l): the sets are p_x, p_y, p_z and w r - s, and one more sum per set,
 // of l w F Q, serves the second term.
 // ---------------------------------------------------------------------------
-template <typename T, bool NORM>
+template <typename T, bool NORM, int LMAX = 0>
 __global__ __launch_bounds__(kColumnsThreads) void column_rows_kernel(Columns g, const T* __restrict__ xyz, const T* __restrict__ w,
                                                          const T* __restrict__ v, T* __restrict__ out) {
     constexpr unsigned TILE = 16;
@@ -618,8 +728,9 @@ __global__ __launch_bounds__(kColumnsThreads) void column_rows_kernel(Columns g,
     const unsigned wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const unsigned threads = blockDim.x;
     const unsigned waves = threads >> 6;
-    const int L = g.l_max;
-    const unsigned ny = g.ny, w_stride = ny + g.pad, v_stride = 3u * ny + g.pad;
+    const int L = LMAX > 0 ? LMAX : g.l_max;
+    const unsigned ny = LMAX > 0 ? (LMAX + 1) * (LMAX + 1) : g.ny;
+    const unsigned pad = LMAX > 0 ? columns_pad(sizeof(T), ny) : g.pad, w_stride = ny + pad, v_stride = 3u * ny + pad;
     const unsigned group = (blockIdx.x & 7u) * g.tiles_per_xcd + (blockIdx.x >> 3);
     if (group >= g.n_tiles) return;
     const unsigned long long first = static_cast<unsigned long long>(group) * TILE;
@@ -631,16 +742,40 @@ __global__ __launch_bounds__(kColumnsThreads) void column_rows_kernel(Columns g,
     const bool have_w = w != nullptr;
 
     T* w_rows = lds + g.off_rows;
-    rows_to_lds<T>(v + first * 3u * ny, lds, valid * 3u * ny, 3u * ny, g.pad, g.magic_vectors3, tid, threads);
-    if (have_w) {
-        rows_to_lds<T>(w + first * ny, w_rows, valid * ny, ny, g.pad, g.magic_vectors, tid, threads);
-    } else {
-        for (unsigned e = tid; e < TILE * w_stride; e += threads) w_rows[e] = 0;
-    }
     const unsigned mine = point < valid ? point : 0u;
     xyz += first * 3;
     out += first * 3;
-    const Point<T> p = load_point<T, NORM>(xyz + mine * 3u);
+    Point<T> p;
+    auto no_weights = [&]() {
+        for (unsigned e = tid; e < TILE * w_stride; e += threads) w_rows[e] = 0;
+    };
+    if constexpr (LMAX > 0) {
+        constexpr unsigned ROW = (LMAX + 1) * (LMAX + 1), PAD = columns_pad(sizeof(T), ROW);
+        const T raw[3] = {xyz[mine * 3u], xyz[mine * 3u + 1u], xyz[mine * 3u + 2u]};
+        FixedRows<T, 3u * ROW, PAD, column_rounds(COLUMNS_ROWS, sizeof(T), LMAX, TILE * 3u * ROW)> three(
+            v + first * 3u * ny, lds, valid, tid, threads);
+        FixedRows<T, ROW, PAD, column_rounds(COLUMNS_ROWS, sizeof(T), LMAX, TILE * ROW)> one(
+            have_w ? w + first * ny : three.run, w_rows, valid, tid, threads);
+        three.issue();
+        one.issue();
+        p = load_point<T, NORM>(raw);
+        three.put();
+        if (have_w) {
+            one.put();
+            one.rest(tid);
+        } else {
+            no_weights();
+        }
+        three.rest(tid);
+    } else {
+        rows_to_lds<T>(v + first * 3u * ny, lds, valid * 3u * ny, 3u * ny, g.pad, g.magic_vectors3, tid, threads);
+        if (have_w) {
+            rows_to_lds<T>(w + first * ny, w_rows, valid * ny, ny, g.pad, g.magic_vectors, tid, threads);
+        } else {
+            no_weights();
+        }
+        p = load_point<T, NORM>(xyz + mine * 3u);
+    }
     const T rho2 = p.x2 + p.y2;
     // set 0 = v_a - n_a s with a = x or z; set 1 = v_y - y s or w r - s
     const T n0 = second_half ? p.z : p.x, n1 = second_half ? T(1) : p.y;
@@ -650,25 +785,22 @@ __global__ __launch_bounds__(kColumnsThreads) void column_rows_kernel(Columns g,
     PointSums<T, true> sums0, sums1;
     T euler0 = 0, euler1 = 0; // sum of l times the set's values
     Azimuth<T> azimuth;
-    Deal deal(waves);
     const T* v_row = lds + point * v_stride;
     const T* w_row = w_rows + point * w_stride;
-    for (int m = 0; m <= L; ++m) {
-        if (m > 0) azimuth.next(p.x, p.y);
-        if (!deal.next(wave)) continue;
-        const T fm = static_cast<T>(m);
+    auto column = [&](auto m) {
+        const T fm = static_cast<T>(static_cast<int>(m));
         // (m = 0 is one entry: it has s_0 = 0 and m = 0 for factors on the minus side)
         const T u = minus ? azimuth.s : azimuth.c;
         const T u1 = minus ? azimuth.s1 : azimuth.c1, w1 = minus ? azimuth.c1 : -azimuth.s1;
         const T u2 = minus ? azimuth.s2 : azimuth.c2, w2 = minus ? azimuth.c2 : -azimuth.s2;
-        const int side = minus ? -m : m;
+        const int side = minus ? -static_cast<int>(m) : static_cast<int>(m);
         const T* v_at = v_row + side;
         const T* w_at = w_row + side;
         const T* at0 = v_at + (second_half ? 2u * ny : 0u);
         const T* at1 = second_half ? w_at : v_at + ny;
         ColumnSums<T> k0, k1;
         T le0 = 0, le1 = 0;
-        walk_column<T, true>(m, L, p.z, rho2, [&](auto step, int l, T fa, T fb, T fc, T fe, T fg, T fk) {
+        walk_column<T, true, LMAX>(m, L, p.z, rho2, [&](auto step, auto l, T fa, T fb, T fc, T fe, T fg, T fk) {
             constexpr int S = decltype(step)::value;
             const int at = l * (l + 1);
             T set0, set1;
@@ -693,6 +825,19 @@ __global__ __launch_bounds__(kColumnsThreads) void column_rows_kernel(Columns g,
         if constexpr (NORM) {
             euler0 = fma_of(le0, u, euler0);
             euler1 = fma_of(le1, u, euler1);
+        }
+    };
+    if constexpr (LMAX > 0) {
+        const unsigned mine = columns_of(wave, waves, LMAX);
+        each_of(std::make_integer_sequence<int, LMAX + 1>{}, [&](auto m) {
+            if constexpr (m.value > 0) azimuth.next(p.x, p.y);
+            if ((mine >> m.value) & 1u) column(m);
+        });
+    } else {
+        Deal deal(waves);
+        for (int m = 0; m <= L; ++m) {
+            if (m > 0) azimuth.next(p.x, p.y);
+            if (deal.next(wave)) column(m);
         }
     }
 

@@ -49,6 +49,12 @@ static int prepare_device(int device) {
     SPHX_HIP(upload_vjp_tables<double>(t));
     SPHX_HIP(upload_column_tables<float>(t));
     SPHX_HIP(upload_column_tables<double>(t));
+    SPHX_HIP((upload_fixed_columns<float, COLUMNS_VJP>(t)));
+    SPHX_HIP((upload_fixed_columns<float, COLUMNS_VJP_BACKWARD>(t)));
+    SPHX_HIP((upload_fixed_columns<float, COLUMNS_ROWS>(t)));
+    SPHX_HIP((upload_fixed_columns<double, COLUMNS_VJP>(t)));
+    SPHX_HIP((upload_fixed_columns<double, COLUMNS_VJP_BACKWARD>(t)));
+    SPHX_HIP((upload_fixed_columns<double, COLUMNS_ROWS>(t)));
     SPHX_HIP(hipDeviceGetAttribute(&fresh.lds_limit, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
     SPHX_HIP(hipDeviceGetAttribute(&fresh.compute_units, hipDeviceAttributeMultiprocessorCount, device));
     // The kernels deal their workgroups to eight XCDs (`blockIdx.x & 7`): on a device partitioned

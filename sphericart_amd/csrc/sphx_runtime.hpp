@@ -103,6 +103,11 @@ template <typename T>
 hipError_t dispatch_columns(ColumnsKind kind, const ColumnsLaunch& launch, bool normalized, const T* xyz, const T* sph_grad,
                             const T* upstream, T* xyz_grad, T* sph_grad_grad, hipStream_t stream);
 template <typename T> hipError_t upload_column_tables(const HostTables& t);
+// The same kernels with l_max a compile-time number, for the l_max that fixed_columns() names.
+template <typename T, int KIND>
+hipError_t dispatch_columns_fixed(const ColumnsLaunch& launch, bool normalized, const T* xyz, const T* sph_grad,
+                                  const T* upstream, T* xyz_grad, T* sph_grad_grad, hipStream_t stream);
+template <typename T, int KIND> hipError_t upload_fixed_columns(const HostTables& t);
 // Each of those translation units has the constant tables of its arithmetic type to itself; these fill them
 // on the current device. `F` / `Q` (may be null) receive the device addresses.
 template <typename T, int MODE> hipError_t upload_forward_tables(const HostTables& t, const T** F, const T** Q);

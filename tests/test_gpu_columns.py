@@ -101,6 +101,45 @@ def test_second_order_products_equal_the_oracles_arrays_contracted(library, orac
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("l_max", range(1, 22))
+def test_kernels_with_l_max_for_a_constant(library, oracle, dtype, l_max, switches):
+    """Every l_max that has such a kernel (product 7-20, second-order products 1-12) and the neighbours that do not, both
+    parities of the row length; a point less and more than a tile of 16, 32, 64; as planned and with numbers of waves that
+    are no power of two or take more vectors per lane than the kernel has under way at a time; weights on and off 16 bytes."""
+    suffix = "f32" if dtype == np.float32 else "f64"
+    vjp, backward, rows = (getattr(library, f"sphx_{name}_{suffix}") for name in ("vjp", "vjp_backward", "gradients_backward"))
+    stream, rng = torch.cuda.current_stream().cuda_stream, np.random.default_rng(l_max)
+    ny, tolerance, normalized = (l_max + 1) ** 2, _tolerance(dtype, l_max), l_max % 3 != 0
+    for n, waves, tile in ((1, 0, 0), (15, 1, 64), (31, 3, 32), (65, 5, 64), (129, 2, 0)):
+        announce("fixed l_max", suffix, l_max, n, waves, tile)
+        switches("SPHX_COLUMNS_WAVES", waves)
+        switches("SPHX_COLUMNS_TILE", tile)
+        xyz = _cloud(n, dtype, n)
+        w, g, v = (rng.standard_normal(shape).astype(dtype) for shape in ((n, ny), (n, 3), (n, 3, ny)))
+        hess_w, dw, hess_v, grad_w = _expected(oracle, xyz, l_max, normalized, w, g, v)
+        d_xyz, d_g = torch.from_numpy(xyz).cuda(), torch.from_numpy(g).cuda()
+        w_holder, v_holder = (torch.zeros(a.size + 1, dtype=d_xyz.dtype, device="cuda") for a in (w, v))
+        shape = (n, l_max, int(normalized))
+        for shift in (0, 1):
+            d_w = w_holder[shift:shift + w.size].view(w.shape)
+            d_v = v_holder[1 - shift:1 - shift + v.size].view(v.shape)
+            d_w.copy_(torch.from_numpy(w))
+            d_v.copy_(torch.from_numpy(v))
+            out, out_w = torch.full_like(d_xyz, float("nan")), torch.full((n, ny), float("nan"), dtype=d_xyz.dtype, device="cuda")
+            assert vjp(d_xyz.data_ptr(), d_w.data_ptr(), *shape, out.data_ptr(), 0, stream) == 0
+            _close(out, *grad_w, tolerance, (l_max, n, shift, "product"))
+            if l_max > 14:
+                continue
+            assert backward(d_xyz.data_ptr(), d_w.data_ptr(), d_g.data_ptr(), *shape, out.data_ptr(), out_w.data_ptr(), stream) == 0
+            _close(out, *hess_w, tolerance, (l_max, n, shift, "xyz_grad"))
+            _close(out_w, *dw, tolerance, (l_max, n, shift, "sph_grad_grad"))
+            for upstream, pointer in ((True, d_w.data_ptr()), (False, None)):
+                out = torch.full_like(d_xyz, float("nan"))
+                assert rows(d_xyz.data_ptr(), pointer, d_v.data_ptr(), *shape, out.data_ptr(), stream) == 0
+                _close(out, hess_v[0] + upstream * grad_w[0], hess_v[1] + upstream * grad_w[1], tolerance, (l_max, n, shift, upstream))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_second_order_products_of_large_calls(library, oracle, dtype):
     """The plans of calls with more than 64 points for every CU, as they are made: 64-point tiles and few waves for the
     product's derivatives, the rows' waves by l_max."""
