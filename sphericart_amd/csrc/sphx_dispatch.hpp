@@ -134,6 +134,7 @@ static hipError_t dispatch(const Plan& plan, const DeviceState& device, const T*
         }
         if constexpr (MODE == 1) {
             const Launch& l = plan.closed;
+            if (l.g.fixed != 0) return dispatch_gradients_fixed<T>(l, NORM, xyz, sph, dsph, stream);
             if (l.g.l_max < 4) return hipErrorInvalidValue; // never planned
             if (l.threads > (l.g.l_max >= 6 ? 1024u : 512u)) return hipErrorInvalidValue; // never planned
             auto kernel = l.g.l_max >= 6   ? (l.threads > 512 ? gradients_lanes_kernel<T, NORM, 6, 1024>

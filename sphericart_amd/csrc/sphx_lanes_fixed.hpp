@@ -1,0 +1,70 @@
+// What the planner and gradients_fixed_kernel both need to know: which l_max it exists for, how a workgroup's work is cut
+// into units and dealt to its waves, how the rows lie in LDS. Plain C++.
+#ifndef SPHX_LANES_FIXED_HPP
+#define SPHX_LANES_FIXED_HPP
+
+#include <cstddef>
+
+namespace sphx {
+
+// l_max of the kernels
+constexpr int kGradientsFixedFirst = 7;
+constexpr int gradients_fixed_last(size_t elem) { return elem == 4 ? 18 : 15; }
+constexpr bool gradients_fixed(size_t elem, int l_max) {
+    return l_max >= kGradientsFixedFirst && l_max <= gradients_fixed_last(elem);
+}
+constexpr unsigned kGradientsFixedPoints = 32; // the most points of a tile: two lanes each
+
+// elements left free after the rows of a point (ny of the values, 3 ny of the gradients): where ny is even, a multiple of
+// four, rows 8 bytes further apart start on 32 different pairs of banks and can still be read 8 bytes at a time
+constexpr unsigned gradients_fixed_pad(size_t elem, unsigned ny) { return ny % 2u == 0u ? 8u / static_cast<unsigned>(elem) : 0u; }
+
+// The units of a tile's work: the closed forms of l <= 6 in eight slices, then the channels from l_max down, each whole or in
+// two parts, the upper half of its m and the lower one, which runs the recursions bare down to where it begins.
+constexpr int kClosedSlices = 8;
+constexpr int gradients_fixed_parts(int l_max, int waves) { return l_max <= 11 || waves > 8 ? 2 : 1; }
+constexpr int gradients_fixed_units(int l_max, int waves) { return kClosedSlices + (l_max - 6) * gradients_fixed_parts(l_max, waves); }
+struct ChannelPart {
+    int l, m_top, m_bottom;
+};
+constexpr ChannelPart channel_part(int l_max, int waves, int unit) {
+    const int parts = gradients_fixed_parts(l_max, waves), i = unit - kClosedSlices, l = l_max - i / parts;
+    if (parts == 1) return {l, l, 0};
+    return i % 2 == 0 ? ChannelPart{l, l, l / 2} : ChannelPart{l, l / 2 - 1, 0};
+}
+// instructions of a unit, roughly
+constexpr int unit_cost(bool normalized, int l_max, int waves, int unit) {
+    if (unit < kClosedSlices) return normalized ? 190 : 110;
+    const ChannelPart c = channel_part(l_max, waves, unit);
+    return (normalized ? 44 : 30) * (c.m_top - c.m_bottom + 1) + 8 * (c.l - c.m_top) + 20;
+}
+
+// Which units each of `waves` waves takes, one bit each: the longest unit left to the wave with the least so far.
+constexpr int kFixedMostWaves = 16;
+struct UnitMasks {
+    unsigned of[kFixedMostWaves];
+};
+constexpr UnitMasks deal_units(bool normalized, int l_max, int waves) {
+    UnitMasks masks{};
+    int load[kFixedMostWaves] = {};
+    bool taken[32] = {};
+    const int units = gradients_fixed_units(l_max, waves);
+    for (int round = 0; round < units; ++round) {
+        int longest = -1;
+        for (int u = 0; u < units; ++u) {
+            if (!taken[u] && (longest < 0 || unit_cost(normalized, l_max, waves, u) > unit_cost(normalized, l_max, waves, longest))) longest = u;
+        }
+        int least = 0;
+        for (int w = 1; w < waves; ++w) {
+            if (load[w] < load[least]) least = w;
+        }
+        taken[longest] = true;
+        load[least] += unit_cost(normalized, l_max, waves, longest);
+        masks.of[least] |= 1u << longest;
+    }
+    return masks;
+}
+
+} // namespace sphx
+
+#endif

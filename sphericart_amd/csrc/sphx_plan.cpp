@@ -8,6 +8,7 @@
 #include <mutex>
 
 #include "../../include/sphx_launch.h"
+#include "sphx_lanes_fixed.hpp"
 #include "sphx_plan_shapes.hpp"
 
 namespace sphx {
@@ -20,7 +21,7 @@ int fail(int code, const std::string& what) {
 }
 
 static const char* const kSwitchNames[SW_COUNT] = {
-    "SPHX_AZ_SHIFT", "SPHX_CHUNK_SHIFT", "SPHX_COLUMNS_TILE", "SPHX_COLUMNS_WAVES", "SPHX_GRADIENT_LANES",
+    "SPHX_AZ_SHIFT", "SPHX_CHUNK_SHIFT", "SPHX_COLUMNS_TILE", "SPHX_COLUMNS_WAVES", "SPHX_GRADIENT_LANES", "SPHX_GRADIENT_LANES_FIXED",
     "SPHX_GRADIENT_LANES_PARTS", "SPHX_GRADIENT_LANES_TILE", "SPHX_GRADIENT_LANES_WAVES", "SPHX_GROUP_THREADS",
     "SPHX_HESSIAN_LANES",
     "SPHX_HESSIAN_LANES_PARTS", "SPHX_HESSIAN_LANES_TILE", "SPHX_JOB_LIST",
@@ -256,6 +257,69 @@ static bool plan_values(size_t n_samples, int l_max, size_t elem, int lds_limit,
     int want = (l_max - 6 + static_cast<int>(pack) - 1) / static_cast<int>(pack);
     if (!with_sums && want < 2) want = switch_or(SW_VALUES_MIN_WAVES, 2);
     out->threads = 64u * static_cast<unsigned>(want < waves ? want : waves);
+    out->lds_bytes = bytes;
+    return true;
+}
+
+// gradients_fixed_kernel: the rows of up to 32 points per workgroup in LDS. SPHX_GRADIENT_LANES_FIXED: 0 never, 2 wherever
+// there is a kernel.
+static bool plan_gradients_fixed(size_t n_samples, int l_max, size_t elem, int lds_limit, int cus, bool normalized, Launch* out) {
+    const int wanted = switch_or(SW_GRADIENT_LANES_FIXED, 1);
+    if (wanted == 0 || !gradients_fixed(elem, l_max)) return false;
+    Tiling& g = out->g;
+    std::memset(&g, 0, sizeof(g));
+    const unsigned esize = static_cast<unsigned>(elem), vec = 16u / esize;
+    const unsigned ny = static_cast<unsigned>(l_max + 1) * (l_max + 1), pad = gradients_fixed_pad(elem, ny);
+    unsigned off_d = 0;
+    auto bytes_of = [&](unsigned t) {
+        off_d = (t * (ny + pad) + vec - 1u) / vec * vec;
+        return (off_d + t * (3u * ny + pad)) * esize;
+    };
+    const unsigned limit = static_cast<unsigned>(lds_limit);
+    const unsigned forced = static_cast<unsigned>(switch_or(SW_GRADIENT_LANES_TILE, 0));
+    unsigned tile = 0, waves = 8;
+    // Calls that one round of workgroups takes: as few of them per CU as hold the points, each with an equal share (a multiple
+    // of four: whole vectors), at least eight. A workgroup that has its CU to itself has sixteen waves where there are enough
+    // units of work for them and a channel is long (l_max = 8, 6 000 points, float32 4.46 with eight, 4.30 with sixteen; 7
+    // 3.92 4.19; 10 5.41 5.15; 13 6.39 6.75: from l_max = 12 eight waves take a channel whole, without the bare steps).
+    for (unsigned beside = 1; cus > 0 && forced != 1u && beside <= 4u; ++beside) {
+        const size_t share = static_cast<size_t>(cus) * beside;
+        const size_t t = ((n_samples + share - 1) / share + 3u) & ~static_cast<size_t>(3u);
+        if (t > kGradientsFixedPoints) continue;
+        const unsigned few = t < 8u ? 8u : static_cast<unsigned>(t);
+        // (LDS is handed out in pieces of 1 280 bytes)
+        if (beside * ((bytes_of(few) + 1279u) / 1280u * 1280u) > limit) continue;
+        tile = few;
+        waves = beside == 1u && l_max >= 8 && l_max <= 11 ? 16u : 8u;
+        break;
+    }
+    if (tile == 0) {
+        for (const FixedGradientsRow& row : kFixedGradientsRows) {
+            if (row.elem != static_cast<int>(elem) || l_max < row.l_from || l_max > row.l_to || n_samples < row.points_from) continue;
+            if (row.harmonics >= 0 && row.harmonics != static_cast<int>(normalized)) continue;
+            tile = row.tile;
+            waves = row.waves;
+            break;
+        }
+        if (tile == 0 && wanted == 2) {
+            tile = kGradientsFixedPoints;
+            while (tile > 8u && bytes_of(tile) > limit / 2u) tile -= 4u;
+        }
+    }
+    if (forced >= 4u && forced <= kGradientsFixedPoints) tile = forced;
+    if (tile == 0) return false;
+    const unsigned bytes = bytes_of(tile);
+    if (bytes > limit || ((n_samples + tile - 1) / tile + 7u) / 8u * 8u > 0xffffffffull / 1024u) return false; // (fewer than 2^32 threads)
+    g.n_samples = n_samples;
+    g.l_max = l_max;
+    g.ny = static_cast<int>(ny);
+    g.tile = static_cast<int>(tile);
+    g.n_tiles = static_cast<unsigned>((n_samples + tile - 1) / tile);
+    g.tiles_per_xcd = (g.n_tiles + 7u) / 8u;
+    g.off_dsph = off_d;
+    g.fixed = 1u;
+    out->workgroups = g.tiles_per_xcd * 8u;
+    out->threads = switch_or(SW_GRADIENT_LANES_WAVES, static_cast<int>(waves)) > 8 ? 1024u : 512u;
     out->lds_bytes = bytes;
     return true;
 }
@@ -940,13 +1004,20 @@ int make_plan(size_t n_samples, int l_max, int mode, size_t elem, int lds_limit,
             }
         }
     }
-    // Gradients just above the closed forms: the lanes kernel (one point per lane, the channels dealt to the
+    // Gradients just above the closed forms: the kernels that have l_max for a constant, where they were measured ahead
+    // (sphx_plan_shapes.hpp).
+    const int gradient_lanes = switch_or(SW_GRADIENT_LANES, 1);
+    if (lane_kernels && mode == 1 && gradient_lanes != 0 && switch_or(SW_TILE, 0) == 0 &&
+        plan_gradients_fixed(n_samples, l_max, elem, lds_limit, cus, normalized, &plan->closed)) {
+        plan->lanes = true;
+        return SPHX_OK;
+    }
+    // Without those: the lanes kernel (one point per lane, the channels dealt to the
     // waves) up to l_max = 13 in float32 and wherever its tiles fit in float64; from there the recursion kernel with
     // its jobs as a list ordered by kind is ahead. Where the recursion kernel runs in workgroups of 1024 threads
     // (calls of 32 768 points or more) it is ahead from l_max = 8 on (3-20 %): the lanes keep l_max = 7; at
     // 20 000 points from l_max = 10 on (6-30 %).
     // SPHX_GRADIENT_LANES: 0 never, 2 wherever the rows fit.
-    const int gradient_lanes = switch_or(SW_GRADIENT_LANES, 1);
     const bool large_groups = group_threads(n_samples, mode, elem, lane_kernels) > kRecursionThreads && n_samples >= 32768;
     // (float64, normalised, l_max = 7: the recursion kernel is 8 % ahead there, 203 against 219 us per 1.2 GB)
     const bool lanes_by_shape = large_groups ? l_max <= (elem == 8 && normalized ? 6 : 7)
@@ -1056,7 +1127,7 @@ std::string describe(const Plan& plan, int l_max, int mode, bool is_f64, bool no
     const std::string t = is_f64 ? "double" : "float";
     const std::string head = t + ", " + std::to_string(mode) + ", " + (normalized ? "true" : "false");
     auto geometry = [](const Launch& l) {
-        return " [" + std::to_string(l.g.tile) + " points per tile, " + std::to_string(l.threads) + " threads, " +
+        return std::string(l.g.fixed != 0 ? " [l_max a constant, " : " [") + std::to_string(l.g.tile) + " points per tile, " + std::to_string(l.threads) + " threads, " +
                std::to_string(l.lds_bytes) + " B LDS, " + std::to_string(l.workgroups) + " workgroups]";
     };
     std::string text;

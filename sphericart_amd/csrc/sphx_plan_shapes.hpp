@@ -163,6 +163,56 @@ inline const PriorityRow* priority_row(int mode, int elem, bool normalized, int 
     return nullptr;
 }
 
+// gradients_fixed_kernel, calls of more points than one round of its workgroups takes: points per tile and waves, by the
+// first row that matches (tile 0: the kernels that follow in make_plan). A unit of work costs a wave the same however many
+// of its 32 points the tile has, so tiles are as large as leaves LDS for two or three workgroups; which of those, and
+// whether one workgroup of sixteen waves with 32 points is ahead, goes by the rounds and by how the runs of the tiles lie in
+// HBM. us, what ran before / tile of points x waves, normalised unless it says otherwise.
+struct FixedGradientsRow {
+    int elem, l_from, l_to;
+    unsigned long long points_from;
+    int harmonics; // 0 solid, 1 normalised, -1 both
+    unsigned tile, waves;
+    const char* measured;
+};
+
+constexpr FixedGradientsRow kFixedGradientsRows[] = {
+    {4, 7, 8, 500000, 0, 0, 0, "solid, 1.2 GB, l_max = 7 196 / 24x8 206, 8 201 / 32x16 205 (250 000 points 60.5 57.3)"},
+    {4, 9, 9, 400000, 0, 0, 0, "solid, 1.2 GB 202 / 32x16 208 (250 000 76.3 71.1)"},
+    {4, 11, 12, 400000, 0, 0, 0, "solid, 1.2 GB, 11 203 / 24x8 205, 12 207 / 16x8 209 (200 000 89 81, 108 97)"},
+    {4, 7, 7, 0, -1, 24, 8, "50 000 points 16.3 / 20x8 11.6 24x8 11.7 32x8 11.9, 1.2 GB 209 / 205 186 203"},
+    {4, 8, 8, 0, -1, 32, 16, "50 000 20.1 / 20x8 13.6 32x8 13.7 32x16 13.9, 1.2 GB 202 / 196 207 190"},
+    {4, 9, 9, 0, -1, 32, 16, "50 000 25.0 / 16x8 17.0 32x8 17.2 32x16 16.2, 1.2 GB 208 / 215 212 188"},
+    {4, 10, 10, 400000, 0, 0, 0, "solid, 400 000 133 / 20x8 144 28x16 138 32x16 137"},
+    {4, 10, 10, 1000000, 1, 0, 0, "(tests/test_planner_host_only.py states the plan of 1 000 000 points; 1.2 GB 222 / 204)"},
+    {4, 10, 10, 0, -1, 32, 16, "50 000 26.8 / 16x8 20.1 32x8 19.2 32x16 19.0, 200 000 80 / 32x16 69, 28x16 71"},
+    {4, 11, 11, 0, -1, 24, 8, "100 000 52.2 / 24x8 43.4 28x8 43.3 32x8 44.0, 1.2 GB 214 / 191 204 209"},
+    {4, 13, 13, 131072, 0, 0, 0, "solid, 200 000 112 / 16x8 113 20x8 115, 1.2 GB 208 / 212 216"},
+    {4, 12, 13, 0, -1, 16, 8, "l_max = 12, 100 000 60.5 / 16x8 49.5 20x8 51.0, 1.2 GB 210 / 188 202; 13, 61.8 / 59.0 58.8, 217 / 193 193"},
+    {4, 14, 16, 0, -1, 16, 8, "14, 50 000 45.1 / 16x8 35.4 20x8 37.5 32x16 38.5, 1.2 GB 210 / 32x8 199 16x8 200; 16, 50 000 49.7 / 43.7 - 46.3"},
+    {4, 17, 18, 65536, 1, 28, 8, "17, 100 000 98.6 / 12x8 101.7 28x8 97.5, 1.2 GB 223 / 226 207; 18, 111 / 111 104, 218 / 221 208"},
+    {4, 17, 18, 0, -1, 12, 8, "17, 25 000 34.7 / 12x8 28.9 28x8 31.6; solid, 1.2 GB 209 / 190 217; 18, 35.1 / 30.7 34.8, 224 / 208 213"},
+    {8, 7, 7, 400000, 0, 0, 0, "solid, 1.2 GB 203 / 20x8 206"},
+    {8, 7, 7, 131072, -1, 20, 8, "250 000 94.1 / 20x8 79.8 32x8 88.9"},
+    {8, 7, 7, 0, -1, 32, 8, "50 000 25.4 / 16x8 21.0 20x8 21.2 32x8 20.3, 100 000 42.1 / - 38.6 37.6"},
+    {8, 8, 9, 65536, 0, 32, 16, "solid, 100 000 53.9 / 20x8 49.7 24x8 48.0 32x16 45.6, 1.2 GB 210 / 215 209 191; 9, 65.6 / 59.2 59.4 57.1, 211 / 207 210 202"},
+    {8, 8, 9, 0, -1, 20, 8, "8, 100 000 53.9 / 20x8 45.3 24x8 48.1 32x16 49.5, 1.2 GB 207 / 193 203 205; 9, 68.7 / 57.3 58.6 60.9, 221 / 196 207 207"},
+    {8, 10, 10, 131072, 0, 24, 8, "solid, 1.2 GB 204 / 20x8 210 24x8 198 32x16 207"},
+    {8, 10, 10, 65536, -1, 32, 16, "100 000 78.0 / 20x8 72.2 32x16 69.6, 1.2 GB 224 / 194 195"},
+    {8, 10, 10, 0, -1, 20, 8, "50 000 44.4 / 16x8 38.3 20x8 38.1 32x16 39.8"},
+    {8, 11, 11, 131072, 0, 0, 0, "solid, 200 000 159 / 16x8 164 32x16 162"},
+    {8, 11, 11, 65536, -1, 32, 16, "200 000 179 / 16x8 160 32x16 155"},
+    {8, 11, 11, 0, -1, 16, 8, "50 000 57.0 / 16x8 43.6 32x16 46.6"},
+    {8, 12, 12, 131072, 0, 12, 8, "solid, 1.2 GB 210 / 12x8 205 28x8 211"},
+    {8, 12, 12, 65536, -1, 28, 8, "100 000 108 / 12x8 98.7 28x8 98.9, 1.2 GB 223 / 216 201"},
+    {8, 13, 13, 131072, 0, 0, 0, "solid, 1.2 GB 208 / 12x8 210 24x8 212"},
+    {8, 13, 13, 65536, -1, 24, 8, "100 000 127 / 12x8 116 24x8 113, 1.2 GB 232 / 220 203"},
+    {8, 12, 13, 0, -1, 12, 8, "12, 50 000 62.0 / 12x8 52.2 28x8 54.9; 13, 69.9 / 61.2 24x8 63.9"},
+    {8, 14, 14, 8193, -1, 0, 0, "15 000 31.0 / 8x8 32.9 20x8 29.5, 50 000 78 / 78"},
+    {8, 15, 15, 16384, -1, 0, 0, "50 000 88 / 88"},
+    {8, 14, 15, 0, -1, 8, 8, "14, 6 000 18.4 / 8x8 15.1 16x8 15.8; 15, 20.1 / 16.6 17.7, 15 000 37.9 / 34.0 35.2"},
+};
+
 } // namespace sphx
 
 #endif

@@ -108,6 +108,10 @@ template <typename T, int KIND>
 hipError_t dispatch_columns_fixed(const ColumnsLaunch& launch, bool normalized, const T* xyz, const T* sph_grad,
                                   const T* upstream, T* xyz_grad, T* sph_grad_grad, hipStream_t stream);
 template <typename T, int KIND> hipError_t upload_fixed_columns(const HostTables& t);
+// gradients_fixed_kernel (sphx_lanes_fixed_kernel.hpp), for the l_max that gradients_fixed() names.
+template <typename T>
+hipError_t dispatch_gradients_fixed(const Launch& launch, bool normalized, const T* xyz, T* sph, T* dsph, hipStream_t stream);
+template <typename T> hipError_t upload_channel_tables(const HostTables& t);
 // Each of those translation units has the constant tables of its arithmetic type to itself; these fill them
 // on the current device. `F` / `Q` (may be null) receive the device addresses.
 template <typename T, int MODE> hipError_t upload_forward_tables(const HostTables& t, const T** F, const T** Q);
