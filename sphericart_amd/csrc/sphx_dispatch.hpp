@@ -78,8 +78,6 @@ static hipError_t launch_recursion(const Launch& l, const typename AsGiven<O>::t
             switch (l.g.l_max) {
             case 4: return with(std::integral_constant<int, 4>{});
             case 5: return with(std::integral_constant<int, 5>{});
-            case 6: return with(std::integral_constant<int, 6>{});
-            case 7: return with(std::integral_constant<int, 7>{});
             default: return hipErrorInvalidValue; // never planned
             }
         }
@@ -152,6 +150,7 @@ static hipError_t dispatch(const Plan& plan, const DeviceState& device, const T*
         }
         if constexpr (MODE == 2) {
             const Launch& l = plan.closed;
+            if (l.g.fixed != 0) return dispatch_hessians_fixed<T>(l, NORM, xyz, sph, dsph, ddsph, stream);
             if (l.threads > hessian_lane_threads<T>()) return hipErrorInvalidValue; // never planned
             auto kernel = hessians_lanes_kernel<T, NORM>;
             if (l.lds_bytes > 64u * 1024u) {

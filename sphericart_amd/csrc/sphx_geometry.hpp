@@ -47,7 +47,7 @@ struct Tiling {
     // in the job table when they are moved to wave boundaries of the entry lanes (0: they follow
     // the bulk without gaps); jobs_per_point then counts the gaps too
     unsigned kind_at[3];
-    unsigned fixed;       // values and gradients: gradients_fixed_kernel, which has l_max for a constant
+    unsigned fixed;       // gradients_fixed_kernel or hessians_fixed_kernel, which have l_max for a constant
     unsigned point_lanes; // recursion_kernel, normalised second derivatives: one point per lane, a job for a whole wave
 };
 

@@ -1,0 +1,9 @@
+// hessians_fixed_kernel in double: a translation unit of its own, so that the kernels of the library compile side by side.
+#include "sphx_hessians_fixed_kernel.hpp"
+
+namespace sphx {
+
+template hipError_t dispatch_hessians_fixed<double>(const Launch&, bool, const double*, double*, double*, double*, hipStream_t);
+template hipError_t upload_hessian_channel_tables<double>(const HostTables&);
+
+} // namespace sphx

@@ -65,6 +65,65 @@ constexpr UnitMasks deal_units(bool normalized, int l_max, int waves) {
     return masks;
 }
 
+// ---- second derivatives --------------------------------------------------------------------------------------
+constexpr int kHessiansFixedFirst = 2;
+// (normalised in float64: from l_max = 8 on the entries need more registers than sixteen waves on a CU leave a lane)
+constexpr int kHessiansFixedLast = 10;
+constexpr int hessians_fixed_last(size_t elem, bool normalized) { return elem == 8 && normalized ? 7 : kHessiansFixedLast; }
+constexpr bool hessians_fixed(size_t elem, int l_max, bool normalized) {
+    return l_max >= kHessiansFixedFirst && l_max <= hessians_fixed_last(elem, normalized);
+}
+
+// The units: l <= 1 in closed form, then the channels l = l_max .. 2, each in equal parts of at most `longest` entries m
+// (an entry is a hundred operations and more, the bare steps down to where a part begins twelve each).
+constexpr int hessians_fixed_longest(int l_max, int waves) {
+    const int entries = (l_max + 1) * (l_max + 2) / 2 - 3, longest = (2 * entries + 3 * waves - 1) / (3 * waves);
+    return longest < 2 ? 2 : longest;
+}
+constexpr int channel_parts(int l_max, int waves, int l) {
+    const int longest = hessians_fixed_longest(l_max, waves);
+    return (l + longest) / longest;
+}
+constexpr int hessians_fixed_units(int l_max, int waves) {
+    int units = 1;
+    for (int l = 2; l <= l_max; ++l) units += channel_parts(l_max, waves, l);
+    return units;
+}
+constexpr ChannelPart hessian_part(int l_max, int waves, int unit) {
+    int i = unit - 1;
+    for (int l = l_max; l >= 2; --l) {
+        const int parts = channel_parts(l_max, waves, l);
+        if (i < parts) return {l, l - i * (l + 1) / parts, l + 1 - (i + 1) * (l + 1) / parts};
+        i -= parts;
+    }
+    return {0, 0, 0};
+}
+constexpr int hessian_unit_cost(bool normalized, int l_max, int waves, int unit) {
+    if (unit == 0) return normalized ? 260 : 60;
+    const ChannelPart c = hessian_part(l_max, waves, unit);
+    return (normalized ? 170 : 65) * (c.m_top - c.m_bottom + 1) + 12 * (c.l - c.m_top) + 20;
+}
+constexpr UnitMasks deal_hessian_units(bool normalized, int l_max, int waves) {
+    UnitMasks masks{};
+    int load[kFixedMostWaves] = {};
+    bool taken[32] = {};
+    const int units = hessians_fixed_units(l_max, waves);
+    for (int round = 0; round < units; ++round) {
+        int longest = -1;
+        for (int u = 0; u < units; ++u) {
+            if (!taken[u] && (longest < 0 || hessian_unit_cost(normalized, l_max, waves, u) > hessian_unit_cost(normalized, l_max, waves, longest))) longest = u;
+        }
+        int least = 0;
+        for (int w = 1; w < waves; ++w) {
+            if (load[w] < load[least]) least = w;
+        }
+        taken[longest] = true;
+        load[least] += hessian_unit_cost(normalized, l_max, waves, longest);
+        masks.of[least] |= 1u << longest;
+    }
+    return masks;
+}
+
 } // namespace sphx
 
 #endif

@@ -49,14 +49,40 @@ template <int... I, typename F> __host__ __device__ __forceinline__ void for_eac
     (f(std::integral_constant<int, I>{}), ...);
 }
 
+// The rows of `points` points, ROW elements each and PAD elements apart, to one run in HBM.
+template <typename T, unsigned ROW, unsigned PAD>
+__device__ __forceinline__ void flush_fixed_rows(const T* staged, T* dst, unsigned points, unsigned tid, unsigned threads) {
+    using V = typename Pack<T>::type;
+    constexpr unsigned W = Pack<T>::width;
+    const unsigned len = points * ROW;
+    if constexpr (PAD == 0) {
+        copy_out<T, SPHX_STREAMING_STORES, false, 1, true>(staged, dst, len, ROW, 0, 0, tid, threads);
+    } else if ((reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
+        typedef T Half __attribute__((ext_vector_type(8 / sizeof(T))));
+        V* out = reinterpret_cast<V*>(dst);
+        const unsigned nvec = len / W; // (a row is a whole number of vectors)
+        for (unsigned v = tid; v < nvec; v += threads) {
+            const Half* from = reinterpret_cast<const Half*>(staged + v * W + PAD * (v / (ROW / W)));
+            const Half a = from[0], b = from[1];
+            V both;
+#pragma unroll
+            for (unsigned e = 0; e < W / 2; ++e) {
+                both[e] = a[e];
+                both[W / 2 + e] = b[e];
+            }
+            emit<T, SPHX_STREAMING_STORES>(both, out + v);
+        }
+    } else {
+        for (unsigned e = tid; e < len; e += threads) dst[e] = staged[e + PAD * (e / ROW)];
+    }
+}
+
 template <typename T, bool NORM, int L, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void gradients_fixed_kernel(Tiling g, const T* __restrict__ xyz, T* __restrict__ sph,
                                                                                T* __restrict__ dsph) {
     constexpr unsigned NY = (L + 1) * (L + 1), PAD = gradients_fixed_pad(sizeof(T), NY);
     constexpr unsigned S_STRIDE = NY + PAD, D_STRIDE = 3 * NY + PAD;
     constexpr int UNITS = gradients_fixed_units(L, WAVES);
-    using V = typename Pack<T>::type;
-    constexpr unsigned W = Pack<T>::width;
     T* lds = reinterpret_cast<T*>(lds_raw);
     const unsigned tid = threadIdx.x;
     const unsigned lane = tid & 63u;
@@ -190,33 +216,8 @@ __global__ __launch_bounds__(64 * WAVES) void gradients_fixed_kernel(Tiling g, c
         }
     }
     __syncthreads(); // the rows
-    // one run of valid * row elements per array
-    auto flush = [&](const T* staged, auto row_elements, T* dst) {
-        constexpr unsigned ROW = decltype(row_elements)::value;
-        const unsigned len = valid * ROW;
-        if constexpr (PAD == 0) {
-            copy_out<T, SPHX_STREAMING_STORES, false, 1, true>(staged, dst, len, ROW, 0, 0, tid, threads);
-        } else if ((reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
-            V* out = reinterpret_cast<V*>(dst);
-            const unsigned nvec = len / W; // (a row is a whole number of vectors)
-            for (unsigned v = tid; v < nvec; v += threads) {
-                typedef T Half __attribute__((ext_vector_type(8 / sizeof(T))));
-                const Half* from = reinterpret_cast<const Half*>(staged + v * W + PAD * (v / (ROW / W)));
-                const Half a = from[0], b = from[1];
-                V both;
-#pragma unroll
-                for (unsigned e = 0; e < W / 2; ++e) {
-                    both[e] = a[e];
-                    both[W / 2 + e] = b[e];
-                }
-                emit<T, SPHX_STREAMING_STORES>(both, out + v);
-            }
-        } else {
-            for (unsigned e = tid; e < len; e += threads) dst[e] = staged[e + PAD * (e / ROW)];
-        }
-    };
-    flush(lds, std::integral_constant<unsigned, NY>{}, sph + first * NY);
-    flush(lds + g.off_dsph, std::integral_constant<unsigned, 3 * NY>{}, dsph + first * 3 * NY);
+    flush_fixed_rows<T, NY, PAD>(lds, sph + first * NY, valid, tid, threads);
+    flush_fixed_rows<T, 3 * NY, PAD>(lds + g.off_dsph, dsph + first * 3 * NY, valid, tid, threads);
 }
 
 template <typename T> static hipError_t fill_channel_table(const HostTables& t) {

@@ -23,8 +23,8 @@ int fail(int code, const std::string& what) {
 static const char* const kSwitchNames[SW_COUNT] = {
     "SPHX_AZ_SHIFT", "SPHX_CHUNK_SHIFT", "SPHX_COLUMNS_TILE", "SPHX_COLUMNS_WAVES", "SPHX_GRADIENT_LANES", "SPHX_GRADIENT_LANES_FIXED",
     "SPHX_GRADIENT_LANES_PARTS", "SPHX_GRADIENT_LANES_TILE", "SPHX_GRADIENT_LANES_WAVES", "SPHX_GROUP_THREADS",
-    "SPHX_HESSIAN_LANES",
-    "SPHX_HESSIAN_LANES_PARTS", "SPHX_HESSIAN_LANES_TILE", "SPHX_JOB_LIST",
+    "SPHX_HESSIAN_LANES", "SPHX_HESSIAN_LANES_FIXED",
+    "SPHX_HESSIAN_LANES_PARTS", "SPHX_HESSIAN_LANES_TILE", "SPHX_HESSIAN_LANES_WAVES", "SPHX_JOB_LIST",
     "SPHX_PAIRS", "SPHX_PAIRS_BATCH", "SPHX_PAIRS_CHUNK", "SPHX_PAIRS_PREP_WAVES", "SPHX_PAIRS_SEQUENCE_WAVES", "SPHX_PAIRS_TILE",
     "SPHX_POINT_LANES", "SPHX_PREFIX_INSIDE", "SPHX_RECURSIONS_TOGETHER", "SPHX_ROW_PAD", "SPHX_SEQUENCE_WAVES", "SPHX_SLICE_WAVES", "SPHX_SPLIT_BELOW",
     "SPHX_SPLIT_RATIO", "SPHX_SPLIT_SIDES", "SPHX_SPREAD_KINDS", "SPHX_TILE", "SPHX_TILE_LDS_BUDGET", "SPHX_TILE_POW2",
@@ -261,27 +261,38 @@ static bool plan_values(size_t n_samples, int l_max, size_t elem, int lds_limit,
     return true;
 }
 
-// gradients_fixed_kernel: the rows of up to 32 points per workgroup in LDS. SPHX_GRADIENT_LANES_FIXED: 0 never, 2 wherever
-// there is a kernel.
-static bool plan_gradients_fixed(size_t n_samples, int l_max, size_t elem, int lds_limit, int cus, bool normalized, Launch* out) {
-    const int wanted = switch_or(SW_GRADIENT_LANES_FIXED, 1);
-    if (wanted == 0 || !gradients_fixed(elem, l_max)) return false;
+// gradients_fixed_kernel (mode 1), hessians_fixed_kernel (mode 2): the rows of up to 32 points per workgroup in LDS.
+// SPHX_GRADIENT_LANES_FIXED, SPHX_HESSIAN_LANES_FIXED: 0 never, 2 wherever there is a kernel.
+static bool plan_fixed(size_t n_samples, int l_max, int mode, size_t elem, int lds_limit, int cus, bool normalized, Launch* out) {
+    const int wanted = switch_or(mode == 1 ? SW_GRADIENT_LANES_FIXED : SW_HESSIAN_LANES_FIXED, 1);
+    if (wanted == 0 || !(mode == 1 ? gradients_fixed(elem, l_max) : hessians_fixed(elem, l_max, normalized))) return false;
     Tiling& g = out->g;
     std::memset(&g, 0, sizeof(g));
     const unsigned esize = static_cast<unsigned>(elem), vec = 16u / esize;
     const unsigned ny = static_cast<unsigned>(l_max + 1) * (l_max + 1), pad = gradients_fixed_pad(elem, ny);
-    unsigned off_d = 0;
+    unsigned off_d = 0, off_dd = 0;
     auto bytes_of = [&](unsigned t) {
         off_d = (t * (ny + pad) + vec - 1u) / vec * vec;
-        return (off_d + t * (3u * ny + pad)) * esize;
+        off_dd = off_d + (t * (3u * ny + pad) + vec - 1u) / vec * vec;
+        return (mode == 1 ? off_d + t * (3u * ny + pad) : off_dd + t * (9u * ny + pad)) * esize;
     };
     const unsigned limit = static_cast<unsigned>(lds_limit);
-    const unsigned forced = static_cast<unsigned>(switch_or(SW_GRADIENT_LANES_TILE, 0));
+    const unsigned forced = static_cast<unsigned>(switch_or(mode == 1 ? SW_GRADIENT_LANES_TILE : SW_HESSIAN_LANES_TILE, 0));
+    const FixedRow* row = nullptr;
+    for (const FixedRow& r : kFixedRows) {
+        if (r.mode != mode || r.elem != static_cast<int>(elem) || l_max < r.l_from || l_max > r.l_to) continue;
+        if (n_samples < r.points_from || n_samples >= r.points_below) continue;
+        if (r.harmonics >= 0 && r.harmonics != static_cast<int>(normalized)) continue;
+        row = &r;
+        break;
+    }
+    if (wanted != 2 && (row == nullptr || row->tile == 0)) return false;
     unsigned tile = 0, waves = 8;
     // Calls that one round of workgroups takes: as few of them per CU as hold the points, each with an equal share (a multiple
     // of four: whole vectors), at least eight. A workgroup that has its CU to itself has sixteen waves where there are enough
-    // units of work for them and a channel is long (l_max = 8, 6 000 points, float32 4.46 with eight, 4.30 with sixteen; 7
-    // 3.92 4.19; 10 5.41 5.15; 13 6.39 6.75: from l_max = 12 eight waves take a channel whole, without the bare steps).
+    // units of work for them and a channel is long (gradients, l_max = 8, 6 000 points, float32 4.46 with eight, 4.30 with
+    // sixteen; 7 3.92 4.19; 10 5.41 5.15; 13 6.39 6.75: from l_max = 12 eight waves take a channel whole, without the bare
+    // steps; second derivatives, 5 000 points, float32 5 5.15 4.99, 7 6.38 6.71, 8 8.15 7.88; float64 5 7.21 7.07, 7 10.8 12.2).
     for (unsigned beside = 1; cus > 0 && forced != 1u && beside <= 4u; ++beside) {
         const size_t share = static_cast<size_t>(cus) * beside;
         const size_t t = ((n_samples + share - 1) / share + 3u) & ~static_cast<size_t>(3u);
@@ -290,24 +301,19 @@ static bool plan_gradients_fixed(size_t n_samples, int l_max, size_t elem, int l
         // (LDS is handed out in pieces of 1 280 bytes)
         if (beside * ((bytes_of(few) + 1279u) / 1280u * 1280u) > limit) continue;
         tile = few;
-        waves = beside == 1u && l_max >= 8 && l_max <= 11 ? 16u : 8u;
+        const bool pays = mode == 1 ? l_max >= 8 && l_max <= 11 : (elem == 4 ? l_max >= 4 && l_max != 7 : l_max == 4 || l_max == 5);
+        waves = beside == 1u && pays ? 16u : 8u;
         break;
     }
-    if (tile == 0) {
-        for (const FixedGradientsRow& row : kFixedGradientsRows) {
-            if (row.elem != static_cast<int>(elem) || l_max < row.l_from || l_max > row.l_to || n_samples < row.points_from) continue;
-            if (row.harmonics >= 0 && row.harmonics != static_cast<int>(normalized)) continue;
-            tile = row.tile;
-            waves = row.waves;
-            break;
-        }
-        if (tile == 0 && wanted == 2) {
-            tile = kGradientsFixedPoints;
-            while (tile > 8u && bytes_of(tile) > limit / 2u) tile -= 4u;
-        }
+    if (tile == 0 && row != nullptr) {
+        tile = row->tile;
+        waves = row->waves;
+    }
+    if (tile == 0 && wanted == 2) {
+        tile = kGradientsFixedPoints;
+        while (tile > 8u && bytes_of(tile) > limit / 2u) tile -= 4u;
     }
     if (forced >= 4u && forced <= kGradientsFixedPoints) tile = forced;
-    if (tile == 0) return false;
     const unsigned bytes = bytes_of(tile);
     if (bytes > limit || ((n_samples + tile - 1) / tile + 7u) / 8u * 8u > 0xffffffffull / 1024u) return false; // (fewer than 2^32 threads)
     g.n_samples = n_samples;
@@ -317,9 +323,11 @@ static bool plan_gradients_fixed(size_t n_samples, int l_max, size_t elem, int l
     g.n_tiles = static_cast<unsigned>((n_samples + tile - 1) / tile);
     g.tiles_per_xcd = (g.n_tiles + 7u) / 8u;
     g.off_dsph = off_d;
+    g.off_ddsph = mode == 2 ? off_dd : 0u;
     g.fixed = 1u;
     out->workgroups = g.tiles_per_xcd * 8u;
-    out->threads = switch_or(SW_GRADIENT_LANES_WAVES, static_cast<int>(waves)) > 8 ? 1024u : 512u;
+    if (waves == 0) waves = 8; // (a row without a tile and SPHX_.._FIXED = 2)
+    out->threads = switch_or(mode == 1 ? SW_GRADIENT_LANES_WAVES : SW_HESSIAN_LANES_WAVES, static_cast<int>(waves)) > 8 ? 1024u : 512u;
     out->lds_bytes = bytes;
     return true;
 }
@@ -564,7 +572,7 @@ static bool plan_recursion(size_t n_samples, int l_max, int mode, bool whole, si
     // 395 / 415. Solid harmonics, whose jobs are mostly stores, gain below 100 000 points and lose beyond (500 000,
     // l_max = 4-7: 111 / 128, 160 / 181, 222 / 241, 283 / 313). Fewer points than 64 for every CU leave lanes idle.
     const bool point_lanes = mode == 2 && whole && elem == 4 && osize == 4 && normalized && threads > kRecursionThreads &&
-                             l_max >= 4 && l_max <= 7 && switch_or(SW_JOB_LIST, 2) == 2 &&
+                             l_max >= 4 && l_max <= 5 && switch_or(SW_JOB_LIST, 2) == 2 &&
                              switch_or(SW_POINT_LANES, n_samples >= 16384 ? 1 : 0) != 0;
     const unsigned row_pad = point_lanes ? 1u - ny % 2u
                              : whole && l_max >= 7 && (ny * osize) % 64u == 0 && switch_or(SW_ROW_PAD, 1) != 0 ? 16u / osize : 0u;
@@ -959,7 +967,14 @@ int make_plan(size_t n_samples, int l_max, int mode, size_t elem, int lds_limit,
         plan->lanes = true;
         return SPHX_OK;
     }
-    // Second derivatives at small l_max: one point per lane where that was measured to be faster
+    // Second derivatives at small l_max: the kernels that have l_max for a constant, where they were measured ahead
+    // (sphx_plan_shapes.hpp).
+    if (lane_kernels && mode == 2 && switch_or(SW_HESSIAN_LANES, 1) != 0 && switch_or(SW_TILE, 0) == 0 && switch_or(SW_POINT_LANES, 0) == 0 &&
+        plan_fixed(n_samples, l_max, mode, elem, lds_limit, cus, normalized, &plan->closed)) {
+        plan->lanes = true;
+        return SPHX_OK;
+    }
+    // Without those: one point per lane where that was measured to be faster
     // than the recursion kernel (SPHX_HESSIAN_LANES: 0 never, 2 wherever the rows fit).
     const int hessian_lanes = switch_or(SW_HESSIAN_LANES, 1);
     // (Since the recursion kernel takes its jobs as a list ordered by kind it wins from l_max = 4 on; the lanes keep
@@ -1008,7 +1023,7 @@ int make_plan(size_t n_samples, int l_max, int mode, size_t elem, int lds_limit,
     // (sphx_plan_shapes.hpp).
     const int gradient_lanes = switch_or(SW_GRADIENT_LANES, 1);
     if (lane_kernels && mode == 1 && gradient_lanes != 0 && switch_or(SW_TILE, 0) == 0 &&
-        plan_gradients_fixed(n_samples, l_max, elem, lds_limit, cus, normalized, &plan->closed)) {
+        plan_fixed(n_samples, l_max, mode, elem, lds_limit, cus, normalized, &plan->closed)) {
         plan->lanes = true;
         return SPHX_OK;
     }

@@ -163,54 +163,107 @@ inline const PriorityRow* priority_row(int mode, int elem, bool normalized, int 
     return nullptr;
 }
 
-// gradients_fixed_kernel, calls of more points than one round of its workgroups takes: points per tile and waves, by the
-// first row that matches (tile 0: the kernels that follow in make_plan). A unit of work costs a wave the same however many
+// gradients_fixed_kernel and hessians_fixed_kernel, calls of more points than one round of workgroups takes: points per tile and waves, by the
+// first row that matches (tile 0: the kernels that follow in make_plan, whatever the number of rounds). A unit of work costs a wave the same however many
 // of its 32 points the tile has, so tiles are as large as leaves LDS for two or three workgroups; which of those, and
 // whether one workgroup of sixteen waves with 32 points is ahead, goes by the rounds and by how the runs of the tiles lie in
 // HBM. us, what ran before / tile of points x waves, normalised unless it says otherwise.
-struct FixedGradientsRow {
+struct FixedRow {
+    int mode; // derivatives: 1, 2
     int elem, l_from, l_to;
     unsigned long long points_from;
     int harmonics; // 0 solid, 1 normalised, -1 both
     unsigned tile, waves;
     const char* measured;
+    unsigned long long points_below = ~0ull;
 };
 
-constexpr FixedGradientsRow kFixedGradientsRows[] = {
-    {4, 7, 8, 500000, 0, 0, 0, "solid, 1.2 GB, l_max = 7 196 / 24x8 206, 8 201 / 32x16 205 (250 000 points 60.5 57.3)"},
-    {4, 9, 9, 400000, 0, 0, 0, "solid, 1.2 GB 202 / 32x16 208 (250 000 76.3 71.1)"},
-    {4, 11, 12, 400000, 0, 0, 0, "solid, 1.2 GB, 11 203 / 24x8 205, 12 207 / 16x8 209 (200 000 89 81, 108 97)"},
-    {4, 7, 7, 0, -1, 24, 8, "50 000 points 16.3 / 20x8 11.6 24x8 11.7 32x8 11.9, 1.2 GB 209 / 205 186 203"},
-    {4, 8, 8, 0, -1, 32, 16, "50 000 20.1 / 20x8 13.6 32x8 13.7 32x16 13.9, 1.2 GB 202 / 196 207 190"},
-    {4, 9, 9, 0, -1, 32, 16, "50 000 25.0 / 16x8 17.0 32x8 17.2 32x16 16.2, 1.2 GB 208 / 215 212 188"},
-    {4, 10, 10, 400000, 0, 0, 0, "solid, 400 000 133 / 20x8 144 28x16 138 32x16 137"},
-    {4, 10, 10, 1000000, 1, 0, 0, "(tests/test_planner_host_only.py states the plan of 1 000 000 points; 1.2 GB 222 / 204)"},
-    {4, 10, 10, 0, -1, 32, 16, "50 000 26.8 / 16x8 20.1 32x8 19.2 32x16 19.0, 200 000 80 / 32x16 69, 28x16 71"},
-    {4, 11, 11, 0, -1, 24, 8, "100 000 52.2 / 24x8 43.4 28x8 43.3 32x8 44.0, 1.2 GB 214 / 191 204 209"},
-    {4, 13, 13, 131072, 0, 0, 0, "solid, 200 000 112 / 16x8 113 20x8 115, 1.2 GB 208 / 212 216"},
-    {4, 12, 13, 0, -1, 16, 8, "l_max = 12, 100 000 60.5 / 16x8 49.5 20x8 51.0, 1.2 GB 210 / 188 202; 13, 61.8 / 59.0 58.8, 217 / 193 193"},
-    {4, 14, 16, 0, -1, 16, 8, "14, 50 000 45.1 / 16x8 35.4 20x8 37.5 32x16 38.5, 1.2 GB 210 / 32x8 199 16x8 200; 16, 50 000 49.7 / 43.7 - 46.3"},
-    {4, 17, 18, 65536, 1, 28, 8, "17, 100 000 98.6 / 12x8 101.7 28x8 97.5, 1.2 GB 223 / 226 207; 18, 111 / 111 104, 218 / 221 208"},
-    {4, 17, 18, 0, -1, 12, 8, "17, 25 000 34.7 / 12x8 28.9 28x8 31.6; solid, 1.2 GB 209 / 190 217; 18, 35.1 / 30.7 34.8, 224 / 208 213"},
-    {8, 7, 7, 400000, 0, 0, 0, "solid, 1.2 GB 203 / 20x8 206"},
-    {8, 7, 7, 131072, -1, 20, 8, "250 000 94.1 / 20x8 79.8 32x8 88.9"},
-    {8, 7, 7, 0, -1, 32, 8, "50 000 25.4 / 16x8 21.0 20x8 21.2 32x8 20.3, 100 000 42.1 / - 38.6 37.6"},
-    {8, 8, 9, 65536, 0, 32, 16, "solid, 100 000 53.9 / 20x8 49.7 24x8 48.0 32x16 45.6, 1.2 GB 210 / 215 209 191; 9, 65.6 / 59.2 59.4 57.1, 211 / 207 210 202"},
-    {8, 8, 9, 0, -1, 20, 8, "8, 100 000 53.9 / 20x8 45.3 24x8 48.1 32x16 49.5, 1.2 GB 207 / 193 203 205; 9, 68.7 / 57.3 58.6 60.9, 221 / 196 207 207"},
-    {8, 10, 10, 131072, 0, 24, 8, "solid, 1.2 GB 204 / 20x8 210 24x8 198 32x16 207"},
-    {8, 10, 10, 65536, -1, 32, 16, "100 000 78.0 / 20x8 72.2 32x16 69.6, 1.2 GB 224 / 194 195"},
-    {8, 10, 10, 0, -1, 20, 8, "50 000 44.4 / 16x8 38.3 20x8 38.1 32x16 39.8"},
-    {8, 11, 11, 131072, 0, 0, 0, "solid, 200 000 159 / 16x8 164 32x16 162"},
-    {8, 11, 11, 65536, -1, 32, 16, "200 000 179 / 16x8 160 32x16 155"},
-    {8, 11, 11, 0, -1, 16, 8, "50 000 57.0 / 16x8 43.6 32x16 46.6"},
-    {8, 12, 12, 131072, 0, 12, 8, "solid, 1.2 GB 210 / 12x8 205 28x8 211"},
-    {8, 12, 12, 65536, -1, 28, 8, "100 000 108 / 12x8 98.7 28x8 98.9, 1.2 GB 223 / 216 201"},
-    {8, 13, 13, 131072, 0, 0, 0, "solid, 1.2 GB 208 / 12x8 210 24x8 212"},
-    {8, 13, 13, 65536, -1, 24, 8, "100 000 127 / 12x8 116 24x8 113, 1.2 GB 232 / 220 203"},
-    {8, 12, 13, 0, -1, 12, 8, "12, 50 000 62.0 / 12x8 52.2 28x8 54.9; 13, 69.9 / 61.2 24x8 63.9"},
-    {8, 14, 14, 8193, -1, 0, 0, "15 000 31.0 / 8x8 32.9 20x8 29.5, 50 000 78 / 78"},
-    {8, 15, 15, 16384, -1, 0, 0, "50 000 88 / 88"},
-    {8, 14, 15, 0, -1, 8, 8, "14, 6 000 18.4 / 8x8 15.1 16x8 15.8; 15, 20.1 / 16.6 17.7, 15 000 37.9 / 34.0 35.2"},
+constexpr FixedRow kFixedRows[] = {
+    {1, 4, 7, 8, 500000, 0, 0, 0, "solid, 1.2 GB, l_max = 7 196 / 24x8 206, 8 201 / 32x16 205 (250 000 points 60.5 57.3)"},
+    {1, 4, 9, 9, 400000, 0, 0, 0, "solid, 1.2 GB 202 / 32x16 208 (250 000 76.3 71.1)"},
+    {1, 4, 11, 12, 400000, 0, 0, 0, "solid, 1.2 GB, 11 203 / 24x8 205, 12 207 / 16x8 209 (200 000 89 81, 108 97)"},
+    {1, 4, 7, 7, 0, -1, 24, 8, "50 000 points 16.3 / 20x8 11.6 24x8 11.7 32x8 11.9, 1.2 GB 209 / 205 186 203"},
+    {1, 4, 8, 8, 0, -1, 32, 16, "50 000 20.1 / 20x8 13.6 32x8 13.7 32x16 13.9, 1.2 GB 202 / 196 207 190"},
+    {1, 4, 9, 9, 0, -1, 32, 16, "50 000 25.0 / 16x8 17.0 32x8 17.2 32x16 16.2, 1.2 GB 208 / 215 212 188"},
+    {1, 4, 10, 10, 400000, 0, 0, 0, "solid, 400 000 133 / 20x8 144 28x16 138 32x16 137"},
+    {1, 4, 10, 10, 1000000, 1, 0, 0, "(tests/test_planner_host_only.py states the plan of 1 000 000 points; 1.2 GB 222 / 204)"},
+    {1, 4, 10, 10, 0, -1, 32, 16, "50 000 26.8 / 16x8 20.1 32x8 19.2 32x16 19.0, 200 000 80 / 32x16 69, 28x16 71"},
+    {1, 4, 11, 11, 0, -1, 24, 8, "100 000 52.2 / 24x8 43.4 28x8 43.3 32x8 44.0, 1.2 GB 214 / 191 204 209"},
+    {1, 4, 13, 13, 131072, 0, 0, 0, "solid, 200 000 112 / 16x8 113 20x8 115, 1.2 GB 208 / 212 216"},
+    {1, 4, 12, 13, 0, -1, 16, 8, "l_max = 12, 100 000 60.5 / 16x8 49.5 20x8 51.0, 1.2 GB 210 / 188 202; 13, 61.8 / 59.0 58.8, 217 / 193 193"},
+    {1, 4, 14, 16, 0, -1, 16, 8, "14, 50 000 45.1 / 16x8 35.4 20x8 37.5 32x16 38.5, 1.2 GB 210 / 32x8 199 16x8 200; 16, 50 000 49.7 / 43.7 - 46.3"},
+    {1, 4, 17, 18, 65536, 1, 28, 8, "17, 100 000 98.6 / 12x8 101.7 28x8 97.5, 1.2 GB 223 / 226 207; 18, 111 / 111 104, 218 / 221 208"},
+    {1, 4, 17, 18, 0, -1, 12, 8, "17, 25 000 34.7 / 12x8 28.9 28x8 31.6; solid, 1.2 GB 209 / 190 217; 18, 35.1 / 30.7 34.8, 224 / 208 213"},
+    {1, 8, 7, 7, 400000, 0, 0, 0, "solid, 1.2 GB 203 / 20x8 206"},
+    {1, 8, 7, 7, 131072, -1, 20, 8, "250 000 94.1 / 20x8 79.8 32x8 88.9"},
+    {1, 8, 7, 7, 0, -1, 32, 8, "50 000 25.4 / 16x8 21.0 20x8 21.2 32x8 20.3, 100 000 42.1 / - 38.6 37.6"},
+    {1, 8, 8, 9, 65536, 0, 32, 16, "solid, 100 000 53.9 / 20x8 49.7 24x8 48.0 32x16 45.6, 1.2 GB 210 / 215 209 191; 9, 65.6 / 59.2 59.4 57.1, 211 / 207 210 202"},
+    {1, 8, 8, 9, 0, -1, 20, 8, "8, 100 000 53.9 / 20x8 45.3 24x8 48.1 32x16 49.5, 1.2 GB 207 / 193 203 205; 9, 68.7 / 57.3 58.6 60.9, 221 / 196 207 207"},
+    {1, 8, 10, 10, 131072, 0, 24, 8, "solid, 1.2 GB 204 / 20x8 210 24x8 198 32x16 207"},
+    {1, 8, 10, 10, 65536, -1, 32, 16, "100 000 78.0 / 20x8 72.2 32x16 69.6, 1.2 GB 224 / 194 195"},
+    {1, 8, 10, 10, 0, -1, 20, 8, "50 000 44.4 / 16x8 38.3 20x8 38.1 32x16 39.8"},
+    {1, 8, 11, 11, 131072, 0, 0, 0, "solid, 200 000 159 / 16x8 164 32x16 162"},
+    {1, 8, 11, 11, 65536, -1, 32, 16, "200 000 179 / 16x8 160 32x16 155"},
+    {1, 8, 11, 11, 0, -1, 16, 8, "50 000 57.0 / 16x8 43.6 32x16 46.6"},
+    {1, 8, 12, 12, 131072, 0, 12, 8, "solid, 1.2 GB 210 / 12x8 205 28x8 211"},
+    {1, 8, 12, 12, 65536, -1, 28, 8, "100 000 108 / 12x8 98.7 28x8 98.9, 1.2 GB 223 / 216 201"},
+    {1, 8, 13, 13, 131072, 0, 0, 0, "solid, 1.2 GB 208 / 12x8 210 24x8 212"},
+    {1, 8, 13, 13, 65536, -1, 24, 8, "100 000 127 / 12x8 116 24x8 113, 1.2 GB 232 / 220 203"},
+    {1, 8, 12, 13, 0, -1, 12, 8, "12, 50 000 62.0 / 12x8 52.2 28x8 54.9; 13, 69.9 / 61.2 24x8 63.9"},
+    {1, 8, 14, 14, 8193, -1, 0, 0, "15 000 31.0 / 8x8 32.9 20x8 29.5, 50 000 78 / 78"},
+    {1, 8, 15, 15, 16384, -1, 0, 0, "50 000 88 / 88"},
+    {1, 8, 14, 15, 0, -1, 8, 8, "14, 6 000 18.4 / 8x8 15.1 16x8 15.8; 15, 20.1 / 16.6 17.7, 15 000 37.9 / 34.0 35.2"},
+    // second derivatives
+    {2, 4, 2, 2, 500000, -1, 0, 0, "1.2 GB 217 / 24x8 266 32x8 215-221 32x16 321; solid 200 / 32x8 201-204"},
+    {2, 4, 2, 2, 0, -1, 32, 8, "30 000 7.5 / 24x8 6.6 32x8 5.4 32x16 7.2, 300 000 34.4 / 32x8 26.9"},
+    {2, 4, 3, 3, 131072, 1, 28, 8, "1.2 GB 291 / 24x8 200 28x8 189 32x8 210"},
+    {2, 4, 3, 3, 131072, 0, 24, 16, "solid, 1.2 GB 248 / 12x8 191 24x16 178 28x16 195"},
+    {2, 4, 3, 3, 0, -1, 32, 8, "30 000 9.3 / 24x8 6.6 32x8 6.2; solid 8.8 / 5.9 5.9"},
+    {2, 4, 4, 4, 400000, -1, 0, 0, "1.2 GB 205 / 32x8 209 32x16 209; solid 203 / 24x16 205 32x16 207"},
+    {2, 4, 4, 4, 0, -1, 32, 16, "30 000 12.8 / 24x8 9.3 32x8 9.8 32x16 9.4; solid 13.1 / 9.2 8.5 8.4"},
+    {2, 4, 5, 5, 500000, 1, 0, 0, "(tests/test_planner_host_only.py states the plan of 500 000 points; 1.2 GB 212 / 28x16 203)"},
+    {2, 4, 5, 5, 400000, 0, 0, 0, "solid, 1.2 GB 206 / 16x16 204-207 32x16 210"},
+    {2, 4, 5, 5, 0, -1, 32, 16, "30 000 17.1 / 24x8 12.6 32x8 12.7 32x16 12.5; solid 17.7 / 11.9 11.8 11.6, 1.2 GB 207 / 8x8 196 16x16 204 32x8 209"},
+    {2, 4, 6, 6, 0, 1, 24, 8, "30 000 25.5 / 20x8 16.8 24x8 18.9 32x8 16.7, 1.2 GB 223 / 207 200 212"},
+    {2, 4, 6, 6, 65536, 0, 16, 16, "solid, 1.2 GB 210 / 16x8 213 16x16 186 28x16 211"},
+    {2, 4, 6, 6, 0, 0, 32, 16, "solid, 30 000 24.1 / 16x16 16.0 32x8 15.8 32x16 15.5"},
+    {2, 4, 7, 7, 0, 1, 20, 8, "30 000 33.1 / 16x8 21.7 20x8 21.2 24x8 21.4, 1.2 GB 234 / 218 207 213"},
+    {2, 4, 7, 7, 0, 0, 12, 16, "solid, 30 000 31.1 / 12x16 19.8 20x16 19.7, 1.2 GB 208 / 191 -"},
+    {2, 4, 8, 8, 65536, 1, 32, 8, "1.2 GB 236 / 16x8 228 32x8 217"},
+    {2, 4, 8, 8, 65536, 0, 20, 16, "solid, 1.2 GB 207 / 20x8 201 20x16 201 28x16 203"},
+    {2, 4, 8, 8, 0, 1, 16, 8, "30 000 35.0 / 12x8 29.7 16x8 27.7 32x8 31.8"},
+    {2, 4, 8, 8, 0, 0, 16, 16, "solid, 30 000 31.3 / 16x8 26.1 16x16 24.9 32x16 25.1"},
+    {2, 4, 9, 10, 250000, 0, 0, 0, "(tests/test_planner_host_only.py states the plans of 300 000 points)"},
+    {2, 4, 9, 9, 65536, 1, 28, 8, "1.2 GB 244 / 24x8 225 28x8 225"},
+    {2, 4, 9, 9, 65536, 0, 16, 16, "solid, 1.2 GB 210 / 8x16 204 16x8 196 16x16 197"},
+    {2, 4, 9, 9, 0, 0, 8, 16, "solid, 30 000 37.9 / 8x16 30.2 12x16 31.6 24x8 31.3"},
+    {2, 4, 9, 10, 0, 1, 12, 8, "9, 30 000 44.5 / 12x8 37.6 24x16 38.7; 10, 51.0 / 43.8 47.3", 65536},
+    {2, 4, 10, 10, 65536, 1, 24, 16, "1.2 GB 249 / 24x8 236 24x16 234"},
+    {2, 4, 10, 10, 65536, 0, 16, 16, "solid, 1.2 GB 208 / 16x8 202 16x16 196"},
+    {2, 4, 10, 10, 0, 0, 24, 16, "solid, 30 000 43.7 / 12x8 39.7 24x8 38.7 24x16 38.2"},
+    {2, 8, 7, 7, 0, 1, 0, 0, "300 points 9.5 / 11.0", 1024},
+    {2, 8, 9, 10, 0, 0, 0, 0, "solid, 300 points, 9 7.7 / 7.8, 10 8.5 / 9.5", 1024},
+    {2, 8, 2, 2, 0, 1, 32, 8, "30 000 11.8 / 24x8 8.9 32x8 7.7 32x16 10.5, 1.2 GB 255 / 241 208 -"},
+    {2, 8, 2, 2, 0, 0, 32, 16, "solid, 30 000 11.6 / 32x8 6.5 32x16 6.6, 1.2 GB 251 / 212 189"},
+    {2, 8, 3, 3, 131072, 1, 28, 8, "1.2 GB 266 / 24x8 189 28x8 182 32x8 204"},
+    {2, 8, 3, 3, 65536, 0, 16, 16, "solid, 1.2 GB 248 / 16x16 186 28x16 202"},
+    {2, 8, 3, 3, 0, 1, 24, 8, "30 000 19.7 / 20x8 11.1 24x8 10.7 32x8 10.7"},
+    {2, 8, 3, 3, 0, 0, 32, 16, "solid, 30 000 15.3 / 12x8 10.4 32x8 10.6 32x16 10.4"},
+    {2, 8, 4, 5, 0, 1, 20, 8, "4, 30 000 26.7 / 16x8 17.4 20x8 17.2 24x8 17.9, 1.2 GB 236 / 210 199 205; 5, 36.7 / 24.6 23.3 -, 249 / 216 201 -"},
+    {2, 8, 4, 4, 65536, 0, 20, 16, "solid, 1.2 GB 209 / 8x8 190 20x16 190 24x16 202"},
+    {2, 8, 4, 4, 0, 0, 24, 8, "solid, 30 000 22.6 / 16x8 15.9 24x8 15.8 32x16 16.1"},
+    {2, 8, 5, 5, 65536, 0, 16, 16, "solid, 1.2 GB 213 / 8x8 201 16x16 188 20x16 202"},
+    {2, 8, 5, 5, 0, 0, 24, 16, "solid, 30 000 30.1 / 12x8 22.7 24x16 22.2 32x8 22.6"},
+    {2, 8, 6, 6, 0, 1, 16, 8, "30 000 44.2 / 12x8 33.4 16x8 30.4 32x16 35.2, 1.2 GB 255 / - 205 207"},
+    {2, 8, 6, 6, 65536, 0, 16, 16, "solid, 1.2 GB 222 / 8x8 206 16x16 189 28x16 204"},
+    {2, 8, 6, 6, 0, 0, 32, 8, "solid, 30 000 36.7 / 16x16 30.4 32x8 29.3 32x16 29.5"},
+    {2, 8, 7, 7, 65536, 1, 24, 8, "1.2 GB 264 / 12x8 236 20x8 234 24x8 219"},
+    {2, 8, 7, 7, 65536, 0, 16, 8, "solid, 1.2 GB 222 / 8x8 197 16x8 192 16x16 194"},
+    {2, 8, 7, 7, 0, 1, 12, 8, "30 000 60.2 / 12x8 42.6 24x8 46.2"},
+    {2, 8, 7, 8, 0, 0, 8, 8, "solid, 7, 30 000 49.5 / 8x8 39.0 24x8 39.4; 8, 58.9 / 49.0 16x16 51.0, 1.2 GB 225 / 199 208"},
+    {2, 8, 9, 9, 0, 0, 12, 16, "solid, 30 000 69.2 / 12x8 65.6 12x16 63.9, 1.2 GB 230 / 207 200"},
+    {2, 8, 10, 10, 65536, 0, 12, 16, "solid, 1.2 GB 223 / 12x8 216 12x16 209"},
+    {2, 8, 10, 10, 0, 0, 12, 16, "solid, 5 000 20.7 / 12x8 19.3 12x16 18.8 (30 000 78.0 / 78 and more)", 8192},
 };
 
 } // namespace sphx

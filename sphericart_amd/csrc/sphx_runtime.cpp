@@ -49,6 +49,8 @@ static int prepare_device(int device) {
     SPHX_HIP(upload_vjp_tables<double>(t));
     SPHX_HIP(upload_channel_tables<float>(t));
     SPHX_HIP(upload_channel_tables<double>(t));
+    SPHX_HIP(upload_hessian_channel_tables<float>(t));
+    SPHX_HIP(upload_hessian_channel_tables<double>(t));
     SPHX_HIP(upload_column_tables<float>(t));
     SPHX_HIP(upload_column_tables<double>(t));
     SPHX_HIP((upload_fixed_columns<float, COLUMNS_VJP>(t)));

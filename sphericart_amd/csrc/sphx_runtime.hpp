@@ -112,6 +112,10 @@ template <typename T, int KIND> hipError_t upload_fixed_columns(const HostTables
 template <typename T>
 hipError_t dispatch_gradients_fixed(const Launch& launch, bool normalized, const T* xyz, T* sph, T* dsph, hipStream_t stream);
 template <typename T> hipError_t upload_channel_tables(const HostTables& t);
+// hessians_fixed_kernel (sphx_hessians_fixed_kernel.hpp), for the l_max that hessians_fixed() names.
+template <typename T>
+hipError_t dispatch_hessians_fixed(const Launch& launch, bool normalized, const T* xyz, T* sph, T* dsph, T* ddsph, hipStream_t stream);
+template <typename T> hipError_t upload_hessian_channel_tables(const HostTables& t);
 // Each of those translation units has the constant tables of its arithmetic type to itself; these fill them
 // on the current device. `F` / `Q` (may be null) receive the device addresses.
 template <typename T, int MODE> hipError_t upload_forward_tables(const HostTables& t, const T** F, const T** Q);

@@ -1,0 +1,61 @@
+"""hessians_fixed_kernel (second derivatives with l_max a compile-time number) against the oracle, number for number."""
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_utils import announce, run_launch_layer
+from helpers import special_points
+from test_gpu_parity import check
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("normalized", [True, False])
+@pytest.mark.parametrize("l_max", range(2, 11))
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_every_l_max(oracle, library, switches, dtype, l_max, normalized):
+    """The smallest and largest tile, tiles that are no power of two, one point less and more than a tile, both numbers of
+    waves; arrays that start at a multiple of 16 bytes and one element past it, nothing written outside them."""
+    if dtype == np.float64 and normalized and l_max > 7:
+        pytest.skip("no kernel")
+    ny = (l_max + 1) ** 2
+    most = min(32, 160 * 1024 // (13 * (ny + 2) * np.dtype(dtype).itemsize) // 4 * 4)
+    for n, tile, waves in ((1, 8, 8), (33, 8, 16), (most - 1, most, 8), (most + 1, most, 16), (50, 12, 8), (263, 20, 16)):
+        library.sphx_reset_switches()
+        switches("SPHX_HESSIAN_LANES_FIXED", 2)
+        switches("SPHX_HESSIAN_LANES_TILE", min(tile, most))
+        switches("SPHX_HESSIAN_LANES_WAVES", waves)
+        text = ctypes.create_string_buffer(512)
+        assert library.sphx_describe_plan(n, l_max, 2, int(dtype == np.float64), int(normalized), text, 512) == 0
+        assert "> [l_max a constant, " in text.value.decode(), text.value
+        xyz = special_points(dtype, np.random.default_rng(l_max), n)
+        want = oracle.compute(xyz, l_max, normalized, "hessians")
+        for offset in (0, 1):
+            announce("second derivatives, l_max a constant", np.dtype(dtype).name, l_max, normalized, n, tile, waves, offset)
+            d_xyz = torch.from_numpy(xyz).cuda()
+            out = [torch.full((n * c * ny + 2,), -7.0, dtype=d_xyz.dtype, device="cuda") for c in (1, 3, 9)]
+            views = tuple(o[offset:offset + n * c * ny] for o, c in zip(out, (1, 3, 9)))
+            status, _ = run_launch_layer(library, d_xyz, l_max, normalized, "hessians", out=views)
+            torch.cuda.synchronize()
+            assert status == 0, library.sphx_last_error()
+            check(tuple(v.reshape(w.shape).cpu().numpy() for v, w in zip(views, want)), want, (l_max, n, tile, waves, offset))
+            for o in out:
+                assert (o[:offset] == -7.0).all() and (o[offset - 2:] == -7.0).all()
+
+
+@pytest.mark.parametrize("dtype, l_max, n", [(np.float32, 3, 131_072), (np.float32, 4, 9_001), (np.float32, 6, 65_536),
+                                             (np.float32, 9, 65_536), (np.float64, 2, 20_000), (np.float64, 5, 65_536),
+                                             (np.float64, 7, 1_024), (np.float64, 9, 1_024), (np.float64, 10, 8_192)])
+def test_as_planned(oracle, library, dtype, l_max, n):
+    """Plans on both sides of the table's lines, and their neighbours that take another kernel."""
+    for normalized in (True, False):
+        for points in (n - 1, n):
+            announce("second derivatives as planned", np.dtype(dtype).name, l_max, normalized, points)
+            xyz = special_points(dtype, np.random.default_rng(l_max), points)
+            want = oracle.compute(xyz, l_max, normalized, "hessians")
+            status, out = run_launch_layer(library, torch.from_numpy(xyz).cuda(), l_max, normalized, "hessians")
+            assert status == 0, library.sphx_last_error()
+            check(tuple(o.cpu().numpy() for o in out), want, (l_max, points))
