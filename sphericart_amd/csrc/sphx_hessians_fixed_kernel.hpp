@@ -15,6 +15,8 @@ namespace sphx {
 // still (170 instructions for one side of 32 points, normalised; 65 solid). us, before and after: float32 normalised l_max =
 // 3 30 000 points 9.3 6.2, 1.2 GB 291 189; 5 2 000 9.9 4.3, 30 000 17.1 12.5, 300 000 108 102; 7 30 000 33 21, 1.2 GB 243
 // 210; float64 4 30 000 26.7 17.2, 1.2 GB 237 199; 6 30 000 44 30, 1.2 GB 255 207; solid 8 30 000 59 49, 1.2 GB 223 201.
+// From l_max = 11 in float32 (one workgroup per CU holds the rows) 2 500 12.2 9.5, solid 10 000 24.2 17.0, 1.2 GB 209 190;
+// beyond 13, and in float64 beyond 10, level or behind.
 //
 // Same operations in the same order as the reference, hence the same numbers. LDS: the rows of the three arrays.
 // ---------------------------------------------------------------------------

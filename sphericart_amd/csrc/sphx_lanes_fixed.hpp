@@ -9,10 +9,12 @@ namespace sphx {
 
 // l_max of the kernels
 constexpr int kGradientsFixedFirst = 7;
-constexpr int gradients_fixed_last(size_t elem) { return elem == 4 ? 18 : 15; }
+constexpr int gradients_fixed_last(size_t elem) { return elem == 4 ? 24 : 20; }
 constexpr bool gradients_fixed(size_t elem, int l_max) {
     return l_max >= kGradientsFixedFirst && l_max <= gradients_fixed_last(elem);
 }
+// (beyond, only the form with eight waves is of use)
+constexpr int gradients_fixed_last_sixteen(size_t elem) { return elem == 4 ? 16 : 11; }
 constexpr unsigned kGradientsFixedPoints = 32; // the most points of a tile: two lanes each
 
 // elements left free after the rows of a point (ny of the values, 3 ny of the gradients): where ny is even, a multiple of
@@ -68,8 +70,8 @@ constexpr UnitMasks deal_units(bool normalized, int l_max, int waves) {
 // ---- second derivatives --------------------------------------------------------------------------------------
 constexpr int kHessiansFixedFirst = 2;
 // (normalised in float64: from l_max = 8 on the entries need more registers than sixteen waves on a CU leave a lane)
-constexpr int kHessiansFixedLast = 10;
-constexpr int hessians_fixed_last(size_t elem, bool normalized) { return elem == 8 && normalized ? 7 : kHessiansFixedLast; }
+constexpr int kHessiansFixedLast = 13;
+constexpr int hessians_fixed_last(size_t elem, bool normalized) { return elem == 4 ? kHessiansFixedLast : (normalized ? 7 : 10); }
 constexpr bool hessians_fixed(size_t elem, int l_max, bool normalized) {
     return l_max >= kHessiansFixedFirst && l_max <= hessians_fixed_last(elem, normalized);
 }

@@ -29,7 +29,9 @@ namespace sphx {
 // are dispatched in the order of the addresses they write: 1.2 GB leave at 5.9-6.5 TB/s where persistent workgroups reached
 // 5.3-5.9. us, normalised, before and after: float32 l_max = 7 3 000 points 6.0 4.3, 50 000 16.3 11.7, 1.2 GB 209 186; 9
 // 20 000 14.0 7.7, 750 000 208 188; 12 15 000 17.2 9.6, 444 000 210 188; float64 8 10 000 points 9.0 7.6, 463 000 207 193;
-// 9 20 000 24.6 15.0; 13 191 000 232 203.
+// 9 20 000 24.6 15.0; 13 191 000 232 203. At larger l_max a tile holds few points and half of the lanes are idle (float32 from
+// l_max = 20, float64 from 16 with more than one tile per CU): there it is ahead only while the call is latency, float32 22
+// 2 500 13.2 9.0, 14 000 32.9 31.3, solid 20 000 40.9 34.4; float64 17 200 32.4 8.4, 4 000 22.3 18.1.
 //
 // Same operations in the same order as the reference (templates_core.hpp:122-426, through finish()), hence the same numbers.
 // LDS: the value rows, then (g.off_dsph) the gradient rows, in HBM layout, an even row length padded by 8 bytes.
@@ -248,7 +250,12 @@ static hipError_t launch_gradients_fixed(const Launch& l, const T* xyz, T* sph, 
     for_each_number(std::make_integer_sequence<int, gradients_fixed_last(sizeof(T)) - kGradientsFixedFirst + 1>{}, [&](auto i) {
         constexpr int L = kGradientsFixedFirst + decltype(i)::value;
         if (l.g.l_max != L) return;
-        auto kernel = l.threads == 512u ? gradients_fixed_kernel<T, NORM, L, 8> : gradients_fixed_kernel<T, NORM, L, 16>;
+        auto kernel = gradients_fixed_kernel<T, NORM, L, 8>;
+        if constexpr (L <= gradients_fixed_last_sixteen(sizeof(T))) {
+            if (l.threads == 1024u) kernel = gradients_fixed_kernel<T, NORM, L, 16>;
+        } else if (l.threads != 512u) {
+            return; // never planned
+        }
         if (l.lds_bytes > 64u * 1024u) {
             unsigned unused = 0;
             status = kernel_facts(reinterpret_cast<const void*>(kernel), l.threads, l.lds_bytes, &unused);

@@ -328,6 +328,7 @@ static bool plan_fixed(size_t n_samples, int l_max, int mode, size_t elem, int l
     out->workgroups = g.tiles_per_xcd * 8u;
     if (waves == 0) waves = 8; // (a row without a tile and SPHX_.._FIXED = 2)
     out->threads = switch_or(mode == 1 ? SW_GRADIENT_LANES_WAVES : SW_HESSIAN_LANES_WAVES, static_cast<int>(waves)) > 8 ? 1024u : 512u;
+    if (mode == 1 && l_max > gradients_fixed_last_sixteen(elem)) out->threads = 512u;
     out->lds_bytes = bytes;
     return true;
 }

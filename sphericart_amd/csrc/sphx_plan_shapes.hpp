@@ -210,9 +210,20 @@ constexpr FixedRow kFixedRows[] = {
     {1, 8, 13, 13, 131072, 0, 0, 0, "solid, 1.2 GB 208 / 12x8 210 24x8 212"},
     {1, 8, 13, 13, 65536, -1, 24, 8, "100 000 127 / 12x8 116 24x8 113, 1.2 GB 232 / 220 203"},
     {1, 8, 12, 13, 0, -1, 12, 8, "12, 50 000 62.0 / 12x8 52.2 28x8 54.9; 13, 69.9 / 61.2 24x8 63.9"},
-    {1, 8, 14, 14, 8193, -1, 0, 0, "15 000 31.0 / 8x8 32.9 20x8 29.5, 50 000 78 / 78"},
-    {1, 8, 15, 15, 16384, -1, 0, 0, "50 000 88 / 88"},
-    {1, 8, 14, 15, 0, -1, 8, 8, "14, 6 000 18.4 / 8x8 15.1 16x8 15.8; 15, 20.1 / 16.6 17.7, 15 000 37.9 / 34.0 35.2"},
+    {1, 8, 14, 14, 0, 1, 8, 8, "6 000 18.4 / 8x8 15.1 16x8 15.8, 12 000 26.6 / 25.2, 15 000 30.7 / 31.3, 50 000 78 / 78", 14000},
+    {1, 8, 15, 15, 0, 1, 8, 8, "12 000 32.2 / 27.7, 15 000 38.3 / 34.2, 30 000 59.2 / 59.2", 16384},
+    {1, 8, 14, 15, 0, 0, 8, 8, "solid, 14, 12 000 25.6 / 8x8 20.7 20x8 23.5, 30 000 49.6 / 43.4 45.8; 15, 30 000 56.6 / 48.2", 32768},
+    {1, 8, 16, 16, 0, 1, 16, 8, "200 28.6 / 8.1, 4 000 16.7 / 16x8 12.1, 12 000 31.5 / 32.4", 4097},
+    {1, 8, 16, 16, 0, 0, 16, 8, "solid, 4 000 15.2 / 10.7, 12 000 30.5 / 16x8 28.8, 30 000 61.4 / 60.8", 16384},
+    {1, 8, 17, 18, 0, 1, 12, 8, "17, 1 000 16.6 / 9.1, 4 000 22.3 / 12x8 18.1, 12 000 38.0 / 39.2; 18, 25.6 / 19.3", 5000},
+    {1, 8, 19, 19, 0, 1, 12, 8, "1 100 19.6 / 10.6, 2 500 19.3 / 12.9, 4 000 25.7 / 22.0, 4 096 21.2 / 22.4", 3073},
+    {1, 8, 17, 19, 0, 0, 12, 8, "solid, 17, 4 000 17.9 / 15.3, 7 000 25.2 / 23.6, 12 500 36.7 / 37.9; 18, 7 000 25.9 / 25.4, 12 500 36.9 / 40.3; 19, 31.1 / 27.8, 42.8 / 45.1", 8192},
+    {1, 8, 20, 20, 0, 1, 8, 8, "1 100 20.2 / 11.0, 2 500 25.4 / 22.9, 4 000 26.5 / 8x8 23.6, 4 096 21.6 / 23.9, 4 900 26.4 / 31.5", 3073},
+    {1, 8, 20, 20, 0, 0, 8, 8, "solid, 2 500 24.6 / 19.7, 4 000 25.9 / 20.0, 4 900 24.6 / 26.1", 4097},
+    {1, 4, 19, 19, 0, 1, 12, 8, "4 000 13.3 / 9.0, 12 000 25.0 / 8x8 20.9 12x8 18.5, 30 000 45.3 / 43.6 39.5", 65536},
+    {1, 4, 19, 19, 0, 0, 8, 8, "solid, 12 000 24.2 / 8x8 17.9 12x8 19.0, 30 000 43.8 / 37.0 39.8", 65536},
+    {1, 4, 20, 24, 0, 1, 8, 8, "20, 4 000 13.6 / 9.5, 12 000 25.5 / 8x8 23.9 16x8 25.2; 22, 31.2 / 27.6 29.4; 24, 33.2 / 31.5 33.9, 30 000 64 / 68", 16384},
+    {1, 4, 20, 24, 0, 0, 8, 8, "solid, 20, 12 000 24.7 / 8x8 20.2 16x8 23.2, 30 000 47.1 / 42.1; 24, 31.8 / 26.6 30.8, 61.0 / 55.9", 32768},
     // second derivatives
     {2, 4, 2, 2, 500000, -1, 0, 0, "1.2 GB 217 / 24x8 266 32x8 215-221 32x16 321; solid 200 / 32x8 201-204"},
     {2, 4, 2, 2, 0, -1, 32, 8, "30 000 7.5 / 24x8 6.6 32x8 5.4 32x16 7.2, 300 000 34.4 / 32x8 26.9"},
@@ -241,6 +252,12 @@ constexpr FixedRow kFixedRows[] = {
     {2, 4, 10, 10, 65536, 1, 24, 16, "1.2 GB 249 / 24x8 236 24x16 234"},
     {2, 4, 10, 10, 65536, 0, 16, 16, "solid, 1.2 GB 208 / 16x8 202 16x16 196"},
     {2, 4, 10, 10, 0, 0, 24, 16, "solid, 30 000 43.7 / 12x8 39.7 24x8 38.7 24x16 38.2"},
+    {2, 4, 11, 11, 131072, 1, 20, 8, "1.2 GB 252 / 16x8 266 20x8 237 24x8 252"},
+    {2, 4, 11, 11, 0, 1, 20, 8, "2 500 12.2 / 9.1, 10 000 28.6 / 8x8 25.8 20x8 22.5, 16 000 36.0 / 38.1, 30 000 55.6 / 55.5", 12288},
+    {2, 4, 12, 13, 0, 1, 0, 0, "300 points, 12 9.0 / 9.8, 13 9.6 / 11.3; 500 9.3 / 8.8, level", 768},
+    {2, 4, 12, 12, 0, 1, 8, 8, "2 500 12.7 / 10.5, 7 000 23.2 / 24.8, 10 000 30.6 / 30.1", 4097},
+    {2, 4, 13, 13, 0, 1, 8, 8, "2 500 13.2 / 11.7, 7 000 29.8 / 28.4, 9 000 31.1 / 34.6, 10 000 37.8 / 35.5, 16 000 45.4 / 52.6", 7169},
+    {2, 4, 11, 13, 0, 0, 8, 8, "solid, 11, 10 000 24.2 / 17.0, 30 000 47.6 / 8x8 39.9 20x8 44.5, 1.2 GB 210 / 193; 12, 54.2 / 50.4, 210 / 198; 13, 65.5 / 54.7, 215 / 193"},
     {2, 8, 7, 7, 0, 1, 0, 0, "300 points 9.5 / 11.0", 1024},
     {2, 8, 9, 10, 0, 0, 0, 0, "solid, 300 points, 9 7.7 / 7.8, 10 8.5 / 9.5", 1024},
     {2, 8, 2, 2, 0, 1, 32, 8, "30 000 11.8 / 24x8 8.9 32x8 7.7 32x16 10.5, 1.2 GB 255 / 241 208 -"},

@@ -14,12 +14,12 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("normalized", [True, False])
-@pytest.mark.parametrize("l_max", range(2, 11))
+@pytest.mark.parametrize("l_max", range(2, 14))
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_every_l_max(oracle, library, switches, dtype, l_max, normalized):
     """The smallest and largest tile, tiles that are no power of two, one point less and more than a tile, both numbers of
     waves; arrays that start at a multiple of 16 bytes and one element past it, nothing written outside them."""
-    if dtype == np.float64 and normalized and l_max > 7:
+    if dtype == np.float64 and l_max > (7 if normalized else 10):
         pytest.skip("no kernel")
     ny = (l_max + 1) ** 2
     most = min(32, 160 * 1024 // (13 * (ny + 2) * np.dtype(dtype).itemsize) // 4 * 4)
@@ -48,7 +48,8 @@ def test_every_l_max(oracle, library, switches, dtype, l_max, normalized):
 
 @pytest.mark.parametrize("dtype, l_max, n", [(np.float32, 3, 131_072), (np.float32, 4, 9_001), (np.float32, 6, 65_536),
                                              (np.float32, 9, 65_536), (np.float64, 2, 20_000), (np.float64, 5, 65_536),
-                                             (np.float64, 7, 1_024), (np.float64, 9, 1_024), (np.float64, 10, 8_192)])
+                                             (np.float64, 7, 1_024), (np.float64, 9, 1_024), (np.float64, 10, 8_192),
+                                             (np.float32, 11, 12_287), (np.float32, 12, 4_097), (np.float32, 13, 3_000)])
 def test_as_planned(oracle, library, dtype, l_max, n):
     """Plans on both sides of the table's lines, and their neighbours that take another kernel."""
     for normalized in (True, False):
