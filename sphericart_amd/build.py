@@ -22,7 +22,7 @@ OBJECTS = os.path.join(HERE, "build")
 
 # the translation units with the most kernels first: they take longest
 SOURCES = [
-    "sphx_lanes_fixed_f64.hip", "sphx_lanes_fixed_f32.hip", "sphx_hessians_fixed_f64.hip", "sphx_hessians_fixed_f32.hip",
+    "sphx_values_fixed_f64.hip", "sphx_values_fixed_f32.hip", "sphx_lanes_fixed_f64.hip", "sphx_lanes_fixed_f32.hip", "sphx_hessians_fixed_f64.hip", "sphx_hessians_fixed_f32.hip",
     *(f"sphx_columns_fixed_{kind}_{t}.hip" for kind in ("rows", "vjp_backward", "vjp") for t in ("f64", "f32")),
     "sphx_forward_f64_hessians.hip", "sphx_forward_f32_hessians.hip", "sphx_wide_hessians.hip",
     "sphx_forward_f64_gradients.hip", "sphx_forward_f32_gradients.hip", "sphx_wide_gradients.hip",

@@ -116,6 +116,7 @@ static hipError_t dispatch(const Plan& plan, const DeviceState& device, const T*
     if (plan.lanes) {
         if constexpr (MODE == 0) {
             const Launch& l = plan.closed;
+            if (l.g.fixed != 0) return dispatch_values_fixed<T>(l, NORM, xyz, sph, stream);
             auto kernel = l.g.points_per_pass == 8   ? values_kernel<T, NORM, 8>
                           : l.g.points_per_pass == 4 ? values_kernel<T, NORM, 4>
                           : l.g.points_per_pass == 2 ? (l.threads > 512 ? values_kernel<T, NORM, 2, 1024> : values_kernel<T, NORM, 2>)

@@ -9,7 +9,7 @@ namespace sphx {
 
 // l_max of the kernels
 constexpr int kGradientsFixedFirst = 7;
-constexpr int gradients_fixed_last(size_t elem) { return elem == 4 ? 24 : 20; }
+constexpr int gradients_fixed_last(size_t elem) { return elem == 4 ? 30 : 24; }
 constexpr bool gradients_fixed(size_t elem, int l_max) {
     return l_max >= kGradientsFixedFirst && l_max <= gradients_fixed_last(elem);
 }
@@ -44,12 +44,12 @@ constexpr int unit_cost(bool normalized, int l_max, int waves, int unit) {
 // Which units each of `waves` waves takes, one bit each: the longest unit left to the wave with the least so far.
 constexpr int kFixedMostWaves = 16;
 struct UnitMasks {
-    unsigned of[kFixedMostWaves];
+    unsigned long long of[kFixedMostWaves];
 };
 constexpr UnitMasks deal_units(bool normalized, int l_max, int waves) {
     UnitMasks masks{};
     int load[kFixedMostWaves] = {};
-    bool taken[32] = {};
+    bool taken[64] = {};
     const int units = gradients_fixed_units(l_max, waves);
     for (int round = 0; round < units; ++round) {
         int longest = -1;
@@ -62,7 +62,34 @@ constexpr UnitMasks deal_units(bool normalized, int l_max, int waves) {
         }
         taken[longest] = true;
         load[least] += unit_cost(normalized, l_max, waves, longest);
-        masks.of[least] |= 1u << longest;
+        masks.of[least] |= 1ull << longest;
+    }
+    return masks;
+}
+
+// ---- values ------------------------------------------------------------------------------------------------------
+constexpr int values_fixed_last(size_t elem) { return elem == 4 ? 32 : 28; }
+constexpr bool values_fixed(size_t elem, int l_max) { return l_max >= kGradientsFixedFirst && l_max <= values_fixed_last(elem); }
+// units: two slices of the closed forms, then the channels from l_max down; a wave that has any of those makes c_m, s_m and
+// 2(m+1)z first
+constexpr int kValueSlices = 2;
+constexpr int value_unit_cost(int l_max, int unit) { return unit < kValueSlices ? 90 : 9 * (l_max - (unit - kValueSlices) + 1); }
+constexpr UnitMasks deal_value_units(int l_max, int waves) {
+    UnitMasks masks{};
+    int load[kFixedMostWaves] = {};
+    const int units = kValueSlices + l_max - 6;
+    for (int i = 0; i < units; ++i) {
+        const int u = (i + kValueSlices) % units; // the channels, longest first, then the slices
+        int least = 0, least_load = 1 << 30;
+        for (int w = 0; w < waves; ++w) {
+            const int with = load[w] + (u >= kValueSlices && load[w] == 0 ? 7 * l_max : 0);
+            if (with < least_load) {
+                least = w;
+                least_load = with;
+            }
+        }
+        masks.of[least] |= 1ull << u;
+        load[least] = least_load + value_unit_cost(l_max, u);
     }
     return masks;
 }
@@ -121,7 +148,7 @@ constexpr UnitMasks deal_hessian_units(bool normalized, int l_max, int waves) {
         }
         taken[longest] = true;
         load[least] += hessian_unit_cost(normalized, l_max, waves, longest);
-        masks.of[least] |= 1u << longest;
+        masks.of[least] |= 1ull << longest;
     }
     return masks;
 }

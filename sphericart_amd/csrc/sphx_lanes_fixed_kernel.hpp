@@ -31,7 +31,8 @@ namespace sphx {
 // 20 000 14.0 7.7, 750 000 208 188; 12 15 000 17.2 9.6, 444 000 210 188; float64 8 10 000 points 9.0 7.6, 463 000 207 193;
 // 9 20 000 24.6 15.0; 13 191 000 232 203. At larger l_max a tile holds few points and half of the lanes are idle (float32 from
 // l_max = 20, float64 from 16 with more than one tile per CU): there it is ahead only while the call is latency, float32 22
-// 2 500 13.2 9.0, 14 000 32.9 31.3, solid 20 000 40.9 34.4; float64 17 200 32.4 8.4, 4 000 22.3 18.1.
+// 2 500 13.2 9.0, 14 000 32.9 31.3, solid 20 000 40.9 34.4, 28 2 000 14.5 12.1; float64 17 200
+// 32.4 8.4, 4 000 22.3 18.1, 23 200 55.8 13.1.
 //
 // Same operations in the same order as the reference (templates_core.hpp:122-426, through finish()), hence the same numbers.
 // LDS: the value rows, then (g.off_dsph) the gradient rows, in HBM layout, an even row length padded by 8 bytes.
@@ -100,7 +101,7 @@ __global__ __launch_bounds__(64 * WAVES) void gradients_fixed_kernel(Tiling g, c
     const unsigned point = lane & (kGradientsFixedPoints - 1u);
     const bool minus = lane >= kGradientsFixedPoints;
     static constexpr UnitMasks kMasks = deal_units(NORM, L, WAVES);
-    const unsigned mine = kMasks.of[wave];
+    const unsigned long long mine = kMasks.of[wave];
     T* row_s = lds + point * S_STRIDE;
     T* row_d = lds + g.off_dsph + point * D_STRIDE;
     if (point < valid) {

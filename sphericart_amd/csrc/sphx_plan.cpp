@@ -28,7 +28,7 @@ static const char* const kSwitchNames[SW_COUNT] = {
     "SPHX_PAIRS", "SPHX_PAIRS_BATCH", "SPHX_PAIRS_CHUNK", "SPHX_PAIRS_PREP_WAVES", "SPHX_PAIRS_SEQUENCE_WAVES", "SPHX_PAIRS_TILE",
     "SPHX_POINT_LANES", "SPHX_PREFIX_INSIDE", "SPHX_RECURSIONS_TOGETHER", "SPHX_ROW_PAD", "SPHX_SEQUENCE_WAVES", "SPHX_SLICE_WAVES", "SPHX_SPLIT_BELOW",
     "SPHX_SPLIT_RATIO", "SPHX_SPLIT_SIDES", "SPHX_SPREAD_KINDS", "SPHX_TILE", "SPHX_TILE_LDS_BUDGET", "SPHX_TILE_POW2",
-    "SPHX_TILE_SMALL_N", "SPHX_VALUES_ALONE", "SPHX_VALUES_LDS", "SPHX_VALUES_MIN_TILE", "SPHX_VALUES_MIN_WAVES",
+    "SPHX_TILE_SMALL_N", "SPHX_VALUES_ALONE", "SPHX_VALUES_FIXED", "SPHX_VALUES_FIXED_TILE", "SPHX_VALUES_FIXED_WAVES", "SPHX_VALUES_LDS", "SPHX_VALUES_MIN_TILE", "SPHX_VALUES_MIN_WAVES",
     "SPHX_VALUES_PACK", "SPHX_VALUES_TILE_STEP", "SPHX_VALUES_WAVES", "SPHX_VJP_GROUPS_BELOW", "SPHX_VJP_LANES", "SPHX_VJP_MIN_TILE", "SPHX_VJP_STEP_FLOOR", "SPHX_VJP_TILE_STEP", "SPHX_WAVE_PRIORITIES",
 };
 struct Switches {
@@ -261,11 +261,18 @@ static bool plan_values(size_t n_samples, int l_max, size_t elem, int lds_limit,
     return true;
 }
 
-// gradients_fixed_kernel (mode 1), hessians_fixed_kernel (mode 2): the rows of up to 32 points per workgroup in LDS.
-// SPHX_GRADIENT_LANES_FIXED, SPHX_HESSIAN_LANES_FIXED: 0 never, 2 wherever there is a kernel.
+// values_fixed_kernel (mode 0), gradients_fixed_kernel (1), hessians_fixed_kernel (2): the rows of up to 32 points per workgroup in LDS.
+// SPHX_VALUES_FIXED, SPHX_GRADIENT_LANES_FIXED, SPHX_HESSIAN_LANES_FIXED: 0 never, 2 wherever there is a kernel.
 static bool plan_fixed(size_t n_samples, int l_max, int mode, size_t elem, int lds_limit, int cus, bool normalized, Launch* out) {
-    const int wanted = switch_or(mode == 1 ? SW_GRADIENT_LANES_FIXED : SW_HESSIAN_LANES_FIXED, 1);
-    if (wanted == 0 || !(mode == 1 ? gradients_fixed(elem, l_max) : hessians_fixed(elem, l_max, normalized))) return false;
+    static constexpr Switch kWanted[3] = {SW_VALUES_FIXED, SW_GRADIENT_LANES_FIXED, SW_HESSIAN_LANES_FIXED};
+    static constexpr Switch kTile[3] = {SW_VALUES_FIXED_TILE, SW_GRADIENT_LANES_TILE, SW_HESSIAN_LANES_TILE};
+    static constexpr Switch kWaves[3] = {SW_VALUES_FIXED_WAVES, SW_GRADIENT_LANES_WAVES, SW_HESSIAN_LANES_WAVES};
+    const int wanted = switch_or(kWanted[mode], 1);
+    if (wanted == 0 || !(mode == 0   ? values_fixed(elem, l_max)
+                         : mode == 1 ? gradients_fixed(elem, l_max)
+                                     : hessians_fixed(elem, l_max, normalized))) {
+        return false;
+    }
     Tiling& g = out->g;
     std::memset(&g, 0, sizeof(g));
     const unsigned esize = static_cast<unsigned>(elem), vec = 16u / esize;
@@ -274,10 +281,10 @@ static bool plan_fixed(size_t n_samples, int l_max, int mode, size_t elem, int l
     auto bytes_of = [&](unsigned t) {
         off_d = (t * (ny + pad) + vec - 1u) / vec * vec;
         off_dd = off_d + (t * (3u * ny + pad) + vec - 1u) / vec * vec;
-        return (mode == 1 ? off_d + t * (3u * ny + pad) : off_dd + t * (9u * ny + pad)) * esize;
+        return (mode == 0 ? off_d : mode == 1 ? off_d + t * (3u * ny + pad) : off_dd + t * (9u * ny + pad)) * esize;
     };
     const unsigned limit = static_cast<unsigned>(lds_limit);
-    const unsigned forced = static_cast<unsigned>(switch_or(mode == 1 ? SW_GRADIENT_LANES_TILE : SW_HESSIAN_LANES_TILE, 0));
+    const unsigned forced = static_cast<unsigned>(switch_or(kTile[mode], 0));
     const FixedRow* row = nullptr;
     for (const FixedRow& r : kFixedRows) {
         if (r.mode != mode || r.elem != static_cast<int>(elem) || l_max < r.l_from || l_max > r.l_to) continue;
@@ -297,11 +304,13 @@ static bool plan_fixed(size_t n_samples, int l_max, int mode, size_t elem, int l
         const size_t share = static_cast<size_t>(cus) * beside;
         const size_t t = ((n_samples + share - 1) / share + 3u) & ~static_cast<size_t>(3u);
         if (t > kGradientsFixedPoints) continue;
-        const unsigned few = t < 8u ? 8u : static_cast<unsigned>(t);
+        // (values: fewer than sixteen cost more than they spread, float64 l_max = 18, 300 points 5.86 with 8, 4.67 with 16)
+        const unsigned least = mode == 0 ? 16u : 8u;
+        const unsigned few = t < least ? least : static_cast<unsigned>(t);
         // (LDS is handed out in pieces of 1 280 bytes)
         if (beside * ((bytes_of(few) + 1279u) / 1280u * 1280u) > limit) continue;
         tile = few;
-        const bool pays = mode == 1 ? l_max >= 8 && l_max <= 11 : (elem == 4 ? l_max >= 4 && l_max != 7 : l_max == 4 || l_max == 5);
+        const bool pays = mode == 0 ? false : mode == 1 ? l_max >= 8 && l_max <= 11 : (elem == 4 ? l_max >= 4 && l_max != 7 : l_max == 4 || l_max == 5);
         waves = beside == 1u && pays ? 16u : 8u;
         break;
     }
@@ -322,12 +331,13 @@ static bool plan_fixed(size_t n_samples, int l_max, int mode, size_t elem, int l
     g.tile = static_cast<int>(tile);
     g.n_tiles = static_cast<unsigned>((n_samples + tile - 1) / tile);
     g.tiles_per_xcd = (g.n_tiles + 7u) / 8u;
-    g.off_dsph = off_d;
+    g.off_dsph = mode >= 1 ? off_d : 0u;
     g.off_ddsph = mode == 2 ? off_dd : 0u;
     g.fixed = 1u;
     out->workgroups = g.tiles_per_xcd * 8u;
     if (waves == 0) waves = 8; // (a row without a tile and SPHX_.._FIXED = 2)
-    out->threads = switch_or(mode == 1 ? SW_GRADIENT_LANES_WAVES : SW_HESSIAN_LANES_WAVES, static_cast<int>(waves)) > 8 ? 1024u : 512u;
+    const int asked = switch_or(kWaves[mode], static_cast<int>(waves));
+    out->threads = mode == 0 ? (asked > 4 ? 512u : 256u) : (asked > 8 ? 1024u : 512u);
     if (mode == 1 && l_max > gradients_fixed_last_sixteen(elem)) out->threads = 512u;
     out->lds_bytes = bytes;
     return true;
@@ -942,6 +952,20 @@ int make_plan(size_t n_samples, int l_max, int mode, size_t elem, int lds_limit,
     // three of its workgroups or more (1.2 GB, us, pairs_kernel / values_kernel: float32 l_max = 24 266 / 208, 25 245 /
     // 203, 26 239 / 220 (50 000 points 37.2 / 38.4), 27 255 / 233, 28 251 / 236, 29 220 / 226, 31 222 / 239, 33 260 / 343; float64 19 221 / 240,
     // 20 217 / 218, 21 281 / 218, 22 279 / 227, 23 324 / 270, 24 243 / 238, 25 211 / 291).
+    // Values: the kernels that have l_max for a constant, where they were measured ahead (sphx_plan_shapes.hpp). An override of
+    // another kernel's shape asks for that kernel.
+    const auto values_overridden = [&] {
+        for (Switch s : {SW_VALUES_ALONE, SW_VALUES_LDS, SW_VALUES_MIN_TILE, SW_VALUES_MIN_WAVES, SW_VALUES_PACK, SW_VALUES_TILE_STEP,
+                         SW_VALUES_WAVES, SW_TILE, SW_POINT_LANES}) {
+            if (switch_or(s, -1) != -1) return true;
+        }
+        return switch_or(SW_PAIRS, 1) == 2;
+    };
+    if (lane_kernels && mode == 0 && l_max > hard && !values_overridden() &&
+        plan_fixed(n_samples, l_max, mode, elem, lds_limit, cus, normalized, &plan->closed)) {
+        plan->lanes = true;
+        return SPHX_OK;
+    }
     if (lane_kernels && mode == 0 && l_max > hard) {
         const int pairs = switch_or(SW_PAIRS, 1);
         const bool pairs_by_shape = n_samples >= 32768 && (elem == 4 ? l_max == 26 || l_max >= 28 : l_max >= 24 || l_max == 19 || l_max == 20);
@@ -1158,7 +1182,7 @@ std::string describe(const Plan& plan, int l_max, int mode, bool is_f64, bool no
     } else if (plan.lanes) {
         const char* names[3] = {"values_kernel", "gradients_lanes_kernel", "hessians_lanes_kernel"};
         text = std::string(names[mode]) + "<" + t + ", " + (normalized ? "true" : "false") +
-               (mode == 0 ? ", " + std::to_string(plan.closed.g.points_per_pass) : std::string()) + ">" +
+               (mode == 0 && plan.closed.g.fixed == 0 ? ", " + std::to_string(plan.closed.g.points_per_pass) : std::string()) + ">" +
                geometry(plan.closed);
     } else {
         if (!plan.whole && plan.rec.g.prefix_inside == 0) {

@@ -47,6 +47,8 @@ static int prepare_device(int device) {
     SPHX_HIP(upload_wide_tables<2>(t));
     SPHX_HIP(upload_vjp_tables<float>(t));
     SPHX_HIP(upload_vjp_tables<double>(t));
+    SPHX_HIP(upload_value_channel_tables<float>(t));
+    SPHX_HIP(upload_value_channel_tables<double>(t));
     SPHX_HIP(upload_channel_tables<float>(t));
     SPHX_HIP(upload_channel_tables<double>(t));
     SPHX_HIP(upload_hessian_channel_tables<float>(t));

@@ -112,6 +112,9 @@ template <typename T, int KIND> hipError_t upload_fixed_columns(const HostTables
 template <typename T>
 hipError_t dispatch_gradients_fixed(const Launch& launch, bool normalized, const T* xyz, T* sph, T* dsph, hipStream_t stream);
 template <typename T> hipError_t upload_channel_tables(const HostTables& t);
+// values_fixed_kernel (sphx_values_fixed_kernel.hpp), for the l_max that values_fixed() names.
+template <typename T> hipError_t dispatch_values_fixed(const Launch& launch, bool normalized, const T* xyz, T* sph, hipStream_t stream);
+template <typename T> hipError_t upload_value_channel_tables(const HostTables& t);
 // hessians_fixed_kernel (sphx_hessians_fixed_kernel.hpp), for the l_max that hessians_fixed() names.
 template <typename T>
 hipError_t dispatch_hessians_fixed(const Launch& launch, bool normalized, const T* xyz, T* sph, T* dsph, T* ddsph, hipStream_t stream);

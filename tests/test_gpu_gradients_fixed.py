@@ -14,12 +14,12 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("normalized", [True, False])
-@pytest.mark.parametrize("l_max", range(7, 25))
+@pytest.mark.parametrize("l_max", range(7, 31))
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_every_l_max(oracle, library, switches, dtype, l_max, normalized):
     """The smallest and largest tile, tiles that are no power of two, one point less and more than a tile, both numbers of
     waves; arrays that start at a multiple of 16 bytes and one element past it, nothing written outside them."""
-    if dtype == np.float64 and l_max > 20:
+    if dtype == np.float64 and l_max > 24:
         pytest.skip("no kernel")
     ny = (l_max + 1) ** 2
     most = min(32, 160 * 1024 // (4 * (ny + 2) * np.dtype(dtype).itemsize) // 4 * 4)
@@ -51,7 +51,7 @@ def test_every_l_max(oracle, library, switches, dtype, l_max, normalized):
                                              (np.float32, 17, 65_536), (np.float64, 8, 10_000), (np.float64, 8, 65_537),
                                              (np.float64, 12, 65_536), (np.float64, 15, 16_384), (np.float32, 19, 65_536),
                                              (np.float32, 22, 16_384), (np.float32, 24, 4_097), (np.float64, 16, 4_097),
-                                             (np.float64, 18, 5_000), (np.float64, 20, 2_049)])
+                                             (np.float64, 18, 5_000), (np.float64, 20, 2_049), (np.float32, 30, 2_049), (np.float64, 24, 2_049)])
 def test_as_planned(oracle, library, dtype, l_max, n):
     """Plans of mid-sized calls on both sides of the table's lines, and their neighbours that take another kernel."""
     for normalized in (True, False):
