@@ -1181,9 +1181,15 @@ std::string describe(const Plan& plan, int l_max, int mode, bool is_f64, bool no
         text = "closed_form_kernel<" + head + ", " + std::to_string(l_max) + ", false>" + geometry(plan.closed);
     } else if (plan.lanes) {
         const char* names[3] = {"values_kernel", "gradients_lanes_kernel", "hessians_lanes_kernel"};
-        text = std::string(names[mode]) + "<" + t + ", " + (normalized ? "true" : "false") +
-               (mode == 0 && plan.closed.g.fixed == 0 ? ", " + std::to_string(plan.closed.g.points_per_pass) : std::string()) + ">" +
-               geometry(plan.closed);
+        const char* fixed_names[3] = {"values_fixed_kernel", "gradients_fixed_kernel", "hessians_fixed_kernel"};
+        const Launch& l = plan.closed;
+        text = std::string(l.g.fixed != 0 ? fixed_names[mode] : names[mode]) + "<" + t + ", " + (normalized ? "true" : "false");
+        if (l.g.fixed != 0) {
+            text += ", " + std::to_string(l_max) + ", " + std::to_string(l.threads / 64u);
+        } else if (mode == 0) {
+            text += ", " + std::to_string(l.g.points_per_pass);
+        }
+        text += ">" + geometry(l);
     } else {
         if (!plan.whole && plan.rec.g.prefix_inside == 0) {
             text = "closed_form_kernel<" + head + ", 6, true>" + geometry(plan.closed) + " + ";

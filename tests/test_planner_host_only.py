@@ -15,7 +15,7 @@ SHAPES = [
     # n_samples, l_max, mode, is_f64, normalized, the kernel it is meant to get
     (1_000_000, 6, 1, 0, 1, "gradients_lanes_kernel<float, true>"),
     (1_000_000, 3, 0, 0, 1, "closed_form_kernel<float, 0, true, 3, false>"),
-    (10_000, 8, 1, 1, 1, "gradients_lanes_kernel<double, true>"),
+    (10_000, 8, 1, 1, 1, "gradients_fixed_kernel<double, true, 8, 8>"),
     (100_000, 16, 2, 1, 0, "recursion_kernel<double, 2, false, true, true, false, true>"),
     (200_000, 32, 1, 0, 1, "pairs_kernel<float, 1, true>"),
     (200_000, 32, 0, 0, 1, "pairs_kernel<float, 0, true>"),
@@ -23,7 +23,11 @@ SHAPES = [
     (1_000_000, 10, 0, 0, 1, "values_kernel<float, true, 1>"),
     (1_000_000, 22, 0, 0, 1, "values_kernel<float, true, 2>"),
     (500_000, 5, 2, 0, 1, "recursion_kernel<float, 2, true, true, false, false, true>"),
-    (500_000, 3, 2, 0, 1, "hessians_lanes_kernel<float, true>"),
+    (500_000, 3, 2, 0, 1, "hessians_fixed_kernel<float, true, 3, 8>"),
+    (600_000, 2, 2, 0, 1, "hessians_lanes_kernel<float, true>"),
+    (1_000_000, 7, 0, 0, 0, "values_fixed_kernel<float, false, 7, 4>"),
+    (2_000, 5, 2, 0, 1, "hessians_fixed_kernel<float, true, 5, 16>"),
+    (600_000, 7, 1, 0, 0, "gradients_lanes_kernel<float, false>"),
     (1_000_000, 10, 1, 0, 1, "recursion_kernel<float, 1, true, true, false, false, true>"),
     (50_000, 20, 2, 1, 1, "pairs_kernel<double, 2, true>"),
     (2_000, 32, 1, 0, 1, "recursion_kernel<float, 1, true, true, false, false, true>"),
