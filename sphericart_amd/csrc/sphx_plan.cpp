@@ -22,9 +22,9 @@ int fail(int code, const std::string& what) {
 
 static const char* const kSwitchNames[SW_COUNT] = {
     "SPHX_AZ_SHIFT", "SPHX_CHUNK_SHIFT", "SPHX_COLUMNS_TILE", "SPHX_COLUMNS_WAVES", "SPHX_GRADIENT_LANES", "SPHX_GRADIENT_LANES_FIXED",
-    "SPHX_GRADIENT_LANES_PARTS", "SPHX_GRADIENT_LANES_TILE", "SPHX_GRADIENT_LANES_WAVES", "SPHX_GROUP_THREADS",
-    "SPHX_HESSIAN_LANES", "SPHX_HESSIAN_LANES_FIXED",
-    "SPHX_HESSIAN_LANES_PARTS", "SPHX_HESSIAN_LANES_TILE", "SPHX_HESSIAN_LANES_WAVES", "SPHX_JOB_LIST",
+    "SPHX_GRADIENT_LANES_FIXED_TILE", "SPHX_GRADIENT_LANES_FIXED_WAVES", "SPHX_GRADIENT_LANES_PARTS", "SPHX_GRADIENT_LANES_TILE", "SPHX_GRADIENT_LANES_WAVES", "SPHX_GROUP_THREADS",
+    "SPHX_HESSIAN_LANES", "SPHX_HESSIAN_LANES_FIXED", "SPHX_HESSIAN_LANES_FIXED_TILE", "SPHX_HESSIAN_LANES_FIXED_WAVES",
+    "SPHX_HESSIAN_LANES_PARTS", "SPHX_HESSIAN_LANES_TILE", "SPHX_JOB_LIST",
     "SPHX_PAIRS", "SPHX_PAIRS_BATCH", "SPHX_PAIRS_CHUNK", "SPHX_PAIRS_PREP_WAVES", "SPHX_PAIRS_SEQUENCE_WAVES", "SPHX_PAIRS_TILE",
     "SPHX_POINT_LANES", "SPHX_PREFIX_INSIDE", "SPHX_RECURSIONS_TOGETHER", "SPHX_ROW_PAD", "SPHX_SEQUENCE_WAVES", "SPHX_SLICE_WAVES", "SPHX_SPLIT_BELOW",
     "SPHX_SPLIT_RATIO", "SPHX_SPLIT_SIDES", "SPHX_SPREAD_KINDS", "SPHX_TILE", "SPHX_TILE_LDS_BUDGET", "SPHX_TILE_POW2",
@@ -261,13 +261,26 @@ static bool plan_values(size_t n_samples, int l_max, size_t elem, int lds_limit,
     return true;
 }
 
+// The kernels with l_max for a constant: 0 never, 1 where their table names them, 2 wherever there is one
+// (SPHX_VALUES_FIXED, SPHX_GRADIENT_LANES_FIXED, SPHX_HESSIAN_LANES_FIXED). An override of any other kernel's choice or
+// shape asks for that kernel.
+static int fixed_wanted(Switch asked) {
+    if (t_switches.set[asked] && t_switches.value[asked] >= 0) return t_switches.value[asked];
+    for (int i = 0; i < SW_COUNT; ++i) {
+        if (!t_switches.set[i] || t_switches.value[i] == -1) continue;
+        const char* name = kSwitchNames[i];
+        const bool elsewhere = std::strncmp(name, "SPHX_COLUMNS", 12) == 0 || std::strncmp(name, "SPHX_VJP", 8) == 0; // (products)
+        if (!elsewhere && std::strstr(name, "_FIXED") == nullptr) return 0;
+    }
+    return 1;
+}
+
 // values_fixed_kernel (mode 0), gradients_fixed_kernel (1), hessians_fixed_kernel (2): the rows of up to 32 points per workgroup in LDS.
-// SPHX_VALUES_FIXED, SPHX_GRADIENT_LANES_FIXED, SPHX_HESSIAN_LANES_FIXED: 0 never, 2 wherever there is a kernel.
 static bool plan_fixed(size_t n_samples, int l_max, int mode, size_t elem, int lds_limit, int cus, bool normalized, Launch* out) {
     static constexpr Switch kWanted[3] = {SW_VALUES_FIXED, SW_GRADIENT_LANES_FIXED, SW_HESSIAN_LANES_FIXED};
-    static constexpr Switch kTile[3] = {SW_VALUES_FIXED_TILE, SW_GRADIENT_LANES_TILE, SW_HESSIAN_LANES_TILE};
-    static constexpr Switch kWaves[3] = {SW_VALUES_FIXED_WAVES, SW_GRADIENT_LANES_WAVES, SW_HESSIAN_LANES_WAVES};
-    const int wanted = switch_or(kWanted[mode], 1);
+    static constexpr Switch kTile[3] = {SW_VALUES_FIXED_TILE, SW_GRADIENT_LANES_FIXED_TILE, SW_HESSIAN_LANES_FIXED_TILE};
+    static constexpr Switch kWaves[3] = {SW_VALUES_FIXED_WAVES, SW_GRADIENT_LANES_FIXED_WAVES, SW_HESSIAN_LANES_FIXED_WAVES};
+    const int wanted = fixed_wanted(kWanted[mode]);
     if (wanted == 0 || !(mode == 0   ? values_fixed(elem, l_max)
                          : mode == 1 ? gradients_fixed(elem, l_max)
                                      : hessians_fixed(elem, l_max, normalized))) {
@@ -947,25 +960,17 @@ int make_plan(size_t n_samples, int l_max, int mode, size_t elem, int lds_limit,
         plan_closed(n_samples, l_max, l_max, mode, elem, &plan->closed);
         return SPHX_OK;
     }
+    // The kernels that have l_max for a constant, where they were measured ahead (sphx_plan_shapes.hpp).
+    if (lane_kernels && l_max > hard &&
+        plan_fixed(n_samples, l_max, mode, elem, lds_limit, cus, normalized, &plan->closed)) {
+        plan->lanes = true;
+        return SPHX_OK;
+    }
     // Values alone where the rows of few points fill LDS: pairs_kernel (below, with the derivatives), which keeps
     // the recursions of the next tile and the flush of this one side by side. values_kernel is ahead where LDS holds
     // three of its workgroups or more (1.2 GB, us, pairs_kernel / values_kernel: float32 l_max = 24 266 / 208, 25 245 /
     // 203, 26 239 / 220 (50 000 points 37.2 / 38.4), 27 255 / 233, 28 251 / 236, 29 220 / 226, 31 222 / 239, 33 260 / 343; float64 19 221 / 240,
     // 20 217 / 218, 21 281 / 218, 22 279 / 227, 23 324 / 270, 24 243 / 238, 25 211 / 291).
-    // Values: the kernels that have l_max for a constant, where they were measured ahead (sphx_plan_shapes.hpp). An override of
-    // another kernel's shape asks for that kernel.
-    const auto values_overridden = [&] {
-        for (Switch s : {SW_VALUES_ALONE, SW_VALUES_LDS, SW_VALUES_MIN_TILE, SW_VALUES_MIN_WAVES, SW_VALUES_PACK, SW_VALUES_TILE_STEP,
-                         SW_VALUES_WAVES, SW_TILE, SW_POINT_LANES}) {
-            if (switch_or(s, -1) != -1) return true;
-        }
-        return switch_or(SW_PAIRS, 1) == 2;
-    };
-    if (lane_kernels && mode == 0 && l_max > hard && !values_overridden() &&
-        plan_fixed(n_samples, l_max, mode, elem, lds_limit, cus, normalized, &plan->closed)) {
-        plan->lanes = true;
-        return SPHX_OK;
-    }
     if (lane_kernels && mode == 0 && l_max > hard) {
         const int pairs = switch_or(SW_PAIRS, 1);
         const bool pairs_by_shape = n_samples >= 32768 && (elem == 4 ? l_max == 26 || l_max >= 28 : l_max >= 24 || l_max == 19 || l_max == 20);
@@ -992,14 +997,7 @@ int make_plan(size_t n_samples, int l_max, int mode, size_t elem, int lds_limit,
         plan->lanes = true;
         return SPHX_OK;
     }
-    // Second derivatives at small l_max: the kernels that have l_max for a constant, where they were measured ahead
-    // (sphx_plan_shapes.hpp).
-    if (lane_kernels && mode == 2 && switch_or(SW_HESSIAN_LANES, 1) != 0 && switch_or(SW_TILE, 0) == 0 && switch_or(SW_POINT_LANES, 0) == 0 &&
-        plan_fixed(n_samples, l_max, mode, elem, lds_limit, cus, normalized, &plan->closed)) {
-        plan->lanes = true;
-        return SPHX_OK;
-    }
-    // Without those: one point per lane where that was measured to be faster
+    // Second derivatives at small l_max: one point per lane where that was measured to be faster
     // than the recursion kernel (SPHX_HESSIAN_LANES: 0 never, 2 wherever the rows fit).
     const int hessian_lanes = switch_or(SW_HESSIAN_LANES, 1);
     // (Since the recursion kernel takes its jobs as a list ordered by kind it wins from l_max = 4 on; the lanes keep
@@ -1044,20 +1042,13 @@ int make_plan(size_t n_samples, int l_max, int mode, size_t elem, int lds_limit,
             }
         }
     }
-    // Gradients just above the closed forms: the kernels that have l_max for a constant, where they were measured ahead
-    // (sphx_plan_shapes.hpp).
-    const int gradient_lanes = switch_or(SW_GRADIENT_LANES, 1);
-    if (lane_kernels && mode == 1 && gradient_lanes != 0 && switch_or(SW_TILE, 0) == 0 &&
-        plan_fixed(n_samples, l_max, mode, elem, lds_limit, cus, normalized, &plan->closed)) {
-        plan->lanes = true;
-        return SPHX_OK;
-    }
-    // Without those: the lanes kernel (one point per lane, the channels dealt to the
+    // Gradients just above the closed forms: the lanes kernel (one point per lane, the channels dealt to the
     // waves) up to l_max = 13 in float32 and wherever its tiles fit in float64; from there the recursion kernel with
     // its jobs as a list ordered by kind is ahead. Where the recursion kernel runs in workgroups of 1024 threads
     // (calls of 32 768 points or more) it is ahead from l_max = 8 on (3-20 %): the lanes keep l_max = 7; at
     // 20 000 points from l_max = 10 on (6-30 %).
     // SPHX_GRADIENT_LANES: 0 never, 2 wherever the rows fit.
+    const int gradient_lanes = switch_or(SW_GRADIENT_LANES, 1);
     const bool large_groups = group_threads(n_samples, mode, elem, lane_kernels) > kRecursionThreads && n_samples >= 32768;
     // (float64, normalised, l_max = 7: the recursion kernel is 8 % ahead there, 203 against 219 us per 1.2 GB)
     const bool lanes_by_shape = large_groups ? l_max <= (elem == 8 && normalized ? 6 : 7)

@@ -1,5 +1,7 @@
 """Helpers of the GPU tests: run the library on torch device buffers through its C entry points."""
 
+import ctypes
+
 import numpy as np
 import torch
 
@@ -12,6 +14,14 @@ METHOD = {"values": "compute", "gradients": "compute_with_gradients", "hessians"
 def announce(*what):
     """Name the case before touching the GPU, so that a fault can be traced to it."""
     print("[gpu case]", *what, flush=True)
+
+
+def plan_text(library, n, l_max, mode, dtype, normalized):
+    """What the library would launch for the call, under the switches that are set (no GPU involved)."""
+    text = ctypes.create_string_buffer(1024)
+    f64 = int(np.dtype(dtype) == np.float64)
+    assert library.sphx_describe_plan(n, l_max, MODE_INDEX[mode], f64, int(bool(normalized)), text, len(text)) == 0
+    return text.value.decode()
 
 
 def run_calculator(xyz, l_max, normalized, mode):

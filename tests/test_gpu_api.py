@@ -9,7 +9,7 @@ import pytest
 import torch
 
 import sphericart_amd
-from gpu_utils import announce, run_calculator, run_launch_layer
+from gpu_utils import announce, plan_text, run_calculator, run_launch_layer
 from helpers import MODES, same_numbers, special_points
 
 pytestmark = pytest.mark.gpu
@@ -116,6 +116,9 @@ def test_second_derivatives_at_small_l_max_by_both_kernels(oracle, library, rout
         for n, shift in ((1, 0), (31, 1), (64, 0), (65, 2), (2049, 0), (4133, 3)):
             normalized = bool((l_max + n) & 1)
             announce("small l_max hessians", route, np.dtype(dtype).name, l_max, n, shift, normalized)
+            planned = plan_text(library, n, l_max, "hessians", dtype, normalized)
+            fits = route == "lanes" and (dtype == np.float32 or l_max <= 5)  # (a tile's rows in LDS)
+            assert planned.startswith("hessians_lanes_kernel<" if fits else "recursion_kernel<"), planned
             ny = (l_max + 1) ** 2
             xyz = special_points(dtype, rng, n)
             want = oracle.compute(xyz, l_max, normalized, "hessians")

@@ -1,12 +1,10 @@
 """gradients_fixed_kernel (values and gradients with l_max a compile-time number) against the oracle, number for number."""
 
-import ctypes
-
 import numpy as np
 import pytest
 import torch
 
-from gpu_utils import announce, run_launch_layer
+from gpu_utils import announce, plan_text, run_launch_layer
 from helpers import special_points
 from test_gpu_parity import check
 
@@ -26,11 +24,13 @@ def test_every_l_max(oracle, library, switches, dtype, l_max, normalized):
     for n, tile, waves in ((1, 8, 8), (33, 8, 16), (most - 1, most, 8), (most + 1, most, 16), (50, 12, 8), (263, 20, 16)):
         library.sphx_reset_switches()
         switches("SPHX_GRADIENT_LANES_FIXED", 2)
-        switches("SPHX_GRADIENT_LANES_TILE", min(tile, most))
-        switches("SPHX_GRADIENT_LANES_WAVES", waves)
-        text = ctypes.create_string_buffer(512)
-        assert library.sphx_describe_plan(n, l_max, 1, int(dtype == np.float64), int(normalized), text, 512) == 0
-        assert "> [l_max a constant, " in text.value.decode(), text.value
+        switches("SPHX_GRADIENT_LANES_FIXED_TILE", min(tile, most))
+        switches("SPHX_GRADIENT_LANES_FIXED_WAVES", waves)
+        sixteen = waves == 16 and l_max <= (16 if dtype == np.float32 else 11)
+        planned = plan_text(library, n, l_max, "gradients", dtype, normalized)
+        name = "double" if dtype == np.float64 else "float"
+        assert planned.startswith(f"gradients_fixed_kernel<{name}, {str(normalized).lower()}, {l_max}, {16 if sixteen else 8}> "
+                                  f"[l_max a constant, {min(tile, most)} points"), planned
         xyz = special_points(dtype, np.random.default_rng(l_max), n)
         want = oracle.compute(xyz, l_max, normalized, "gradients")
         for offset in (0, 1):

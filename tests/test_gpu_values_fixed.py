@@ -1,12 +1,10 @@
 """values_fixed_kernel (values with l_max a compile-time number) against the oracle, number for number."""
 
-import ctypes
-
 import numpy as np
 import pytest
 import torch
 
-from gpu_utils import announce, run_launch_layer
+from gpu_utils import announce, plan_text, run_launch_layer
 from helpers import special_points
 from test_gpu_parity import check
 
@@ -28,9 +26,10 @@ def test_every_l_max(oracle, library, switches, dtype, l_max, normalized):
         switches("SPHX_VALUES_FIXED", 2)
         switches("SPHX_VALUES_FIXED_TILE", min(tile, most))
         switches("SPHX_VALUES_FIXED_WAVES", waves)
-        text = ctypes.create_string_buffer(512)
-        assert library.sphx_describe_plan(n, l_max, 0, int(dtype == np.float64), int(normalized), text, 512) == 0
-        assert "> [l_max a constant, " in text.value.decode(), text.value
+        planned = plan_text(library, n, l_max, "values", dtype, normalized)
+        name = "double" if dtype == np.float64 else "float"
+        assert planned.startswith(f"values_fixed_kernel<{name}, {str(normalized).lower()}, {l_max}, {waves}> "
+                                  f"[l_max a constant, {min(tile, most)} points"), planned
         xyz = special_points(dtype, np.random.default_rng(l_max), n)
         want = oracle.compute(xyz, l_max, normalized, "values")
         for offset in (0, 1):

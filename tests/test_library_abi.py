@@ -152,6 +152,32 @@ def test_planner_overrides(library, switches):
         status, (tile, threads, _, _) = _plan(library, 100_000, l_max, 0, False)
         assert status == 0 and threads <= 512, (l_max, tile, threads)
     library.sphx_reset_switches()
+    # the kernels with l_max for a constant stand back where another kernel is asked for by a switch of its own, in every
+    # mode, and have switches of their own
+    def kernel_of(n, l_max, mode, **asked):
+        for name, value in asked.items():
+            switches(name, value)
+        text = ctypes.create_string_buffer(512)
+        assert library.sphx_describe_plan(n, l_max, mode, 0, 1, text, 512) == 0
+        library.sphx_reset_switches()
+        return text.value.decode()
+
+    for l_max, mode, name in ((7, 1, "gradients"), (10, 1, "gradients"), (3, 2, "hessians"), (5, 2, "hessians"), (12, 0, "values")):
+        assert kernel_of(1_001, l_max, mode).startswith(name + "_fixed_kernel<")
+    for parts, waves in ((1, 8), (2, 16)):
+        lanes = kernel_of(1_001, 10, 1, SPHX_GRADIENT_LANES=2, SPHX_GRADIENT_LANES_PARTS=parts, SPHX_GRADIENT_LANES_WAVES=waves)
+        assert lanes.startswith("gradients_lanes_kernel<") and f" {64 * waves} threads" in lanes, lanes
+    assert kernel_of(1_001, 7, 1, SPHX_GRADIENT_LANES_PARTS=1).startswith("gradients_lanes_kernel<")
+    assert kernel_of(1_001, 3, 2, SPHX_HESSIAN_LANES=2, SPHX_HESSIAN_LANES_PARTS=2).startswith("hessians_lanes_kernel<")
+    assert kernel_of(1_001, 5, 2, SPHX_HESSIAN_LANES=0).startswith("recursion_kernel<")
+    assert kernel_of(1_001, 5, 2, SPHX_JOB_LIST=0).startswith("recursion_kernel<")
+    assert kernel_of(1_001, 10, 0, SPHX_VALUES_PACK=2).startswith("values_kernel<float, true, 2>")
+    assert kernel_of(1_001, 7, 1, SPHX_GRADIENT_LANES_TILE=16).startswith("gradients_lanes_kernel<float, true> [16 ")
+    fixed = kernel_of(1_001, 10, 1, SPHX_GRADIENT_LANES_FIXED=2, SPHX_GRADIENT_LANES_FIXED_TILE=12, SPHX_GRADIENT_LANES=0)
+    assert fixed.startswith("gradients_fixed_kernel<float, true, 10, 16> [l_max a constant, 12 "), fixed
+    fixed = kernel_of(1_001, 5, 2, SPHX_HESSIAN_LANES_FIXED_TILE=20, SPHX_HESSIAN_LANES_FIXED_WAVES=8)
+    assert fixed.startswith("hessians_fixed_kernel<float, true, 5, 8> [l_max a constant, 20 "), fixed
+    assert kernel_of(1_001, 10, 1, SPHX_VALUES_FIXED=0, SPHX_COLUMNS_WAVES=4, SPHX_VJP_LANES=0).startswith("gradients_fixed_kernel<")
     assert library.sphx_set_switch(b"SPHX_NO_SUCH_SWITCH", 1) == 1
     assert b"unknown switch" in library.sphx_last_error()
     assert library.sphx_set_switch(None, 1) == 1
