@@ -196,12 +196,13 @@ def test_planned_by_shape(library):
     assert _plan_text(library, 100_000, 16, True, True).startswith("recursion_kernel")
     assert _plan_text(library, 50_000, 22, True, True, mode=2).startswith("recursion_kernel")
     assert _plan_text(library, 20_000, 32, False, True).startswith("recursion_kernel")  # few points
-    assert _plan_text(library, 200_000, 32, False, True, mode=0).startswith("pairs_kernel<float, 0, true>")
-    assert _plan_text(library, 200_000, 20, True, False, mode=0).startswith("pairs_kernel<double, 0, false>")
+    assert _plan_text(library, 200_000, 34, False, True, mode=0).startswith("pairs_kernel<float, 0, true>")
+    assert _plan_text(library, 200_000, 25, True, False, mode=0).startswith("pairs_kernel<double, 0, false>")
     assert _plan_text(library, 200_000, 22, False, True, mode=0).startswith("values_fixed_kernel<float, true, 22, 8>")
     assert _plan_text(library, 200_000, 18, True, True, mode=0).startswith("values_fixed_kernel<double, true, 18, 8>")
     assert _plan_text(library, 200_000, 23, False, True, mode=0).startswith("values_fixed_kernel<float, true, 23, 8>")
     assert _plan_text(library, 1_000_000, 17, False, True, mode=0).startswith("values_kernel<float, true, 4>")
-    assert _plan_text(library, 20_000, 32, False, True, mode=0).startswith("values_kernel")  # few points
+    assert _plan_text(library, 200_000, 32, False, True, mode=0).startswith("values_fixed_kernel<float, true, 32, 8>")
+    assert _plan_text(library, 10_000, 34, False, True, mode=0).startswith("values_kernel<float, true, 8>")  # few points
     # second derivatives in float32 stay where they were
     assert not _plan_text(library, 200_000, 24, False, True, mode=2).startswith("pairs")

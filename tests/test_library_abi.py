@@ -97,24 +97,27 @@ def test_launch_plans(library):
     assert text.value.decode().startswith("recursion_kernel<double, 2, false, true, true, false, true> [4 points per tile, 1024 threads")
     assert library.sphx_describe_plan(100_000, 16, 2, 1, 1, text, 512) == 0
     assert "512 threads" in text.value.decode()
-    # values: as many points per workgroup as fit in half a CU's LDS, in steps of four; in float32
-    # one workgroup with all of LDS while 40 points fit; from l_max = 24 (float64: 19) pairs_kernel with as
-    # many points per tile as fit (and the lanes kernel again where there are few points)
+    # values, where no kernel with l_max for a constant is ahead: as many points per workgroup as fit in half a CU's LDS,
+    # in steps of four; at large l_max pairs_kernel with as many points per tile as fit (and the lanes kernel again where
+    # there are few points)
     status, (tile, threads, lds, groups) = _plan(library, 1_000_000, 16, 0, False)
     assert status == 0 and (tile, threads) == (60, 512) and lds == 60 * (289 + 51) * 4
-    status, (tile, threads, lds, groups) = _plan(library, 1_000_000, 28, 0, False)
-    assert status == 0 and (tile, threads, groups) == (25, 1024, 256) and 150_000 < lds <= 160 * 1024
-    status, (tile, threads, lds, groups) = _plan(library, 20_000, 28, 0, False)
-    assert status == 0 and (tile, threads) == (44, 768) and 80 * 1024 < lds <= 160 * 1024
-    # tiles of 32 and 16 points: two and four channels side by side in a wave
-    assert _plan(library, 1_000_000, 22, 0, False)[1][:2] == [32, 512]
-    assert _plan(library, 20_000, 26, 0, False)[1][:2] == [16, 320]
-    assert _plan(library, 20_000, 32, 0, False)[1][:2] == [32, 832]
-    assert _plan(library, 20_000, 34, 0, False)[1][1] == 1024
-    assert _plan(library, 20_000, 22, 0, True)[1][:2] == [32, 1024]
-    assert _plan(library, 20_000, 23, 0, True)[1][1] == 1024
-    assert _plan(library, 1_000_000, 32, 0, False)[1][:2] == [20, 1024]
-    assert _plan(library, 1_000_000, 24, 0, True)[1][0] == 16
+    status, (tile, threads, lds, groups) = _plan(library, 1_000_000, 34, 0, False)
+    assert status == 0 and (tile, threads, groups) == (18, 1024, 256) and 150_000 < lds <= 160 * 1024
+    # tiles of 32, 16 and 8 points: two, four and eight channels side by side in a wave
+    assert _plan(library, 1_000_000, 13, 0, False)[1][:2] == [32, 256]
+    assert _plan(library, 1_000_000, 18, 0, False)[1][:2] == [16, 192]
+    assert _plan(library, 10_000, 34, 0, False)[1][:2] == [8, 256]
+    assert _plan(library, 500_000, 14, 0, True)[1][:2] == [32, 256]
+    assert _plan(library, 20_000, 29, 0, True)[1][:2] == [16, 384]
+    assert _plan(library, 20_000, 34, 0, False)[1][1] == 1024  # recursion_kernel
+    assert _plan(library, 1_000_000, 29, 0, True)[1][:2] == [11, 1024]
+    # with l_max for a constant: small tiles, many workgroups
+    for n, l_max, f64, tile, lds in ((1_000_000, 22, False, 20, 20 * 529 * 4), (20_000, 26, False, 16, 16 * 729 * 4),
+                                     (1_000_000, 28, False, 16, 16 * 841 * 4), (1_000_000, 32, False, 16, 16 * 1089 * 4),
+                                     (20_000, 22, True, 16, 16 * 529 * 8), (20_000, 23, True, 16, 16 * (576 + 1) * 8)):
+        status, plan = _plan(library, n, l_max, 0, f64)
+        assert status == 0 and plan[:3] == [tile, 512, lds] and (plan[3] - 8) * tile < n <= plan[3] * tile, (n, l_max, f64)
     assert _plan(library, 10, 65, 0, False)[0] == 2       # beyond the tables
     assert _plan(library, 10, 64, 2, True)[0] == 2        # one point's rows no longer fit in LDS
     assert b"LDS" in library.sphx_last_error()

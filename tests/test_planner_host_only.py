@@ -18,39 +18,55 @@ SHAPES = [
     (10_000, 8, 1, 1, 1, "gradients_fixed_kernel<double, true, 8, 8>"),
     (100_000, 16, 2, 1, 0, "recursion_kernel<double, 2, false, true, true, false, true>"),
     (200_000, 32, 1, 0, 1, "pairs_kernel<float, 1, true>"),
-    (200_000, 32, 0, 0, 1, "pairs_kernel<float, 0, true>"),
-    (200_000, 20, 0, 1, 0, "pairs_kernel<double, 0, false>"),
+    (200_000, 32, 0, 0, 1, "values_fixed_kernel<float, true, 32, 8>"),
+    (200_000, 34, 0, 0, 1, "pairs_kernel<float, 0, true>"),
+    (200_000, 20, 0, 1, 0, "values_fixed_kernel<double, false, 20, 8>"),
+    (200_000, 25, 0, 1, 0, "pairs_kernel<double, 0, false>"),
     (1_000_000, 10, 0, 0, 1, "values_kernel<float, true, 1>"),
-    (1_000_000, 22, 0, 0, 1, "values_kernel<float, true, 2>"),
-    (500_000, 5, 2, 0, 1, "recursion_kernel<float, 2, true, true, false, false, true>"),
+    (3_000_000, 9, 0, 0, 1, "values_kernel<float, true, 1>"),
+    (1_000_000, 22, 0, 0, 1, "values_fixed_kernel<float, true, 22, 8>"),
+    (1_000_000, 13, 0, 0, 1, "values_kernel<float, true, 2>"),
+    (100_000, 8, 0, 0, 1, "values_fixed_kernel<float, true, 8, 4>"),
+    (500_000, 5, 2, 0, 1, "hessians_fixed_kernel<float, true, 5, 16>"),
+    (1_000_000, 4, 2, 0, 1, "recursion_kernel<float, 2, true, true, false, false, true>"),
     (500_000, 3, 2, 0, 1, "hessians_fixed_kernel<float, true, 3, 8>"),
-    (600_000, 2, 2, 0, 1, "hessians_lanes_kernel<float, true>"),
+    (4_000_000, 2, 2, 0, 1, "hessians_lanes_kernel<float, true>"),
     (1_000_000, 7, 0, 0, 0, "values_fixed_kernel<float, false, 7, 4>"),
     (2_000, 5, 2, 0, 1, "hessians_fixed_kernel<float, true, 5, 16>"),
     (600_000, 7, 1, 0, 0, "gradients_lanes_kernel<float, false>"),
-    (1_000_000, 10, 1, 0, 1, "recursion_kernel<float, 1, true, true, false, false, true>"),
+    (1_000_000, 10, 1, 0, 1, "gradients_fixed_kernel<float, true, 10, 16>"),
+    (1_000_000, 10, 1, 0, 0, "recursion_kernel<float, 1, false, true, false, false, true>"),
+    (100_000, 19, 1, 0, 1, "recursion_kernel<float, 1, true, true, false, false, true>"),
     (50_000, 20, 2, 1, 1, "pairs_kernel<double, 2, true>"),
     (2_000, 32, 1, 0, 1, "recursion_kernel<float, 1, true, true, false, false, true>"),
     (2_000, 40, 1, 1, 1, "recursion_kernel<double, 1, true, false, false, false, false>"),
     (5, 24, 2, 1, 1, "recursion_kernel<double, 2, true, true, false, false, false>"),
     (1, 0, 0, 0, 1, "closed_form_kernel<float, 0, true, 0, false>"),
-    # values: channels side by side by the rounds that the tiles take on the CUs
-    (45_000, 12, 0, 0, 1, "values_kernel<float, true, 1>"),
-    (60_000, 12, 0, 0, 1, "values_kernel<float, true, 2>"),
-    (200_000, 12, 0, 0, 1, "values_kernel<float, true, 2>"),
-    (8_000, 18, 0, 1, 1, "values_kernel<double, true, 4>"),
-    (10_000, 18, 0, 1, 1, "values_kernel<double, true, 8>"),
-    (12_000, 18, 0, 1, 1, "values_kernel<double, true, 1>"),
-    (9_000, 21, 0, 1, 1, "values_kernel<double, true, 1>"),
-    (9_000, 26, 0, 0, 1, "values_kernel<float, true, 8>"),
-    (12_000, 26, 0, 0, 1, "values_kernel<float, true, 4>"),
+    # values: channels side by side, four or eight by the rounds that the tiles take on the CUs
+    (600_000, 16, 0, 0, 1, "values_kernel<float, true, 2>"),
+    (300_000, 17, 0, 0, 1, "values_kernel<float, true, 4>"),
+    (1_000_000, 10, 0, 1, 1, "values_kernel<double, true, 1>"),
+    (500_000, 14, 0, 1, 1, "values_kernel<double, true, 2>"),
+    (9_000, 29, 0, 1, 1, "values_kernel<double, true, 4>"),
+    (4_000, 33, 0, 0, 1, "values_kernel<float, true, 4>"),
+    (9_000, 33, 0, 0, 1, "values_kernel<float, true, 8>"),
+    # values and second derivatives in mid-sized and large calls: no gaps between the ranges
+    (60_000, 12, 0, 0, 1, "values_fixed_kernel<float, true, 12, 8>"),
+    (12_000, 26, 0, 0, 1, "values_fixed_kernel<float, true, 26, 8>"),
+    (20_000, 28, 0, 0, 1, "values_fixed_kernel<float, true, 28, 8>"),
+    (1_000_000, 30, 0, 0, 1, "values_fixed_kernel<float, true, 30, 8>"),
+    (10_000, 18, 0, 1, 1, "values_fixed_kernel<double, true, 18, 8>"),
+    (9_000, 21, 0, 1, 1, "values_fixed_kernel<double, true, 21, 8>"),
+    (20_000, 23, 0, 1, 1, "values_fixed_kernel<double, true, 23, 8>"),
+    (300_000, 9, 2, 0, 0, "hessians_fixed_kernel<float, false, 9, 16>"),
+    (300_000, 10, 2, 0, 0, "hessians_fixed_kernel<float, false, 10, 16>"),
     # the flush at raised priority: by the table of shapes, and only with many tiles per workgroup
     (200_000, 33, 1, 0, 0, "pairs_kernel<float, 1, false>"),
     (40_000, 33, 1, 0, 0, "pairs_kernel<float, 1, false>"),
-    (300_000, 10, 2, 0, 0, "recursion_kernel<float, 2, false, true, false, false, true>"),
-    (300_000, 9, 2, 0, 0, "recursion_kernel<float, 2, false, true, false, false, true>"),
+    (300_000, 14, 2, 0, 0, "recursion_kernel<float, 2, false, true, false, false, true>"),
+    (300_000, 15, 2, 0, 0, "recursion_kernel<float, 2, false, true, false, false, true>"),
 ]
-PRIORITY = {(200_000, 33): True, (40_000, 33): False, (300_000, 10): True, (300_000, 9): False}
+PRIORITY = {(200_000, 33, 1, 0): True, (300_000, 14, 2, 0): True, (1_000_000, 10, 1, 0): True}  # (n, l_max, mode, normalized)
 
 
 @pytest.fixture(scope="module")
@@ -71,7 +87,7 @@ def test_plans_without_a_device_match_the_library_and_name_the_intended_kernels(
         assert library.sphx_describe_plan(n, l_max, mode, is_f64, normalized, text, len(text)) == 0
         assert line == text.value.decode(), (n, l_max, mode, is_f64, normalized)
         assert line.split(" + ")[-1].startswith(kernel + " ["), (line, kernel)
-        assert line.endswith("(flush at raised priority)") == PRIORITY.get((n, l_max), False), line
+        assert line.endswith("(flush at raised priority)") == PRIORITY.get((n, l_max, mode, normalized), False), line
 
 
 def test_shapes_beyond_the_tables_or_lds_are_refused_with_a_message(probe):
