@@ -58,15 +58,16 @@ SHAPES = [
     (10_000, 18, 0, 1, 1, "values_fixed_kernel<double, true, 18, 8>"),
     (9_000, 21, 0, 1, 1, "values_fixed_kernel<double, true, 21, 8>"),
     (20_000, 23, 0, 1, 1, "values_fixed_kernel<double, true, 23, 8>"),
-    (300_000, 9, 2, 0, 0, "hessians_fixed_kernel<float, false, 9, 16>"),
-    (300_000, 10, 2, 0, 0, "hessians_fixed_kernel<float, false, 10, 16>"),
+    (2_000_000, 10, 1, 0, 1, "gradients_fixed_kernel<float, true, 10, 16>"),
     # the flush at raised priority: by the table of shapes, and only with many tiles per workgroup
     (200_000, 33, 1, 0, 0, "pairs_kernel<float, 1, false>"),
     (40_000, 33, 1, 0, 0, "pairs_kernel<float, 1, false>"),
+    (300_000, 10, 2, 0, 0, "recursion_kernel<float, 2, false, true, false, false, true>"),
+    (300_000, 9, 2, 0, 0, "recursion_kernel<float, 2, false, true, false, false, true>"),
     (300_000, 14, 2, 0, 0, "recursion_kernel<float, 2, false, true, false, false, true>"),
     (300_000, 15, 2, 0, 0, "recursion_kernel<float, 2, false, true, false, false, true>"),
 ]
-PRIORITY = {(200_000, 33, 1, 0): True, (300_000, 14, 2, 0): True, (1_000_000, 10, 1, 0): True}  # (n, l_max, mode, normalized)
+PRIORITY = {(200_000, 33, 1, 0): True, (300_000, 14, 2, 0): True, (300_000, 10, 2, 0): True, (1_000_000, 10, 1, 0): True}  # (n, l_max, mode, normalized)
 
 
 @pytest.fixture(scope="module")
