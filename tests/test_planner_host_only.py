@@ -27,6 +27,11 @@ SHAPES = [
     (1_000_000, 22, 0, 0, 1, "values_fixed_kernel<float, true, 22, 8>"),
     (1_000_000, 13, 0, 0, 1, "values_kernel<float, true, 2>"),
     (100_000, 8, 0, 0, 1, "values_fixed_kernel<float, true, 8, 4>"),
+    (3_500_000, 8, 0, 0, 0, "values_fixed_kernel<float, false, 8, 4>"),
+    (300_000, 22, 0, 0, 1, "values_fixed_kernel<float, true, 22, 8>"),
+    (500_000, 22, 0, 0, 0, "values_fixed_kernel<float, false, 22, 8>"),
+    (100_000, 4, 2, 0, 1, "hessians_fixed_kernel<float, true, 4, 8>"),
+    (600_000, 4, 2, 0, 1, "hessians_fixed_kernel<float, true, 4, 8>"),
     (500_000, 5, 2, 0, 1, "hessians_fixed_kernel<float, true, 5, 16>"),
     (1_000_000, 4, 2, 0, 1, "recursion_kernel<float, 2, true, true, false, false, true>"),
     (500_000, 3, 2, 0, 1, "hessians_fixed_kernel<float, true, 3, 8>"),
