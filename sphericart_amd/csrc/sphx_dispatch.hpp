@@ -67,19 +67,10 @@ static hipError_t launch_recursion(const Launch& l, const typename AsGiven<O>::t
         }
     }
     if constexpr (MODE == 2 && NORM && sizeof(T) == 4 && LIST && !SPLIT && NT == 2 * kRecursionThreads && POINTS_L == 0) {
-        // the variants with one point per lane; for odd l_max, whose rows lie one element apart, only where every array starts at a multiple of 16 bytes
-        const bool aligned = ((reinterpret_cast<uintptr_t>(sph) | reinterpret_cast<uintptr_t>(dsph) |
-                               reinterpret_cast<uintptr_t>(ddsph)) & 15u) == 0;
-        if (l.g.point_lanes != 0 && (aligned || l.g.l_max % 2 == 0)) {
-            auto with = [&](auto l_max) {
-                return launch_recursion<T, MODE, NORM, WHOLE, SPLIT, VJP, LIST, O, NT, TOGETHER, decltype(l_max)::value>(
-                    l, xyz, sph, dsph, ddsph, stream);
-            };
-            switch (l.g.l_max) {
-            case 4: return with(std::integral_constant<int, 4>{});
-            case 5: return with(std::integral_constant<int, 5>{});
-            default: return hipErrorInvalidValue; // never planned
-            }
+        // the variant with one point per lane
+        if (l.g.point_lanes != 0) {
+            if (l.g.l_max != 4) return hipErrorInvalidValue; // never planned
+            return launch_recursion<T, MODE, NORM, WHOLE, SPLIT, VJP, LIST, O, NT, TOGETHER, 4>(l, xyz, sph, dsph, ddsph, stream);
         }
     }
     if ((l.g.together != 0) != TOGETHER) return hipErrorInvalidValue; // never planned
@@ -152,16 +143,18 @@ static hipError_t dispatch(const Plan& plan, const DeviceState& device, const T*
         if constexpr (MODE == 2) {
             const Launch& l = plan.closed;
             if (l.g.fixed != 0) return dispatch_hessians_fixed<T>(l, NORM, xyz, sph, dsph, ddsph, stream);
-            if (l.threads > hessian_lane_threads<T>()) return hipErrorInvalidValue; // never planned
-            auto kernel = hessians_lanes_kernel<T, NORM>;
-            if (l.lds_bytes > 64u * 1024u) {
-                unsigned unused = 0;
-                hipError_t e = kernel_facts(reinterpret_cast<const void*>(kernel), l.threads, l.lds_bytes, &unused);
-                if (e != hipSuccess) return e;
+            if constexpr (sizeof(T) == 4) {
+                if (l.threads > kHessianLaneThreads) return hipErrorInvalidValue; // never planned
+                auto kernel = hessians_lanes_kernel<T, NORM>;
+                if (l.lds_bytes > 64u * 1024u) {
+                    unsigned unused = 0;
+                    hipError_t e = kernel_facts(reinterpret_cast<const void*>(kernel), l.threads, l.lds_bytes, &unused);
+                    if (e != hipSuccess) return e;
+                }
+                hipLaunchKernelGGL(kernel, dim3(l.workgroups), dim3(l.threads), l.lds_bytes, stream, l.g, xyz, sph,
+                                   dsph, ddsph);
+                return hipGetLastError();
             }
-            hipLaunchKernelGGL(kernel, dim3(l.workgroups), dim3(l.threads), l.lds_bytes, stream, l.g, xyz, sph,
-                               dsph, ddsph);
-            return hipGetLastError();
         }
         return hipErrorInvalidValue;
     }

@@ -30,7 +30,7 @@ struct Tiling {
     unsigned slice_waves;   // not 0: this many waves of their own (together: and wave 0) evaluate the closed
                             // forms of l <= 6 (whole rows); 0: the slices go round all waves
     unsigned together;      // recursion_kernel, float64: 1 = the recursions run next to the entries (TOGETHER)
-    unsigned row_pad;       // recursion_kernel, whole rows: elements left free after every staged row (0, 16 bytes' worth or, point_lanes, 0 or 1)
+    unsigned row_pad;       // recursion_kernel, whole rows: elements left free after every staged row (0 or 16 bytes' worth)
     unsigned magic_ny;      // ceil(2^32 / ny)
     unsigned priorities;    // recursion_kernel: 1 = the waves that flush run at raised priority, 2 = those that prepare the next tile
     // LDS carve-up, in elements of T: the staged rows come first, rows_elems of them, with the
@@ -47,7 +47,7 @@ struct Tiling {
     // in the job table when they are moved to wave boundaries of the entry lanes (0: they follow
     // the bulk without gaps); jobs_per_point then counts the gaps too
     unsigned kind_at[3];
-    unsigned fixed;       // gradients_fixed_kernel or hessians_fixed_kernel, which have l_max for a constant
+    unsigned fixed;       // values_fixed_kernel, gradients_fixed_kernel or hessians_fixed_kernel, which have l_max for a constant
     unsigned point_lanes; // recursion_kernel, normalised second derivatives: one point per lane, a job for a whole wave
 };
 
@@ -84,10 +84,9 @@ constexpr unsigned closed_form_phases(unsigned elem, int mode, int H) {
     return phases;
 }
 
-// threads of a workgroup of hessians_lanes_kernel (float64 entries need more than 128 registers; float32 with
-// 512 threads and 128 registers per lane was 5-15 % slower at l_max = 2-5 with the same number of waves)
+// threads of a workgroup of hessians_lanes_kernel (with 512 threads and 128 registers per lane 5-15 % slower at l_max = 2-5
+// with the same number of waves)
 constexpr unsigned kHessianLaneThreads = 256;
-template <typename T> constexpr unsigned hessian_lane_threads() { return kHessianLaneThreads; }
 
 } // namespace sphx
 

@@ -507,7 +507,7 @@ __global__ __launch_bounds__(NT) void gradients_lanes_kernel(Tiling g, const T* 
 // g.sequence_waves (1, 2 or 4): the waves that share one channel, each taking a part of its m.
 // ---------------------------------------------------------------------------
 template <typename T, bool NORM>
-__global__ __launch_bounds__(hessian_lane_threads<T>()) void hessians_lanes_kernel(Tiling g, const T* __restrict__ xyz,
+__global__ __launch_bounds__(kHessianLaneThreads) void hessians_lanes_kernel(Tiling g, const T* __restrict__ xyz,
                                                                             T* __restrict__ sph,
                                                                             T* __restrict__ dsph,
                                                                             T* __restrict__ ddsph) {

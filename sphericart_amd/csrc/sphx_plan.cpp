@@ -165,22 +165,9 @@ static bool plan_values(size_t n_samples, int l_max, size_t elem, int lds_limit,
     const bool four_fit = rounds(16u, 4u) != ~static_cast<size_t>(0);
     if (!with_sums && n_samples < 16384 && l_max >= 16) {
         // Fewer points than 64 for every CU: tiles of 16 reach four times as many of them (us, 3 000 points, one / two /
-        // four channels: float32 l_max = 18 7.2 5.7 5.6, 28 11.6 8.0 7.3; float64 18 8.3 6.9 6.6, 26 16.5 - 8.4), unless
-        // that takes a round more than tiles of 8 (four / eight channels: float32 26, 9 000 points 12.4 10.4; 33, 5 000
-        // 13.7 9.8; float64 23, 4 551 and 14 000 points 13.3 10.1, 25.8 23.5; as many rounds, 23, 8 000 15.1 16.0, 25, 6 000
-        // 14.4 15.4) or, in float64, more than the one in which the largest tiles take all points with one channel per
-        // wave (four / one: 16, 14 000 points 12.4 11.7; 18, 12 000 12.4 11.8; 20, 10 000 13.1 12.6; 21, 9 000 14.3
-        // 12.9; float32 28, 10 000 14.2 15.3).
-        const unsigned largest = allowed / ((row_stride + table_elems) * esize) / 4u * 4u;
+        // four channels: float32 l_max = 28 11.6 8.0 7.3; float64 26 16.5 - 8.4), unless that takes a round more than tiles
+        // of 8 (four / eight channels: float32 33, 5 000 points 13.7 9.8).
         pack_by_shape = four_fit && rounds(8u, 8u) < rounds(16u, 4u) ? 8u : 4u;
-        if (pack_by_shape == 4 && elem == 8 && rounds(16u, 4u) > 1 && largest >= 32 && rounds(largest < 64 ? largest : 64u, 1u) == 1) {
-            pack_by_shape = 1;
-        }
-    } else if (!with_sums && pack_by_shape == 2 && rounds(64u, 1u) <= 3 && rounds(32u, 2u) > rounds(64u, 1u)) {
-        // Two channels where their tiles fill the CUs once more than whole waves of points do, and not often: one (float32,
-        // l_max = 12, us, two / one: 45 000 points 10.1 8.7, 90 000 15.6 15.0, 130 000 19.5 18.7; as many rounds, 60 000
-        // points 11.0 11.7, four and five, 200 000, 26.9 26.8).
-        pack_by_shape = 1;
     }
     const int waves_by_shape = shape ? shape->waves : 0;
     const unsigned floor_by_shape = shape ? shape->floor : 32u;
@@ -446,25 +433,22 @@ static bool plan_gradient_lanes(size_t n_samples, int l_max, size_t elem, int ld
     return true;
 }
 
-// hessians_lanes_kernel: 64 or 32 points per workgroup with their thirteen rows, tables and
+// hessians_lanes_kernel (float32): 64 or 32 points per workgroup with their thirteen rows, tables and
 // iterates in LDS. Returns false when 32 points do not fit.
-static bool plan_hessian_lanes(size_t n_samples, int l_max, size_t elem, int lds_limit, Launch* out,
-                               bool normalized = true) {
+static bool plan_hessian_lanes(size_t n_samples, int l_max, int lds_limit, Launch* out) {
     Tiling& g = out->g;
     std::memset(&g, 0, sizeof(g));
-    const unsigned esize = static_cast<unsigned>(elem);
+    const unsigned esize = 4u;
     const unsigned ny = static_cast<unsigned>(l_max + 1) * (l_max + 1);
     const unsigned vec = 16u / esize;
     auto stride_of = [&](unsigned block) { return (block * (esize / 4u)) % 8u == 0 ? block + vec : block; };
     const unsigned s_stride = stride_of(ny), d_stride = stride_of(3u * ny), dd_stride = stride_of(9u * ny);
     const unsigned table_stride = (3u * static_cast<unsigned>(l_max + 1)) | 1u;
     const unsigned channels = static_cast<unsigned>(l_max - 1);
-    const unsigned most = (elem == 4 ? hessian_lane_threads<float>() : hessian_lane_threads<double>()) / 64u;
-    // Waves per channel, each with a part of its m: two where one or two channels would leave the workgroup with
-    // one or two waves and that measured faster (l_max = 3 in float32 and for solid harmonics in float64, l_max = 2
-    // in float32: 5-20 %).
-    const bool shared = (l_max == 3 && (elem == 4 || !normalized)) || (l_max == 2 && elem == 4);
-    unsigned parts = static_cast<unsigned>(switch_or(SW_HESSIAN_LANES_PARTS, shared ? 2 : 1));
+    const unsigned most = kHessianLaneThreads / 64u;
+    // Waves per channel, each with a part of its m: two where one channel would leave the workgroup with one wave (l_max =
+    // 2: 5-20 %).
+    unsigned parts = static_cast<unsigned>(switch_or(SW_HESSIAN_LANES_PARTS, l_max == 2 ? 2 : 1));
     if (parts != 1 && parts != 2 && parts != 4) parts = 1;
     while (parts > 1 && parts > most) parts /= 2;
     const unsigned slots = channels * parts <= most ? channels : most / parts;
@@ -588,18 +572,15 @@ static bool plan_recursion(size_t n_samples, int l_max, int mode, bool whole, si
     // (whole rows a multiple of 64 bytes long, l_max = 3 mod 4, would all start on one LDS bank: 16 bytes are left
     // free after each, which the flush skips; recursion_kernel, row_pad. Not below l_max = 7, where a tile can be
     // shorter than the line its end is carried in.)
-    // One point per lane and a job for a whole wave (the POINTS_L variants of recursion_kernel, their rows an odd number
-    // of elements apart): normalised second derivatives in float32 at l_max = 4-7, where the rows of 38 to 64 points fit
-    // and the vector units are what a tile waits for. us, list of jobs / this, 20 000, 100 000 and 500 000 points: l_max = 4
-    // 14.4 / 12.5, 35.0 / 31.4, 134 / 118; 5 17.7 / 15.4, 46.8 / 43.3, 187 / 169 (177 / 183 on another box); 6 20.2 / 18.3,
-    // 60.8 / 55.2, 266 / 235; 7 29.4 / 25.8, 84 / 72, 367 / 330; 8, with 35 of 64 lanes at work, 27.7 / 30.1, 87 / 97,
-    // 395 / 415. Solid harmonics, whose jobs are mostly stores, gain below 100 000 points and lose beyond (500 000,
-    // l_max = 4-7: 111 / 128, 160 / 181, 222 / 241, 283 / 313). Fewer points than 64 for every CU leave lanes idle.
+    // One point per lane and a job for a whole wave (the POINTS_L variant of recursion_kernel): normalised second derivatives
+    // in float32 at l_max = 4, where the rows of 64 points fit and the vector units are what a tile waits for, in calls too
+    // large for hessians_fixed_kernel. us, list of jobs / this, 20 000, 100 000 and 500 000 points: 14.4 / 12.5, 35.0 / 31.4,
+    // 134 / 118. Solid harmonics, whose jobs are mostly stores, lose there (500 000: 111 / 128). Fewer points than 64 for
+    // every CU leave lanes idle.
     const bool point_lanes = mode == 2 && whole && elem == 4 && osize == 4 && normalized && threads > kRecursionThreads &&
-                             l_max >= 4 && l_max <= 5 && switch_or(SW_JOB_LIST, 2) == 2 &&
+                             l_max == 4 && switch_or(SW_JOB_LIST, 2) == 2 &&
                              switch_or(SW_POINT_LANES, n_samples >= 16384 ? 1 : 0) != 0;
-    const unsigned row_pad = point_lanes ? 1u - ny % 2u
-                             : whole && l_max >= 7 && (ny * osize) % 64u == 0 && switch_or(SW_ROW_PAD, 1) != 0 ? 16u / osize : 0u;
+    const unsigned row_pad = whole && l_max >= 7 && (ny * osize) % 64u == 0 && switch_or(SW_ROW_PAD, 1) != 0 ? 16u / osize : 0u;
     const unsigned row_stride = nrow + (whole ? row_pad : nyh % (16u / osize));
     g.row_pad = row_pad;
     g.magic_ny = magic_of(ny);
@@ -815,7 +796,6 @@ static bool plan_recursion(size_t n_samples, int l_max, int mode, bool whole, si
         g.points_per_pass = 0;
     }
     g.point_lanes = point_lanes && !*split_sides && g.points_per_pass == 0 ? 1u : 0u;
-    if (point_lanes && g.point_lanes == 0) g.row_pad = 0; // (not the list after all: its rows lie back to back)
 
     // in front of every staging region, room for the part of a 128-byte line that precedes the
     // tile's run (recursion_kernel, flush_run)
@@ -968,12 +948,11 @@ int make_plan(size_t n_samples, int l_max, int mode, size_t elem, int lds_limit,
     }
     // Values alone where the rows of few points fill LDS: pairs_kernel (below, with the derivatives), which keeps
     // the recursions of the next tile and the flush of this one side by side. values_kernel is ahead where LDS holds
-    // three of its workgroups or more (1.2 GB, us, pairs_kernel / values_kernel: float32 l_max = 24 266 / 208, 25 245 /
-    // 203, 26 239 / 220 (50 000 points 37.2 / 38.4), 27 255 / 233, 28 251 / 236, 29 220 / 226, 31 222 / 239, 33 260 / 343; float64 19 221 / 240,
-    // 20 217 / 218, 21 281 / 218, 22 279 / 227, 23 324 / 270, 24 243 / 238, 25 211 / 291).
+    // three of its workgroups or more, values_fixed_kernel where it exists but for float64 l_max = 25 in large calls (1.2 GB,
+    // us, pairs_kernel / values_kernel: float32 l_max = 33 260 / 343; float64 25 211 / 291).
     if (lane_kernels && mode == 0 && l_max > hard) {
         const int pairs = switch_or(SW_PAIRS, 1);
-        const bool pairs_by_shape = n_samples >= 32768 && (elem == 4 ? l_max == 26 || l_max >= 28 : l_max >= 24 || l_max == 19 || l_max == 20);
+        const bool pairs_by_shape = n_samples >= 32768 && l_max >= (elem == 4 ? 33 : 25);
         if (pairs == 2 || (pairs == 1 && pairs_by_shape)) {
             PairsChoice want;
             want.tile = static_cast<unsigned>(switch_or(SW_PAIRS_TILE, 0));
@@ -997,14 +976,11 @@ int make_plan(size_t n_samples, int l_max, int mode, size_t elem, int lds_limit,
         plan->lanes = true;
         return SPHX_OK;
     }
-    // Second derivatives at small l_max: one point per lane where that was measured to be faster
-    // than the recursion kernel (SPHX_HESSIAN_LANES: 0 never, 2 wherever the rows fit).
+    // Second derivatives at l_max = 2 in float32, in calls too large for the kernel with l_max for a constant: one point per
+    // lane (SPHX_HESSIAN_LANES: 0 never, 2 wherever the rows fit; float32 only).
     const int hessian_lanes = switch_or(SW_HESSIAN_LANES, 1);
-    // (Since the recursion kernel takes its jobs as a list ordered by kind it wins from l_max = 4 on; the lanes keep
-    // l_max <= 3 in float32 and, for calls too small for workgroups of 1024 threads, solid l_max = 3 in float64.)
-    const bool hessian_lanes_pay = elem == 4 ? l_max <= 3 : (l_max == 3 && !normalized && n_samples < 32768);
-    if (lane_kernels && mode == 2 && (hessian_lanes == 2 || (hessian_lanes == 1 && hessian_lanes_pay)) &&
-        plan_hessian_lanes(n_samples, l_max, elem, lds_limit, &plan->closed, normalized)) {
+    if (lane_kernels && mode == 2 && elem == 4 && (hessian_lanes == 2 || (hessian_lanes == 1 && l_max == 2)) &&
+        plan_hessian_lanes(n_samples, l_max, lds_limit, &plan->closed)) {
         plan->lanes = true;
         return SPHX_OK;
     }
@@ -1042,18 +1018,11 @@ int make_plan(size_t n_samples, int l_max, int mode, size_t elem, int lds_limit,
             }
         }
     }
-    // Gradients just above the closed forms: the lanes kernel (one point per lane, the channels dealt to the
-    // waves) up to l_max = 13 in float32 and wherever its tiles fit in float64; from there the recursion kernel with
-    // its jobs as a list ordered by kind is ahead. Where the recursion kernel runs in workgroups of 1024 threads
-    // (calls of 32 768 points or more) it is ahead from l_max = 8 on (3-20 %): the lanes keep l_max = 7; at
-    // 20 000 points from l_max = 10 on (6-30 %).
-    // SPHX_GRADIENT_LANES: 0 never, 2 wherever the rows fit.
+    // Gradients at l_max = 7 in calls too large for the kernel with l_max for a constant (solid harmonics): the lanes kernel,
+    // one point per lane, the channels dealt to the waves. From l_max = 8 on the recursion kernel is ahead of it in such
+    // calls (3-20 %). SPHX_GRADIENT_LANES: 0 never, 2 wherever the rows fit.
     const int gradient_lanes = switch_or(SW_GRADIENT_LANES, 1);
-    const bool large_groups = group_threads(n_samples, mode, elem, lane_kernels) > kRecursionThreads && n_samples >= 32768;
-    // (float64, normalised, l_max = 7: the recursion kernel is 8 % ahead there, 203 against 219 us per 1.2 GB)
-    const bool lanes_by_shape = large_groups ? l_max <= (elem == 8 && normalized ? 6 : 7)
-                                             : (n_samples >= 16384 ? l_max <= 9 : elem == 8 || l_max <= 13);
-    if (lane_kernels && mode == 1 && gradient_lanes != 0 && (gradient_lanes == 2 || lanes_by_shape) &&
+    if (lane_kernels && mode == 1 && gradient_lanes != 0 && (gradient_lanes == 2 || l_max == 7) &&
         plan_gradient_lanes(n_samples, l_max, elem, lds_limit, cus, &plan->closed)) {
         plan->lanes = true;
         return SPHX_OK;

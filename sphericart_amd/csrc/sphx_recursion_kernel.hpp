@@ -83,7 +83,7 @@ __global__ __launch_bounds__(NT, MODE < 2 ? 4 : 1) void recursion_kernel(Tiling 
                                                                      O* __restrict__ ddsph) {
     static_assert(!VJP || (MODE == 1 && !SPLIT), "the fused product is built on the gradient kernel");
     static_assert(!VJP || std::is_same<T, O>::value, "the fused product stages what it computes");
-    static_assert(POINTS_L == 0 || (LIST && MODE == 2 && WHOLE && !SPLIT && sizeof(O) == 4), "one point per lane");
+    static_assert(POINTS_L == 0 || (POINTS_L % 2 == 0 && LIST && MODE == 2 && WHOLE && !SPLIT && sizeof(O) == 4), "one point per lane");
     static_assert(!TOGETHER || sizeof(T) == 8, "float32 has the recursions in the flush only");
     constexpr int H = MODE == 2 ? 1 : 6;
     constexpr unsigned NYH = (H + 1) * (H + 1);
@@ -110,10 +110,10 @@ __global__ __launch_bounds__(NT, MODE < 2 ? 4 : 1) void recursion_kernel(Tiling 
     // and 12). The host then asks for 16 bytes between the staged rows, g.row_pad elements; the flush skips them
     // (flush_run). They keep a row's 16-byte vectors whole only where the arrays start at multiples of 16 bytes:
     // for other pointers the rows stay back to back.
-    // POINTS_L: rows an odd number of elements apart, so that the lanes of a wave, which store the same entry of their
-    // points, spread over all banks (the arrays then start at multiples of 16 bytes).
+    // POINTS_L (even): rows of an odd number of elements back to back, so that the lanes of a wave, which store the same
+    // entry of their points, spread over all banks.
     const unsigned row_pad =
-        POINTS_L != 0 ? static_cast<unsigned>(POINTS_L % 2)
+        POINTS_L != 0 ? 0u
         : WHOLE && !VJP && ((reinterpret_cast<uintptr_t>(sph) | reinterpret_cast<uintptr_t>(dsph) |
                              reinterpret_cast<uintptr_t>(ddsph)) & 15u) == 0
             ? g.row_pad
@@ -597,16 +597,8 @@ __global__ __launch_bounds__(NT, MODE < 2 ? 4 : 1) void recursion_kernel(Tiling 
                     V* out = reinterpret_cast<V*>(line0 + full_lo);
                     // (two or four loads in flight per lane ahead of their stores: no faster on any shape)
                     for (unsigned v = ft; v < nvec; v += count) {
-                        if constexpr (POINTS_L % 2 != 0) { // (a vector lies inside one row)
-                            const O* from = region + staged_at(full_lo + v * W);
-                            V hold;
-#pragma unroll
-                            for (unsigned k = 0; k < W; ++k) hold[k] = from[k];
-                            emit<O, SPHX_STREAMING_STORES>(hold, out + v);
-                        } else {
-                            emit<O, SPHX_STREAMING_STORES>(*reinterpret_cast<const V*>(region + staged_at(full_lo + v * W)),
-                                                           out + v);
-                        }
+                        emit<O, SPHX_STREAMING_STORES>(*reinterpret_cast<const V*>(region + staged_at(full_lo + v * W)),
+                                                       out + v);
                     }
                     tail_from = full_hi;
                 } else {

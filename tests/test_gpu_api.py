@@ -117,8 +117,8 @@ def test_second_derivatives_at_small_l_max_by_both_kernels(oracle, library, rout
             normalized = bool((l_max + n) & 1)
             announce("small l_max hessians", route, np.dtype(dtype).name, l_max, n, shift, normalized)
             planned = plan_text(library, n, l_max, "hessians", dtype, normalized)
-            fits = route == "lanes" and (dtype == np.float32 or l_max <= 5)  # (a tile's rows in LDS)
-            assert planned.startswith("hessians_lanes_kernel<" if fits else "recursion_kernel<"), planned
+            lanes = route == "lanes" and dtype == np.float32  # (there is no such kernel in float64)
+            assert planned.startswith("hessians_lanes_kernel<" if lanes else "recursion_kernel<"), planned
             ny = (l_max + 1) ** 2
             xyz = special_points(dtype, rng, n)
             want = oracle.compute(xyz, l_max, normalized, "hessians")

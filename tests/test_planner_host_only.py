@@ -96,6 +96,15 @@ def test_plans_without_a_device_match_the_library_and_name_the_intended_kernels(
         assert line.endswith("(flush at raised priority)") == PRIORITY.get((n, l_max, mode, normalized), False), line
 
 
+def test_every_row_of_the_planners_tables_is_reached(tmp_path):
+    """No row, and no l_max of one, that no call is planned by: such a row is a figure nobody can check by calling."""
+    binary = tmp_path / "rows_probe"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", os.path.join(ROOT, "tests", "rows_probe.cpp"),
+                    *(os.path.join(CSRC, name) for name in ("sphx_plan.cpp", "sphx_columns.cpp")), "-o", str(binary)], check=True)
+    out = subprocess.run([str(binary)], capture_output=True, text=True, check=True).stdout.splitlines()
+    assert out == ["done"], out
+
+
 def test_shapes_beyond_the_tables_or_lds_are_refused_with_a_message(probe):
     out = subprocess.run([probe, "10", "65", "0", "0", "1", "10", "64", "2", "1", "1"], capture_output=True, text=True,
                          check=True).stdout.splitlines()
