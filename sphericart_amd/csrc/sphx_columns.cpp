@@ -120,6 +120,7 @@ bool plan_columns(ColumnsKind kind, size_t n_samples, int l_max, size_t elem, in
     out->threads = 64u * static_cast<unsigned>(waves);
     out->lds_bytes = bytes;
     out->groups = kind == COLUMNS_ROWS ? 4 : static_cast<int>(64u / tile);
+    out->fixed = fixed_columns(kind, l_max) && fixed_columns_on(kind, elem, l_max, out->groups);
     return true;
 }
 

@@ -35,6 +35,7 @@ struct ColumnsLaunch {
     Columns g;
     unsigned workgroups, threads, lds_bytes;
     int groups; // lanes per point (columns_kernel: 1 or 2)
+    bool fixed; // the kernel that has l_max for a constant (not where the product is added to the output)
 };
 
 enum ColumnsKind {

@@ -22,7 +22,7 @@ static hipError_t launch_columns(Kernel kernel, const ColumnsLaunch& l, hipStrea
 template <typename T>
 hipError_t dispatch_columns(ColumnsKind kind, const ColumnsLaunch& l, bool normalized, const T* xyz, const T* sph_grad,
                             const T* upstream, T* xyz_grad, T* sph_grad_grad, hipStream_t s) {
-    if (fixed_columns(kind, l.g.l_max) && fixed_columns_on(kind, sizeof(T), l.g.l_max, l.groups) && l.g.accumulate == 0) {
+    if (l.fixed && l.g.accumulate == 0) {
         auto go = [&](auto dispatch) { return dispatch(l, normalized, xyz, sph_grad, upstream, xyz_grad, sph_grad_grad, s); };
         if (kind == COLUMNS_VJP) return go(dispatch_columns_fixed<T, COLUMNS_VJP>);
         if (kind == COLUMNS_VJP_BACKWARD) return go(dispatch_columns_fixed<T, COLUMNS_VJP_BACKWARD>);

@@ -1,7 +1,7 @@
 // The planner of columns_kernel and column_rows_kernel compiled on its own with a host compiler: for every shape given on
 // the command line as "kind n_samples l_max bytes" quadruples one line of numbers, for an MI355X (160 KB of LDS per
 // workgroup, 256 CUs): whether there is a plan, lanes per point, workgroups, threads, bytes of LDS, tiles, pad, the two
-// offsets, and for the vector-Jacobian product whether it is taken.
+// offsets, for the vector-Jacobian product whether it is taken, and whether the kernel has l_max for a constant.
 #include <cstdio>
 #include <cstdlib>
 
@@ -22,8 +22,8 @@ int main(int argc, char** argv) {
         if (kind == sphx::COLUMNS_VJP && sphx::make_vjp_plan(n, l_max, elem, 160 * 1024, 256, &other) == 0) {
             by_columns = sphx::vjp_by_columns(n, l_max, elem, 160 * 1024, 256, other, &taken);
         }
-        std::printf("%d %d %u %u %u %u %u %u %u %d\n", there, c.groups, c.workgroups, c.threads, c.lds_bytes, c.g.n_tiles,
-                    c.g.pad, c.g.off_rows, c.g.off_sums, by_columns);
+        std::printf("%d %d %u %u %u %u %u %u %u %d %d\n", there, c.groups, c.workgroups, c.threads, c.lds_bytes, c.g.n_tiles,
+                    c.g.pad, c.g.off_rows, c.g.off_sums, by_columns, there && c.fixed);
     }
     return 0;
 }

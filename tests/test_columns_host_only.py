@@ -17,10 +17,12 @@ def plans(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", os.path.join(ROOT, "tests", "columns_probe.cpp"),
                     *(os.path.join(CSRC, name) for name in ("sphx_columns.cpp", "sphx_plan.cpp")), "-o", str(binary)], check=True)
 
-    def run(shapes):
-        names = "there groups workgroups threads lds tiles pad off_rows off_sums by_columns".split()
+    def run(shapes, **switches):
+        """`switches`: overrides, read from the environment under SPHX_DEBUG_SWITCHES."""
+        names = "there groups workgroups threads lds tiles pad off_rows off_sums by_columns fixed".split()
+        env = dict(os.environ, SPHX_DEBUG_SWITCHES="1", **{name: str(value) for name, value in switches.items()})
         out = subprocess.run([str(binary)] + [str(v) for shape in shapes for v in shape], capture_output=True, text=True,
-                             check=True).stdout.splitlines()
+                             check=True, env=env).stdout.splitlines()
         assert len(out) == len(shapes)
         return [dict(zip(names, map(int, line.split()))) for line in out]
 
@@ -40,6 +42,23 @@ def test_which_kernel_a_product_gets(plans):
     }
     for shape, plan in zip(wanted, plans([(VJP, *shape) for shape in wanted])):
         assert bool(plan["by_columns"]) == wanted[shape], shape
+
+
+@pytest.mark.parametrize("elem", [4, 8])
+def test_which_products_have_a_kernel_with_l_max_for_a_constant(plans, elem):
+    """The product at l_max = 7-20, the second-order ones at 1-12, on two lanes per point and, where three tiles of 64 points
+    fit a CU, on one; calls of every size, and the settings that tests/test_gpu_columns.py forces on small ones."""
+    first_last = {VJP: (7, 20), VJP_BACKWARD: (1, 12), ROWS: (1, 12)}
+    for waves, tile, points in ((0, 0, (1, 129, 16_384, 16_385, 400_003)), (1, 64, (15,)), (3, 32, (31,)), (5, 64, (65,)), (2, 0, (129,))):
+        shapes = [(kind, n, l_max, elem) for kind in first_last for l_max in range(28) for n in points]
+        for (kind, n, l_max, _), plan in zip(shapes, plans(shapes, SPHX_COLUMNS_WAVES=waves, SPHX_COLUMNS_TILE=tile)):
+            ny = (l_max + 1) ** 2
+            row = (ny + (1 if ny % 2 == 0 and ny > 16 // elem else 0)) * elem
+            lanes = kind == ROWS or plan["groups"] == 2 or 3 * 64 * row <= 160 * 1024
+            wanted = plan["there"] and first_last[kind][0] <= l_max <= first_last[kind][1] and lanes
+            assert bool(plan["fixed"]) == bool(wanted), (kind, n, l_max, waves, tile)
+            if l_max <= 6 and tile == 64 and kind != ROWS:
+                assert plan["groups"] == 1 and plan["fixed"] == (kind == VJP_BACKWARD and l_max > 0)
 
 
 @pytest.mark.parametrize("elem", [4, 8])
