@@ -53,7 +53,7 @@ def test_every_l_max(oracle, library, switches, dtype, l_max, normalized):
                                              (np.float32, 22, 16_384), (np.float32, 24, 4_097), (np.float64, 16, 4_097),
                                              (np.float64, 18, 5_000), (np.float64, 20, 2_049), (np.float32, 30, 2_049), (np.float64, 24, 2_049)])
 def test_as_planned(oracle, library, dtype, l_max, n):
-    """Plans of mid-sized calls on both sides of the table's lines, and their neighbours that take another kernel."""
+    """Calls of sizes between the table's lines, as they are planned."""
     for normalized in (True, False):
         for points in (n - 1, n):
             announce("gradients as planned", np.dtype(dtype).name, l_max, normalized, points)
@@ -62,3 +62,38 @@ def test_as_planned(oracle, library, dtype, l_max, n):
             status, out = run_launch_layer(library, torch.from_numpy(xyz).cuda(), l_max, normalized, "gradients")
             assert status == 0, library.sphx_last_error()
             check(tuple(o.cpu().numpy() if o is not None else None for o in out), want, (l_max, points))
+
+
+@pytest.mark.parametrize("dtype, l_max, normalized, n, below, at", [
+    # (kernel<waves> tile, or the kernel without l_max for a constant that is ahead there)
+    (np.float32, 13, False, 131_072, "gradients_fixed_kernel<8> 16", "recursion_kernel"),
+    (np.float32, 17, True, 65_536, "gradients_fixed_kernel<8> 12", "gradients_fixed_kernel<8> 28"),
+    (np.float32, 19, True, 65_536, "gradients_fixed_kernel<8> 12", "recursion_kernel"),
+    (np.float32, 22, True, 16_384, "gradients_fixed_kernel<8> 8", "recursion_kernel"),
+    (np.float32, 24, False, 32_768, "gradients_fixed_kernel<8> 8", "pairs_kernel"),
+    (np.float32, 30, True, 2_049, "gradients_fixed_kernel<8> 8", "recursion_kernel"),
+    (np.float64, 14, True, 14_000, "gradients_fixed_kernel<8> 8", "recursion_kernel"),
+    (np.float64, 15, True, 16_384, "gradients_fixed_kernel<8> 8", "recursion_kernel"),
+    (np.float64, 16, True, 4_097, "gradients_fixed_kernel<8> 16", "recursion_kernel"),
+    (np.float64, 18, True, 5_000, "gradients_fixed_kernel<8> 12", "recursion_kernel"),
+    (np.float64, 20, True, 3_073, "gradients_fixed_kernel<8> 8", "recursion_kernel"),
+    (np.float64, 19, False, 8_192, "gradients_fixed_kernel<8> 12", "recursion_kernel"),
+    (np.float64, 20, False, 4_097, "gradients_fixed_kernel<8> 8", "recursion_kernel"),
+    (np.float64, 24, False, 2_049, "gradients_fixed_kernel<8> 8", "recursion_kernel"),
+    (np.float64, 8, False, 65_536, "gradients_fixed_kernel<8> 20", "gradients_fixed_kernel<16> 32"),
+    (np.float64, 12, True, 65_536, "gradients_fixed_kernel<8> 12", "gradients_fixed_kernel<8> 28"),
+])
+def test_both_sides_of_the_tables_lines(oracle, library, dtype, l_max, normalized, n, below, at):
+    for points, wanted in ((n - 1, below), (n, at)):
+        announce("gradients at a line", np.dtype(dtype).name, l_max, normalized, points, wanted)
+        planned = plan_text(library, points, l_max, "gradients", dtype, normalized)
+        if "_fixed_kernel" in wanted:
+            kernel, waves, tile = wanted.replace("<", " ").replace(">", "").split()
+            assert planned.startswith(kernel + "<") and f", {l_max}, {waves}> [l_max a constant, {tile} points" in planned, planned
+        else:
+            assert planned.startswith(wanted + "<"), planned
+        xyz = special_points(dtype, np.random.default_rng(l_max), points)
+        want = oracle.compute(xyz, l_max, normalized, "gradients")
+        status, out = run_launch_layer(library, torch.from_numpy(xyz).cuda(), l_max, normalized, "gradients")
+        assert status == 0, library.sphx_last_error()
+        check(tuple(o.cpu().numpy() if o is not None else None for o in out), want, (l_max, points))

@@ -50,7 +50,7 @@ def test_every_l_max(oracle, library, switches, dtype, l_max, normalized):
                                              (np.float64, 7, 1_024), (np.float64, 9, 1_024), (np.float64, 10, 8_192),
                                              (np.float32, 11, 12_287), (np.float32, 12, 4_097), (np.float32, 13, 3_000)])
 def test_as_planned(oracle, library, dtype, l_max, n):
-    """Plans on both sides of the table's lines, and their neighbours that take another kernel."""
+    """Calls of sizes between the table's lines, as they are planned."""
     for normalized in (True, False):
         for points in (n - 1, n):
             announce("second derivatives as planned", np.dtype(dtype).name, l_max, normalized, points)
@@ -59,3 +59,36 @@ def test_as_planned(oracle, library, dtype, l_max, n):
             status, out = run_launch_layer(library, torch.from_numpy(xyz).cuda(), l_max, normalized, "hessians")
             assert status == 0, library.sphx_last_error()
             check(tuple(o.cpu().numpy() for o in out), want, (l_max, points))
+
+
+@pytest.mark.parametrize("dtype, l_max, normalized, n, below, at", [
+    # (kernel<waves> tile, or the kernel without l_max for a constant that is ahead there)
+    (np.float32, 3, True, 131_072, "hessians_fixed_kernel<8> 32", "hessians_fixed_kernel<8> 28"),
+    (np.float32, 3, False, 131_072, "hessians_fixed_kernel<8> 32", "hessians_fixed_kernel<16> 24"),
+    (np.float32, 4, True, 32_768, "hessians_fixed_kernel<16> 32", "hessians_fixed_kernel<8> 32"),
+    (np.float32, 6, False, 65_536, "hessians_fixed_kernel<16> 32", "hessians_fixed_kernel<16> 16"),
+    (np.float32, 9, True, 65_536, "hessians_fixed_kernel<8> 12", "hessians_fixed_kernel<8> 28"),
+    (np.float32, 11, True, 12_288, "hessians_fixed_kernel<8> 20", "recursion_kernel"),
+    (np.float32, 12, True, 768, "recursion_kernel", "hessians_fixed_kernel<16> 8"),
+    (np.float32, 12, True, 4_097, "hessians_fixed_kernel<16> 16", "recursion_kernel"),
+    (np.float32, 13, True, 7_169, "hessians_fixed_kernel<8> 8", "recursion_kernel"),
+    (np.float64, 3, False, 65_536, "hessians_fixed_kernel<16> 32", "hessians_fixed_kernel<16> 16"),
+    (np.float64, 7, True, 1_024, "recursion_kernel", "hessians_fixed_kernel<8> 8"),
+    (np.float64, 9, False, 1_024, "recursion_kernel", "hessians_fixed_kernel<8> 8"),
+    (np.float64, 10, False, 8_192, "hessians_fixed_kernel<16> 12", "recursion_kernel"),
+    (np.float64, 5, False, 65_536, "hessians_fixed_kernel<16> 24", "hessians_fixed_kernel<16> 16"),
+])
+def test_both_sides_of_the_tables_lines(oracle, library, dtype, l_max, normalized, n, below, at):
+    for points, wanted in ((n - 1, below), (n, at)):
+        announce("second derivatives at a line", np.dtype(dtype).name, l_max, normalized, points, wanted)
+        planned = plan_text(library, points, l_max, "hessians", dtype, normalized)
+        if "_fixed_kernel" in wanted:
+            kernel, waves, tile = wanted.replace("<", " ").replace(">", "").split()
+            assert planned.startswith(kernel + "<") and f", {l_max}, {waves}> [l_max a constant, {tile} points" in planned, planned
+        else:
+            assert planned.startswith(wanted + "<"), planned
+        xyz = special_points(dtype, np.random.default_rng(l_max), points)
+        want = oracle.compute(xyz, l_max, normalized, "hessians")
+        status, out = run_launch_layer(library, torch.from_numpy(xyz).cuda(), l_max, normalized, "hessians")
+        assert status == 0, library.sphx_last_error()
+        check(tuple(o.cpu().numpy() if o is not None else None for o in out), want, (l_max, points))

@@ -138,6 +138,7 @@ def test_values_kernel_with_tiles_of_any_size(oracle, library, switches, dtype):
                 for step, least, pack, alone in ((None, None, None, None), (1, 8, 1, 0), (0, 32, 1, 0), (4, 8, 1, 1),
                                                  (4, 8, 2, 0), (4, 8, 4, 0), (4, 8, 2, 1)):
                     library.sphx_reset_switches()
+                    switches("SPHX_VALUES_FIXED", 0)  # (not the kernels with l_max for a constant)
                     if step is not None:
                         switches("SPHX_VALUES_TILE_STEP", step)
                         switches("SPHX_VALUES_MIN_TILE", least)
@@ -325,15 +326,17 @@ def test_literal_clouds_of_the_reference_at_full_size(oracle, library):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-def test_values_with_fewer_points_than_a_channel_has_prefactors(oracle, library, dtype):
+def test_values_with_fewer_points_than_a_channel_has_prefactors(oracle, library, switches, dtype):
     """values_kernel hands a channel's prefactors from lane to lane: with one, two or five points in a tile (or a
     last tile that holds so few) most of the lanes that hold a prefactor have no point. Every l_max the kernel
-    takes, to the largest of the tables."""
+    takes, to the largest of the tables; and the calls as they are planned."""
     rng = np.random.default_rng(53)
     for l_max in (7, 10, 20, 33, 40, 63):
         for n in (1, 2, 5, 25, 45, 64 + 3):
-            for normalized in (True, False):
-                announce("values, few points", np.dtype(dtype).name, normalized, l_max, n)
+            for normalized, fixed in ((True, 0), (False, 0), (True, 1), (False, 1)):
+                switches("SPHX_VALUES_FIXED", fixed)
+                assert fixed == 1 or "_fixed_kernel" not in plan_text(library, n, l_max, "values", dtype, normalized)
+                announce("values, few points", np.dtype(dtype).name, normalized, l_max, n, "fixed", fixed)
                 xyz = special_points(dtype, rng, n)
                 want = oracle.compute(xyz, l_max, normalized, "values")
                 status, got = run_launch_layer(library, torch.from_numpy(xyz).cuda(), l_max, normalized, "values")

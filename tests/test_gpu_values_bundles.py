@@ -20,6 +20,7 @@ def test_bundles_of_channels(oracle, library, switches, dtype, l_max, pack):
     padded rows (l_max = 15, 23), tiles with one point, one short of full, full, and one more."""
     rng = np.random.default_rng(61)
     library.sphx_reset_switches()
+    switches("SPHX_VALUES_FIXED", 0)  # (not the kernels with l_max for a constant)
     if pack is not None:
         switches("SPHX_VALUES_PACK", pack)
         switches("SPHX_PAIRS", 0)

@@ -49,7 +49,7 @@ def test_every_l_max(oracle, library, switches, dtype, l_max, normalized):
                                              (np.float64, 9, 65_537), (np.float64, 18, 6_144), (np.float64, 22, 32_768),
                                              (np.float64, 25, 20_000), (np.float64, 28, 4_097), (np.float64, 29, 3_000)])
 def test_as_planned(oracle, library, dtype, l_max, n):
-    """Plans on both sides of the table's lines, and their neighbours that take another kernel."""
+    """Calls of sizes between the table's lines, as they are planned."""
     for normalized in (True, False):
         for points in (n - 1, n):
             announce("values as planned", np.dtype(dtype).name, l_max, normalized, points)
@@ -58,3 +58,27 @@ def test_as_planned(oracle, library, dtype, l_max, n):
             status, out = run_launch_layer(library, torch.from_numpy(xyz).cuda(), l_max, normalized, "values")
             assert status == 0, library.sphx_last_error()
             check(tuple(o.cpu().numpy() if o is not None else None for o in out), want, (l_max, points))
+
+
+@pytest.mark.parametrize("dtype, l_max, normalized, n, below, at", [
+    # (kernel<waves> tile, or the kernel without l_max for a constant that is ahead there)
+    (np.float32, 24, False, 65_536, "values_fixed_kernel<8> 16", "values_fixed_kernel<8> 24"),
+    (np.float32, 18, True, 262_144, "values_fixed_kernel<8> 20", "values_kernel"),
+    (np.float32, 10, False, 524_288, "values_fixed_kernel<8> 32", "values_kernel"),
+    (np.float64, 12, True, 300_000, "values_fixed_kernel<8> 32", "values_kernel"),
+    (np.float32, 13, False, 400_000, "values_fixed_kernel<8> 24", "values_kernel"),
+])
+def test_both_sides_of_the_tables_lines(oracle, library, dtype, l_max, normalized, n, below, at):
+    for points, wanted in ((n - 1, below), (n, at)):
+        announce("values at a line", np.dtype(dtype).name, l_max, normalized, points, wanted)
+        planned = plan_text(library, points, l_max, "values", dtype, normalized)
+        if "_fixed_kernel" in wanted:
+            kernel, waves, tile = wanted.replace("<", " ").replace(">", "").split()
+            assert planned.startswith(kernel + "<") and f", {l_max}, {waves}> [l_max a constant, {tile} points" in planned, planned
+        else:
+            assert planned.startswith(wanted + "<"), planned
+        xyz = special_points(dtype, np.random.default_rng(l_max), points)
+        want = oracle.compute(xyz, l_max, normalized, "values")
+        status, out = run_launch_layer(library, torch.from_numpy(xyz).cuda(), l_max, normalized, "values")
+        assert status == 0, library.sphx_last_error()
+        check(tuple(o.cpu().numpy() if o is not None else None for o in out), want, (l_max, points))
