@@ -47,12 +47,15 @@ namespace sphx {
 // The products are sums in another order than the entries' own, with fused multiply-adds: they agree with the
 // contraction of the derivative arrays to rounding.
 //
-// LMAX > 0: kernels for one l_max each (fixed_columns(), sphx_columns.hpp), the same operations in the same order. What the
-// general kernel is bound by is the issue of instructions and, in small calls, the wait at every step: per step it loads the
-// entry's factors through the scalar unit and the weights from LDS, which share a counter, and waits for both (l_max = 8 in
-// float32: as many scalar as vector instructions, 31 + 30 per pair of entries). With l_max a constant a column is one run
-// of 16 instructions per pair, the loads of several steps ahead, the offsets of the weights part of the instructions, and
-// the rows come into LDS without a branch between the loads. us, general and fixed: the product, 400 000 points, float32
+// LMAX > 0: kernels for one l_max each (fixed_columns(), sphx_columns.hpp), the same operations in the same order within a
+// wave; where the columns are dealt to another number of waves than in the general kernel (the product in float32 at l_max =
+// 10, its derivatives at 3), the waves' sums are as many fewer or more, added in that other order: rounding of the same width.
+// What the general kernel is bound by is the issue of instructions and, in small calls, the wait at every step: per step it
+// loads the entry's factors through the scalar unit and the weights from LDS, which share a counter, and waits for both. With
+// l_max a constant a column is one run of instructions, the loads of several steps ahead, the offsets of the weights part of
+// the instructions, and the rows come into LDS without a branch between the loads (SQ counters, general / fixed, e6: the
+// product, 400 003 points, float32 l_max = 8, vector 8.6 6.3, scalar 8.5 2.3; 100 000 points at 17, 10.0 8.4, 8.5 1.4). The
+// derivatives of the product in float64 at l_max = 11 and 12 on two lanes per point spill 2-9 vector registers. us, general and fixed: the product, 400 000 points, float32
 // l_max = 8 27.3 22.5 (floor 20.2), 12 56 43 (41), 17 134 101 (77), float64 8 50 42 (40), 12 130 106 (81), 20 000 points
 // at 14 in float32 8.8 5.1; its derivatives, float32 8 51.6 43.9 (39.7), float64 10 169 147 (116); the rows, float32 8 144
 // 108 (77), float64 9 295 236 (177), 20 000 points 22.9 18.2.
@@ -757,7 +760,7 @@ __global__ __launch_bounds__(kColumnsThreads) void column_rows_kernel(Columns g,
         FixedRows<T, ROW, PAD, column_rounds(COLUMNS_ROWS, sizeof(T), LMAX, TILE * ROW)> one(
             have_w ? w + first * ny : three.run, w_rows, valid, tid, threads);
         three.issue();
-        one.issue();
+        one.issue(); // (without weights a part of v once more, thrown away: no branch among the loads)
         p = load_point<T, NORM>(raw);
         three.put();
         if (have_w) {

@@ -9,10 +9,12 @@ namespace sphx {
 // ---------------------------------------------------------------------------
 // gradients_fixed_kernel with second derivatives: two lanes per point (+m and -m), up to 32 points per workgroup, the channels
 // l = 2 .. l_max in parts of a few entries m dealt to the waves at compile time, the three recursions of a channel in
-// registers. An entry is entry_job_from (sphx_device.hpp) with l and m literals: of the 350 vector instructions that
-// recursion_kernel spends on the two sides of an entry a hundred were look-up and addresses, and its one workgroup per CU
-// stores nothing while it computes; here two to five workgroups per CU do both. The entries are bound by the vector units
-// still (170 instructions for one side of 32 points, normalised; 65 solid). us, before and after: float32 normalised l_max =
+// registers. An entry is entry_job_from (sphx_device.hpp) with l and m literals. recursion_kernel's one workgroup per CU
+// stores nothing while it computes; here two to five workgroups per CU do both. What the entries issue to the vector units is
+// about the same (SQ counters, recursion_kernel / here, e6: float32 normalised l_max = 5, 500 000 points, vector 80 80, scalar
+// 32 23, LDS 7.8 4.0; 7, 300 000, 98 108, 33 13, 9.3 5.7; solid 5, 300 000, 29 21, 21 14, 4.5 2.4; float64 6, 100 000, 30 36, 10
+// 7.5, 2.9 2.1): look-up and addresses are gone, the recursions are run by both sides of an entry. Normalised in float64 at
+// l_max = 6, 7 and solid at 10 2 to 8 vector registers are spilled to scratch (128 per lane). us, before and after: float32 normalised l_max =
 // 3 30 000 points 9.3 6.2, 1.2 GB 291 189; 5 2 000 9.9 4.3, 30 000 17.1 12.5, 300 000 108 102; 7 30 000 33 21, 1.2 GB 243
 // 210; float64 4 30 000 26.7 17.2, 1.2 GB 237 199; 6 30 000 44 30, 1.2 GB 255 207; solid 8 30 000 59 49, 1.2 GB 223 201.
 // From l_max = 11 in float32 (one workgroup per CU holds the rows) 2 500 12.2 9.5, solid 10 000 24.2 17.0, 1.2 GB 209 190;

@@ -96,7 +96,8 @@ constexpr UnitMasks deal_value_units(int l_max, int waves) {
 
 // ---- second derivatives --------------------------------------------------------------------------------------
 constexpr int kHessiansFixedFirst = 2;
-// (normalised in float64: from l_max = 8 on the entries need more registers than sixteen waves on a CU leave a lane)
+// (normalised in float64 the entries outgrow the 128 registers that sixteen waves on a CU leave a lane: 4 spilled at l_max = 6,
+// 8 at 7, where the kernel is still ahead)
 constexpr int kHessiansFixedLast = 13;
 constexpr int hessians_fixed_last(size_t elem, bool normalized) { return elem == 4 ? kHessiansFixedLast : (normalized ? 7 : 10); }
 constexpr bool hessians_fixed(size_t elem, int l_max, bool normalized) {

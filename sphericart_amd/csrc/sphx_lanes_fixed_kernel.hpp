@@ -22,12 +22,13 @@ namespace sphx {
 //
 // With l_max a constant everything around the arithmetic goes: c_m, s_m and 2(m+1)z of all m stay in registers, the
 // constants of an entry come as one scalar load, several entries ahead, the places of its four numbers in the rows are
-// offsets in the instructions, and no loop, job table or iterate in LDS is left: 44 (solid 30) vector instructions for
-// the entries of 32 points, 8 of them recursion. gradients_lanes_kernel waited at every step of a channel for a scalar
-// load and an LDS read, recursion_kernel worked its jobs out (122 cycles of a CU per point at l_max = 10 in float32, here
-// 60) and stores nothing meanwhile. Workgroups are small and many, so one computes while another stores, and they
-// are dispatched in the order of the addresses they write: 1.2 GB leave at 5.9-6.5 TB/s where persistent workgroups reached
-// 5.3-5.9. us, normalised, before and after: float32 l_max = 7 3 000 points 6.0 4.3, 50 000 16.3 11.7, 1.2 GB 209 186; 9
+// offsets in the instructions, and no loop, job table or iterate in LDS is left. gradients_lanes_kernel waited at every step of
+// a channel for a scalar load and an LDS read, recursion_kernel stores nothing while it works out its entries. The vector
+// instructions are about as many as there, the recursions being run by +m and -m, those to LDS and to the scalar unit fewer
+// (SQ counters, 400 000 points of l_max = 10 in float32, recursion_kernel / here: vector 57e6 63e6, scalar 25e6 20e6, LDS 7.7e6
+// 4.7e6, bank conflicts 7.9e6 0 cycles): the gain is that workgroups are small and many, so one computes while another
+// stores, and that they are dispatched in the order of the addresses they write: 1.2 GB leave at 5.9-6.5 TB/s in a loop where
+// persistent workgroups reached 5.3-5.9 (behind another kernel: sphx_plan_shapes.hpp). us, normalised, before and after: float32 l_max = 7 3 000 points 6.0 4.3, 50 000 16.3 11.7, 1.2 GB 209 186; 9
 // 20 000 14.0 7.7, 750 000 208 188; 12 15 000 17.2 9.6, 444 000 210 188; float64 8 10 000 points 9.0 7.6, 463 000 207 193;
 // 9 20 000 24.6 15.0; 13 191 000 232 203. At larger l_max a tile holds few points and half of the lanes are idle (float32 from
 // l_max = 20, float64 from 16 with more than one tile per CU): there it is ahead only while the call is latency, float32 22

@@ -11,9 +11,10 @@ namespace sphx {
 // l > 6 and two slices of the closed forms dealt to the waves at compile time. c_m, s_m, 2(m+1)z and the constants of an entry
 // come from registers and scalar loads where values_kernel reads them from LDS or from a lane at every step, behind a barrier
 // that waits for one wave to make the tables, and pairs_kernel's one workgroup per CU stores in turn with its recursions. Half
-// of the recursions are done twice (by +m and -m), 9 instructions an entry of 32 points, and that is still a fraction of the
-// time its row takes to HBM: tiles are small, so that some workgroups store while others compute, and no smaller, since c_m
-// and 2(m+1)z of all m are made anew by every wave. us, normalised, before and after: float32 l_max = 12 30 000 points 7.0
+// of the recursions are done twice (by +m and -m), and that is still a fraction of the time its row takes to HBM (SQ counters,
+// values_kernel / here, e6: 500 000 points of l_max = 12 in float32, two channels, vector 18 27, scalar 11 8, LDS 3.5 1.7; of
+// 22, one channel, 83 96, 78 19, 16 8): tiles are small, so that some workgroups store while others compute, and no smaller, since c_m and 2(m+1)z of all m are made anew by every
+// wave. us, normalised, before and after: float32 l_max = 12 30 000 points 7.0
 // 5.7; 18 3 000 5.6 4.0; 22 30 000 17.4 13.7, 500 000 171 163; 28 30 000 40.4 21.3, 1.2 GB 251 198; 32 12 000 17.0 13.7, 1.2 GB
 // 227 190; float64 7 100 000 16.0 10.2; 13 1.2 GB 223 191; 23 100 000 110 81, 1.2 GB 272 189; 28 1.2 GB 227 203.
 //
